@@ -114,6 +114,18 @@ def _collapse_axes(a: ndarray, axes: tuple[int, ...]) -> tuple[int, ndarray]:
     return first, ndarray(thunk.shape, thunk.dtype, thunk=thunk)
 
 
+# Vectors from this length on are selected from (`cpn_quantile_select`) instead of sorted.  us per call,
+# selected / sorted: five percentiles of 10^4 float32 47 / 88, float64 78 / 90, of 4 * 10^4 float64 77 / 128; sixteen
+# of 10^4 int64 108 / 79, of 10^6 123 / 210.  Vectors of up to 16 384 elements are sorted by one kernel, in less
+# time than the launches of a selection of many quantiles take.
+SELECT_MIN_SIZE = 32768
+
+
+def _select_bytes(a: ndarray, num_q: int) -> int:
+    """Workspace of a selection of `num_q` quantiles from `a`; 0: it has to be sorted."""
+    return int(_lib.load().cpn_quantile_select_temp_bytes(_lib.DTYPE_CODES[a.dtype], a.size, num_q))
+
+
 def quantile(
     a: Any,
     q: Any,
@@ -150,11 +162,14 @@ def quantile(
 
     from . import sort  # (the module-level function; imported here to keep the import order free)
 
+    # A long vector of which only a few elements are needed is not sorted (SELECT_MIN_SIZE)
+    flat = real_axis is None or a_rr.ndim == 1
+    select = flat and not overwrite_input and a_rr.size >= SELECT_MIN_SIZE and _select_bytes(a_rr, q_arr.size) != 0
     if overwrite_input:
         a_rr.sort(axis=real_axis)
         arr = a_rr
     else:
-        arr = sort(a_rr, axis=real_axis)
+        arr = a_rr if select else sort(a_rr, axis=real_axis)
     if arr.dtype.kind == "c":
         raise TypeError("input array cannot be of complex type")
     to_dtype = arr.dtype if method in _KEEP_DTYPE else np.dtype(np.float64)
@@ -203,6 +218,25 @@ def quantile(
         lib = _lib.load()
         torch = runtime.torch
         dev = runtime.require_device()
+    if result.size and select:
+        temp_bytes = _select_bytes(arr, q_arr.size)
+        temp = runtime.empty_bytes(temp_bytes)
+        status = lib.cpn_quantile_select(
+            _lib.DTYPE_CODES[arr.dtype],
+            arr._thunk.base.ptr(),
+            n,
+            q_arr.size,
+            left.ctypes.data,
+            right.ctypes.data,
+            gamma.ctypes.data,
+            int(interpolate),
+            result.base.ptr(),
+            temp.data_ptr(),
+            temp_bytes,
+            ctypes.c_void_p(runtime.stream_handle()),
+        )
+        _lib.check(status, "cpn_quantile_select")
+    elif result.size:
         d_left = torch.from_numpy(left).to(dev)
         d_right = torch.from_numpy(right).to(dev)
         d_gamma = torch.from_numpy(gamma).to(dev)

@@ -30,6 +30,7 @@ SOURCES = [
     "searchsorted.hip",
     "unique.hip",
     "quantile.hip",
+    "select.hip",
     "sort_keys8.hip",
     "sort_keys16.hip",
     "sort_keys32.hip",

@@ -255,6 +255,18 @@ int cpn_quantile_sorted(int dtype, const void* sorted, uint64_t outer, uint64_t 
                         int interpolate, void* out, void* stream);
 
 /*
+ * The same for one long vector that is not sorted (outer == inner == 1): the elements that would stand
+ * at left[q] and right[q] of the stable ascending sort are selected without sorting, bit for bit.
+ * left, right and gamma are HOST arrays of num_q entries (read before the call returns).  Real types
+ * of 4 and 8 bytes, n < 2^31, 1 <= num_q <= 16; for anything else the size query returns 0 and the call
+ * CPN_ERR_UNSUPPORTED.  values is not modified; temp: cpn_quantile_select_temp_bytes bytes, 256-byte aligned.
+ */
+uint64_t cpn_quantile_select_temp_bytes(int dtype, uint64_t n, uint64_t num_q);
+int cpn_quantile_select(int dtype, const void* values, uint64_t n, uint64_t num_q, const int64_t* left,
+                        const int64_t* right, const double* gamma, int interpolate, void* out, void* temp,
+                        uint64_t temp_bytes, void* stream);
+
+/*
  * The quantiles of nanquantile / nanpercentile / nanmedian, which ignore NaNs
  * (cupynumeric/_module/stats_order.py:653-951, cupynumeric/_module/stats_avgs_vars.py:445-512).
  * `sorted` is a dense [outer][n][inner] array of float16 / float32 / float64 sorted along the middle
