@@ -623,7 +623,7 @@ class UniqueJob:
         self.stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         distinct = min(n, max(n >> 6, 2))
         self.alg = {"total": n * 4 + 4 * n * 8 + 2 * n * 4 + distinct * 4, "onesweep": n * 8,
-                    "unique_count": n * 4, "unique_scatter": n * 4 + distinct * 4, "histogram": n * 4}
+                    "unique_mark": n * 4 + n // 8, "unique_scatter": n // 8 + 2 * distinct * 4, "histogram": n * 4}
         self.dominant = "onesweep"
         self.dtype = "u32"
 
