@@ -17,7 +17,9 @@
 // sorted first (with their positions, by the library's own sort, in the caller's workspace):
 // neighbouring lanes then search for neighbouring values, their probes fall into the same
 // cache lines, and the array is read about once instead of once per probe.  The answers go
-// back to the positions the values came from.
+// back to the positions the values came from.  Where the values are dense in the array the sorted
+// values are served in tiles: the part of the array between the answers of two tiles' first
+// values goes to LDS in one coalesced read, and the search runs there.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -27,6 +29,10 @@ namespace cpn {
 
 constexpr int SEARCH_BLOCK  = 256;
 constexpr int SEARCH_PIVOTS = 2048;
+
+constexpr uint32_t WINDOW_BYTES    = 40960;
+constexpr uint32_t WINDOW_TILE_MAX = 1024;
+constexpr int BOUNDS_BLOCK         = 64;
 
 template <int NW>
 __device__ __forceinline__ bool words_less(const uint64_t (&a)[NW], const uint64_t (&b)[NW])
@@ -112,10 +118,173 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_kernel(const KeyT* 
   }
 }
 
+// bounds[b] = answer for the first value of tile b (values sorted, `tile` of them per tile); bounds[tiles] = n
+template <typename KeyT, int CODEC, bool LEFT>
+__global__ __launch_bounds__(BOUNDS_BLOCK) void window_bounds_kernel(const KeyT* __restrict__ sorted,
+                                                                     uint64_t n,
+                                                                     const KeyT* __restrict__ values,
+                                                                     uint32_t tile,
+                                                                     uint64_t tiles,
+                                                                     uint64_t* __restrict__ bounds)
+{
+  const uint64_t b = static_cast<uint64_t>(blockIdx.x) * BOUNDS_BLOCK + threadIdx.x;
+  if (b < tiles) {
+    uint64_t v[1];
+    KeyTraits<CODEC, KeyT>::words(values[b * tile], v);
+    uint64_t lo = 0, hi = n;
+    while (lo < hi) {
+      const uint64_t mid = lo + (hi - lo) / 2;
+      uint64_t a[1];
+      KeyTraits<CODEC, KeyT>::words(sorted[mid], a);
+      if (go_right<LEFT, 1>(a, v)) {
+        lo = mid + 1;
+      } else {
+        hi = mid;
+      }
+    }
+    bounds[b] = lo;
+  } else if (b == tiles) {
+    bounds[tiles] = n;
+  }
+}
+
+// One tile of sorted values per workgroup.  The answers of the tile lie in [bounds[b], bounds[b + 1]]; if that
+// window of the array fits, its ordered keys go to LDS and the search runs there, else (values
+// sparse in this part of the array) it runs in the array.
+//
+// Bound by the read of the array, once, and by the 8-byte stores at the values' own positions.
+// 40 KB of window let four workgroups share a CU, so that one searches while others load; the
+// loads of eight elements per lane are issued together.  Two values per lane search side by side,
+// with a step count that is the same for all lanes.  2^24 float32 values in 2^28: 518 + 23 us for the
+// windows' bounds, against 837 us for probes of the array by lanes with neighbouring values.
+template <typename KeyT, int CODEC, bool LEFT>
+__global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const KeyT* __restrict__ sorted,
+                                                                           const KeyT* __restrict__ values,
+                                                                           uint64_t num_values,
+                                                                           int64_t* __restrict__ out,
+                                                                           const int64_t* __restrict__ origin,
+                                                                           uint32_t tile,
+                                                                           const uint64_t* __restrict__ bounds)
+{
+  constexpr uint32_t CAPACITY = WINDOW_BYTES / sizeof(KeyT);
+  __shared__ KeyT s_key[CAPACITY];
+  const uint64_t from   = bounds[blockIdx.x];
+  const uint64_t extent = bounds[blockIdx.x + 1] - from;
+  const uint64_t first  = static_cast<uint64_t>(blockIdx.x) * tile;
+  const uint32_t count  = static_cast<uint32_t>(num_values - first < tile ? num_values - first : tile);
+  if (extent > CAPACITY) {  // the same for every lane of the workgroup
+    for (uint32_t t = threadIdx.x; t < count; t += SEARCH_BLOCK) {
+      uint64_t v[1];
+      KeyTraits<CODEC, KeyT>::words(values[first + t], v);
+      uint64_t lo = from, hi = from + extent;
+      while (lo < hi) {
+        const uint64_t mid = lo + (hi - lo) / 2;
+        uint64_t a[1];
+        KeyTraits<CODEC, KeyT>::words(sorted[mid], a);
+        if (go_right<LEFT, 1>(a, v)) {
+          lo = mid + 1;
+        } else {
+          hi = mid;
+        }
+      }
+      out[origin[first + t]] = static_cast<int64_t>(lo);
+    }
+    return;
+  }
+  const uint32_t width = static_cast<uint32_t>(extent);
+  for (uint32_t start = 0; start < width; start += 8 * SEARCH_BLOCK) {
+    KeyT key[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t j = start + k * SEARCH_BLOCK + threadIdx.x;
+      key[k]           = sorted[from + (j < width ? j : width - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t j = start + k * SEARCH_BLOCK + threadIdx.x;
+      if (j < width) {
+        s_key[j] = ordered_bits<CODEC, KeyT>(key[k]);
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t largest_step = (width != 0) ? 1u << (31 - __builtin_clz(width)) : 0u;
+  for (uint32_t start = 0; start < count; start += 2 * SEARCH_BLOCK) {
+    KeyT v[2];
+    uint32_t pos[2] = {0, 0};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t t = start + k * SEARCH_BLOCK + threadIdx.x;
+      v[k]             = ordered_bits<CODEC, KeyT>(values[first + (t < count ? t : count - 1)]);
+    }
+    for (uint32_t step = largest_step; step != 0; step >>= 1) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const uint32_t to = pos[k] + step;  // every element before `to` is left of the answer?
+        if (to <= width) {
+          const KeyT a = s_key[to - 1];
+          if (LEFT ? a < v[k] : a <= v[k]) {
+            pos[k] = to;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t t = start + k * SEARCH_BLOCK + threadIdx.x;
+      if (t < count) {
+        out[origin[first + t]] = static_cast<int64_t>(from + pos[k]);
+      }
+    }
+  }
+}
+
+// Values per tile of the window search for `key_bytes`-byte keys, 0 where it does not pay.  A window is
+// planned to fill four fifths of its LDS, which leaves room for values that are not spread
+// evenly.  Below 128 values per tile a value has more than 256 bytes of the array to itself, and reading
+// all of it costs more than the cache lines that the probes of a value touch.
+static uint32_t window_tile(int key_bytes, uint64_t n, uint64_t num_values)
+{
+  const double per_value = static_cast<double>(n) * key_bytes / static_cast<double>(num_values);
+  const double fits      = 0.8 * WINDOW_BYTES / per_value;
+  return fits >= WINDOW_TILE_MAX ? WINDOW_TILE_MAX : static_cast<uint32_t>(fits) / 128 * 128;
+}
+
+template <typename KeyT, int CODEC>
+static int launch_window_search(const void* sorted, uint64_t n, const void* values, uint64_t num_values, bool left,
+                                int64_t* out, const int64_t* origin, uint32_t tile, uint64_t* bounds,
+                                hipStream_t stream)
+{
+  const uint64_t tiles = (num_values + tile - 1) / tile;
+  const auto bounds_of = left ? &window_bounds_kernel<KeyT, CODEC, true> : &window_bounds_kernel<KeyT, CODEC, false>;
+  const auto search =
+    left ? &searchsorted_window_kernel<KeyT, CODEC, true> : &searchsorted_window_kernel<KeyT, CODEC, false>;
+  {
+    ProfileScope prof("window_bounds", stream);
+    hipLaunchKernelGGL(bounds_of, dim3(static_cast<uint32_t>(tiles / BOUNDS_BLOCK + 1)), dim3(BOUNDS_BLOCK), 0, stream,
+                       static_cast<const KeyT*>(sorted), n, static_cast<const KeyT*>(values), tile, tiles, bounds);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    ProfileScope prof("searchsorted", stream);
+    hipLaunchKernelGGL(search, dim3(static_cast<uint32_t>(tiles)), dim3(SEARCH_BLOCK), 0, stream,
+                       static_cast<const KeyT*>(sorted), static_cast<const KeyT*>(values), num_values, out, origin, tile,
+                       bounds);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  return CPN_OK;
+}
+
 template <typename KeyT, int CODEC>
 static int launch_searchsorted(const void* sorted, uint64_t n, const void* values, uint64_t num_values, bool left,
-                               int64_t* out, const int64_t* origin, hipStream_t stream)
+                               int64_t* out, const int64_t* origin, uint64_t* bounds, hipStream_t stream)
 {
+  if constexpr (CODEC != CODEC_COMPLEX) {
+    const uint32_t tile = window_tile(static_cast<int>(sizeof(KeyT)), n, num_values);
+    if (origin != nullptr && tile != 0 && num_values / tile < (1ull << 31) - 1) {
+      return launch_window_search<KeyT, CODEC>(sorted, n, values, num_values, left, out, origin, tile, bounds, stream);
+    }
+  }
   uint64_t step       = 0;
   uint32_t num_pivots = 0;
   if (n >= 8192 && num_values >= 2048) {
@@ -151,16 +320,20 @@ static bool presort_pays(int key_bytes, uint64_t n, uint64_t num_values)
 }
 
 struct SearchLayout {
-  uint64_t sort_bytes, off_values, off_origin, total;
+  uint64_t sort_bytes, off_values, off_origin, off_bounds, total;
 };
 
-static SearchLayout search_layout(int dtype, int key_bytes, uint64_t num_values)
+static SearchLayout search_layout(int dtype, int key_bytes, uint64_t n, uint64_t num_values)
 {
   SearchLayout L{};
   L.sort_bytes = cpn_local_sort_temp_bytes(dtype, num_values, num_values, 1, 1, 0);
   L.off_values = align_up(L.sort_bytes, WORKSPACE_ALIGN);
   L.off_origin = L.off_values + align_up(num_values * static_cast<uint64_t>(key_bytes), WORKSPACE_ALIGN);
-  L.total      = L.off_origin + align_up(num_values * 8, WORKSPACE_ALIGN);
+  L.off_bounds = L.off_origin + align_up(num_values * 8, WORKSPACE_ALIGN);
+  L.total      = L.off_bounds;
+  if (const uint32_t tile = window_tile(key_bytes, n, num_values); tile != 0) {
+    L.total += align_up(((num_values + tile - 1) / tile + 1) * 8, WORKSPACE_ALIGN);
+  }
   return L;
 }
 
@@ -172,7 +345,7 @@ extern "C" uint64_t cpn_searchsorted_temp_bytes(int dtype, uint64_t n, uint64_t 
   if (k.bytes == 0 || k.codec < 0 || !cpn::presort_pays(k.bytes, n, num_values)) {
     return 0;
   }
-  const cpn::SearchLayout L = cpn::search_layout(dtype, k.bytes, num_values);
+  const cpn::SearchLayout L = cpn::search_layout(dtype, k.bytes, n, num_values);
   return L.sort_bytes == 0 ? 0 : L.total;
 }
 
@@ -196,8 +369,9 @@ extern "C" int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const
     return CPN_ERR_ALIGN;
   }
   const int64_t* origin = nullptr;
+  uint64_t* bounds      = nullptr;
   if (temp != nullptr && presort_pays(k.bytes, n, num_values)) {
-    const SearchLayout L = search_layout(dtype, k.bytes, num_values);
+    const SearchLayout L = search_layout(dtype, k.bytes, n, num_values);
     if (L.sort_bytes != 0 && temp_bytes >= L.total) {
       if ((reinterpret_cast<uintptr_t>(temp) % WORKSPACE_ALIGN) != 0) {
         return CPN_ERR_TEMP;
@@ -212,12 +386,13 @@ extern "C" int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const
       }
       values = sorted_vals;
       origin = where;
+      bounds = reinterpret_cast<uint64_t*>(ws + L.off_bounds);
     }
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool l  = left != 0;
 #define CPN_SEARCH_CASE(T, C) \
-  return launch_searchsorted<T, C>(sorted, n, values, num_values, l, positions_out, origin, s)
+  return launch_searchsorted<T, C>(sorted, n, values, num_values, l, positions_out, origin, bounds, s)
   switch (k.codec) {
     case CODEC_UNSIGNED:
       switch (k.bytes) {
