@@ -154,11 +154,12 @@ __global__ __launch_bounds__(BOUNDS_BLOCK) void window_bounds_kernel(const KeyT*
 //
 // Bound by the read of the array, once, and by the 8-byte stores at the values' own positions.
 // 40 KB of window let four workgroups share a CU, so that one searches while others load; the
-// loads of eight elements per lane are issued together.  Two values per lane search side by side,
-// with a step count that is the same for all lanes.  2^24 float32 values in 2^28: 518 + 23 us for the
-// windows' bounds, against 837 us for probes of the array by lanes with neighbouring values.
+// loads of the whole window, 16 bytes each, are issued together.  Two values per lane search side by side,
+// with a step count that is the same for all lanes.  2^24 float32 values in 2^28: 512 us (518 with loads
+// of one element) + 23 us for the windows' bounds, against 837 us for probes of the array by lanes with neighbouring values.
 template <typename KeyT, int CODEC, bool LEFT>
 __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const KeyT* __restrict__ sorted,
+                                                                           uint64_t n,
                                                                            const KeyT* __restrict__ values,
                                                                            uint64_t num_values,
                                                                            int64_t* __restrict__ out,
@@ -167,12 +168,23 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const
                                                                            const uint64_t* __restrict__ bounds)
 {
   constexpr uint32_t CAPACITY = WINDOW_BYTES / sizeof(KeyT);
-  __shared__ KeyT s_key[CAPACITY];
+  constexpr uint32_t PACK     = 16 / sizeof(KeyT);
+  constexpr int PACKS         = WINDOW_BYTES / 16 / SEARCH_BLOCK;  // per lane
+  struct alignas(16) Pack {
+    KeyT key[PACK];
+  };
+  static_assert(PACKS * 16 * SEARCH_BLOCK == WINDOW_BYTES, "one batch of loads covers the window");
+  __shared__ Pack s_pack[CAPACITY / PACK];
+  KeyT* s_key = s_pack[0].key;
   const uint64_t from   = bounds[blockIdx.x];
   const uint64_t extent = bounds[blockIdx.x + 1] - from;
   const uint64_t first  = static_cast<uint64_t>(blockIdx.x) * tile;
   const uint32_t count  = static_cast<uint32_t>(num_values - first < tile ? num_values - first : tile);
-  if (extent > CAPACITY) {  // the same for every lane of the workgroup
+  // elements between the 16-byte boundary below the window and the window
+  const uint32_t head = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(sorted + from) % 16 / sizeof(KeyT));
+  // Room for whole packs at both ends.  An array that is not sorted can have bounds that fall: that
+  // extent wraps to a large one and the search in the array ends at once.
+  if (extent > CAPACITY - 2 * PACK) {  // the same for every lane of the workgroup
     for (uint32_t t = threadIdx.x; t < count; t += SEARCH_BLOCK) {
       uint64_t v[1];
       KeyTraits<CODEC, KeyT>::words(values[first + t], v);
@@ -192,19 +204,30 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const
     return;
   }
   const uint32_t width = static_cast<uint32_t>(extent);
-  for (uint32_t start = 0; start < width; start += 8 * SEARCH_BLOCK) {
-    KeyT key[8];
+  const uint32_t packs = (head + width + PACK - 1) / PACK;
+  uint32_t skip        = 0;  // elements in LDS before the window
+  if (width != 0 && from >= head && from - head + static_cast<uint64_t>(packs) * PACK <= n) {
+    // whole packs inside the array
+    const Pack* __restrict__ source = reinterpret_cast<const Pack*>(sorted + (from - head));
+    Pack p[PACKS];
+    skip = head;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t j = start + k * SEARCH_BLOCK + threadIdx.x;
-      key[k]           = sorted[from + (j < width ? j : width - 1)];
+    for (int k = 0; k < PACKS; ++k) {
+      const uint32_t j = k * SEARCH_BLOCK + threadIdx.x;
+      p[k]             = source[j < packs ? j : packs - 1];
     }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t j = start + k * SEARCH_BLOCK + threadIdx.x;
-      if (j < width) {
-        s_key[j] = ordered_bits<CODEC, KeyT>(key[k]);
+    for (int k = 0; k < PACKS; ++k) {
+#pragma unroll
+      for (uint32_t e = 0; e < PACK; ++e) {
+        p[k].key[e] = ordered_bits<CODEC, KeyT>(p[k].key[e]);
       }
+      // (past the window: copies of its last pack; a store under a condition would pull its load along)
+      s_pack[k * SEARCH_BLOCK + threadIdx.x] = p[k];
+    }
+  } else {  // the first or last window of an array that does not begin or end on a 16-byte boundary
+    for (uint32_t j = threadIdx.x; j < width; j += SEARCH_BLOCK) {
+      s_key[j] = ordered_bits<CODEC, KeyT>(sorted[from + j]);
     }
   }
   __syncthreads();
@@ -222,7 +245,7 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const
       for (int k = 0; k < 2; ++k) {
         const uint32_t to = pos[k] + step;  // every element before `to` is left of the answer?
         if (to <= width) {
-          const KeyT a = s_key[to - 1];
+          const KeyT a = s_key[skip + to - 1];
           if (LEFT ? a < v[k] : a <= v[k]) {
             pos[k] = to;
           }
@@ -268,8 +291,8 @@ static int launch_window_search(const void* sorted, uint64_t n, const void* valu
   {
     ProfileScope prof("searchsorted", stream);
     hipLaunchKernelGGL(search, dim3(static_cast<uint32_t>(tiles)), dim3(SEARCH_BLOCK), 0, stream,
-                       static_cast<const KeyT*>(sorted), static_cast<const KeyT*>(values), num_values, out, origin, tile,
-                       bounds);
+                       static_cast<const KeyT*>(sorted), n, static_cast<const KeyT*>(values), num_values, out, origin,
+                       tile, bounds);
   }
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;

@@ -9,12 +9,14 @@ from cupynumeric_amd import _lib
 pytestmark = pytest.mark.gpu
 
 
-def _search(table, values, left):
+def _search(table, values, left, shift=0):
     import torch
 
     lib = _lib.load()
     code = _lib.DTYPE_CODES[table.dtype]
-    d_a = torch.from_numpy(table.view(np.uint8)).cuda()
+    memory = torch.empty(table.nbytes + shift * table.itemsize, dtype=torch.uint8, device="cuda")
+    d_a = memory[shift * table.itemsize :]  # off a 16-byte boundary by `shift` elements
+    d_a.copy_(torch.from_numpy(table.view(np.uint8)))
     d_v = torch.from_numpy(values.view(np.uint8)).cuda()
     out = torch.full((values.size,), -1, dtype=torch.int64, device="cuda")
     tb = lib.cpn_searchsorted_temp_bytes(code, table.size, values.size)
@@ -52,9 +54,9 @@ def test_searchsorted_window_tiles(dtype, spread):
             v = np.where(rng.random(m) < 0.5, a[0], a[-1]).astype(dtype)
         else:
             v = np.full(m, a[n // 2])
-        for left in (True, False):
+        for left, shift in ((True, 0), (False, 1)):
             if dtype == np.float16:
                 want = np.searchsorted(a.astype(np.float32), v.astype(np.float32), "left" if left else "right")
             else:
                 want = np.searchsorted(a, v, "left" if left else "right")
-            assert np.array_equal(_search(a, v, left), want), (m, left)
+            assert np.array_equal(_search(a, v, left, shift), want), (m, left)
