@@ -157,6 +157,8 @@ __global__ __launch_bounds__(BOUNDS_BLOCK) void window_bounds_kernel(const KeyT*
 // loads of the whole window, 16 bytes each, are issued together.  Two values per lane search side by side,
 // with a step count that is the same for all lanes.  2^24 float32 values in 2^28: 512 us (518 with loads
 // of one element) + 23 us for the windows' bounds, against 837 us for probes of the array by lanes with neighbouring values.
+// The stores stay ordinary ones: with non-temporal stores, which the L2 does not gather, the whole call
+// took 1395 us instead of 891.
 template <typename KeyT, int CODEC, bool LEFT>
 __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const KeyT* __restrict__ sorted,
                                                                            uint64_t n,
