@@ -21,58 +21,15 @@
 #include <stdint.h>
 
 #include "lerp.h"
+#include "select_plan.h"
 #include "sort_driver.h"
 
 namespace cpn {
 
 constexpr int SELECT_BLOCK      = 1024;
 constexpr int SELECT_WAVES      = SELECT_BLOCK / WAVE;
-constexpr int SELECT_MAX_Q      = 16;
-constexpr int SELECT_MAX_RANKS  = 2 * SELECT_MAX_Q;
-constexpr int SELECT_BINS       = 16384;  // counters in LDS, shared by the prefixes of a round
-constexpr int SELECT_FIRST_BITS = 12;
 constexpr int SELECT_COPIES     = SELECT_BINS >> SELECT_FIRST_BITS;  // first round: copies of every counter, by lane
-constexpr int SELECT_MAX_BITS   = 11;     // later rounds
-constexpr int SELECT_MAX_ROUNDS = 8;
 constexpr int SELECT_CHUNKS     = 1024;   // select_count_class_kernel
-
-// Bits that a round after the first resolves for `prefixes` different prefixes.
-__host__ __device__ constexpr uint32_t select_bits(uint32_t prefixes)
-{
-  uint32_t w = SELECT_MAX_BITS;
-  while ((prefixes << w) > static_cast<uint32_t>(SELECT_BINS)) {
-    --w;
-  }
-  return w;
-}
-// Rounds that resolve `bits` bits of `ranks` targets.
-__host__ __device__ constexpr int select_rounds(int bits, uint32_t ranks)
-{
-  const int w = static_cast<int>(select_bits(ranks));
-  return bits <= SELECT_FIRST_BITS ? 1 : 1 + (bits - SELECT_FIRST_BITS + w - 1) / w;
-}
-static_assert(select_rounds(64, SELECT_MAX_RANKS) <= SELECT_MAX_ROUNDS, "counters for every round");
-
-// Device-side state, written by select_init_kernel and by the last workgroup of every round.
-struct SelectPlan {
-  uint64_t key_or, key_and;            // over all images (first round)
-  uint64_t prefix[SELECT_MAX_RANKS];   // different prefixes: the resolved top bits of an image
-  uint64_t image[SELECT_MAX_RANKS];    // per target, once done
-  uint32_t rank[SELECT_MAX_RANKS];     // per target: position among the keys with its prefix
-  uint32_t which[SELECT_MAX_RANKS];    // per target: its prefix
-  uint32_t chunk[SELECT_MAX_RANKS];    // per target: where a key that ties with other bits is found
-  uint32_t n_prefix;
-  uint32_t bits_left;
-  uint32_t list_len;                   // keys of the list that the next round reads
-  uint32_t from_copy;                  // that list is the copy, not the input
-  uint32_t copy_now;                   // the next round makes the copy
-  uint32_t copied;                     // keys in the copy so far
-  uint32_t done;
-  uint32_t ties;                       // float targets among the NaNs or the zeros: bit 0, bit 1
-  uint32_t blocks_done[SELECT_MAX_ROUNDS + 1];
-};
-constexpr uint64_t SELECT_PLAN_BYTES = 2048;
-static_assert(sizeof(SelectPlan) <= SELECT_PLAN_BYTES, "plan slot");
 
 struct SelectRanks {
   uint32_t rank[SELECT_MAX_RANKS];  // ascending, all different
@@ -211,7 +168,8 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
     }
   };
   // the keys of one iteration that go to the copy: staged, then stored side by side.  copy_cap is at least
-  // the number of keys that match (the plan compares), the test below is a second safety.
+  // the number of keys that match (the plan compares) unless the caller writes to the input meanwhile: keys
+  // without room are dropped, and the next round reads no more than copy_cap (select_advance).
   auto flush = [&]() {
     __syncthreads();
     const uint32_t staged = s_staged;
@@ -368,6 +326,10 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
     const uint32_t which = plan->which[t];
     const uint32_t rank  = plan->rank[t];
     uint32_t run         = 0;
+    if (lane == 0) {  // (no key at this rank: only if the caller has written to the input during the call)
+      s_new[t]   = 0;
+      s_count[t] = 0;
+    }
     for (uint32_t b0 = 0; b0 <= mask; b0 += WAVE) {  // uniform for the wavefront
       const uint32_t b    = b0 + lane;
       const uint32_t c    = b <= mask ? s_hist[(which << w) + b] : 0u;
@@ -385,41 +347,15 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
   }
   __syncthreads();
   if (tid == 0) {
-    uint32_t left  = shift;
-    uint64_t total = 0;
+    uint64_t common = 0, varying = 0;
     if constexpr (FIRST) {
-      const uint64_t all     = agent_load(&plan->key_and);
-      const uint64_t varying = all ^ agent_load(&plan->key_or);
-      const uint32_t top     = varying == 0 ? 0u : 64u - static_cast<uint32_t>(__builtin_clzll(varying));
-      if (top < left) {  // every key agrees on the bits above: one bin, whose prefix takes them in
-        left = top;
-        for (uint32_t t = 0; t < n_ranks; ++t) {
-          s_new[t] = all >> left;
-        }
-      }
+      common  = agent_load(&plan->key_and);
+      varying = common ^ agent_load(&plan->key_or);
     }
-    uint32_t n = 0;
-    for (uint32_t t = 0; t < n_ranks; ++t) {  // ascending targets: equal prefixes are neighbours
-      if (t == 0 || s_new[t] != s_new[t - 1]) {
-        plan->prefix[n++] = s_new[t];
-        total += s_count[t];
-      }
-      plan->which[t] = n - 1;
-    }
-    plan->n_prefix  = n;
-    plan->bits_left = left;
-    if (copy_now) {
-      plan->copy_now  = 0;
-      plan->from_copy = 1;
-      plan->list_len  = agent_load(&plan->copied);
-    } else if (!from_copy && total <= copy_cap) {
-      plan->copy_now = 1;
-    }
-    if (left == 0) {
-      plan->done    = 1;
+    select_advance(plan, s_new, s_count, n_ranks, shift, FIRST, common, varying, copy_now ? agent_load(&plan->copied) : 0u, copy_cap);
+    if (plan->done != 0) {
       uint32_t ties = 0;
       for (uint32_t t = 0; t < n_ranks; ++t) {
-        plan->image[t] = s_new[t];
         if constexpr (CODEC == CODEC_FLOAT) {
           ties |= static_cast<KeyT>(s_new[t]) == static_cast<KeyT>(~static_cast<KeyT>(0)) ? 1u : 0u;
           ties |= static_cast<KeyT>(s_new[t]) == FloatLayout<KeyT>::sign ? 2u : 0u;
