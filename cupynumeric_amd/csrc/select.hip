@@ -7,15 +7,15 @@
 //
 // Radix selection from the top: each round counts, for the keys that agree with a target in the bits
 // resolved so far, the next 9 ... 12 bits of their ordered images, and the workgroup that finishes last
-// finds every target's bin.  The first round also learns which bits vary at all and later rounds
-// start below the others (ids held in 64 bits).  Once no more than a quarter of the keys can still be
-// asked for, a round copies them out as it counts them and the following rounds read the copy.
+// finds every target's bin.  A round also learns in which lower bits the keys of every prefix agree: these
+// take no round of their own (ids held in 64 bits, whole numbers held as floats).  Once no more than a
+// quarter of the keys can still be asked for, a round copies them out as it counts them and the
+// following rounds read the copy.
 //
-// Bound by reading the vector: three times for normal or uniform floats (the sign, exponent and first
-// mantissa bits take two rounds, the third makes the copy); the later rounds are launches.
-// Five percentiles of 10^7 normal float64 values: rounds of 35, 34 and 46 us (the copy), then 6 to 16 us
-// each, 152 us per call where the sort took 552; one read of the 80 MB at the rate of a large copy is 15 us.
-// 2^26 float64: 484 us against 2556 (one read: 103 us).
+// Normal or uniform floats are read three times: the sign, exponent and first mantissa bits take two rounds, the
+// third makes the copy; the later rounds are launches.  Us per call, five percentiles, against sort and take:
+//   float64, normal   10^7 elements 130 / 551   2^26 432 / 2560   2^28 1500 / 9370
+//   float64, 0 and 1  10^7 elements  81 / 285   2^26 336 /  771   2^28 1144 / 2538
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -28,7 +28,10 @@ namespace cpn {
 
 constexpr int SELECT_BLOCK      = 1024;
 constexpr int SELECT_WAVES      = SELECT_BLOCK / WAVE;
-constexpr int SELECT_COPIES     = SELECT_BINS >> SELECT_FIRST_BITS;  // first round: copies of every counter, by lane
+constexpr int SELECT_STAGED     = 4;      // 16-byte loads per thread that the copy stages at a time
+constexpr uint32_t SELECT_FIRST_SPREAD = 2;
+static_assert((1 << (SELECT_FIRST_BITS + SELECT_FIRST_SPREAD)) == SELECT_BINS, "copies of the first round's counters");
+constexpr uint32_t SELECT_SPREAD_MIN = 1u << 20;  // keys from which a round spreads its counters
 constexpr int SELECT_CHUNKS     = 1024;   // select_count_class_kernel
 
 struct SelectRanks {
@@ -56,10 +59,10 @@ static __global__ __launch_bounds__(256) void select_init_kernel(SelectPlan* pla
   if (blockIdx.x == 0 && threadIdx.x < SELECT_MAX_RANKS) {
     plan->rank[threadIdx.x]  = ranks.rank[threadIdx.x];
     plan->which[threadIdx.x] = 0;
+    plan->any[threadIdx.x]   = 0;
+    plan->all[threadIdx.x]   = ~0ull;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    plan->key_or    = 0;
-    plan->key_and   = ~0ull;
     plan->prefix[0] = 0;
     plan->n_prefix  = 1;
     plan->bits_left = bits;
@@ -70,6 +73,12 @@ static __global__ __launch_bounds__(256) void select_init_kernel(SelectPlan* pla
     }
   }
 }
+
+// OR and AND of a set of images.
+struct alignas(16) Agreement {
+  uint64_t any, all;
+};
+static_assert(SELECT_WAVES <= SELECT_MAX_RANKS, "first round: one entry per wavefront");
 
 // Is this the last workgroup of the launch to get here?  What the others have written with agent-scope
 // atomics is then seen by agent-scope loads: every wavefront waits until its own are done.  (A fence
@@ -93,10 +102,10 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
 {
   constexpr int VEC = 16 / sizeof(KeyT);
   __shared__ uint32_t s_hist[SELECT_BINS];
-  __shared__ __align__(16) KeyT s_stage[FIRST ? 1 : SELECT_BLOCK * VEC];
-  __shared__ uint64_t s_or[SELECT_WAVES], s_and[SELECT_WAVES];
+  __shared__ __align__(16) KeyT s_stage[FIRST ? 1 : SELECT_STAGED * SELECT_BLOCK * VEC];
+  __shared__ Agreement s_agree[SELECT_MAX_RANKS];  // per prefix; first round: per wavefront
   __shared__ uint64_t s_prefix[SELECT_MAX_RANKS];
-  __shared__ uint32_t s_count[SELECT_MAX_RANKS];
+  __shared__ uint32_t s_count[SELECT_MAX_RANKS], s_which[SELECT_MAX_RANKS], s_rank[SELECT_MAX_RANKS];
   __shared__ uint32_t s_staged, s_base, s_flag;
 
   if (plan->done != 0) {  // (written by earlier launches only: uniform)
@@ -114,19 +123,34 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
   const bool from_copy     = !FIRST && plan->from_copy != 0;
   const KeyT* list         = from_copy ? copy : values;
   const uint32_t len       = plan->list_len;
-  const uint32_t bins      = FIRST ? static_cast<uint32_t>(SELECT_BINS) : (n_prefix << w);
+  // Copies of every counter, by lane: with few prefixes most keys may be of one value, and the lanes of a wave
+  // that add to one counter wait for each other.  Median of 2^28 int64 of five values: 3.1 ms without, 2.7 with
+  // copies; a short list is done before the copies are added up.
+  uint32_t spread = FIRST ? SELECT_FIRST_SPREAD : 0u;  // logarithm of their number
+  if (!FIRST && !from_copy && len >= SELECT_SPREAD_MIN) {
+    while ((n_prefix << (w + spread + 1)) <= static_cast<uint32_t>(SELECT_BINS) && spread < SELECT_FIRST_SPREAD) {
+      ++spread;
+    }
+  }
+  const uint32_t own  = static_cast<uint32_t>(tid) & ((1u << spread) - 1u);
+  const uint32_t bins = n_prefix << (w + spread);
   for (uint32_t j = tid; j < bins; j += SELECT_BLOCK) {
     s_hist[j] = 0;
   }
   if (tid < static_cast<int>(n_prefix)) {
     s_prefix[tid] = plan->prefix[tid];
+    s_agree[tid]  = Agreement{0, ~0ull};
+  }
+  if (tid < static_cast<int>(n_ranks)) {
+    s_which[tid] = plan->which[tid];
+    s_rank[tid]  = plan->rank[tid];
   }
   if (tid == 0) {
     s_staged = 0;
   }
   __syncthreads();
 
-  uint64_t k_or = 0, k_and = ~0ull;
+  Agreement mine = {0, ~0ull};  // first round
   // counts the keys of an array; bit j of the result: key j can still be a target
   auto count = [&](const auto& k) -> uint32_t {
     constexpr int N = sizeof(k) / sizeof(KeyT);
@@ -138,9 +162,9 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
     if constexpr (FIRST) {
 #pragma unroll
       for (int j = 0; j < N; ++j) {
-        k_or |= image[j];
-        k_and &= image[j];
-        atomicAdd(&s_hist[(static_cast<uint32_t>(image[j] >> shift) & mask) * SELECT_COPIES + (tid % SELECT_COPIES)], 1u);
+        mine.any |= image[j];
+        mine.all &= image[j];
+        atomicAdd(&s_hist[((static_cast<uint32_t>(image[j] >> shift) & mask) << spread) + own], 1u);
       }
       return ~0u;
     } else {
@@ -160,8 +184,17 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         if (which[j] != ~0u) {
-          atomicAdd(&s_hist[(which[j] << w) + (static_cast<uint32_t>(image[j] >> shift) & mask)], 1u);
+          atomicAdd(&s_hist[(((which[j] << w) + (static_cast<uint32_t>(image[j] >> shift) & mask)) << spread) + own], 1u);
           hits |= 1u << j;
+          // Does the key add to its prefix's agreement?  After the first few keys hardly ever.  (An entry read while
+          // another lane updates it has fewer bits set, or cleared: that costs an update, no bit is lost.)
+          if (shift != 0) {
+            const Agreement known = s_agree[which[j]];
+            if (((image[j] & ~known.any) | (known.all & ~image[j])) != 0) {
+              __hip_atomic_fetch_or(&s_agree[which[j]].any, image[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              __hip_atomic_fetch_and(&s_agree[which[j]].all, image[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+          }
         }
       }
       return hits;
@@ -229,18 +262,25 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
     }
   }
   if (!FIRST && copy_now) {
-    for (uint32_t v0 = first; v0 < nvec; v0 += step) {  // uniform per workgroup
-      const uint32_t v = v0 + tid;
-      KeyT k[VEC] = {};
-      uint32_t hits = 0;
-      if (v < nvec) {
-        const uint4 q = vp[v];
-        __builtin_memcpy(k, &q, 16);
-        hits = count(k);
+    // four loads in flight and one flush for them, of four barriers and a global atomic: the median of 2^28 int64 of
+    // five values 2.7 -> 1.5 ms against a flush per load, five percentiles of 10^7 normal float64 142 -> 132 us
+    for (uint64_t v0 = first; v0 < nvec; v0 += static_cast<uint64_t>(SELECT_STAGED) * step) {  // uniform per workgroup
+      uint4 q[SELECT_STAGED];
+#pragma unroll
+      for (int i = 0; i < SELECT_STAGED; ++i) {
+        const uint64_t v = v0 + static_cast<uint64_t>(i) * step + tid;
+        q[i]             = vp[v < nvec ? v : nvec - 1];
       }
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        stage(k[j], ((hits >> j) & 1u) != 0);
+      for (int i = 0; i < SELECT_STAGED; ++i) {
+        const uint64_t v = v0 + static_cast<uint64_t>(i) * step + tid;
+        KeyT k[VEC];
+        __builtin_memcpy(k, &q[i], 16);
+        const uint32_t hits = v < nvec ? count(k) : 0u;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+          stage(k[j], ((hits >> j) & 1u) != 0);
+        }
       }
       flush();
     }
@@ -268,34 +308,33 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
     }
   }
   if constexpr (FIRST) {
-    k_or  = wave_reduce_or_dpp(k_or);
-    k_and = wave_reduce_and_dpp(k_and);
+    mine.any = wave_reduce_or_dpp(mine.any);
+    mine.all = wave_reduce_and_dpp(mine.all);
+    __syncthreads();  // (entry 0 was set at the start)
     if (lane == 0) {
-      s_or[tid / WAVE]  = k_or;
-      s_and[tid / WAVE] = k_and;
+      s_agree[tid / WAVE] = mine;
     }
   }
   __syncthreads();
   if constexpr (FIRST) {
     if (tid == 0) {
       for (int i = 1; i < SELECT_WAVES; ++i) {
-        k_or |= s_or[i];
-        k_and &= s_and[i];
+        mine.any |= s_agree[i].any;
+        mine.all &= s_agree[i].all;
       }
-      __hip_atomic_fetch_or(&plan->key_or, k_or, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_fetch_and(&plan->key_and, k_and, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+  } else if (tid < static_cast<int>(n_prefix)) {
+    mine = s_agree[tid];
+  }
+  if (tid < static_cast<int>(n_prefix) && (mine.any | ~mine.all) != 0) {  // (a prefix none of whose keys are here adds nothing)
+    __hip_atomic_fetch_or(&plan->any[tid], mine.any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_fetch_and(&plan->all[tid], mine.all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   uint32_t* out = hist + static_cast<uint32_t>(round) * SELECT_BINS;
   for (uint32_t j = tid; j < (n_prefix << w); j += SELECT_BLOCK) {
     uint32_t c = 0;
-    if constexpr (FIRST) {
-#pragma unroll
-      for (int i = 0; i < SELECT_COPIES; ++i) {
-        c += s_hist[j * SELECT_COPIES + i];
-      }
-    } else {
-      c = s_hist[j];
+    for (uint32_t i = 0; i < (1u << spread); ++i) {
+      c += s_hist[(j << spread) + i];
     }
     if (c != 0) {
       __hip_atomic_fetch_add(&out[j], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -310,6 +349,10 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
   {
     constexpr int EACH = SELECT_BINS / SELECT_BLOCK;
     uint32_t c[EACH];
+    if (tid < static_cast<int>(n_prefix)) {
+      mine.any = agent_load(&plan->any[tid]);
+      mine.all = agent_load(&plan->all[tid]);
+    }
 #pragma unroll
     for (int i = 0; i < EACH; ++i) {
       const uint32_t j = i * SELECT_BLOCK + tid;
@@ -319,13 +362,21 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
     for (int i = 0; i < EACH; ++i) {
       s_hist[i * SELECT_BLOCK + tid] = c[i];
     }
+    if (tid < static_cast<int>(n_prefix)) {
+      s_agree[tid]   = mine;
+      plan->any[tid] = 0;  // for the next round
+      plan->all[tid] = ~0ull;
+    }
   }
   __syncthreads();
   __shared__ uint64_t s_new[SELECT_MAX_RANKS];
   for (uint32_t t = tid / WAVE; t < n_ranks; t += SELECT_WAVES) {
-    const uint32_t which = plan->which[t];
-    const uint32_t rank  = plan->rank[t];
+    const uint32_t which = s_which[t];
+    const uint32_t rank  = s_rank[t];
     uint32_t run         = 0;
+    if (which == SELECT_FINISHED) {  // uniform for the wavefront
+      continue;
+    }
     if (lane == 0) {  // (no key at this rank: only if the caller has written to the input during the call)
       s_new[t]   = 0;
       s_count[t] = 0;
@@ -346,22 +397,47 @@ __global__ __launch_bounds__(SELECT_BLOCK) void select_round_kernel(const KeyT* 
     }
   }
   __syncthreads();
-  if (tid == 0) {
-    uint64_t common = 0, varying = 0;
-    if constexpr (FIRST) {
-      common  = agent_load(&plan->key_and);
-      varying = common ^ agent_load(&plan->key_or);
+  if (tid >= WAVE) {
+    return;
+  }
+  // The plan of the next round by one wavefront, a lane per target (ascending: equal prefixes are neighbours).
+  const uint32_t copied = copy_now ? agent_load(&plan->copied) : 0u;
+  const bool target     = lane < static_cast<int>(n_ranks);
+  const uint32_t before = target ? s_which[lane] : SELECT_FINISHED;
+  const bool active     = before != SELECT_FINISHED;
+  const SelectChild c   = active ? select_child(s_new[lane], shift, s_agree[before].any, s_agree[before].all) : SelectChild{0, 0};
+  const uint32_t left   = select_bits_left(wave_reduce_or_dpp(c.varying));
+  const bool goes_on    = active && c.varying != 0;
+  const uint64_t prefix = c.image >> left;
+  const uint64_t going  = __builtin_amdgcn_ballot_w64(goes_on);
+  const uint64_t lower  = going & ((1ull << lane) - 1);  // the active target before this one
+  const int neighbour   = lower != 0 ? 63 - __builtin_clzll(lower) : lane;
+  const uint64_t theirs = __shfl(prefix, neighbour, WAVE);
+  const bool opens      = goes_on && (lower == 0 || theirs != prefix);
+  const uint64_t heads  = __builtin_amdgcn_ballot_w64(opens);
+  const uint32_t which  = lanes_below(heads) + (opens ? 1u : 0u) - 1u;
+  const uint32_t total  = wave_inclusive_sum_dpp(opens ? s_count[lane] : 0u);  // below 2^31: keys of different prefixes
+  if (active) {
+    plan->which[lane] = goes_on ? which : SELECT_FINISHED;
+    if (!goes_on) {
+      plan->image[lane] = c.image;
     }
-    select_advance(plan, s_new, s_count, n_ranks, shift, FIRST, common, varying, copy_now ? agent_load(&plan->copied) : 0u, copy_cap);
-    if (plan->done != 0) {
-      uint32_t ties = 0;
-      for (uint32_t t = 0; t < n_ranks; ++t) {
-        if constexpr (CODEC == CODEC_FLOAT) {
-          ties |= static_cast<KeyT>(s_new[t]) == static_cast<KeyT>(~static_cast<KeyT>(0)) ? 1u : 0u;
-          ties |= static_cast<KeyT>(s_new[t]) == FloatLayout<KeyT>::sign ? 2u : 0u;
-        }
-      }
-      plan->ties = ties;
+  }
+  if (opens) {
+    plan->prefix[which] = prefix;
+  }
+  const uint32_t all_keys = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(total), WAVE - 1));
+  if (lane == 0) {
+    select_next_list(plan, copy_now, from_copy, static_cast<uint32_t>(__builtin_popcountll(heads)), left, all_keys, copied, copy_cap);
+  }
+  if constexpr (CODEC == CODEC_FLOAT) {
+    // targets whose image keys of other bits share, now or in an earlier round
+    const KeyT image = static_cast<KeyT>(active ? c.image : (target ? plan->image[lane] : 0));
+    const bool whole = target && !goes_on;
+    const uint64_t nans  = __builtin_amdgcn_ballot_w64(whole && image == static_cast<KeyT>(~static_cast<KeyT>(0)));
+    const uint64_t zeros = __builtin_amdgcn_ballot_w64(whole && image == FloatLayout<KeyT>::sign);
+    if (lane == 0) {
+      plan->ties = (nans != 0 ? 1u : 0u) | (zeros != 0 ? 2u : 0u);
     }
   }
 }

@@ -31,13 +31,16 @@ __host__ __device__ constexpr int select_rounds(int bits, uint32_t ranks)
 }
 static_assert(select_rounds(64, SELECT_MAX_RANKS) <= SELECT_MAX_ROUNDS, "counters for every round");
 
+constexpr uint32_t SELECT_FINISHED = ~0u;
+
 // Device-side state, written by select_init_kernel and by the last workgroup of every round.
 struct SelectPlan {
-  uint64_t key_or, key_and;            // over all images (first round)
+  uint64_t any[SELECT_MAX_RANKS];      // per prefix: OR of the images that have it (the round under way)
+  uint64_t all[SELECT_MAX_RANKS];      // per prefix: AND of them
   uint64_t prefix[SELECT_MAX_RANKS];   // different prefixes: the resolved top bits of an image
-  uint64_t image[SELECT_MAX_RANKS];    // per target, once done
+  uint64_t image[SELECT_MAX_RANKS];    // per target, once finished
   uint32_t rank[SELECT_MAX_RANKS];     // per target: position among the keys with its prefix
-  uint32_t which[SELECT_MAX_RANKS];    // per target: its prefix
+  uint32_t which[SELECT_MAX_RANKS];    // per target: its prefix, or SELECT_FINISHED
   uint32_t chunk[SELECT_MAX_RANKS];    // per target: where a key that ties with other bits is found
   uint32_t n_prefix;
   uint32_t bits_left;
@@ -52,47 +55,45 @@ struct SelectPlan {
 constexpr uint64_t SELECT_PLAN_BYTES = 2048;
 static_assert(sizeof(SelectPlan) <= SELECT_PLAN_BYTES, "plan slot");
 
-// The plan after a round.  chosen[t], count[t]: the prefix of target t down to bit `shift` and the
-// keys that have it, 0 where the round counted no key at the target's rank: a caller that writes to
-// the input during the call gets there.  Its result is undefined, but no later round may read
-// outside the lists: list_len never exceeds copy_cap once the copy is read.
-// `common`, `varying`: the bits on which all images of the input agree and differ (first round).
-__host__ __device__ inline void select_advance(SelectPlan* plan, uint64_t* chosen, const uint32_t* count, uint32_t n_ranks, uint32_t shift,
-                                               bool first, uint64_t common, uint64_t varying, uint32_t copied, uint32_t copy_cap)
+// A target after a round that resolved the bits from `shift` on: `chosen` is its prefix down to that bit,
+// `any` and `all` are OR and AND of the images counted under its old prefix.  Lower bits on which all of these
+// agree are known without another round: a target none of whose lower bits vary is finished, and the next
+// round starts at the highest bit that varies for any target.  So a handful of values is told apart in two
+// or three rounds wherever their bits are (whole numbers held as floats, small integers of either sign).  With a
+// round per eleven bits, each over the whole input since no copy is small enough, five percentiles of 2^28
+// zeros and ones in float64 took 4.6 ms, where the sort takes 2.5; now 1.1.
+struct SelectChild {
+  uint64_t image;    // right in the bits on which the keys agree
+  uint64_t varying;  // bits on which they do not; 0: the image is whole
+};
+__host__ __device__ inline SelectChild select_child(uint64_t chosen, uint32_t shift, uint64_t any, uint64_t all)
 {
-  uint32_t left  = shift;
-  uint64_t total = 0;
-  if (first) {
-    const uint32_t top = varying == 0 ? 0u : 64u - static_cast<uint32_t>(__builtin_clzll(varying));
-    if (top < left) {  // every key agrees on the bits above: one bin, whose prefix takes them in
-      left = top;
-      for (uint32_t t = 0; t < n_ranks; ++t) {
-        chosen[t] = common >> left;
-      }
-    }
-  }
-  uint32_t n = 0;
-  for (uint32_t t = 0; t < n_ranks; ++t) {  // ascending targets: equal prefixes are neighbours
-    if (t == 0 || chosen[t] != chosen[t - 1]) {
-      plan->prefix[n++] = chosen[t];
-      total += count[t];
-    }
-    plan->which[t] = n - 1;
-  }
-  plan->n_prefix  = n;
+  const uint64_t low = (1ull << shift) - 1;  // (the first round resolves at least one bit: shift < 64)
+  return SelectChild{(chosen << shift) | (all & low), (any ^ all) & low};
+}
+// Bits that are left to the next round; `varying`: of all its targets.
+__host__ __device__ inline uint32_t select_bits_left(uint64_t varying)
+{
+  return varying == 0 ? 0u : 64u - static_cast<uint32_t>(__builtin_clzll(varying));
+}
+
+// The list of the next round, which asks for `prefixes` prefixes with `total` keys in all and `left` unknown
+// bits: the input, the copy, or the input while the copy is made (unless no round comes after it).  copy_now,
+// from_copy: as the plan had them for this round; `copied`: keys that this round has staged for the copy.  A
+// caller that writes to the input during the call may bring more of them than were counted; the result is
+// undefined then, but no later round reads past the room that the copy has.
+__host__ __device__ inline void select_next_list(SelectPlan* plan, bool copy_now, bool from_copy, uint32_t prefixes, uint32_t left,
+                                                 uint64_t total, uint32_t copied, uint32_t copy_cap)
+{
+  plan->n_prefix  = prefixes;
   plan->bits_left = left;
-  if (plan->copy_now != 0) {
+  plan->done      = prefixes == 0 ? 1u : 0u;
+  if (copy_now) {
     plan->copy_now  = 0;
     plan->from_copy = 1;
     plan->list_len  = copied < copy_cap ? copied : copy_cap;
-  } else if (plan->from_copy == 0 && total <= copy_cap) {
+  } else if (!from_copy && total <= copy_cap && left > select_bits(prefixes)) {
     plan->copy_now = 1;
-  }
-  if (left == 0) {
-    plan->done = 1;
-    for (uint32_t t = 0; t < n_ranks; ++t) {
-      plan->image[t] = chosen[t];
-    }
   }
 }
 

@@ -44,15 +44,19 @@ extern "C" int run_rounds(const uint64_t* before, const uint64_t* after, uint32_
       return -1;
     }
     std::vector<uint32_t> hist(np << w);
-    uint64_t key_or = 0, key_and = ~0ull;
+    uint64_t any[SELECT_MAX_RANKS], all[SELECT_MAX_RANKS];
+    for (int t = 0; t < SELECT_MAX_RANKS; ++t) {
+      any[t] = 0;
+      all[t] = ~0ull;
+    }
     uint32_t copied = 0;
     for (uint32_t i = 0; i < list_len; ++i) {
       const uint64_t k = list[i];
-      key_or |= k;
-      key_and &= k;
       for (uint32_t t = 0; t < np; ++t) {
         if (first || (k >> plan.bits_left) == plan.prefix[t]) {
           ++hist[(t << w) + ((k >> shift) & ((1u << w) - 1))];
+          any[t] |= k;
+          all[t] &= k;
           if (plan.copy_now) {
             if (copied < copy_cap) {
               copy[copied] = k;
@@ -70,6 +74,9 @@ extern "C" int run_rounds(const uint64_t* before, const uint64_t* after, uint32_
       uint64_t run = 0;
       chosen[t] = 0;
       count[t]  = 0;
+      if (p == SELECT_FINISHED) {
+        continue;
+      }
       for (uint32_t b = 0; b < (1u << w); ++b) {
         const uint32_t c = hist[(p << w) + b];
         if (plan.rank[t] >= run && plan.rank[t] < run + c) {
@@ -81,7 +88,33 @@ extern "C" int run_rounds(const uint64_t* before, const uint64_t* after, uint32_
         run += c;
       }
     }
-    select_advance(&plan, chosen, count, n_ranks, shift, first, key_and, key_and ^ key_or, copied, copy_cap);
+    SelectChild child[SELECT_MAX_RANKS];
+    uint64_t varying = 0;
+    for (uint32_t t = 0; t < n_ranks; ++t) {
+      if (plan.which[t] != SELECT_FINISHED) {
+        child[t] = select_child(chosen[t], shift, any[plan.which[t]], all[plan.which[t]]);
+        varying |= child[t].varying;
+      }
+    }
+    const uint32_t left = select_bits_left(varying);
+    uint32_t prefixes = 0;
+    uint64_t total    = 0;
+    for (uint32_t t = 0; t < n_ranks; ++t) {
+      if (plan.which[t] == SELECT_FINISHED) {
+        continue;
+      }
+      if (child[t].varying == 0) {
+        plan.image[t] = child[t].image;
+        plan.which[t] = SELECT_FINISHED;
+        continue;
+      }
+      if (prefixes == 0 || plan.prefix[prefixes - 1] != child[t].image >> left) {
+        plan.prefix[prefixes++] = child[t].image >> left;
+        total += count[t];
+      }
+      plan.which[t] = prefixes - 1;
+    }
+    select_next_list(&plan, plan.copy_now != 0, plan.from_copy != 0, prefixes, left, total, copied, copy_cap);
   }
   for (uint32_t t = 0; t < n_ranks; ++t) {
     images[t]    = plan.image[t];
@@ -183,3 +216,16 @@ def test_no_round_leaves_the_lists_when_the_input_changes_under_way(lib, bits):
     for after in (np.full(n, middle), before ^ np.uint64(1 << (bits - 2)), np.zeros(n, np.uint64)):
         _, rounds, _, _, _ = _run(lib, before, wanted, bits, after=after)
         assert rounds >= 0
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.float64])
+@pytest.mark.parametrize("kind, reads", [("equal", 1), ("binary", 2), ("whole", 2), ("signed", 3), ("twenty", 4), ("ids", 4), ("random", 4)])
+def test_few_values_take_few_passes(lib, dtype, kind, reads):
+    """Vectors whose wanted values cover most of the input are never copied: every round reads all of it, so
+    rounds must not be spent on bits in which the keys of a prefix agree."""
+    rng = np.random.default_rng(7)
+    n = 50_000
+    k = _images(_data(kind, dtype, n, rng))
+    for wanted in ([n // 2], np.linspace(0, n - 1, 32).astype(int)):
+        _, rounds, _, _, read = _run(lib, k, wanted, 64)
+        assert rounds > 0 and read <= reads * n, (rounds, read / n)
