@@ -32,7 +32,8 @@ constexpr int SEARCH_PIVOTS = 2048;
 
 constexpr uint32_t WINDOW_BYTES    = 40960;
 constexpr uint32_t WINDOW_TILE_MAX = 1024;
-constexpr int BOUNDS_BLOCK         = 64;
+constexpr uint64_t WINDOW_WIDE_MAX = 1ull << 26;  // 8-byte keys of an array with the lower limit of values per tile
+constexpr int BOUNDS_BLOCK         = 256;
 
 template <int NW>
 __device__ __forceinline__ bool words_less(const uint64_t (&a)[NW], const uint64_t (&b)[NW])
@@ -118,34 +119,59 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_kernel(const KeyT* 
   }
 }
 
-// bounds[b] = answer for the first value of tile b (values sorted, `tile` of them per tile); bounds[tiles] = n
+// bounds[b] = answer for the first value of tile b (values sorted, `tile` of them per tile); bounds[tiles] = answer for
+// the last value.  Few searches, each a chain of dependent loads: evenly spaced elements in LDS take the first eleven.
 template <typename KeyT, int CODEC, bool LEFT>
 __global__ __launch_bounds__(BOUNDS_BLOCK) void window_bounds_kernel(const KeyT* __restrict__ sorted,
                                                                      uint64_t n,
                                                                      const KeyT* __restrict__ values,
+                                                                     uint64_t num_values,
                                                                      uint32_t tile,
                                                                      uint64_t tiles,
                                                                      uint64_t* __restrict__ bounds)
 {
+  __shared__ KeyT s_pivot[SEARCH_PIVOTS];
+  const uint64_t step = (n + SEARCH_PIVOTS - 1) / SEARCH_PIVOTS;
+  constexpr int EACH  = SEARCH_PIVOTS / BOUNDS_BLOCK;
+  KeyT pivot[EACH];
+#pragma unroll
+  for (int k = 0; k < EACH; ++k) {
+    const uint64_t i = (k * BOUNDS_BLOCK + threadIdx.x) * step;
+    pivot[k]         = sorted[i < n ? i : n - 1];
+  }
   const uint64_t b = static_cast<uint64_t>(blockIdx.x) * BOUNDS_BLOCK + threadIdx.x;
-  if (b < tiles) {
-    uint64_t v[1];
-    KeyTraits<CODEC, KeyT>::words(values[b * tile], v);
-    uint64_t lo = 0, hi = n;
-    while (lo < hi) {
-      const uint64_t mid = lo + (hi - lo) / 2;
-      uint64_t a[1];
-      KeyTraits<CODEC, KeyT>::words(sorted[mid], a);
-      if (go_right<LEFT, 1>(a, v)) {
-        lo = mid + 1;
-      } else {
-        hi = mid;
+  const uint64_t j = b < tiles ? b * tile : num_values - 1;
+  const KeyT v     = ordered_bits<CODEC, KeyT>(values[j]);
+#pragma unroll
+  for (int k = 0; k < EACH; ++k) {
+    s_pivot[k * BOUNDS_BLOCK + threadIdx.x] = ordered_bits<CODEC, KeyT>(pivot[k]);
+  }
+  __syncthreads();
+  if (b > tiles) {
+    return;
+  }
+  const uint32_t pivots = static_cast<uint32_t>((n + step - 1) / step);
+  uint32_t right        = 0;  // pivots left of the answer
+  for (uint32_t at = SEARCH_PIVOTS; at != 0; at >>= 1) {
+    if (right + at <= pivots) {
+      const KeyT a = s_pivot[right + at - 1];
+      if (LEFT ? a < v : a <= v) {
+        right += at;
       }
     }
-    bounds[b] = lo;
-  } else if (b == tiles) {
-    bounds[tiles] = n;
   }
+  uint64_t lo = right == 0 ? 0 : (right - 1) * step + 1;
+  uint64_t hi = right == pivots ? n : right * step;
+  while (lo < hi) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    const KeyT a       = ordered_bits<CODEC, KeyT>(sorted[mid]);
+    if (LEFT ? a < v : a <= v) {
+      lo = mid + 1;
+    } else {
+      hi = mid;
+    }
+  }
+  bounds[b] = lo;
 }
 
 // One tile of sorted values per workgroup.  The answers of the tile lie in [bounds[b], bounds[b + 1]]; if that
@@ -155,8 +181,8 @@ __global__ __launch_bounds__(BOUNDS_BLOCK) void window_bounds_kernel(const KeyT*
 // Bound by the read of the array, once, and by the 8-byte stores at the values' own positions.
 // 40 KB of window let four workgroups share a CU, so that one searches while others load; the
 // loads of the whole window, 16 bytes each, are issued together.  Two values per lane search side by side,
-// with a step count that is the same for all lanes.  2^24 float32 values in 2^28: 512 us (518 with loads
-// of one element) + 23 us for the windows' bounds, against 837 us for probes of the array by lanes with neighbouring values.
+// with a step count that is the same for all lanes.  2^24 float32 values in 2^28: 504 us + 25 us for the
+// windows' bounds, against 837 us for probes of the array by lanes with neighbouring values.
 // The stores stay ordinary ones: with non-temporal stores, which the L2 does not gather, the whole call
 // took 1395 us instead of 891.
 template <typename KeyT, int CODEC, bool LEFT>
@@ -184,6 +210,45 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const
   const uint32_t count  = static_cast<uint32_t>(num_values - first < tile ? num_values - first : tile);
   // elements between the 16-byte boundary below the window and the window
   const uint32_t head = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(sorted + from) % 16 / sizeof(KeyT));
+  if constexpr (sizeof(KeyT) <= 2) {
+    const uint64_t to = from + extent;
+    if (to <= from) {  // one answer for all, most often a value that ends or misses a run
+      for (uint32_t t = threadIdx.x; t < count; t += SEARCH_BLOCK) {
+        out[origin[first + t]] = static_cast<int64_t>(from);
+      }
+      return;
+    }
+    // An array this long has runs of 512 equal elements and more, and a window is mostly the run that the tile's first
+    // value begins.  A value that equals the first one of this tile or of the next has that bound for an answer: if
+    // there is no other, nothing of the array is read.  2^22 float16 values in 2^29: 162 us a call, 244 when the
+    // window is searched all the same, 219 by probes of the array.  (Any lane?  The flag lies in the window's LDS: with
+    // more of it per workgroup only three workgroups share a CU.)
+    const KeyT v_from   = ordered_bits<CODEC, KeyT>(values[first]);
+    const KeyT v_to     = ordered_bits<CODEC, KeyT>(values[first + tile < num_values ? first + tile : num_values - 1]);
+    uint32_t* s_between = reinterpret_cast<uint32_t*>(s_pack);
+    bool between        = false;
+    for (uint32_t t = threadIdx.x; t < count; t += SEARCH_BLOCK) {
+      const KeyT v = ordered_bits<CODEC, KeyT>(values[first + t]);
+      between      = between || (v != v_from && v != v_to);
+    }
+    if (threadIdx.x == 0) {
+      *s_between = 0;
+    }
+    __syncthreads();
+    if (__builtin_amdgcn_ballot_w64(between) != 0 && threadIdx.x % WAVE == 0) {
+      *s_between = 1;
+    }
+    __syncthreads();
+    const bool search = *s_between != 0;
+    __syncthreads();
+    if (!search) {
+      for (uint32_t t = threadIdx.x; t < count; t += SEARCH_BLOCK) {
+        const KeyT v           = ordered_bits<CODEC, KeyT>(values[first + t]);
+        out[origin[first + t]] = static_cast<int64_t>(v == v_from ? from : to);
+      }
+      return;
+    }
+  }
   // Room for whole packs at both ends.  An array that is not sorted can have bounds that fall: that
   // extent wraps to a large one and the search in the array ends at once.
   if (extent > CAPACITY - 2 * PACK) {  // the same for every lane of the workgroup
@@ -267,12 +332,21 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_window_kernel(const
 // Values per tile of the window search for `key_bytes`-byte keys, 0 where it does not pay.  A window is
 // planned to fill four fifths of its LDS, which leaves room for values that are not spread
 // evenly.  Below 128 values per tile a value has more than 256 bytes of the array to itself, and reading
-// all of it costs more than the cache lines that the probes of a value touch.
+// all of it costs more than the cache lines that the probes of a value touch.  8-byte keys of an array past the 512 MiB
+// need 256 values per tile: us per call by windows / by probes at 256 bytes per value, values spread as the
+// array / half of them in a thousandth of it:
+//   float64   512 MiB  387 / 446   390 / 407     1 GiB  582 / 603   577 / 552     4 GiB  2359 / 2375   2296 / 2160
+//   float32   512 MiB  267 / 331   279 / 297     1 GiB  430 / 481   445 / 422     4 GiB  1744 / 1799   1545 / 1509
 static uint32_t window_tile(int key_bytes, uint64_t n, uint64_t num_values)
 {
   const double per_value = static_cast<double>(n) * key_bytes / static_cast<double>(num_values);
   const double fits      = 0.8 * WINDOW_BYTES / per_value;
-  return fits >= WINDOW_TILE_MAX ? WINDOW_TILE_MAX : static_cast<uint32_t>(fits) / 128 * 128;
+  if (fits >= WINDOW_TILE_MAX) {
+    return WINDOW_TILE_MAX;
+  }
+  const uint32_t least = key_bytes == 8 && n > WINDOW_WIDE_MAX ? 256 : 128;
+  const uint32_t tile  = static_cast<uint32_t>(fits) / 128 * 128;
+  return tile >= least ? tile : 0;
 }
 
 template <typename KeyT, int CODEC>
@@ -287,7 +361,7 @@ static int launch_window_search(const void* sorted, uint64_t n, const void* valu
   {
     ProfileScope prof("window_bounds", stream);
     hipLaunchKernelGGL(bounds_of, dim3(static_cast<uint32_t>(tiles / BOUNDS_BLOCK + 1)), dim3(BOUNDS_BLOCK), 0, stream,
-                       static_cast<const KeyT*>(sorted), n, static_cast<const KeyT*>(values), tile, tiles, bounds);
+                       static_cast<const KeyT*>(sorted), n, static_cast<const KeyT*>(values), num_values, tile, tiles, bounds);
   }
   CPN_HIP_TRY(hipGetLastError());
   {

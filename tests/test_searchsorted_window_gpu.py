@@ -60,3 +60,65 @@ def test_searchsorted_window_tiles(dtype, spread):
             else:
                 want = np.searchsorted(a, v, "left" if left else "right")
             assert np.array_equal(_search(a, v, left, shift), want), (m, left)
+
+
+def _labels(call):
+    """The kernels that a call launches, and its result."""
+    import torch
+
+    lib = _lib.load()
+    torch.cuda.synchronize()
+    lib.cpn_profile_enable(1)
+    _lib.profile_collect()
+    try:
+        result = call()
+        torch.cuda.synchronize()
+        return {label for label, _ in _lib.profile_collect()}, result
+    finally:
+        lib.cpn_profile_enable(0)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.float16, np.int32, np.float32, np.float64])
+@pytest.mark.parametrize("windows", [True, False])
+def test_searchsorted_route_at_the_least_values_per_tile(dtype, windows):
+    """128 values per tile are the fewest that go by windows: 250 bytes of the array per value do, 262 do not."""
+    rng = np.random.default_rng(3)
+    n = (64 << 20) // np.dtype(dtype).itemsize + 77
+    m = (64 << 20) // (250 if windows else 262)
+    runs = {1: 200, 2: 3000}.get(np.dtype(dtype).itemsize, n // 3)  # different elements, half of the numbers between them missing
+    step = -(-n // runs)
+    a = np.arange(n) // step * 2 % (1 << 24)
+    v = rng.integers(0, 2 * runs, m)
+    if dtype == np.uint8:
+        a, v = a // 2, v // 2
+    a, v = np.sort(a).astype(dtype), (v % (1 << 24)).astype(dtype)
+    wide = np.float32 if dtype == np.float16 else dtype
+    for left in (True, False):
+        want = np.searchsorted(a.astype(wide), v.astype(wide), "left" if left else "right")
+        for shift in (0, 1):
+            labels, got = _labels(lambda: _search(a, v, left, shift))
+            assert ("window_bounds" in labels) == windows
+            assert np.array_equal(got, want), (left, shift)
+
+
+@pytest.mark.parametrize("n", [1 << 26, (1 << 26) + 1])
+def test_searchsorted_route_of_wide_keys(n):
+    """8-byte keys of more than 512 MiB take windows only from 256 values per tile on."""
+    a = np.arange(n, dtype=np.float64)
+    v = np.random.default_rng(5).integers(0, n, n // 25).astype(np.float64)  # 200 bytes of the array per value
+    labels, got = _labels(lambda: _search(a, v, False))
+    assert ("window_bounds" in labels) == (n == 1 << 26)
+    assert np.array_equal(got, v.astype(np.int64) + 1)
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.int32])
+def test_searchsorted_windows_of_an_array_that_is_not_sorted(dtype):
+    """Bounds that fall from one tile to the next: the answers mean nothing, but they are positions."""
+    rng = np.random.default_rng(9)
+    n = (64 << 20) // np.dtype(dtype).itemsize
+    info = np.iinfo(dtype)
+    a = rng.integers(info.min, info.max, n, dtype=dtype, endpoint=True)
+    v = rng.integers(info.min, info.max, n // 20, dtype=dtype, endpoint=True)
+    for table in (a, np.sort(a)[::-1].copy()):
+        got = _search(table, v, True)
+        assert got.min() >= 0 and got.max() <= n
