@@ -380,7 +380,7 @@ static int launch_searchsorted(const void* sorted, uint64_t n, const void* value
 {
   if constexpr (CODEC != CODEC_COMPLEX) {
     const uint32_t tile = window_tile(static_cast<int>(sizeof(KeyT)), n, num_values);
-    if (origin != nullptr && tile != 0 && num_values / tile < (1ull << 31) - 1) {
+    if (bounds != nullptr && num_values / tile < (1ull << 31) - 1) {
       return launch_window_search<KeyT, CODEC>(sorted, n, values, num_values, left, out, origin, tile, bounds, stream);
     }
   }
@@ -418,21 +418,19 @@ static bool presort_pays(int key_bytes, uint64_t n, uint64_t num_values)
   return n * static_cast<uint64_t>(key_bytes) >= (64ull << 20) && num_values >= (1ull << 16);
 }
 
+// The windows' bounds lie behind the header of the sort's own workspace, which is done with by then and has room for them
+// (a kilobyte of counters per 16384 values): a search by windows asks for no more than one by probes.
 struct SearchLayout {
-  uint64_t sort_bytes, off_values, off_origin, off_bounds, total;
+  uint64_t sort_bytes, off_values, off_origin, total;
 };
 
-static SearchLayout search_layout(int dtype, int key_bytes, uint64_t n, uint64_t num_values)
+static SearchLayout search_layout(int dtype, int key_bytes, uint64_t num_values)
 {
   SearchLayout L{};
   L.sort_bytes = cpn_local_sort_temp_bytes(dtype, num_values, num_values, 1, 1, 0);
   L.off_values = align_up(L.sort_bytes, WORKSPACE_ALIGN);
   L.off_origin = L.off_values + align_up(num_values * static_cast<uint64_t>(key_bytes), WORKSPACE_ALIGN);
-  L.off_bounds = L.off_origin + align_up(num_values * 8, WORKSPACE_ALIGN);
-  L.total      = L.off_bounds;
-  if (const uint32_t tile = window_tile(key_bytes, n, num_values); tile != 0) {
-    L.total += align_up(((num_values + tile - 1) / tile + 1) * 8, WORKSPACE_ALIGN);
-  }
+  L.total      = L.off_origin + align_up(num_values * 8, WORKSPACE_ALIGN);
   return L;
 }
 
@@ -444,7 +442,7 @@ extern "C" uint64_t cpn_searchsorted_temp_bytes(int dtype, uint64_t n, uint64_t 
   if (k.bytes == 0 || k.codec < 0 || !cpn::presort_pays(k.bytes, n, num_values)) {
     return 0;
   }
-  const cpn::SearchLayout L = cpn::search_layout(dtype, k.bytes, n, num_values);
+  const cpn::SearchLayout L = cpn::search_layout(dtype, k.bytes, num_values);
   return L.sort_bytes == 0 ? 0 : L.total;
 }
 
@@ -470,7 +468,7 @@ extern "C" int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const
   const int64_t* origin = nullptr;
   uint64_t* bounds      = nullptr;
   if (temp != nullptr && presort_pays(k.bytes, n, num_values)) {
-    const SearchLayout L = search_layout(dtype, k.bytes, n, num_values);
+    const SearchLayout L = search_layout(dtype, k.bytes, num_values);
     if (L.sort_bytes != 0 && temp_bytes >= L.total) {
       if ((reinterpret_cast<uintptr_t>(temp) % WORKSPACE_ALIGN) != 0) {
         return CPN_ERR_TEMP;
@@ -485,7 +483,10 @@ extern "C" int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const
       }
       values = sorted_vals;
       origin = where;
-      bounds = reinterpret_cast<uint64_t*>(ws + L.off_bounds);
+      if (const uint32_t tile = window_tile(k.bytes, n, num_values);
+          tile != 0 && L.sort_bytes >= HEADER_BYTES + ((num_values + tile - 1) / tile + 1) * 8) {
+        bounds = reinterpret_cast<uint64_t*>(ws + HEADER_BYTES);
+      }
     }
   }
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -365,3 +365,20 @@ def test_no_allocation_calls_in_the_native_sources():
             assert all(h.startswith("hipEventCreate") for h in hits), hits  # events, only while profiling is on
         else:
             assert hits == [], f"{path.name} calls {hits}"
+
+
+def test_searchsorted_workspace_holds_the_sorted_values_and_no_more():
+    """The bounds of the search windows (8 bytes per 128 values or more, and one) lie in the workspace of the values' sort, behind
+    its header of 2048 bytes: a search by windows asks for what one by probes does."""
+    lib = _lib.load()
+    align = lambda n: -(-n // 256) * 256
+    sizes = [65536, 65537, 100_003, 1 << 20, (1 << 24) + 1, 3 * (1 << 26) + 5, 1 << 32] + [(1 << 16) + 4096 * k + k for k in range(60)]
+    for dt, code in _lib.DTYPE_CODES.items():
+        if dt.kind == "c":
+            continue
+        for m in sizes:
+            sort_bytes = lib.cpn_local_sort_temp_bytes(code, m, m, 1, 1, 0)
+            assert sort_bytes >= 2048 + (-(-m // 128) + 1) * 8, (dt, m)
+            for n in (1 << 26, 1 << 28, 1 << 33):
+                want = align(sort_bytes) + align(m * dt.itemsize) + align(m * 8)
+                assert lib.cpn_searchsorted_temp_bytes(code, n, m) == want, (dt, n, m)
