@@ -258,8 +258,11 @@ int cpn_quantile_sorted(int dtype, const void* sorted, uint64_t outer, uint64_t 
  * The same for one long vector that is not sorted (outer == inner == 1): the elements that would stand
  * at left[q] and right[q] of the stable ascending sort are selected without sorting, bit for bit.
  * left, right and gamma are HOST arrays of num_q entries (read before the call returns).  Real types
- * of 4 and 8 bytes, n < 2^31, 1 <= num_q <= 16; for anything else the size query returns 0 and the call
- * CPN_ERR_UNSUPPORTED.  values is not modified; temp: cpn_quantile_select_temp_bytes bytes, 256-byte aligned.
+ * of 4 and 8 bytes, 1 <= n < 2^31, 1 <= num_q <= 16; for anything else the size query returns 0.  The call then
+ * returns CPN_ERR_DTYPE for unknown and complex types, CPN_OK without writing anything for num_q == 0,
+ * CPN_ERR_SHAPE for n == 0 and CPN_ERR_UNSUPPORTED for the rest; CPN_ERR_SHAPE also for a position
+ * outside [0, n).  values is not modified, and must not be written by others until the call's work on the
+ * stream is done: out is undefined otherwise.  temp: cpn_quantile_select_temp_bytes bytes, 256-byte aligned.
  */
 uint64_t cpn_quantile_select_temp_bytes(int dtype, uint64_t n, uint64_t num_q);
 int cpn_quantile_select(int dtype, const void* values, uint64_t n, uint64_t num_q, const int64_t* left,

@@ -382,3 +382,38 @@ def test_searchsorted_workspace_holds_the_sorted_values_and_no_more():
             for n in (1 << 26, 1 << 28, 1 << 33):
                 want = align(sort_bytes) + align(m * dt.itemsize) + align(m * 8)
                 assert lib.cpn_searchsorted_temp_bytes(code, n, m) == want, (dt, n, m)
+
+
+def test_quantile_select_refuses_with_the_codes_of_the_header():
+    lib = _lib.load()
+    select, size = lib.cpn_quantile_select, lib.cpn_quantile_select_temp_bytes
+    f32, f64, f16, c64 = (_lib.DTYPE_CODES[np.dtype(d)] for d in (np.float32, np.float64, np.float16, np.complex64))
+    left, right, gamma = np.array([3, 7]), np.array([4, 8]), np.zeros(2)
+    l, r, g = left.ctypes.data, right.ctypes.data, gamma.ctypes.data
+    need = size(f32, 10, 2)
+    assert need > 0 and need % 256 == 0
+
+    def call(dtype=f32, values=256, n=10, num_q=2, l=l, r=r, g=g, interpolate=1, out=512, temp=1024, temp_bytes=need):
+        return select(dtype, values, n, num_q, l, r, g, interpolate, out, temp, temp_bytes, None)
+
+    unsupported = _lib.CPN_ERR_UNSUPPORTED if hasattr(_lib, "CPN_ERR_UNSUPPORTED") else -8
+    assert call(dtype=99) == _lib.CPN_ERR_DTYPE and call(dtype=c64) == _lib.CPN_ERR_DTYPE
+    assert call(num_q=0, values=None, out=None, temp=None, temp_bytes=0) == _lib.CPN_OK
+    assert call(n=0) == _lib.CPN_ERR_SHAPE
+    assert call(dtype=f16) == _lib.CPN_ERR_UNSUPPORTED and call(num_q=17) == _lib.CPN_ERR_UNSUPPORTED and call(n=1 << 31) == _lib.CPN_ERR_UNSUPPORTED
+    for dtype, n, num_q in ((99, 10, 2), (c64, 10, 2), (f16, 10, 2), (f32, 0, 2), (f32, 1 << 31, 2), (f32, 10, 0), (f32, 10, 17)):
+        assert size(dtype, n, num_q) == 0
+    assert call(values=None) == _lib.CPN_ERR_NULL and call(out=None) == _lib.CPN_ERR_NULL and call(l=None) == _lib.CPN_ERR_NULL
+    assert call(r=None) == _lib.CPN_ERR_NULL and call(g=None) == _lib.CPN_ERR_NULL
+    assert call(temp=None) == _lib.CPN_ERR_TEMP and call(temp_bytes=need - 1) == _lib.CPN_ERR_TEMP and call(temp=1032) == _lib.CPN_ERR_TEMP
+    assert call(values=258) == _lib.CPN_ERR_ALIGN and call(out=516) == _lib.CPN_ERR_ALIGN
+    assert call(dtype=f64, values=260, temp_bytes=size(f64, 10, 2)) == _lib.CPN_ERR_ALIGN
+    for position in (-1, 10):
+        for side in (left, right):
+            kept = side[1]
+            side[1] = position
+            assert call() == _lib.CPN_ERR_SHAPE
+            side[1] = kept
+    # without interpolation right and gamma are not read, and out holds elements: the position is looked at last
+    left[1] = 10
+    assert call(r=None, g=None, interpolate=0, out=516) == _lib.CPN_ERR_SHAPE

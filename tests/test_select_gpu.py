@@ -76,3 +76,26 @@ def test_which_quantiles_are_selected():
     x = np.random.default_rng(1).standard_normal(100_000)
     qs = np.linspace(0, 1, 17)
     assert_same_bits(np.asarray(num.quantile(num.array(x), qs)), oracle.quantile(x, qs), "17 quantiles are read from the sorted vector")
+
+
+@pytest.mark.parametrize("dtype, n", [(np.float32, 8_500_007), (np.float64, 4_300_003), (np.int64, 4_300_003)])
+@pytest.mark.parametrize("kind", ["random", "specials", "few", "ids", "signed", "half"])
+def test_selection_from_vectors_longer_than_one_sweep_of_the_grid(dtype, n, kind):
+    """Every workgroup takes several strides: the loops with four loads in flight, the copy in several pieces, counters
+    with copies by lane, and a tied NaN or zero that is searched for over several steps of a chunk."""
+    rng = np.random.default_rng(n)
+    if kind == "signed":
+        x = rng.integers(-2, 3, n).astype(dtype)
+    elif kind == "half":  # one value for half of the vector, in one bin with the others
+        x = rng.integers(1, 1000, n).astype(dtype) if np.dtype(dtype).kind == "i" else (1 + rng.random(n)).astype(dtype)
+        x[rng.random(n) < 0.5] = 1
+    elif kind == "specials" and np.dtype(dtype).kind == "i":
+        x = np.where(rng.random(n) < 0.001, rng.integers(-(10**12), 10**12, n), rng.integers(1, 6, n)).astype(dtype)
+    else:
+        x = _data(kind, dtype, n, rng)
+    a = num.array(x)
+    assert _stats._select_bytes(a, 9) != 0
+    ordered = oracle.sort(x)
+    for q in ([0.5], [0.0, 0.05, 0.25, 0.31, 0.5, 0.62, 0.75, 0.95, 1.0], np.linspace(0.01, 0.99, 16)):
+        got = np.asarray(num.quantile(a, q, method="lower"))
+        assert_same_bits(got, ordered[(np.asarray(q) * (n - 1)).astype(np.int64)], f"{kind} {len(q)} quantiles")
