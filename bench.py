@@ -622,8 +622,9 @@ class UniqueJob:
         self.temp = torch.empty(self.tb, dtype=torch.uint8, device=dev)
         self.stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         distinct = min(n, max(n >> 6, 2))
-        self.alg = {"total": n * 4 + 4 * n * 8 + 2 * n * 4 + distinct * 4, "onesweep": n * 8,
-                    "unique_mark": n * 4 + n // 8, "unique_scatter": n // 8 + 2 * distinct * 4, "histogram": n * 4}
+        self.alg = {"onesweep": n * 8, "unique_mark": n * 4 + n // 8, "unique_scatter": n // 8 + 2 * distinct * 4, "histogram": n * 4}
+        passes = ((max(n >> 6, 2) - 1).bit_length() + 7) // 8  # (digits that agree in all values are skipped)
+        self.alg["total"] = passes * self.alg["onesweep"] + self.alg["unique_mark"] + self.alg["unique_scatter"] + self.alg["histogram"]
         self.dominant = "onesweep"
         self.dtype = "u32"
 
