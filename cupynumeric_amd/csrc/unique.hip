@@ -70,7 +70,16 @@ __global__ __launch_bounds__(UNIQUE_BLOCK) void unique_mark_kernel(const KeyT* _
   const int wave      = threadIdx.x / WAVE;
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * UNIQUE_TILE;
   constexpr int BATCH = sizeof(KeyT) <= 4 ? UNIQUE_ITEMS : (sizeof(KeyT) == 8 ? 8 : 4);
-  auto mark_batch     = [&](int start) {
+#pragma unroll
+  for (int start = 0; start < UNIQUE_ITEMS; start += BATCH) {
+    // A batch past the end is a round trip to memory for nothing (1000 complex128 values: 71 us a call with them,
+    // 68 without).  The first batch, all there is for keys of up to 4 bytes, is not asked.
+    if (start != 0 && base + static_cast<uint64_t>(start) * UNIQUE_BLOCK >= n) {
+      if (lane < BATCH) {
+        s_mark[(start + lane) * UNIQUE_WAVES + wave] = 0;
+      }
+      continue;
+    }
     KeyT key[BATCH], before[BATCH];
 #pragma unroll
     for (int k = 0; k < BATCH; ++k) {
@@ -86,22 +95,6 @@ __global__ __launch_bounds__(UNIQUE_BLOCK) void unique_mark_kernel(const KeyT* _
       const uint64_t bal = __builtin_amdgcn_ballot_w64(i < n && (i == 0 || differ));
       if (lane == 0) {
         s_mark[(start + k) * UNIQUE_WAVES + wave] = bal;
-      }
-    }
-  };
-  if (base + UNIQUE_TILE <= n) {
-#pragma unroll
-    for (int start = 0; start < UNIQUE_ITEMS; start += BATCH) {
-      mark_batch(start);
-    }
-  } else {
-    // the last tile: a batch past the end is a round trip to memory for nothing (1000 complex128 values: 71 us a call with
-    // them, 68 without)
-    for (int start = 0; start < UNIQUE_ITEMS; start += BATCH) {
-      if (base + static_cast<uint64_t>(start) * UNIQUE_BLOCK < n) {
-        mark_batch(start);
-      } else if (lane < BATCH) {
-        s_mark[(start + lane) * UNIQUE_WAVES + wave] = 0;
       }
     }
   }
