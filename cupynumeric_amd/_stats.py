@@ -114,10 +114,11 @@ def _collapse_axes(a: ndarray, axes: tuple[int, ...]) -> tuple[int, ndarray]:
     return first, ndarray(thunk.shape, thunk.dtype, thunk=thunk)
 
 
-# Vectors from this length on are selected from (`cpn_quantile_select`) instead of sorted.  us per call,
-# selected / sorted: five percentiles of 10^4 float32 47 / 88, float64 78 / 90, of 4 * 10^4 float64 77 / 128; sixteen
-# of 10^4 int64 108 / 79, of 10^6 123 / 210.  Vectors of up to 16 384 elements are sorted by one kernel, in less
-# time than the launches of a selection of many quantiles take.
+# Vectors from this length on are selected from (`cpn_quantile_select`) instead of sorted.  us per call of normal
+# values, selected / sorted, one, five and sixteen quantiles:
+#   32 768 elements   float32 38 / 102, 45 / 103, 65 / 104   float64 46 / 119, 61 / 120, 69 / 121   int64 56, 67, 85 / 115
+#   10 000 elements   float32 37 /  85, 44 /  84, 61 /  83   float64 42 /  89, 61 /  89, 65 /  89   int64 54, 65, 76 /  89
+# so the line could lie lower; only at 5000 int64 elements do sixteen quantiles lose (76 / 74).
 SELECT_MIN_SIZE = 32768
 
 
