@@ -62,6 +62,7 @@ PROTOTYPES: dict[str, tuple] = {
     "cpn_set_wide_row_threshold": (c_int64, [c_int64]),
     "cpn_set_lookback_spin_limit": (c_int64, [c_int64]),
     "cpn_set_virtual_digit_threshold": (c_int64, [c_int64]),
+    "cpn_set_equal_digit_threshold": (c_int64, [c_int64]),
     "cpn_set_wave_row_limit": (c_int64, [c_int64]),
     "cpn_set_merge_rows": (c_int, [c_int]),
     "cpn_set_bitonic_rows": (c_int, [c_int]),

@@ -49,6 +49,7 @@
 #include <limits>
 #include <type_traits>
 
+#include "equal_digits.h"
 #include "radix_common.h"
 #include "wave_row_sort.h"  // wave_all_and / wave_all_or, FIXUP_ROUNDS
 
@@ -120,7 +121,15 @@ __host__ __device__ constexpr int lds_row_waves_per_simd(int block, int items, i
   return (block == 1024 && items <= 8 && key_bytes <= 4) ? 8 : 1;
 }
 
-template <typename KeyT, int CODEC, bool HAS_IDX, int BLOCK, int ITEMS>
+// SEGMENTS: the workgroups share the pieces of one long row on the list of equal_digits.h (`segs`, n_list of the
+// plan), of any length up to the tile; a key's position is looked up in `pos` once its place is known.
+struct LdsSegments {
+  const uint2* segs;
+  uint32_t max_segs;
+  const uint32_t* pos;
+  const EqualPlan* eq;
+};
+template <typename KeyT, int CODEC, bool HAS_IDX, int BLOCK, int ITEMS, bool SEGMENTS = false>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(lds_row_waves_per_simd(BLOCK, ITEMS, sizeof(KeyT)))))
 void lds_row_sort_kernel(const KeyT* keys_in,
                                                               KeyT* keys_out,
@@ -130,9 +139,16 @@ void lds_row_sort_kernel(const KeyT* keys_in,
                                                               uint32_t pieces,
                                                               uint32_t last_piece_len,
                                                               int64_t index_offset,
-                                                              uint32_t* status)
+                                                              uint32_t* status,
+                                                              const LdsSegments sg)
 {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  uint32_t n_pieces = 1;  // SEGMENTS: on the list
+  if constexpr (SEGMENTS) {
+    if (sg.eq->mode == 0 || *status != 0) {
+      return;
+    }
+    n_pieces = sg.eq->n_list < sg.max_segs ? sg.eq->n_list : sg.max_segs;
+  } else if (blockIdx.x == 0 && threadIdx.x == 0) {
     *status = 0;  // the workspace's status word: a per-row sort cannot fail on the device
   }
   constexpr int WAVES  = BLOCK / WAVE;
@@ -174,9 +190,13 @@ void lds_row_sort_kernel(const KeyT* keys_in,
   __shared__ uint32_t s_wsum[DT::WAVES];
   __shared__ SW s_red[2 * WAVES * NW];
 
-  const int tid       = threadIdx.x;
-  const int lane      = tid & (WAVE - 1);
-  const int wave      = tid / WAVE;
+  for (uint32_t entry = SEGMENTS ? blockIdx.x : 0u; entry < n_pieces; entry += SEGMENTS ? gridDim.x : 1u) {
+  int tid = threadIdx.x;
+  if constexpr (SEGMENTS) {
+    asm volatile("" : "+v"(tid));  // (or every address below is worked out ahead of the loop, and spilled)
+  }
+  const int lane = tid & (WAVE - 1);
+  const int wave = tid / WAVE;
   // A workgroup sorts one piece of a row: the whole row (pieces == 1; row_stride == piece_len where the
   // rows are dense), or, for rows that are merged afterwards, piece number blockIdx.x % pieces of row
   // blockIdx.x / pieces; the last piece of a row may be shorter, and positions count from the row's start.
@@ -188,6 +208,11 @@ void lds_row_sort_kernel(const KeyT* keys_in,
     base                 = static_cast<uint64_t>(row) * row_stride + static_cast<uint64_t>(piece) * piece_len;
     index_offset += static_cast<int64_t>(piece) * piece_len;
     seg = piece + 1 == pieces ? last_piece_len : piece_len;
+  }
+  if constexpr (SEGMENTS) {
+    const uint2 piece = sg.segs[entry];
+    base              = piece.x;
+    seg               = piece.y;
   }
   const bool full     = (seg == TILE);
   // A row shorter than the tile is dealt in equal contiguous shares of whole 64-key rounds, so that
@@ -797,6 +822,13 @@ void lds_row_sort_kernel(const KeyT* keys_in,
     }
   }
 
+  if constexpr (SEGMENTS && HAS_IDX) {
+    const uint32_t* const pos = sg.pos + base;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      idx[i] = pos[idx[i] < seg ? idx[i] : 0u];  // (all lookups ahead of the stores; lanes without a key: any)
+    }
+  }
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const uint32_t o = woff + i * WAVE;
@@ -808,6 +840,10 @@ void lds_row_sort_kernel(const KeyT* keys_in,
         idx_out[base + o] = static_cast<int64_t>(idx[i]) + index_offset;
       }
     }
+  }
+  if constexpr (SEGMENTS) {
+    __syncthreads();  // the next piece reuses the shared memory
+  }
   }
 }
 

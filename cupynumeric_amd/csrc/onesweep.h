@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "equal_digits.h"
 #include "radix_common.h"
 #include "virtual_digits.h"
 
@@ -107,10 +108,20 @@ __device__ __forceinline__ bool hist_accumulate(uint32_t* s_hist, KeyT raw, uint
   return special;
 }
 
+// What the byte passes go on from when equalised digits have failed (equal_digits.h): keys and positions, and the
+// buffers that their first pass reads (make_plan).
+template <typename KeyT>
+struct EqualResume {
+  const KeyT* keys;
+  KeyT* keys_to;
+  const uint32_t* pos;  // nullptr: a plain sort
+  uint32_t* pos_to;
+};
+
 // grid = rows * blocks_per_row; block b of a row covers elements [b*chunk, min(seg, (b+1)*chunk)).
 // 128-bit loads over the 16-byte aligned middle of the chunk, scalar head and tail.
 // `vplan` (may be null): nothing to do when the sort already runs on the ranks of the row's
-// different keys (virtual_digits.h).
+// different keys (virtual_digits.h), or when equalised digits have sorted it (`eq`, may be null).
 // SPECIALS (float keys, keys-only sorts): also tells through `specials` whether a NaN or a -0.0 occurs.
 template <typename KeyT, int CODEC, typename OffT, bool SPECIALS = false>
 __global__ __launch_bounds__(HIST_BLOCK) void histogram_kernel(const KeyT* __restrict__ keys,
@@ -119,13 +130,27 @@ __global__ __launch_bounds__(HIST_BLOCK) void histogram_kernel(const KeyT* __res
                                                                  uint32_t blocks_per_row,
                                                                  uint64_t chunk,
                                                                  const VirtPlan* __restrict__ vplan,
-                                                                 uint32_t* __restrict__ specials)
+                                                                 uint32_t* __restrict__ specials,
+                                                                 const EqualPlan* __restrict__ eq,
+                                                                 const EqualResume<KeyT> resume)
 {
   constexpr int PASSES      = KeyTraits<CODEC, KeyT>::PASSES;
   constexpr int VEC         = 16 / sizeof(KeyT);
   constexpr int HIST_COPIES = hist_copies(PASSES);
-  if (vplan != nullptr && vplan->enabled == VIRT_DISTINCT) {
+  if ((vplan != nullptr && vplan->enabled == VIRT_DISTINCT) || eq_sorted(eq)) {
     return;
+  }
+  if (eq_failed(eq)) {
+    // the byte passes go on from what the passes on equalised digits left, in the buffers that suit their plan
+    keys                 = resume.keys;
+    const uint64_t first = static_cast<uint64_t>(blockIdx.x) * chunk;  // (one row)
+    const uint64_t last  = first + chunk < seg ? first + chunk : seg;
+    for (uint64_t i = first + threadIdx.x; i < last; i += HIST_BLOCK) {
+      resume.keys_to[i] = keys[i];
+      if (resume.pos != nullptr) {
+        resume.pos_to[i] = resume.pos[i];
+      }
+    }
   }
   __shared__ uint32_t s_hist[PASSES * RADIX * HIST_COPIES];
 
@@ -252,6 +277,9 @@ struct PlanRequest {
   // keys unless the histogram sweep met a NaN or a -0.0 (*specials != 0).
   uint32_t free_rank;
   const uint32_t* specials;
+  // Requests that may use equalised digits (may be null).  When those have failed, the byte passes start
+  // from the scratch partner of T1 below and from IDX_ALIAS.
+  const EqualPlan* eq;
 };
 
 // One thread.  `varying` is read with device-scope loads: the flags may have been raised by other
@@ -266,6 +294,18 @@ __device__ __forceinline__ void make_plan(const uint32_t* varying, SortPlan* __r
       ++k;
     }
   }
+  const bool resume = eq_failed(rq.eq);
+  if (resume && (k & 1u) != 0) {
+    // The first pass may not write the buffer it reads: an even number of passes, one of them on a
+    // digit on which all keys agree (it copies).
+    for (uint32_t p = 0; p < rq.passes; ++p) {
+      if (((flags >> p) & 1u) == 0) {
+        flags |= 1u << p;
+        ++k;
+        break;
+      }
+    }
+  }
   plan->n_active = k;
   plan->flipped  = (rq.free_rank != 0 && rq.specials != nullptr && rq.want_indices == 0 &&
                    __hip_atomic_load(rq.specials, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
@@ -273,7 +313,7 @@ __device__ __forceinline__ void make_plan(const uint32_t* varying, SortPlan* __r
                      : 0u;
   // scratch partner of T1: the caller's value array when it is free to be overwritten early
   const uint32_t key_x = (rq.want_values && !rq.in_place) ? KEY_OUT : KEY_T2;
-  uint32_t j = 0, key_prev = KEY_IN, idx_prev = BUF_NONE;
+  uint32_t j = 0, key_prev = resume ? key_x : KEY_IN, idx_prev = (resume && rq.want_indices) ? IDX_ALIAS : BUF_NONE;
   for (uint32_t p = 0; p < rq.passes; ++p) {
     PassPlan e{};
     if ((flags >> p) & 1u) {
@@ -303,7 +343,7 @@ __device__ __forceinline__ void make_plan(const uint32_t* varying, SortPlan* __r
 
 static __global__ void plan_kernel(const uint32_t* __restrict__ varying, SortPlan* __restrict__ plan, PlanRequest rq)
 {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
+  if (threadIdx.x == 0 && blockIdx.x == 0 && !eq_sorted(rq.eq)) {
     make_plan(varying, plan, rq);
   }
 }
@@ -327,6 +367,9 @@ __global__ __launch_bounds__(SCAN_BLOCK) void histogram_scan_kernel(OffT* __rest
                                                                     SortPlan* __restrict__ plan,
                                                                     PlanRequest rq)
 {
+  if (eq_sorted(rq.eq)) {
+    return;  // (the plan stays cleared: no byte pass runs)
+  }
   // first use (`second` == 0): nothing when the sort already runs on the ranks of the row's
   // different keys.  Second use, after vplan_kernel: scans the histograms of the grouped virtual
   // digits (one row, histogram = group) and nothing when that plan is not in force.
@@ -405,6 +448,9 @@ __global__ __launch_bounds__(256) void finalize_kernel(const SortPlan* __restric
                                                         int64_t index_offset,
                                                         PlanRequest rq)
 {
+  if (eq_sorted(rq.eq)) {
+    return;
+  }
   const uint32_t k      = plan->n_active;
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   const uint64_t first  = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -559,7 +605,7 @@ struct SweepShared {
 // the images that the first pass stored are mapped back to the keys' bits by the last pass as it
 // stores them.
 template <typename KeyT, int CODEC, bool XFORM, bool BIG, bool HAS_IDX, int BLOCK, int ITEMS, bool FULL, bool VIRT,
-          bool DONLY = false, bool UNFLIP = false>
+          bool DONLY = false, bool UNFLIP = false, bool EQ = false>
 __device__ __forceinline__ void onesweep_tile(
   const SweepArgs<BIG>& a,
   const uint32_t vcount,    // VIRT: positions in this pass's group, their bit offsets (8 bits each)
@@ -570,7 +616,8 @@ __device__ __forceinline__ void onesweep_tile(
   const uint32_t tile,
   const uint64_t row,
   const uint32_t trow,
-  const uint32_t count)
+  const uint32_t count,
+  const EqualDigits<KeyT> equal = {})  // EQ: how the keys' buckets are found
 {
   using OffT = typename RowWidth<BIG>::off_t;
   using DB   = DescBits<OffT>;
@@ -625,10 +672,20 @@ __device__ __forceinline__ void onesweep_tile(
   const uint32_t* rank_base    = free_first ? sh.ctr : wctr;
   uint32_t dpk[ITEMS / 4];   // the digits, four per register
   uint32_t rnk2[ITEMS / 2];  // rank among the wave's keys of the same digit, two per register
+  if constexpr (EQ) {
+    // all lookups first: between the ranking's own LDS accesses each would be waited for by itself
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const uint32_t d = (equal.bucket(ordered_bits<CODEC, KeyT>(key[i])) >> (RADIX_BITS * a.pass)) & 0xFFu;
+      dpk[i / 4]       = (i % 4 == 0) ? d : (dpk[i / 4] | (d << (8 * (i % 4))));
+    }
+  }
   auto rank_item = [&](const int i, const KeyT k) {
     const bool valid = FULL || (woff + i * WAVE < count);
     uint32_t d;
-    if constexpr (DONLY) {
+    if constexpr (EQ) {
+      d = (dpk[i / 4] >> (8 * (i % 4))) & 0xFFu;
+    } else if constexpr (DONLY) {
       uint64_t ow[KeyTraits<DCODEC, KeyT>::NWORDS];
       KeyTraits<DCODEC, KeyT>::words(k, ow);
       d = distinct_rank(ow[0], reinterpret_cast<const uint64_t*>(vlut), vlut + DISTINCT_LOOKUP * 8);
@@ -639,7 +696,9 @@ __device__ __forceinline__ void onesweep_tile(
     } else {
       d = KeyTraits<DCODEC, KeyT>::digit(k, a.pass);
     }
-    dpk[i / 4]       = (i % 4 == 0) ? d : (dpk[i / 4] | (d << (8 * (i % 4))));
+    if constexpr (!EQ) {
+      dpk[i / 4] = (i % 4 == 0) ? d : (dpk[i / 4] | (d << (8 * (i % 4))));
+    }
     uint32_t r;
     if (FREE_FIRST_OK && free_first) {  // uniform
       r = valid ? atomicAdd(&sh.ctr[d], 1u) : 0u;
@@ -726,6 +785,10 @@ __device__ __forceinline__ void onesweep_tile(
   // VIRT kernels, passes that store no keys (the last pass of an index-only sort): only the digits
   // travel, one byte each, and the table lookups for the second use of the digit fall away
   const bool digits_only = DONLY || (VIRT && (a.keys_out == nullptr));
+  // EQ: a digit is a table lookup and some arithmetic, so it is kept for the store instead of being found again:
+  // one byte per key, in the memory of the counters, once every thread has read those.
+  static_assert(!EQ || WAVES * RADIX * 4 >= TILE, "room for the digits");
+  uint8_t* const s_eq_digits = reinterpret_cast<uint8_t*>(sh.ctr);
   uint32_t pos2[ITEMS / 2];  // positions in the sorted tile, two per register
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
@@ -739,6 +802,15 @@ __device__ __forceinline__ void onesweep_tile(
       }
     }
     pos2[i / 2] = (i % 2 == 0) ? pos : (pos2[i / 2] | (pos << 16));
+  }
+  if constexpr (EQ) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      if (FULL || (woff + i * WAVE < count)) {
+        s_eq_digits[(pos2[i / 2] >> (16 * (i % 2))) & 0xFFFFu] = static_cast<uint8_t>(dpk[i / 4] >> (8 * (i % 4)));
+      }
+    }
   }
 
   // ---- decoupled look-back over the earlier tiles of this row ----
@@ -833,6 +905,8 @@ __device__ __forceinline__ void onesweep_tile(
         uint64_t ow[KeyTraits<DCODEC, KeyT>::NWORDS];
         KeyTraits<DCODEC, KeyT>::words(kk[k], ow);
         d = virtual_digit(ow[0], vcount, voffsets, vlut);
+      } else if constexpr (EQ) {
+        d = s_eq_digits[tid + k * BLOCK];  // (past the end of a short tile: not used)
       } else {
         d = KeyTraits<DCODEC, KeyT>::digit(kk[k], a.pass);
       }
@@ -1038,6 +1112,54 @@ void onesweep_kernel(const SweepArgs<BIG> a_in)
       onesweep_tile<KeyT, CODEC, XFORM, BIG, HAS_IDX, BLOCK, ITEMS, false, false>(a, 0u, 0ull, nullptr, sh, tile, row, trow,
                                                                                   static_cast<uint32_t>(remain));
     }
+  }
+}
+
+// A pass on equalised digits (equal_digits.h): a.pass is the byte of the bucket, the buffers are fixed
+// (the caller's a.keys_in, ...), and `specials` (may be null) says whether the first pass of a keys-only
+// sort has to be stable.
+template <typename KeyT, int CODEC, bool HAS_IDX, int BLOCK, int ITEMS>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CPN_ONESWEEP_WAVES_PER_EU)))
+void eq_sweep_kernel(SweepArgs<false> a, const EqualPlan* __restrict__ eq, const uint32_t* __restrict__ specials)
+{
+  constexpr int WAVES      = BLOCK / WAVE;
+  constexpr int TILE       = BLOCK * ITEMS;
+  constexpr int STAGE_ELEM = sweep_stage_elem<KeyT, uint32_t, HAS_IDX, false>();
+  __shared__ SweepShared<KeyT, uint32_t, WAVES, TILE, STAGE_ELEM> sh;
+  __shared__ __align__(16) uint32_t s_table[1 << eq_cell_bits(sizeof(KeyT))];
+  if (eq->mode == 0) {
+    return;
+  }
+  const int tid = threadIdx.x;
+  if (tid == 0) {  // (as in onesweep_kernel)
+    uint32_t ticket;
+    if (a.single_ticket != 0) {
+      ticket = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (ticket >= a.num_tiles) {
+        ticket = 0xFFFFFFFFu;
+      }
+    } else {
+      ticket = claim_tile(a.xcd_tickets, a.num_tiles);
+    }
+    sh.tile = (*a.status != 0) ? 0xFFFFFFFFu : ticket;
+  }
+  const EqualDigits<KeyT> equal = eq_load<KeyT>(eq, s_table, tid, BLOCK);
+  for (int j = tid; j < WAVES * RADIX; j += BLOCK) {
+    sh.ctr[j] = 0;
+  }
+  a.free_rank = (a.free_rank != 0 && (specials == nullptr || *specials == 0)) ? 1 : 0;
+  __syncthreads();
+  const uint32_t tile = sh.tile;
+  if (tile >= a.num_tiles) {
+    return;
+  }
+  const uint64_t remain = a.seg - static_cast<uint64_t>(tile) * TILE;
+  if (remain >= static_cast<uint64_t>(TILE)) {
+    onesweep_tile<KeyT, CODEC, false, false, HAS_IDX, BLOCK, ITEMS, true, false, false, false, true>(
+      a, 0u, 0ull, nullptr, sh, tile, 0, tile, TILE, equal);
+  } else {
+    onesweep_tile<KeyT, CODEC, false, false, HAS_IDX, BLOCK, ITEMS, false, false, false, false, true>(
+      a, 0u, 0ull, nullptr, sh, tile, 0, tile, static_cast<uint32_t>(remain), equal);
   }
 }
 

@@ -122,6 +122,12 @@ static std::atomic<long long> g_virt_threshold{[] {
   return (e != nullptr && *e != 0) ? atoll(e) : static_cast<long long>(VIRT_MIN_ROW_ELEMENTS);
 }()};
 
+static std::atomic<long long> g_equal_threshold{[] {
+  const char* e = getenv("CPN_SORT_EQUAL_DIGIT_THRESHOLD");
+  return (e != nullptr && *e != 0) ? atoll(e) : static_cast<long long>(EQ_MIN_ROW_ELEMENTS);
+}()};
+uint64_t equal_digit_threshold() { return static_cast<uint64_t>(g_equal_threshold.load(std::memory_order_relaxed)); }
+
 uint64_t virtual_digit_threshold() { return static_cast<uint64_t>(g_virt_threshold.load(std::memory_order_relaxed)); }
 
 static const long long g_count16_min_row = [] {
@@ -224,6 +230,12 @@ int64_t cpn_set_virtual_digit_threshold(int64_t elements)
 {
   const long long v = elements < 0 ? static_cast<long long>(cpn::VIRT_MIN_ROW_ELEMENTS) : static_cast<long long>(elements);
   return static_cast<int64_t>(cpn::g_virt_threshold.exchange(v));
+}
+
+int64_t cpn_set_equal_digit_threshold(int64_t elements)
+{
+  const long long v = elements < 0 ? static_cast<long long>(cpn::EQ_MIN_ROW_ELEMENTS) : static_cast<long long>(elements);
+  return static_cast<int64_t>(cpn::g_equal_threshold.exchange(v));
 }
 
 int64_t cpn_set_lookback_spin_limit(int64_t polls)
@@ -350,8 +362,9 @@ int cpn_local_sort_static(int dtype, const void* values_in, void* values_out, in
   const cpn::KeyKind k = cpn::key_kind(dtype);
   if (k.bytes != 0 && k.codec >= 0 && volume != 0 && sort_dim_size != 0 && volume % sort_dim_size == 0) {
     // a well-formed request: does its workspace fit?  (everything else gets cpn_local_sort's own answer)
-    const uint64_t need = cpn_local_sort_temp_bytes(dtype, volume, sort_dim_size, values_out != nullptr,
-                                                    indices_out != nullptr, values_out == values_in);
+    const uint64_t need =
+      cpn::workspace_bytes(k.bytes, cpn::key_passes(k.bytes, k.codec), volume, sort_dim_size, values_out != nullptr,
+                           indices_out != nullptr, values_out == values_in, /*least=*/true);
     if (need > CPN_STATIC_SCRATCH_BYTES) {
       return CPN_ERR_SCRATCH;
     }

@@ -54,6 +54,16 @@ constexpr uint64_t BIG_ROW_ELEMENTS = 1ull << 30;
 constexpr uint64_t VIRT_MIN_ROW_ELEMENTS = 1ull << 26;
 // The threshold in force (cpn_set_virtual_digit_threshold; tests lower it).
 uint64_t virtual_digit_threshold();
+// Row lengths that are tried with equalised digits (equal_digits.h), real keys of 8 bytes: from the threshold in
+// force (cpn_set_equal_digit_threshold; tests move it) to EQ_MAX_ROW_ELEMENTS.
+constexpr uint64_t EQ_MIN_ROW_ELEMENTS = 1ull << 25;
+constexpr uint64_t EQ_MAX_ROW_ELEMENTS = 1ull << 27;
+uint64_t equal_digit_threshold();
+// The stretch of the row whose bucket starts make one piece of the LDS sort (the rest of its tile is for the last
+// bucket to reach into), and the shape of the general sort that takes what that one does not.
+constexpr int EQ_SORT_STRIDE   = EQ_SORT_TILE * 3 / 4;
+constexpr int EQ_MEDIUM_BLOCK  = 1024;
+constexpr int EQ_MEDIUM_ITEMS  = 10;  // (12 and more spill)
 // How the scatter passes hand out their tiles: per XCD (default) or through one counter
 // (cpn_set_tile_order, CPN_SORT_TILE_ORDER=single).
 bool tile_order_single();
@@ -231,6 +241,12 @@ struct GlobalLayout {
   uint64_t off_key1, off_key2, key_bytes_total;
   uint64_t off_idx, idx_bytes_total;
   uint64_t total;
+  // Equalised digits (equal_digits.h): plan, tile counters, histograms and descriptors of their two passes
+  // ([off_eq, off_eq + eq_zero_bytes) is cleared), then the pieces for the LDS sort.  Behind everything else: a
+  // workspace that ends at `total` is enough to sort without them.
+  bool eq;
+  uint32_t eq_segments;
+  uint64_t off_eq, off_eq_tickets, off_eq_hist, off_eq_desc, eq_zero_bytes, off_eq_sample, off_eq_segs, off_eq_large, eq_total;
   bool valid;
 };
 
@@ -285,11 +301,28 @@ inline GlobalLayout global_layout(int key_bytes, int passes, uint64_t volume, ui
     off += L.idx_bytes_total;
   }
   L.total = off;
+  L.eq    = L.rows == 1 && !L.big && key_bytes == 8 && passes == key_bytes && seg >= equal_digit_threshold() &&
+         seg >= EQ_RANGE_SAMPLE && seg <= EQ_MAX_ROW_ELEMENTS;
+  L.eq_total = L.total;
+  if (L.eq) {
+    L.off_eq         = off;
+    L.off_eq_tickets = align_up(L.off_eq + sizeof(EqualPlan), WORKSPACE_ALIGN);
+    L.off_eq_hist    = L.off_eq_tickets + WORKSPACE_ALIGN;
+    L.off_eq_desc    = L.off_eq_hist + align_up(2 * RADIX * sizeof(uint32_t), WORKSPACE_ALIGN);
+    L.eq_zero_bytes  = L.off_eq_desc + 2 * L.desc_bytes_per_pass - L.off_eq;
+    L.eq_segments    = static_cast<uint32_t>((seg + EQ_SORT_STRIDE - 1) / EQ_SORT_STRIDE);
+    L.off_eq_sample  = L.off_eq + L.eq_zero_bytes;
+    L.off_eq_segs    = L.off_eq_sample + static_cast<uint64_t>(2 * EQ_GATHER_GRID + EQ_SAMPLE) * key_bytes;
+    // (pieces, further pieces, and the general sort's list, which may have to take all of them)
+    L.off_eq_large   = align_up(L.off_eq_segs + 4ull * L.eq_segments * sizeof(uint2), WORKSPACE_ALIGN);
+    L.eq_total       = align_up(L.off_eq_large + eq_large_entries(seg, EQ_SORT_TILE) * sizeof(EqualLarge), WORKSPACE_ALIGN);
+  }
   return L;
 }
 
+// What a sort asks for; with `least`, what it can do with.
 inline uint64_t workspace_bytes(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_values,
-                                bool want_indices, bool in_place)
+                                bool want_indices, bool in_place, bool least = false)
 {
   if (volume == 0 || seg <= lds_row_limit(key_bytes, want_indices)) {
     return HEADER_BYTES;
@@ -302,7 +335,7 @@ inline uint64_t workspace_bytes(int key_bytes, int passes, uint64_t volume, uint
     return HEADER_BYTES + merged_row_split_bytes(volume, seg, levels) + (levels >= 2 ? 2 : 1) * copy;
   }
   const GlobalLayout L = global_layout(key_bytes, passes, volume, seg, want_values, want_indices, in_place);
-  return L.valid ? L.total : 0;
+  return L.valid ? (least ? L.total : L.eq_total) : 0;
 }
 
 inline int launch_zero_fill(void* p, uint64_t bytes, hipStream_t stream)
@@ -395,7 +428,7 @@ inline int launch_lds_rows(const SortRequest& r)
                        static_cast<const KeyT*>(r.values_in), static_cast<KeyT*>(r.values_out), r.indices_out,
                        static_cast<uint32_t>(r.seg), r.row_stride != 0 ? r.row_stride : r.seg, r.pieces,
                        r.pieces > 1 ? r.last_seg : static_cast<uint32_t>(r.seg), r.index_offset,
-                       static_cast<uint32_t*>(r.temp));
+                       static_cast<uint32_t*>(r.temp), LdsSegments{});
   }
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;
@@ -729,6 +762,119 @@ inline int sort_rows_in_lds(const SortRequest& r)
 }
 
 // ---- global onesweep path --------------------------------------------------------------
+// The launches of equalised digits (equal_digits.h), ahead of the byte passes, which find nothing left to do when
+// these have sorted the row: keys go in -> key_x -> key buffer 1 -> output, positions through the caller's int64
+// array (as 32-bit scratch) and the index buffer back into it.
+template <typename KeyT, int CODEC, bool HAS_IDX>
+inline int sort_equalised(const SortRequest& r, const GlobalLayout& L, EqualPlan* eq, const VirtPlan* vplan, void* key_x,
+                          const PlanRequest& rq)
+{
+  constexpr int KB         = sizeof(KeyT);
+  constexpr bool SPECIALS  = (CODEC == CODEC_FLOAT) && !HAS_IDX;
+  unsigned char* ws        = static_cast<unsigned char*>(r.temp);
+  const uint32_t n         = static_cast<uint32_t>(r.seg);
+  uint32_t* hist           = reinterpret_cast<uint32_t*>(ws + L.off_eq_hist);
+  uint32_t* tickets        = reinterpret_cast<uint32_t*>(ws + L.off_eq_tickets);  // [0..1] one per pass, [8..23] per XCD
+  uint32_t* varying        = tickets + 32;
+  uint2* segs              = reinterpret_cast<uint2*>(ws + L.off_eq_segs);
+  uint2* extras            = segs + L.eq_segments;
+  uint2* list              = extras + L.eq_segments;
+  constexpr uint32_t medium = EQ_MEDIUM_BLOCK * EQ_MEDIUM_ITEMS;
+  EqualLarge* large        = reinterpret_cast<EqualLarge*>(ws + L.off_eq_large);
+  const uint32_t entries   = static_cast<uint32_t>(eq_large_entries(r.seg, EQ_SORT_TILE));
+  uint32_t* status         = static_cast<uint32_t*>(r.temp);
+  uint32_t* specials       = reinterpret_cast<uint32_t*>(ws + HEADER_SPECIALS);
+  KeyT* key1               = reinterpret_cast<KeyT*>(ws + L.off_key1);
+  uint32_t* idx1           = HAS_IDX ? reinterpret_cast<uint32_t*>(ws + L.off_idx) : nullptr;
+  {
+    // A bucket that the LDS sort can just take holds medium * EQ_SAMPLE / n sampled keys on average, and a bucket of
+    // evenly spread keys a quarter of one: the former and 8 more are a crowd.
+    const uint64_t share = static_cast<uint64_t>(medium) * EQ_SAMPLE / r.seg;
+    const uint32_t crowd = static_cast<uint32_t>(share) + 8;
+    const KeyT* ranges   = reinterpret_cast<const KeyT*>(ws + L.off_eq_sample);
+    ProfileScope prof("equal_plan", r.stream);
+    static_assert(VIRT_DISTINCT == 2, "veto word");
+    hipLaunchKernelGGL((eq_plan_kernel<KeyT, CODEC>), dim3(1), dim3(EQ_SAMPLE_BLOCK), 0, r.stream, ranges,
+                       ranges + 2 * EQ_GATHER_GRID, crowd,
+                       vplan != nullptr ? &vplan->enabled : static_cast<const uint32_t*>(nullptr), eq);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    const uint64_t unit = EQ_HIST_BLOCK * (16 / KB) * 4;  // one round of a workgroup
+    uint64_t chunk      = align_up((r.seg + 2047) / 2048, unit);
+    chunk               = chunk < 4 * unit ? 4 * unit : chunk;
+    ProfileScope prof("equal_histogram", r.stream);
+    hipLaunchKernelGGL((eq_histogram_kernel<KeyT, CODEC, SPECIALS>), dim3(static_cast<uint32_t>((r.seg + chunk - 1) / chunk)),
+                       dim3(EQ_HIST_BLOCK), 0, r.stream, static_cast<const KeyT*>(r.values_in), hist, r.seg, chunk, eq,
+                       specials);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    ProfileScope prof("equal_scan", r.stream);
+    hipLaunchKernelGGL((histogram_scan_kernel<uint32_t>), dim3(1), dim3(SCAN_BLOCK), 0, r.stream, hist, varying, r.seg, 2u,
+                       2ull, static_cast<const VirtPlan*>(nullptr), 0u, static_cast<uint32_t*>(nullptr),
+                       static_cast<SortPlan*>(nullptr), PlanRequest{});
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  for (int p = 0; p < 2; ++p) {
+    SweepArgs<false> a{};
+    a.keys_in         = p == 0 ? r.values_in : key_x;
+    a.keys_out        = p == 0 ? key_x : key1;
+    a.idx_in          = (HAS_IDX && p == 1) ? reinterpret_cast<const uint32_t*>(r.indices_out) : nullptr;
+    a.idx_out         = HAS_IDX ? (p == 0 ? static_cast<void*>(r.indices_out) : static_cast<void*>(idx1)) : nullptr;
+    a.ticket          = tickets + p;
+    a.xcd_tickets     = tickets + 8 + p * XCD_COUNT;
+    a.hist_excl       = hist + p * RADIX;
+    a.desc            = reinterpret_cast<uint32_t*>(ws + L.off_eq_desc + L.desc_bytes_per_pass * p);
+    a.status          = status;
+    a.seg             = r.seg;
+    a.hist_row_stride = 2 * RADIX;
+    a.tiles_per_row   = L.tiles_per_row;
+    a.num_tiles       = static_cast<uint32_t>(L.num_tiles);
+    a.pass            = p;
+    a.spin_limit      = lookback_spin_limit();
+    a.single_ticket   = (r.single_ticket || tile_order_single()) ? 1u : 0u;
+    a.free_rank       = (p == 0 && rq.free_rank != 0) ? 1 : 0;
+    ProfileScope prof("equal_sweep", r.stream);
+    hipLaunchKernelGGL((eq_sweep_kernel<KeyT, CODEC, HAS_IDX, global_block(KB), global_items(KB, false)>),
+                       dim3(static_cast<uint32_t>(L.num_tiles)), dim3(global_block(KB)), 0, r.stream, a, eq,
+                       SPECIALS ? static_cast<const uint32_t*>(specials) : static_cast<const uint32_t*>(nullptr));
+    CPN_HIP_TRY(hipGetLastError());
+  }
+  {
+    ProfileScope prof("equal_segments", r.stream);
+    hipLaunchKernelGGL((eq_segments_kernel<KeyT, CODEC>), dim3((L.eq_segments + EQ_SEGMENT_GROUP - 1) / EQ_SEGMENT_GROUP),
+                       dim3(EQ_SEGMENT_BLOCK), 0, r.stream, static_cast<const KeyT*>(key1), n, L.eq_segments,
+                       static_cast<uint32_t>(EQ_SORT_STRIDE), static_cast<uint32_t>(EQ_SORT_TILE), medium, entries, status, eq,
+                       segs, extras, list, large);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    // (no more workgroups than fit at once: each works through its share of the pieces)
+    const uint32_t grid = 4u * static_cast<uint32_t>(compute_units());
+    ProfileScope prof("equal_sort", r.stream);
+    hipLaunchKernelGGL((eq_sort_kernel<KeyT, CODEC, HAS_IDX>), dim3(grid < L.eq_segments ? grid : L.eq_segments),
+                       dim3(EQ_SORT_BLOCK), 0, r.stream, static_cast<const KeyT*>(key1), static_cast<KeyT*>(r.values_out),
+                       static_cast<const uint32_t*>(idx1), r.indices_out, r.index_offset, L.eq_segments, status, segs, extras,
+                       list, static_cast<const EqualLarge*>(large), entries, eq);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    LdsSegments sg{};
+    sg.segs     = list;
+    sg.max_segs = 2 * L.eq_segments;
+    sg.pos      = idx1;
+    sg.eq       = eq;
+    ProfileScope prof("equal_sort_general", r.stream);
+    hipLaunchKernelGGL((lds_row_sort_kernel<KeyT, CODEC, HAS_IDX, EQ_MEDIUM_BLOCK, EQ_MEDIUM_ITEMS, true>),
+                       dim3(static_cast<uint32_t>(compute_units())), dim3(EQ_MEDIUM_BLOCK), 0, r.stream,
+                       static_cast<const KeyT*>(key1), static_cast<KeyT*>(r.values_out), r.indices_out, 0u, 0ull, 1u, 0u,
+                       r.index_offset, status, sg);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  return CPN_OK;
+}
+
 template <typename KeyT, int CODEC, bool BIG, bool HAS_IDX>
 inline int sort_global(const SortRequest& r, const GlobalLayout& L)
 {
@@ -741,8 +887,21 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   const bool in_place  = (r.values_out == r.values_in);
   const bool want_vals = (r.values_out != nullptr);
 
-  int rc = launch_zero_fill(ws, L.zero_bytes, r.stream);
-  if (rc != CPN_OK) {
+  constexpr bool EQ_OK = !BIG && KB == 8 && KeyTraits<CODEC, KeyT>::PASSES == KB;
+  const bool use_eq    = EQ_OK && L.eq && r.temp_bytes >= L.eq_total;
+  EqualPlan* eq        = use_eq ? reinterpret_cast<EqualPlan*>(ws + L.off_eq) : nullptr;
+  if constexpr (EQ_OK) {
+    if (use_eq) {  // one launch clears the workspace and looks at a sample of the keys
+      KeyT* ranges = reinterpret_cast<KeyT*>(ws + L.off_eq_sample);
+      ProfileScope prof("equal_gather", r.stream);
+      hipLaunchKernelGGL((eq_gather_kernel<KeyT, CODEC>), dim3(EQ_GATHER_GRID), dim3(EQ_GATHER_BLOCK), 0, r.stream,
+                         static_cast<const KeyT*>(r.values_in), r.seg, ranges, ranges + 2 * EQ_GATHER_GRID,
+                         reinterpret_cast<uint4*>(ws), L.zero_bytes / 16, reinterpret_cast<uint4*>(eq), L.eq_zero_bytes / 16);
+    }
+  }
+  if (use_eq) {
+    CPN_HIP_TRY(hipGetLastError());
+  } else if (const int rc = launch_zero_fill(ws, L.zero_bytes, r.stream); rc != CPN_OK) {
     return rc;
   }
   uint32_t* status  = reinterpret_cast<uint32_t*>(ws);
@@ -761,6 +920,9 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   rq.in_place     = in_place ? 1u : 0u;
   rq.free_rank    = (!HAS_IDX && (CODEC == CODEC_UNSIGNED || CODEC == CODEC_SIGNED || CODEC == CODEC_FLOAT)) ? 1u : 0u;
   rq.specials     = (CODEC == CODEC_FLOAT) ? reinterpret_cast<const uint32_t*>(ws + HEADER_SPECIALS) : nullptr;
+  rq.eq           = eq;
+  // what the intermediate byte passes alternate with key buffer 1 (make_plan)
+  void* const key_x = (want_vals && !in_place) ? r.values_out : (L.off_key2 ? ws + L.off_key2 : nullptr);
 
   // histogram sweep: about 2048 blocks in total, at least one per row
   {
@@ -807,13 +969,24 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
         CPN_HIP_TRY(hipGetLastError());
       }
     }
+    if constexpr (EQ_OK) {
+      if (use_eq) {
+        const int eq_rc = sort_equalised<KeyT, CODEC, HAS_IDX>(r, L, eq, vplan, key_x, rq);
+        if (eq_rc != CPN_OK) {
+          return eq_rc;
+        }
+      }
+    }
     {
       ProfileScope prof("histogram", r.stream);
       constexpr bool SPECIALS = (CODEC == CODEC_FLOAT) && !HAS_IDX;  // who may rank its first pass freely
       hipLaunchKernelGGL((histogram_kernel<KeyT, CODEC, OffT, SPECIALS>), dim3(static_cast<uint32_t>(grid)),
                          dim3(HIST_BLOCK), 0, r.stream, static_cast<const KeyT*>(r.values_in), hist, r.seg,
                          static_cast<uint32_t>(bpr), chunk, static_cast<const VirtPlan*>(vplan),
-                         reinterpret_cast<uint32_t*>(ws + HEADER_SPECIALS));
+                         reinterpret_cast<uint32_t*>(ws + HEADER_SPECIALS), static_cast<const EqualPlan*>(eq),
+                         EqualResume<KeyT>{reinterpret_cast<const KeyT*>(ws + L.off_key1), static_cast<KeyT*>(key_x),
+                                           HAS_IDX ? reinterpret_cast<const uint32_t*>(ws + L.off_idx) : nullptr,
+                                           HAS_IDX ? reinterpret_cast<uint32_t*>(r.indices_out) : nullptr});
     }
     CPN_HIP_TRY(hipGetLastError());
     {
@@ -979,7 +1152,8 @@ int sort_typed(const SortRequest& r)
   constexpr int PASSES = KeyTraits<CODEC, KeyT>::PASSES;
   const bool has_idx   = (r.indices_out != nullptr);
   const bool in_place  = (r.values_out == r.values_in);
-  const uint64_t need  = workspace_bytes(KB, PASSES, r.volume, r.seg, r.values_out != nullptr, has_idx, in_place);
+  const uint64_t need  = workspace_bytes(KB, PASSES, r.volume, r.seg, r.values_out != nullptr, has_idx, in_place,
+                                             /*least=*/true);
   if (need == 0) {
     return CPN_ERR_UNSUPPORTED;
   }

@@ -441,6 +441,16 @@ int cpn_set_tile_order(int single);
 int64_t cpn_set_virtual_digit_threshold(int64_t elements);
 
 /*
+ * Process-wide tunable: a 1-D sort of real 8-byte keys with at least `elements` elements (and 2^18, and at most
+ * 2^27) lets the device sort it by two passes on digits made from a sample of the keys and one sort in LDS
+ * instead of the byte passes (cupynumeric_amd/csrc/equal_digits.h).  Results do not depend on it.  The default is
+ * 2^25; a negative value restores it and the previous setting is returned.  It changes the workspace that
+ * cpn_local_sort_temp_bytes asks for; the sort also takes the smaller one, and then runs the byte passes.  Also
+ * initialised from the environment variable CPN_SORT_EQUAL_DIGIT_THRESHOLD.
+ */
+int64_t cpn_set_equal_digit_threshold(int64_t elements);
+
+/*
  * Per-launch timing.  cpn_profile_enable(1) makes every kernel launch of the library record
  * a pair of HIP events on the stream it is launched on; it returns the previous setting.
  * cpn_profile_collect waits for the recorded events, writes up to `max_records` entries --

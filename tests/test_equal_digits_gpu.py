@@ -1,0 +1,118 @@
+"""Sorts of 8-byte keys by equalised digits (csrc/equal_digits.h) against the oracle, bit for bit.
+
+The threshold is lowered so that rows of a few hundred thousand keys take the path.  The inputs are those where it
+can go wrong: digits from a sample that misses the ends of the range, buckets of one value (kept), of many keys
+(larger tile), of a value and a few neighbours of it (the byte passes take over, before or after the passes on
+equalised digits), NaNs and zeros of both signs, and lengths at the ends of tiles and stretches.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+from conftest import assert_same_bits
+from test_sort_gpu import abi_sort, lib, torch_cuda  # noqa: F401 (fixtures)
+
+from oracle import sort_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def lowered_threshold(lib):
+    """(Rows of this length are merged from sorted pieces by default.)"""
+    prev, merged = lib.cpn_set_equal_digit_threshold(1 << 18), lib.cpn_set_merge_rows(0)
+    yield
+    lib.cpn_set_equal_digit_threshold(prev)
+    lib.cpn_set_merge_rows(merged)
+
+
+def _keys(kind, dtype, n, rng):
+    dt = np.dtype(dtype)
+    if dt.kind == "f":
+        x = rng.standard_normal(n)
+        u = rng.random(n)
+        if kind == "spread":
+            return rng.random(n)
+        if kind == "bits":  # every magnitude, NaNs of many payloads
+            return rng.integers(0, 1 << 63, n, dtype=np.int64).view(np.float64) * np.where(u < 0.5, -1.0, 1.0)
+        if kind == "specials":
+            x[u < 0.02] = np.nan
+            x[(u >= 0.02) & (u < 0.03)] = 0.0
+            x[(u >= 0.03) & (u < 0.04)] = -0.0
+            x[(u >= 0.04) & (u < 0.05)] = np.inf
+            x[(u >= 0.05) & (u < 0.06)] = -np.inf
+        elif kind == "crowd":  # a quarter is one value, and two neighbours of it are too few for the sample
+            x[u < 0.25] = 50.0
+            x[n // 3], x[n // 2] = np.nextafter(50.0, 51.0), np.nextafter(50.0, 49.0)
+        elif kind == "repeated":
+            x = rng.standard_normal(n // 40)[rng.integers(0, n // 40, n)]
+        return x
+    info = np.iinfo(dtype)
+    x = rng.integers(info.min, info.max, n, dtype=dtype, endpoint=True)
+    if kind == "specials":  # the smallest and largest key, often
+        x[rng.random(n) < 0.02] = info.min
+        x[rng.random(n) < 0.02] = info.max
+    elif kind == "crowd":
+        mid = dt.type(info.max // 3)
+        x[rng.random(n) < 0.25] = mid
+        x[n // 3], x[n // 2] = mid + dt.type(1), mid - dt.type(1)
+    elif kind == "repeated":
+        x = x[: n // 40][rng.integers(0, n // 40, n)]
+    elif kind == "bits":  # few bytes vary: the byte passes keep it
+        x = (x.view(np.uint64) >> np.uint64(33)).astype(dtype)
+    return x
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.int64, np.uint64])
+@pytest.mark.parametrize("kind", ["spread", "bits", "normal", "specials", "crowd", "repeated"])
+def test_kinds_of_keys(lib, torch_cuda, dtype, kind):
+    if kind == "normal" and np.dtype(dtype).kind != "f":
+        pytest.skip("float keys only")
+    rng = np.random.default_rng(len(kind) + np.dtype(dtype).num)
+    n = 700_001
+    x = _keys(kind, dtype, n, rng).astype(dtype, copy=False)
+    want_v = oracle.local_sort(x, argsort=False, threads=8)
+    want_i = oracle.local_sort(x, argsort=True, threads=8)
+    v, _ = abi_sort(lib, torch_cuda, x, want_values=True, want_indices=False)
+    assert_same_bits(v, want_v, "values")
+    _, i = abi_sort(lib, torch_cuda, x, want_values=False, want_indices=True, offset=7)
+    assert_same_bits(i, want_i + 7, "positions")
+    v, i = abi_sort(lib, torch_cuda, x, want_values=True, want_indices=True)
+    assert_same_bits(v, want_v, "both: values")
+    assert_same_bits(i, want_i, "both: positions")
+    v, i = abi_sort(lib, torch_cuda, x, want_values=True, want_indices=True, in_place=True)
+    assert_same_bits(v, want_v, "in place")
+    assert_same_bits(i, want_i, "in place: positions")
+    v, _ = abi_sort(lib, torch_cuda, x, want_values=True, in_place=True)
+    assert_same_bits(v, want_v, "in place, values only")
+
+
+@pytest.mark.parametrize("n", [(1 << 18), (1 << 18) + 1, 16384 * 17 - 1, 16384 * 17, 2304 * 120, 2304 * 120 + 1, 3072 * 100 - 1])
+def test_lengths(lib, torch_cuda, n):
+    """The shortest row that is sampled, ends of the scatter tiles (16384) and of the LDS sort's stretches (2304)."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n)
+    _, i = abi_sort(lib, torch_cuda, x, want_values=False, want_indices=True)
+    assert_same_bits(i, oracle.local_sort(x, argsort=True, threads=8), "positions")
+    v, _ = abi_sort(lib, torch_cuda, x, want_values=True)
+    assert_same_bits(v, oracle.local_sort(x, argsort=False, threads=8), "values")
+
+
+def test_the_smaller_workspace_is_still_taken(lib, torch_cuda):
+    """A caller that asked for the workspace while the path was out of use gets the byte passes."""
+    torch = torch_cuda
+    n = 300_000
+    x = np.random.default_rng(0).standard_normal(n)
+    lib.cpn_set_equal_digit_threshold(1 << 40)
+    small = lib.cpn_local_sort_temp_bytes(11, n, n, 1, 0, 0)
+    lib.cpn_set_equal_digit_threshold(1 << 18)
+    assert small < lib.cpn_local_sort_temp_bytes(11, n, n, 1, 0, 0)
+    a = torch.from_numpy(x).cuda()
+    out = torch.empty_like(a)
+    ws = torch.empty(small, dtype=torch.uint8, device="cuda")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.cpn_local_sort(11, a.data_ptr(), out.data_ptr(), None, n, n, 0, 1, ws.data_ptr(), small, stream) == 0
+    assert lib.cpn_local_sort_check(ws.data_ptr(), stream) == 0
+    assert_same_bits(out.cpu().numpy(), np.sort(x), "values")
