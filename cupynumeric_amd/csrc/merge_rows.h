@@ -231,4 +231,175 @@ __global__ __launch_bounds__(merge_block(HAS_IDX)) void merge_halves_kernel(cons
   }
 }
 
+// ---- short requests: all pieces of a row merged in one launch, by rank ----------------------------
+// A key's place in the row is its place in its own piece plus, for every other piece, the number of that piece's
+// keys that come before it.  A workgroup takes RANK_CHUNK neighbouring keys of one piece; what lies between the
+// first and the last of them in another piece (about as many keys, where the pieces are alike) is copied into LDS
+// and searched there by every key of the chunk.  The work grows with the number of pieces, so this is for
+// requests that leave most of the chip idle, whose time is the chain of launches: 100 000 float64 keys with
+// positions took 48 us for sorting eight pieces and three pairs of launches for merging them level by level, 59 us;
+// now 22 us for thirteen pieces and 26 us for this kernel (which waits for memory and LDS in turn: the windows'
+// ends, the windows, the searches).
+constexpr int RANK_CHUNK      = 256;
+constexpr int RANK_MAX_PIECES = 64;
+// Keys of other pieces in LDS at a time (more are taken in turns), and how many of them a thread reads at once.
+constexpr uint32_t RANK_STAGE = 8192;
+constexpr int RANK_LOADS      = 8;
+constexpr int RANK_ILP        = 4;  // pieces searched at once by a thread
+
+// keys / idx: the rows, [rows][n], in sorted pieces of `piece` elements (the last one of a row may be shorter); idx
+// holds row positions.  Outputs may not alias them.  Grid: rows x pieces x chunks workgroups of RANK_CHUNK threads.
+template <typename KeyT, int CODEC, bool HAS_IDX>
+__global__ __launch_bounds__(RANK_CHUNK) void merge_ranks_kernel(const KeyT* __restrict__ keys,
+                                                                 const int64_t* __restrict__ idx,
+                                                                 KeyT* __restrict__ keys_out,
+                                                                 int64_t* __restrict__ idx_out,
+                                                                 uint32_t n,
+                                                                 uint32_t piece,
+                                                                 uint32_t pieces,
+                                                                 uint32_t chunks)
+{
+  static_assert(2 * RANK_MAX_PIECES <= RANK_CHUNK, "a thread per end of a window");
+  __shared__ KeyT s_keys[RANK_STAGE];                  // ordered images
+  __shared__ uint32_t s_end[2][RANK_MAX_PIECES + RANK_ILP];  // of every piece: keys before the chunk's first / last key
+  __shared__ uint32_t s_at[RANK_MAX_PIECES + 1];       // where its window starts, all windows one after the other
+  const uint32_t tid  = threadIdx.x;
+  const uint32_t lane = tid % WAVE, wave = tid / WAVE;
+  const uint32_t per_row = pieces * chunks;
+  const uint64_t row     = blockIdx.x / per_row;
+  const uint32_t rest    = blockIdx.x - static_cast<uint32_t>(row * per_row);
+  const uint32_t mine    = rest / chunks;
+  const uint32_t first   = (rest - mine * chunks) * RANK_CHUNK;  // of the chunk in its piece
+  const KeyT* const row_keys = keys + row * n;
+  auto length = [&](uint32_t j) { return n - j * piece < piece ? n - j * piece : piece; };
+  if (first >= length(mine)) {
+    return;  // (the whole workgroup: the last piece may be short)
+  }
+  const uint32_t count = length(mine) - first < RANK_CHUNK ? length(mine) - first : RANK_CHUNK;
+  auto image           = [](KeyT k) { return ordered_bits<CODEC, KeyT>(k); };
+  const uint64_t own   = row * n + static_cast<uint64_t>(mine) * piece + first;  // of the chunk
+  const KeyT raw       = keys[own + (tid < count ? tid : count - 1)];
+  const KeyT key       = image(raw);
+  int64_t position     = 0;
+  if constexpr (HAS_IDX) {
+    position = idx[own + (tid < count ? tid : count - 1)];
+  }
+  // a key k of piece j comes before x of this chunk when it is smaller, or equal and j is the earlier piece:
+  // k < x + (j < mine), where x + 1 may wrap, so as two comparisons
+  auto before = [&](KeyT k, KeyT x, uint32_t j) { return k < x || (k == x && j < mine); };
+
+  // ---- the windows: thread 2j + e counts the keys of piece j before the chunk's first (e = 0) or last key ----
+  if (tid < 2 * pieces) {
+    const uint32_t j = tid / 2;
+    const KeyT x     = image(keys[own + ((tid & 1u) ? count - 1 : 0u)]);
+    const KeyT* p    = row_keys + static_cast<uint64_t>(j) * piece;
+    uint32_t lo = 0, hi = length(j);
+    if (j == mine) {
+      hi = 0;  // (not searched)
+    }
+    while (lo < hi) {  // three probes at once: half the dependent reads
+      const uint32_t d = (hi - lo) / 4;
+      const uint32_t m1 = lo + d, m2 = lo + (hi - lo) / 2, m3 = hi - 1 - d;
+      const bool b1 = before(image(p[m1]), x, j), b2 = before(image(p[m2]), x, j), b3 = before(image(p[m3]), x, j);
+      // m1 <= m2; m3 may stand before m2 in a short range, where the answers are still those of a sorted array
+      uint32_t l = lo, h = hi;
+      if (b1) { l = m1 + 1 > l ? m1 + 1 : l; } else { h = m1 < h ? m1 : h; }
+      if (b2) { l = m2 + 1 > l ? m2 + 1 : l; } else { h = m2 < h ? m2 : h; }
+      if (b3) { l = m3 + 1 > l ? m3 + 1 : l; } else { h = m3 < h ? m3 : h; }
+      lo = l;
+      hi = h;
+    }
+    s_end[tid & 1u][j] = lo;
+  }
+  __syncthreads();
+  // window of piece j: keys [s_end[0][j], s_end[1][j]) of it; before a key of the chunk come s_end[0][j] of its keys
+  // and some of the window
+  uint32_t rank = first + tid;
+  if (wave == 0) {
+    uint32_t run = 0;
+    for (uint32_t j0 = 0; j0 < pieces; j0 += WAVE) {
+      const uint32_t j    = j0 + lane;
+      const uint32_t s    = j < pieces ? s_end[1][j] - s_end[0][j] : 0u;
+      const uint32_t incl = wave_inclusive_sum_dpp(s);
+      if (j < pieces) {
+        s_at[j] = run + incl - s;
+      }
+      run += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), WAVE - 1));
+    }
+    if (lane == 0) {
+      s_at[pieces] = run;
+    }
+  }
+  __syncthreads();
+  for (uint32_t j = 0; j < pieces; ++j) {
+    rank += s_end[0][j];
+  }
+  const uint32_t total = s_at[pieces];
+  for (uint32_t from = 0; from < total; from += RANK_STAGE) {
+    const uint32_t to = total - from < RANK_STAGE ? total : from + RANK_STAGE;
+    // keys [from, to) of the windows laid end to end, RANK_LOADS of a thread's share in flight
+    {
+      uint32_t j = 0;
+      for (uint32_t i0 = from + tid; i0 < to; i0 += RANK_LOADS * RANK_CHUNK) {
+        KeyT k[RANK_LOADS];
+#pragma unroll
+        for (int l = 0; l < RANK_LOADS; ++l) {
+          const uint32_t i = i0 + l * RANK_CHUNK < to ? i0 + l * RANK_CHUNK : to - 1;
+          while (s_at[j + 1] <= i) {  // (s_at[pieces] == total > i)
+            ++j;
+          }
+          k[l] = row_keys[static_cast<uint64_t>(j) * piece + s_end[0][j] + (i - s_at[j])];
+        }
+#pragma unroll
+        for (int l = 0; l < RANK_LOADS; ++l) {
+          if (i0 + l * RANK_CHUNK < to) {
+            s_keys[i0 + l * RANK_CHUNK - from] = image(k[l]);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    for (uint32_t j0 = 0; j0 < pieces; j0 += RANK_ILP) {
+      uint32_t base[RANK_ILP], len[RANK_ILP], found[RANK_ILP], most = 0;
+#pragma unroll
+      for (int k = 0; k < RANK_ILP; ++k) {
+        const uint32_t j = j0 + k < pieces ? j0 + k : pieces;
+        const uint32_t a = s_at[j] > from ? s_at[j] : from;
+        const uint32_t e = s_at[j < pieces ? j + 1 : j];
+        const uint32_t b = e < to ? e : to;
+        base[k]  = a - from;
+        len[k]   = b > a ? b - a : 0u;
+        found[k] = 0;
+        most     = len[k] > most ? len[k] : most;
+      }
+      if (most == 0) {
+        continue;  // uniform
+      }
+      for (uint32_t step = 1u << (31 - __builtin_clz(most)); step != 0; step >>= 1) {
+#pragma unroll
+        for (int k = 0; k < RANK_ILP; ++k) {
+          const uint32_t at  = found[k] + step;
+          const bool inside  = at <= len[k];
+          const KeyT other   = s_keys[inside ? base[k] + at - 1 : 0u];
+          const bool earlier = before(other, key, j0 + k);
+          found[k]           = (inside && earlier) ? at : found[k];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < RANK_ILP; ++k) {
+        rank += found[k];
+      }
+    }
+    __syncthreads();
+  }
+  if (tid < count) {
+    if (keys_out != nullptr) {
+      keys_out[row * n + rank] = raw;
+    }
+    if constexpr (HAS_IDX) {
+      idx_out[row * n + rank] = position;
+    }
+  }
+}
+
 }  // namespace cpn

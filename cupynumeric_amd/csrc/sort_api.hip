@@ -64,6 +64,7 @@ static std::atomic<int> g_merge_rows{[] {
   return v < 0 ? 1 : v;
 }()};
 
+bool merge_rows_default() { return g_merge_rows.load(std::memory_order_relaxed) == 1; }
 bool merge_rows_enabled() { return g_merge_rows.load(std::memory_order_relaxed) != 0; }
 
 // Measured on 2^26 keys: a level of merging costs 0.17 ms for 4-byte keys (0.27 with positions) and

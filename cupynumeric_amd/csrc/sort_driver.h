@@ -179,6 +179,34 @@ inline uint64_t merged_row_split_bytes(uint64_t volume, uint64_t seg, int levels
   return align_up((volume / seg) * per_row * sizeof(uint32_t), WORKSPACE_ALIGN);
 }
 
+// Requests of few keys, real keys of 4 and 8 bytes: rows cut into short pieces, all merged by rank in one launch
+// (merge_rows.h).  Returns the pieces' length, 0: another path.  (cpn_set_merge_rows: in the default mode only.)
+// Where the lines lie (us per call through the Python API, this way / the way it took before, sort and argsort):
+//   from where one workgroup per row is left: 14 000 uint32 23, 23 / 24, 24, float32 25, 25 / 34, 33, float64 26,
+//   28 / 46, 51; 8192 float64 26, 28 / 27, 21.  (Only single rows of up to lds_row_capacity keys: the other way
+//   needs no workspace, and several rows keep as many workgroups busy.)
+//   to where the work, which grows with the square of the row, eats the launches saved: 262 144 uint32 68, 72 /
+//   86, 98, float32 75, 80 / 89, 99, 400 000 uint32 147, 152 / 86, 106; float64 200 000 104, 96 / 124, 132,
+//   262 144 127, 119 / 123, 131.
+//   pieces of 4096 or 8192 keys: fewer pieces to search against a longer sort of each: 32 768 uint32 26, 26
+//   (4096) and 27, 31 (8192), 65 536 34, 35 and 31, 35, 131 072 56, 58 and 39, 44; float64 sort 65 536 40 and 47,
+//   131 072 65 and 59, argsort 32 768 33 and 38, 65 536 41 and 41, 131 072 67 and 51.
+constexpr uint64_t RANK_MAX_VOLUME = 1ull << 18;
+bool merge_rows_default();
+inline uint64_t ranked_row_piece(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_indices)
+{
+  const uint64_t cap = lds_row_capacity(key_bytes, want_indices);
+  if (!merge_rows_default() || (key_bytes != 4 && key_bytes != 8) || passes != key_bytes ||
+      lds_row_limit(key_bytes, want_indices) != cap || volume > RANK_MAX_VOLUME ||
+      seg <= (key_bytes == 4 ? 12288u : 8192u) || (seg <= cap && volume != seg) ||
+      (key_bytes == 8 && !want_indices && volume > 26 * 8192)) {
+    return 0;
+  }
+  const uint64_t few    = key_bytes == 4 ? 40000 : (want_indices ? 40000 : 80000);
+  const uint64_t tile   = seg <= few ? 4096 : 8192;
+  const uint64_t pieces = (seg + tile - 1) / tile;  // (of equal length: a short one would be searched far more widely)
+  return (seg + pieces - 1) / pieces;
+}
 // Element type code (enum cpn_dtype) -> key width and codec.
 struct KeyKind {
   int bytes;  // 0 = unknown code
@@ -320,10 +348,20 @@ inline GlobalLayout global_layout(int key_bytes, int passes, uint64_t volume, ui
   return L;
 }
 
+// Rows merged by rank: the rows with their pieces sorted, and the positions.
+inline uint64_t ranked_workspace_bytes(int key_bytes, uint64_t volume, bool want_indices)
+{
+  return HEADER_BYTES + align_up(volume * key_bytes, WORKSPACE_ALIGN) + (want_indices ? align_up(volume * 8, WORKSPACE_ALIGN) : 0);
+}
 // What a sort asks for; with `least`, what it can do with.
 inline uint64_t workspace_bytes(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_values,
                                 bool want_indices, bool in_place, bool least = false)
 {
+  if (!least && volume != 0 && ranked_row_piece(key_bytes, passes, volume, seg, want_indices) != 0) {
+    const uint64_t own = workspace_bytes(key_bytes, passes, volume, seg, want_values, want_indices, in_place, true);
+    const uint64_t all = ranked_workspace_bytes(key_bytes, volume, want_indices);
+    return own > all ? own : all;
+  }
   if (volume == 0 || seg <= lds_row_limit(key_bytes, want_indices)) {
     return HEADER_BYTES;
   }
@@ -429,6 +467,45 @@ inline int launch_lds_rows(const SortRequest& r)
                        static_cast<uint32_t>(r.seg), r.row_stride != 0 ? r.row_stride : r.seg, r.pieces,
                        r.pieces > 1 ? r.last_seg : static_cast<uint32_t>(r.seg), r.index_offset,
                        static_cast<uint32_t*>(r.temp), LdsSegments{});
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  return CPN_OK;
+}
+
+// ---- requests of few keys: pieces merged by rank -----------------------------------------
+template <typename KeyT, int CODEC, bool HAS_IDX>
+int sort_rows_ranked(const SortRequest& r, uint64_t piece)
+{
+  const uint64_t n = r.seg, rows = r.volume / n, pieces = (n + piece - 1) / piece;
+  uint8_t* ws  = static_cast<uint8_t*>(r.temp) + HEADER_BYTES;
+  KeyT* keys   = reinterpret_cast<KeyT*>(ws);
+  int64_t* idx = HAS_IDX ? reinterpret_cast<int64_t*>(ws + align_up(r.volume * sizeof(KeyT), WORKSPACE_ALIGN)) : nullptr;
+  SortRequest c = r;
+  c.values_out  = keys;
+  c.indices_out = idx;
+  c.seg         = piece;
+  c.volume      = rows * piece;
+  c.row_stride  = n;
+  c.pieces      = static_cast<uint32_t>(pieces);
+  c.last_seg    = static_cast<uint32_t>(n - (pieces - 1) * piece);
+  int rc;
+  if (piece <= 4096) {
+    rc = launch_lds_rows<KeyT, CODEC, HAS_IDX, 512, 8>(c);
+  } else if constexpr (sizeof(KeyT) == 8 && HAS_IDX) {
+    rc = launch_lds_rows<KeyT, CODEC, HAS_IDX, 1024, 8>(c);
+  } else {
+    rc = launch_lds_rows<KeyT, CODEC, HAS_IDX, 512, 16>(c);
+  }
+  if (rc != CPN_OK) {
+    return rc;
+  }
+  const uint64_t chunks = (piece + RANK_CHUNK - 1) / RANK_CHUNK;
+  {
+    ProfileScope prof("merge_ranks", r.stream);
+    hipLaunchKernelGGL((merge_ranks_kernel<KeyT, CODEC, HAS_IDX>), dim3(static_cast<uint32_t>(rows * pieces * chunks)),
+                       dim3(RANK_CHUNK), 0, r.stream, keys, idx, static_cast<KeyT*>(r.values_out), r.indices_out,
+                       static_cast<uint32_t>(n), static_cast<uint32_t>(piece), static_cast<uint32_t>(pieces),
+                       static_cast<uint32_t>(chunks));
   }
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;
@@ -1159,6 +1236,12 @@ int sort_typed(const SortRequest& r)
   }
   if (r.temp == nullptr || r.temp_bytes < need || (reinterpret_cast<uintptr_t>(r.temp) % WORKSPACE_ALIGN) != 0) {
     return CPN_ERR_TEMP;
+  }
+  if constexpr ((KB == 4 || KB == 8) && KeyTraits<CODEC, KeyT>::NWORDS == 1) {
+    const uint64_t piece = ranked_row_piece(KB, PASSES, r.volume, r.seg, has_idx);
+    if (piece != 0 && r.temp_bytes >= ranked_workspace_bytes(KB, r.volume, has_idx)) {
+      return has_idx ? sort_rows_ranked<KeyT, CODEC, true>(r, piece) : sort_rows_ranked<KeyT, CODEC, false>(r, piece);
+    }
   }
   if (r.seg <= lds_row_limit(KB, has_idx)) {
     // one launch: the row kernels clear the status word of the workspace themselves.  (More rows than a

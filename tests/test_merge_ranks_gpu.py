@@ -1,0 +1,56 @@
+"""Requests of few keys whose sorted pieces are merged by rank in one launch (csrc/merge_rows.h), against the
+oracle, bit for bit: lengths at the ends of pieces, chunks and of the path itself, ties across pieces, rows whose
+pieces do not overlap or lie inside one another (windows of no key and of whole pieces), special values."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+from conftest import assert_same_bits, make_input
+from test_sort_gpu import abi_sort, lib, torch_cuda  # noqa: F401 (fixtures)
+
+from oracle import sort_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(lib, torch, x, what):
+    want_v = oracle.local_sort(x, argsort=False, threads=8)
+    want_i = oracle.local_sort(x, argsort=True, threads=8)
+    v, _ = abi_sort(lib, torch, x, want_values=True)
+    assert_same_bits(v, want_v, f"{what}: values")
+    _, i = abi_sort(lib, torch, x, want_values=False, want_indices=True, offset=3)
+    assert_same_bits(i, want_i + 3, f"{what}: positions")
+    v, i = abi_sort(lib, torch, x, want_values=True, want_indices=True, in_place=True)
+    assert_same_bits(v, want_v, f"{what}: in place")
+    assert_same_bits(i, want_i, f"{what}: in place, positions")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.uint64])
+@pytest.mark.parametrize("n", [8193, 12289, 16385, 40000, 40001, 80001, 100000, 131071, 212992, 262144])
+def test_lengths(lib, torch_cuda, dtype, n):
+    _check(lib, torch_cuda, make_input(dtype, (1, n), seed=n), f"{np.dtype(dtype)} {n}")
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.int32])
+def test_rows_and_arrangements(lib, torch_cuda, dtype):
+    n = 30_000
+    rng = np.random.default_rng(3)
+    rows = np.stack([
+        np.arange(n), np.arange(n)[::-1], np.full(n, 4), rng.integers(0, 3, n),
+        # one piece spread thinly over what the others hold densely, and the reverse
+        np.where(np.arange(n) < 4000, rng.integers(0, 1 << 30, n), rng.integers(5000, 6000, n)),
+        np.where(np.arange(n) < 4000, rng.integers(5000, 6000, n), rng.integers(0, 1 << 30, n)),
+        np.arange(n) // 300,
+    ]).astype(dtype)
+    _check(lib, torch_cuda, rows, f"{np.dtype(dtype)} arrangements")
+    _check(lib, torch_cuda, make_input(dtype, (3, 70_001), seed=9), f"{np.dtype(dtype)} three rows")
+
+
+def test_level_by_level_still_agrees(lib, torch_cuda):
+    """The other way of merging at lengths that the default no longer sends there."""
+    prev = lib.cpn_set_merge_rows(8)
+    try:
+        _check(lib, torch_cuda, make_input(np.float64, (2, 60_001), seed=5), "level by level")
+        _check(lib, torch_cuda, make_input(np.float32, (1, 33_000), seed=6), "level by level")
+    finally:
+        lib.cpn_set_merge_rows(prev)
