@@ -59,6 +59,9 @@ uint32_t lookback_spin_limit();
 #define CPN_LOOKBACK_WINDOW 4
 #endif
 constexpr int LOOKBACK_WINDOW = CPN_LOOKBACK_WINDOW;
+// In small tiles: many of them start at once, and none has a prefix yet (2 10^6 uint32 keys in tiles of 4096: 111 us
+// with windows of 4, 107 with 16; argsort of 10^6 int64 ids 124 -> 106).
+constexpr int LOOKBACK_WINDOW_SMALL = 16;
 
 // Status word values written by kernels into the workspace header.
 constexpr uint32_t DEVICE_ERR_LOOKBACK = 1u;
@@ -496,7 +499,8 @@ __global__ __launch_bounds__(SCAN_BLOCK) void histogram_scan_kernel(OffT* __rest
 
 // What the scatter passes leave undone: nothing ran (all keys of every row are equal: the
 // output is the input, the indices are 0..seg-1), or a single pass sorted in place into
-// scratch buffer 1 and its result still has to reach the caller's array.
+// scratch buffer 1 and its result still has to reach the caller's array.  (In small tiles the launch of the last
+// pass sees to the former, and this is launched for in-place requests only.)
 template <typename KeyT>
 __global__ __launch_bounds__(256) void finalize_kernel(const SortPlan* __restrict__ plan,
                                                         const KeyT* in,
@@ -568,6 +572,13 @@ struct SweepArgs {
   // is to run, has been done by a launch of its own in a shape that stages one byte per key (DONLY
   // below), and the launch of the pass itself has nothing left to do.
   uint32_t distinct_pass_done;
+  // Small tiles: the launch of the last pass gives the caller the input itself when no pass ran (all keys of every
+  // row equal, and not sorted by equalised digits).  A launch of its own that finds nothing to do takes 4.6 of the
+  // 91 us of 10^6 uint32 keys.  (In the kernels of large tiles, which have no register to spare, the same code made
+  // 2^24 float32 keys with positions 40 us slower.)
+  uint32_t finish;
+  uint64_t volume;
+  const EqualPlan* eq;
 };
 
 // ---- which tile a workgroup takes ----
@@ -629,6 +640,9 @@ __device__ __forceinline__ uint32_t claim_tile(uint32_t* xcd_tickets, uint32_t n
 #define CPN_ONESWEEP_WAVES_PER_EU 4
 #endif
 
+// The shapes of small_sweep_items.
+__host__ __device__ constexpr bool small_tile(bool big, int block, int items) { return !big && block == 512 && items <= 16; }
+
 // Bytes per key of the LDS staging area: the wider of key and row position; DONLY kernels stage one
 // byte per key (its digit) and the row positions.
 template <typename KeyT, typename OffT, bool HAS_IDX, bool DONLY>
@@ -684,6 +698,8 @@ __device__ __forceinline__ void onesweep_tile(
   constexpr int WAVES = BLOCK / WAVE;
   constexpr int TILE  = BLOCK * ITEMS;
   constexpr int WTILE = ITEMS * WAVE;  // keys of one wave, contiguous in the tile
+  constexpr bool SMALL = small_tile(BIG, BLOCK, ITEMS);
+  constexpr int WINDOW = SMALL ? LOOKBACK_WINDOW_SMALL : LOOKBACK_WINDOW;
   constexpr int DCODEC = XFORM ? static_cast<int>(CODEC_UNSIGNED) : CODEC;  // codec at digit extraction
 
   const int tid           = threadIdx.x;
@@ -801,7 +817,7 @@ __device__ __forceinline__ void onesweep_tile(
   // ---- per digit: start of every wave's keys, tile total, publish, first look-back reads:
   //      the answers travel while the tile is scattered into LDS ----
   uint32_t dsum = 0, dincl = 0;
-  OffT window[LOOKBACK_WINDOW];
+  OffT window[WINDOW];
   OffT* my_desc     = a.desc + static_cast<uint64_t>(tile) * RADIX + tid;
   const uint32_t t0 = tile - trow;  // first tile of the row, always published INCLUSIVE
   if (tid < RADIX) {
@@ -815,7 +831,7 @@ __device__ __forceinline__ void onesweep_tile(
     __hip_atomic_store(my_desc, static_cast<OffT>(first | dsum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (trow != 0) {
 #pragma unroll
-      for (int j = 0; j < LOOKBACK_WINDOW; ++j) {
+      for (int j = 0; j < WINDOW; ++j) {
         // tiles before the row start are replaced by the row's first tile (the sum stops there)
         const uint32_t t = (tile - 1 >= t0 + j) ? tile - 1 - j : t0;
         window[j] = __hip_atomic_load(a.desc + static_cast<uint64_t>(t) * RADIX + tid, __ATOMIC_RELAXED,
@@ -884,9 +900,45 @@ __device__ __forceinline__ void onesweep_tile(
       uint32_t hi = tile - 1;  // nearest predecessor not yet accounted for
       bool done   = false;
       bool failed = false;
-      while (true) {
+      // Small tiles: most of a window is not there yet at the first look.  What is there up to the first gap counts,
+      // and the window is read again from the gap on: polling the missing ones one after the other would take a
+      // round trip for each.
+      for (uint32_t spins = 0; SMALL;) {
+        bool gap       = false;
+        uint32_t taken = 0;
 #pragma unroll
-        for (int j = 0; j < LOOKBACK_WINDOW; ++j) {
+        for (int j = 0; j < WINDOW; ++j) {
+          const OffT w = window[j];
+          gap |= (w & DB::STATUS) == 0;
+          if (!gap && !done) {
+            before += (w & DB::VALUE);
+            done = (w & DB::INCLUSIVE) != 0;
+            ++taken;
+          }
+        }
+        if (done) {
+          break;
+        }
+        if (gap) {
+          spins = taken != 0 ? 1 : spins + 1;
+          if (spins >= a.spin_limit || ((spins & 255u) == 0 && __hip_atomic_load(a.status, __ATOMIC_RELAXED,
+                                                                                 __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+            failed = true;  // (or another tile gave up: drain quickly)
+            break;
+          }
+          __builtin_amdgcn_s_sleep(2);
+        }
+        hi = (hi >= t0 + taken) ? hi - taken : t0;
+#pragma unroll
+        for (int j = 0; j < WINDOW; ++j) {
+          const uint32_t t = (hi >= t0 + j) ? hi - j : t0;
+          window[j]        = __hip_atomic_load(a.desc + static_cast<uint64_t>(t) * RADIX + tid, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      while (!SMALL) {
+#pragma unroll
+        for (int j = 0; j < WINDOW; ++j) {
           if (!done) {
             OffT w = window[j];
             if ((w & DB::STATUS) == 0) {
@@ -920,9 +972,9 @@ __device__ __forceinline__ void onesweep_tile(
         if (done) {
           break;
         }
-        hi = (hi >= t0 + LOOKBACK_WINDOW) ? hi - LOOKBACK_WINDOW : t0;
+        hi = (hi >= t0 + WINDOW) ? hi - WINDOW : t0;
 #pragma unroll
-        for (int j = 0; j < LOOKBACK_WINDOW; ++j) {
+        for (int j = 0; j < WINDOW; ++j) {
           const uint32_t t = (hi >= t0 + j) ? hi - j : t0;
           window[j] = __hip_atomic_load(a.desc + static_cast<uint64_t>(t) * RADIX + tid, __ATOMIC_RELAXED,
                                         __HIP_MEMORY_SCOPE_AGENT);
@@ -1063,8 +1115,24 @@ void onesweep_kernel(const SweepArgs<BIG> a_in)
   uint64_t voffsets = 0;
 
   const PassPlan pp = a_in.plan->pass[a_in.pass];
-  if (pp.active == 0) {
-    return;  // every key of every row has the same digit here
+  if (pp.active == 0) {  // every key of every row has the same digit here
+    if constexpr (small_tile(BIG, BLOCK, ITEMS)) {
+      if (a_in.finish != 0 && a_in.plan->n_active == 0 && !eq_sorted(a_in.eq)) {
+        const KeyT* in        = static_cast<const KeyT*>(a_in.key_buf[KEY_IN]);
+        KeyT* out             = static_cast<KeyT*>(const_cast<void*>(a_in.key_buf[KEY_OUT]));
+        int64_t* positions    = HAS_IDX ? static_cast<int64_t*>(a_in.idx_buf[IDX_FINAL]) : nullptr;
+        const uint64_t stride = static_cast<uint64_t>(gridDim.x) * BLOCK;
+        for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * BLOCK + threadIdx.x; i < a_in.volume; i += stride) {
+          if (out != nullptr && out != in) {
+            out[i] = in[i];
+          }
+          if (positions != nullptr) {
+            positions[i] = static_cast<int64_t>(i % a_in.seg) + a_in.index_offset;
+          }
+        }
+      }
+    }
+    return;
   }
   if constexpr (VIRT) {
     // the index-only pass on the ranks of the row's different keys belongs to the DONLY launch,

@@ -99,6 +99,24 @@ __host__ __device__ constexpr int global_tile(int key_bytes, bool big)
   return global_block(key_bytes) * global_items(key_bytes, big);
 }
 
+// Requests that leave compute units without a tile of that size take smaller ones, real keys of 4 and 8 bytes:
+// 512 threads with 8 or 16 keys each.  Returns the keys per thread, 0: the tiles above.  A smaller tile shortens a
+// pass until the look-back over more of them, and the shorter runs they write, take longer.
+// Where the lines lie (us per call through the Python API, normal float keys; tiles above / 16 per thread / 8):
+//   4 bytes, sort     300 000 84, 69, 62;  600 000 86, 71, 71;  10^6 90, 80, 82;  2 10^6 102, 95, 111;  4 10^6 119, 124
+//   4 bytes, argsort  300 000 99, 78, 67;  600 000 111, 80, 79;  10^6 105, 90, 90;  2 10^6 117, 103, 116;  4 10^6 133, 135
+//   8 bytes, argsort  600 000 192, 173, 161;  10^6 203, 189, 180;  1.5 10^6 215, 196, 210;  2 10^6 219, 208, 231;
+//                     3 10^6 234, 257;  sort 1.5 10^6 198, 188, 203;  2 10^6 208, 201, 222;  3 10^6 212, 232
+constexpr int SMALL_BLOCK = 512;
+inline int small_sweep_items(int key_bytes, int passes, uint64_t volume)
+{
+  if ((key_bytes != 4 && key_bytes != 8) || passes != key_bytes) {
+    return 0;
+  }
+  const uint64_t eight = key_bytes == 4 ? 3ull << 18 : 1ull << 20, sixteen = key_bytes == 4 ? 5ull << 19 : 1ull << 21;
+  return volume <= eight ? 8 : (volume <= sixteen ? 16 : 0);
+}
+
 // Longest row the LDS kernel can take, per key width: 1024 threads with the row, the staged row
 // positions of an argsort (2 bytes each) and 16 KiB of per-wave digit counters in the CU's 160 KiB
 // of LDS.  Keys of up to 4 bytes: 16 per thread (64 + 32 + 16 KiB).  8-byte keys: 16 per thread for
@@ -261,6 +279,7 @@ struct GlobalLayout {
   uint64_t off_virt;
   int passes;
   uint64_t rows;
+  int small_items;    // keys per thread where the request takes small tiles, otherwise 0
   uint32_t tiles_per_row;
   uint64_t num_tiles;
   uint64_t off_hist, hist_bytes;
@@ -273,29 +292,33 @@ struct GlobalLayout {
   // ([off_eq, off_eq + eq_zero_bytes) is cleared), then the pieces for the LDS sort.  Behind everything else: a
   // workspace that ends at `total` is enough to sort without them.
   bool eq;
-  uint32_t eq_segments;
+  uint32_t eq_segments, eq_tiles;
+  uint64_t eq_desc_bytes;  // of a pass
   uint64_t off_eq, off_eq_tickets, off_eq_hist, off_eq_desc, eq_zero_bytes, off_eq_sample, off_eq_segs, off_eq_large, eq_total;
   bool valid;
 };
 
 inline GlobalLayout global_layout(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_values,
-                                  bool want_indices, bool in_place)
+                                  bool want_indices, bool in_place, bool small_tiles)
 {
   GlobalLayout L{};
   L.big           = seg >= wide_row_threshold();
   L.passes        = passes;
   L.rows          = volume / seg;
-  const uint64_t tile = static_cast<uint64_t>(global_tile(key_bytes, L.big));
-  const uint64_t tpr  = (seg + tile - 1) / tile;
-  L.num_tiles         = tpr * L.rows;
-  L.valid             = (tpr < (1ull << 32)) && (L.num_tiles < (1ull << 32));
-  L.tiles_per_row     = static_cast<uint32_t>(tpr);
-  const uint64_t ow   = L.big ? 8 : 4;
   // virtual digits: one long row of real 8-byte keys.  Their extra launches (three small kernels
   // and one early-exiting twin per pass, about 10 us each at this grid size) cost a 2^28-key sort
   // of 4-byte keys 2 %, more than four passes can win back on average; eight passes can.
   L.virt     = (L.rows == 1) && !L.big && (key_bytes == 8) && (passes == key_bytes) && (seg >= virtual_digit_threshold());
   L.off_virt = L.virt ? HEADER_BYTES : 0;
+  L.eq       = L.rows == 1 && !L.big && key_bytes == 8 && passes == key_bytes && seg >= equal_digit_threshold() &&
+         seg >= EQ_RANGE_SAMPLE && seg <= EQ_MAX_ROW_ELEMENTS;
+  L.small_items = (small_tiles && !L.big && !L.virt) ? small_sweep_items(key_bytes, passes, volume) : 0;
+  const uint64_t tile = static_cast<uint64_t>(L.small_items != 0 ? SMALL_BLOCK * L.small_items : global_tile(key_bytes, L.big));
+  const uint64_t tpr  = (seg + tile - 1) / tile;
+  L.num_tiles         = tpr * L.rows;
+  L.valid             = (tpr < (1ull << 32)) && (L.num_tiles < (1ull << 32));
+  L.tiles_per_row     = static_cast<uint32_t>(tpr);
+  const uint64_t ow   = L.big ? 8 : 4;
   L.off_hist          = HEADER_BYTES + (L.virt ? VIRT_WORKSPACE_BYTES : 0);
   L.hist_bytes        = align_up(L.rows * L.passes * RADIX * ow, WORKSPACE_ALIGN);
   L.off_desc          = L.off_hist + L.hist_bytes;
@@ -329,15 +352,15 @@ inline GlobalLayout global_layout(int key_bytes, int passes, uint64_t volume, ui
     off += L.idx_bytes_total;
   }
   L.total = off;
-  L.eq    = L.rows == 1 && !L.big && key_bytes == 8 && passes == key_bytes && seg >= equal_digit_threshold() &&
-         seg >= EQ_RANGE_SAMPLE && seg <= EQ_MAX_ROW_ELEMENTS;
   L.eq_total = L.total;
   if (L.eq) {
     L.off_eq         = off;
     L.off_eq_tickets = align_up(L.off_eq + sizeof(EqualPlan), WORKSPACE_ALIGN);
     L.off_eq_hist    = L.off_eq_tickets + WORKSPACE_ALIGN;
     L.off_eq_desc    = L.off_eq_hist + align_up(2 * RADIX * sizeof(uint32_t), WORKSPACE_ALIGN);
-    L.eq_zero_bytes  = L.off_eq_desc + 2 * L.desc_bytes_per_pass - L.off_eq;
+    L.eq_tiles       = static_cast<uint32_t>((seg + global_tile(key_bytes, false) - 1) / global_tile(key_bytes, false));
+    L.eq_desc_bytes  = align_up(static_cast<uint64_t>(L.eq_tiles) * RADIX * sizeof(uint32_t), WORKSPACE_ALIGN);
+    L.eq_zero_bytes  = L.off_eq_desc + 2 * L.eq_desc_bytes - L.off_eq;
     L.eq_segments    = static_cast<uint32_t>((seg + EQ_SORT_STRIDE - 1) / EQ_SORT_STRIDE);
     L.off_eq_sample  = L.off_eq + L.eq_zero_bytes;
     L.off_eq_segs    = L.off_eq_sample + static_cast<uint64_t>(2 * EQ_GATHER_GRID + EQ_SAMPLE) * key_bytes;
@@ -372,7 +395,7 @@ inline uint64_t workspace_bytes(int key_bytes, int passes, uint64_t volume, uint
       align_up(volume * key_bytes, WORKSPACE_ALIGN) + (want_indices ? align_up(volume * 8, WORKSPACE_ALIGN) : 0);
     return HEADER_BYTES + merged_row_split_bytes(volume, seg, levels) + (levels >= 2 ? 2 : 1) * copy;
   }
-  const GlobalLayout L = global_layout(key_bytes, passes, volume, seg, want_values, want_indices, in_place);
+  const GlobalLayout L = global_layout(key_bytes, passes, volume, seg, want_values, want_indices, in_place, !least);
   return L.valid ? (least ? L.total : L.eq_total) : 0;
 }
 
@@ -902,19 +925,19 @@ inline int sort_equalised(const SortRequest& r, const GlobalLayout& L, EqualPlan
     a.ticket          = tickets + p;
     a.xcd_tickets     = tickets + 8 + p * XCD_COUNT;
     a.hist_excl       = hist + p * RADIX;
-    a.desc            = reinterpret_cast<uint32_t*>(ws + L.off_eq_desc + L.desc_bytes_per_pass * p);
+    a.desc            = reinterpret_cast<uint32_t*>(ws + L.off_eq_desc + L.eq_desc_bytes * p);
     a.status          = status;
     a.seg             = r.seg;
     a.hist_row_stride = 2 * RADIX;
-    a.tiles_per_row   = L.tiles_per_row;
-    a.num_tiles       = static_cast<uint32_t>(L.num_tiles);
+    a.tiles_per_row   = L.eq_tiles;
+    a.num_tiles       = L.eq_tiles;
     a.pass            = p;
     a.spin_limit      = lookback_spin_limit();
     a.single_ticket   = (r.single_ticket || tile_order_single()) ? 1u : 0u;
     a.free_rank       = (p == 0 && rq.free_rank != 0) ? 1 : 0;
     ProfileScope prof("equal_sweep", r.stream);
     hipLaunchKernelGGL((eq_sweep_kernel<KeyT, CODEC, HAS_IDX, global_block(KB), global_items(KB, false)>),
-                       dim3(static_cast<uint32_t>(L.num_tiles)), dim3(global_block(KB)), 0, r.stream, a, eq,
+                       dim3(L.eq_tiles), dim3(global_block(KB)), 0, r.stream, a, eq,
                        SPECIALS ? static_cast<const uint32_t*>(specials) : static_cast<const uint32_t*>(nullptr));
     CPN_HIP_TRY(hipGetLastError());
   }
@@ -952,6 +975,31 @@ inline int sort_equalised(const SortRequest& r, const GlobalLayout& L, EqualPlan
   return CPN_OK;
 }
 
+// A pass in small tiles.
+template <typename KeyT, int CODEC, bool HAS_IDX, bool CAN_ORDER_KEYS>
+inline bool launch_small_sweep(const SweepArgs<false>& a, int items, bool ordered_keys, dim3 grid, hipStream_t stream)
+{
+  auto launch = [&](auto xform, auto count) {
+    hipLaunchKernelGGL((onesweep_kernel<KeyT, CODEC, decltype(xform)::value, false, HAS_IDX, SMALL_BLOCK, decltype(count)::value>),
+                       grid, dim3(SMALL_BLOCK), 0, stream, a);
+  };
+  auto shape = [&](auto xform) {
+    if (items == 8) {
+      launch(xform, std::integral_constant<int, 8>{});
+    } else {
+      launch(xform, std::integral_constant<int, 16>{});
+    }
+  };
+  if constexpr (CAN_ORDER_KEYS) {
+    if (ordered_keys) {
+      shape(std::true_type{});
+      return true;
+    }
+  }
+  shape(std::false_type{});
+  return true;
+}
+
 template <typename KeyT, int CODEC, bool BIG, bool HAS_IDX>
 inline int sort_global(const SortRequest& r, const GlobalLayout& L)
 {
@@ -985,6 +1033,7 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   uint32_t* tickets = reinterpret_cast<uint32_t*>(ws + HEADER_TICKETS);
   uint32_t* varying = reinterpret_cast<uint32_t*>(ws + HEADER_VARYING);
   SortPlan* plan    = reinterpret_cast<SortPlan*>(ws + HEADER_PLAN);
+  constexpr bool SMALL_OK = !BIG && (KB == 4 || KB == 8) && KeyTraits<CODEC, KeyT>::PASSES == KB;
   constexpr bool VIRT_OK = !BIG && KB == 8 && KeyTraits<CODEC, KeyT>::PASSES == KB;
   VirtPlan* vplan   = L.virt ? reinterpret_cast<VirtPlan*>(ws + L.off_virt) : nullptr;
   DistinctTable* dtable = L.virt ? reinterpret_cast<DistinctTable*>(ws + L.off_virt + VIRT_PLAN_BYTES) : nullptr;
@@ -1132,6 +1181,7 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   // whose one workgroup per CU runs its phases one after the other.
   constexpr bool DISTINCT_SPECIAL = VIRT_OK && HAS_IDX && global_block(KB) * global_items(KB, BIG) == 512 * 32;
   const bool distinct_special     = DISTINCT_SPECIAL && L.virt && !want_vals;
+  const bool last_pass_finishes   = L.small_items != 0 && !(in_place && want_vals);
   auto pass_args = [&](int p) {
     SweepArgs<BIG> a{};
     a.key_buf[KEY_IN]    = r.values_in;
@@ -1159,6 +1209,9 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
     a.vplan              = vplan;
     a.dtable             = dtable;
     a.distinct_pass_done = distinct_special ? 1u : 0u;
+    a.volume             = r.volume;
+    a.finish             = (last_pass_finishes && p == PASSES - 1) ? 1u : 0u;
+    a.eq                 = eq;
     return a;
   };
   if constexpr (DISTINCT_SPECIAL) {
@@ -1178,6 +1231,11 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
       // requests that may run on virtual digits get the kernel that can do both (the device-side
       // plan decides); everything else the plain one
       bool launched = false;
+      if constexpr (SMALL_OK) {
+        if (L.small_items != 0) {
+          launched = launch_small_sweep<KeyT, CODEC, HAS_IDX, CAN_ORDER_KEYS>(a, L.small_items, ordered_keys, grid, r.stream);
+        }
+      }
       if constexpr (VIRT_OK) {
         if (L.virt) {
           if constexpr (CAN_ORDER_KEYS) {
@@ -1208,7 +1266,7 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
     }
     CPN_HIP_TRY(hipGetLastError());
   }
-  {
+  if (!last_pass_finishes) {
     uint64_t blocks = (r.volume + 1023) / 1024;
     if (blocks > 8192) {
       blocks = 8192;
@@ -1267,7 +1325,10 @@ int sort_typed(const SortRequest& r)
       return has_idx ? sort_rows_merged<KeyT, CODEC, true>(r, levels) : sort_rows_merged<KeyT, CODEC, false>(r, levels);
     }
   }
-  const GlobalLayout L = global_layout(KB, PASSES, r.volume, r.seg, r.values_out != nullptr, has_idx, in_place);
+  GlobalLayout L = global_layout(KB, PASSES, r.volume, r.seg, r.values_out != nullptr, has_idx, in_place, true);
+  if (L.small_items != 0 && r.temp_bytes < L.total) {  // (small tiles have more descriptors)
+    L = global_layout(KB, PASSES, r.volume, r.seg, r.values_out != nullptr, has_idx, in_place, false);
+  }
   if (L.big) {
     return has_idx ? sort_global<KeyT, CODEC, true, true>(r, L) : sort_global<KeyT, CODEC, true, false>(r, L);
   }
