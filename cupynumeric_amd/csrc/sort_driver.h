@@ -99,7 +99,8 @@ __host__ __device__ constexpr int global_tile(int key_bytes, bool big)
   return global_block(key_bytes) * global_items(key_bytes, big);
 }
 
-// Requests that leave compute units without a tile of that size take smaller ones, real keys of 4 and 8 bytes:
+// Single rows that leave compute units without a tile of that size take smaller ones, real keys of 4 and 8 bytes
+// (several rows, whose look-back is short anyway, keep the tiles above: the lines below are those of one row):
 // 512 threads with 8 or 16 keys each.  Returns the keys per thread, 0: the tiles above.  A smaller tile shortens a
 // pass until the look-back over more of them, and the shorter runs they write, take longer.
 // Where the lines lie (us per call through the Python API, normal float keys; tiles above / 16 per thread / 8):
@@ -312,7 +313,7 @@ inline GlobalLayout global_layout(int key_bytes, int passes, uint64_t volume, ui
   L.off_virt = L.virt ? HEADER_BYTES : 0;
   L.eq       = L.rows == 1 && !L.big && key_bytes == 8 && passes == key_bytes && seg >= equal_digit_threshold() &&
          seg >= EQ_RANGE_SAMPLE && seg <= EQ_MAX_ROW_ELEMENTS;
-  L.small_items = (small_tiles && !L.big && !L.virt) ? small_sweep_items(key_bytes, passes, volume) : 0;
+  L.small_items = (small_tiles && L.rows == 1 && !L.big && !L.virt) ? small_sweep_items(key_bytes, passes, volume) : 0;
   const uint64_t tile = static_cast<uint64_t>(L.small_items != 0 ? SMALL_BLOCK * L.small_items : global_tile(key_bytes, L.big));
   const uint64_t tpr  = (seg + tile - 1) / tile;
   L.num_tiles         = tpr * L.rows;

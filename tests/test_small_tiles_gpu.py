@@ -46,7 +46,7 @@ def test_lengths(lib, torch_cuda, dtype, n):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.int64])
 def test_rows(lib, torch_cuda, dtype):
-    """The look-back stops at the row's first tile."""
+    """Several rows keep the large tiles."""
     _check(lib, torch_cuda, make_input(dtype, (5, 70_001), seed=3), f"{np.dtype(dtype)} five rows")
 
 
