@@ -129,6 +129,11 @@ struct LdsSegments {
   const uint32_t* pos;
   const EqualPlan* eq;
 };
+struct NoSegments {};
+// Nothing of this may reach the row kernels: their loop is a `do ... while` that clang drops, since its condition is
+// false by itself.  As a `for` over a single entry it gave 512 x 24, plain float32, 131 registers instead of 128, so
+// one workgroup per CU instead of two, and 2^26 keys in rows of 8193 took 0.83 ms instead of 0.45; the body as an
+// inlined function of two kernels makes 1024 x 16 spill and costs most 8-byte shapes a wave.
 template <typename KeyT, int CODEC, bool HAS_IDX, int BLOCK, int ITEMS, bool SEGMENTS = false>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(lds_row_waves_per_simd(BLOCK, ITEMS, sizeof(KeyT)))))
 void lds_row_sort_kernel(const KeyT* keys_in,
@@ -140,14 +145,18 @@ void lds_row_sort_kernel(const KeyT* keys_in,
                                                               uint32_t last_piece_len,
                                                               int64_t index_offset,
                                                               uint32_t* status,
-                                                              const LdsSegments sg)
+                                                              const typename std::conditional<SEGMENTS, LdsSegments, NoSegments>::type sg)
 {
-  uint32_t n_pieces = 1;  // SEGMENTS: on the list
+  uint32_t entry = 0, entries = 0;  // SEGMENTS: of the list
   if constexpr (SEGMENTS) {
     if (sg.eq->mode == 0 || *status != 0) {
       return;
     }
-    n_pieces = sg.eq->n_list < sg.max_segs ? sg.eq->n_list : sg.max_segs;
+    entry   = blockIdx.x;
+    entries = sg.eq->n_list < sg.max_segs ? sg.eq->n_list : sg.max_segs;
+    if (entry >= entries) {
+      return;
+    }
   } else if (blockIdx.x == 0 && threadIdx.x == 0) {
     *status = 0;  // the workspace's status word: a per-row sort cannot fail on the device
   }
@@ -190,7 +199,7 @@ void lds_row_sort_kernel(const KeyT* keys_in,
   __shared__ uint32_t s_wsum[DT::WAVES];
   __shared__ SW s_red[2 * WAVES * NW];
 
-  for (uint32_t entry = SEGMENTS ? blockIdx.x : 0u; entry < n_pieces; entry += SEGMENTS ? gridDim.x : 1u) {
+  do {
   int tid = threadIdx.x;
   if constexpr (SEGMENTS) {
     asm volatile("" : "+v"(tid));  // (or every address below is worked out ahead of the loop, and spilled)
@@ -843,8 +852,9 @@ void lds_row_sort_kernel(const KeyT* keys_in,
   }
   if constexpr (SEGMENTS) {
     __syncthreads();  // the next piece reuses the shared memory
+    entry += gridDim.x;
   }
-  }
+  } while (SEGMENTS && entry < entries);
 }
 
 }  // namespace cpn

@@ -490,7 +490,7 @@ inline int launch_lds_rows(const SortRequest& r)
                        static_cast<const KeyT*>(r.values_in), static_cast<KeyT*>(r.values_out), r.indices_out,
                        static_cast<uint32_t>(r.seg), r.row_stride != 0 ? r.row_stride : r.seg, r.pieces,
                        r.pieces > 1 ? r.last_seg : static_cast<uint32_t>(r.seg), r.index_offset,
-                       static_cast<uint32_t*>(r.temp), LdsSegments{});
+                       static_cast<uint32_t*>(r.temp), NoSegments{});
   }
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;

@@ -293,6 +293,29 @@ def test_built_row_kernels_do_not_spill():
     assert seen_row_kernels > 100  # the row kernels of five key widths were all looked at
 
 
+# Waves per SIMD that shapes of the row kernel were chosen for: mangled key type, codec and positions, threads, keys
+# per thread.  (4 in the first: two workgroups of 512 threads per CU.)
+ROW_KERNEL_WAVES = [("jLi2ELb0", 512, 24, 4), ("jLi2ELb1", 256, 8, 7), ("jLi0ELb1", 64, 4, 8), ("jLi1ELb1", 64, 4, 8),
+                    ("jLi0ELb1", 128, 8, 8), ("jLi0ELb1", 128, 12, 5), ("jLi1ELb1", 128, 12, 5),
+                    ("mLi0ELb0", 64, 4, 8), ("mLi1ELb0", 64, 4, 8), ("mLi1ELb0", 512, 16, 4), ("mLi2ELb0", 64, 8, 5)]
+
+
+@pytest.mark.parametrize("key,block,items,waves", ROW_KERNEL_WAVES)
+def test_built_row_kernels_keep_their_waves(key, block, items, waves):
+    """A row kernel with a few registers more loses a workgroup per CU without failing any other test."""
+    import json
+
+    from cupynumeric_amd import build as B
+
+    reports = sorted(B.OBJ_DIR.glob("sort_keys*.resources.json"))
+    if not reports:
+        pytest.skip("no build reports in this tree")
+    pattern = f"19lds_row_sort_kernelI{key}ELi{block}ELi{items}E"
+    found = [use["waves_per_simd"] for r in reports for kernel, use in json.loads(r.read_text()).items() if pattern in kernel]
+    assert found, pattern
+    assert min(found) >= waves, (pattern, found)
+
+
 def test_setter_between_size_query_and_sort_is_refused(lib):
     """A test hook that enlarges the workspace a request needs, called between the size query and the
     sort: the sort works the size out again and returns CPN_ERR_TEMP before it launches anything (the
