@@ -1013,7 +1013,7 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   const bool in_place  = (r.values_out == r.values_in);
   const bool want_vals = (r.values_out != nullptr);
 
-  constexpr bool EQ_OK = !BIG && KB == 8 && KeyTraits<CODEC, KeyT>::PASSES == KB;
+  constexpr bool EQ_OK = eq_keys<KeyT, CODEC, OffT>();
   const bool use_eq    = EQ_OK && L.eq && r.temp_bytes >= L.eq_total;
   EqualPlan* eq        = use_eq ? reinterpret_cast<EqualPlan*>(ws + L.off_eq) : nullptr;
   if constexpr (EQ_OK) {

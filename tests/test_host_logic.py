@@ -300,6 +300,22 @@ ROW_KERNEL_WAVES = [("jLi2ELb0", 512, 24, 4), ("jLi2ELb1", 256, 8, 7), ("jLi0ELb
                     ("mLi0ELb0", 64, 4, 8), ("mLi1ELb0", 64, 4, 8), ("mLi1ELb0", 512, 16, 4), ("mLi2ELb0", 64, 8, 5)]
 
 
+@pytest.mark.parametrize("offsets", ["j", "m"])
+@pytest.mark.parametrize("specials", [0, 1])
+def test_built_float16_histogram_keeps_its_waves(offsets, specials):
+    """(It was chosen for 64 registers: 8 waves per SIMD.)"""
+    import json
+
+    from cupynumeric_amd import build as B
+
+    report = B.OBJ_DIR / "sort_keys16.resources.json"
+    if not report.exists():
+        pytest.skip("no build reports in this tree")
+    pattern = f"16histogram_kernelItLi2E{offsets}Lb{specials}E"
+    found = [use["waves_per_simd"] for kernel, use in json.loads(report.read_text()).items() if pattern in kernel]
+    assert found and min(found) >= 8, (pattern, found)
+
+
 @pytest.mark.parametrize("key,block,items,waves", ROW_KERNEL_WAVES)
 def test_built_row_kernels_keep_their_waves(key, block, items, waves):
     """A row kernel with a few registers more loses a workgroup per CU without failing any other test."""
