@@ -246,6 +246,15 @@ constexpr int RANK_MAX_PIECES = 64;
 constexpr uint32_t RANK_STAGE = 8192;
 constexpr int RANK_LOADS      = 8;
 constexpr int RANK_ILP        = 4;  // pieces searched at once by a thread
+// When the windows fill RANK_STAGE keys more often than this, those of more than RANK_WIDE keys are searched where they
+// lie.  Where pieces are unlike (their values drift, or change halfway), neighbouring keys of one can have most of
+// another between them, and a workgroup that copied all of that took as long as there was to copy: 262 144 float32
+// keys, 8192 of them spread over the narrow range of the others, 366 us, now 68 (level by level: 88); the second half
+// in a thousandth of the range of the first, 242 and 66 (88).  (Fewer keys are copied sooner than searched: a random walk
+// of 9000 float64 keys, three pieces, 26 us against 32.)
+constexpr uint32_t RANK_MAX_STAGES = 2;
+constexpr uint32_t RANK_WIDE       = 4 * RANK_CHUNK;
+constexpr int RANK_WIDE_ILP        = 8;  // windows searched at once
 
 // keys / idx: the rows, [rows][n], in sorted pieces of `piece` elements (the last one of a row may be shorter); idx
 // holds row positions.  Outputs may not alias them.  Grid: rows x pieces x chunks workgroups of RANK_CHUNK threads.
@@ -262,7 +271,8 @@ __global__ __launch_bounds__(RANK_CHUNK) void merge_ranks_kernel(const KeyT* __r
   static_assert(2 * RANK_MAX_PIECES <= RANK_CHUNK, "a thread per end of a window");
   __shared__ KeyT s_keys[RANK_STAGE];                  // ordered images
   __shared__ uint32_t s_end[2][RANK_MAX_PIECES + RANK_ILP];  // of every piece: keys before the chunk's first / last key
-  __shared__ uint32_t s_at[RANK_MAX_PIECES + 1];       // where its window starts, all windows one after the other
+  __shared__ uint32_t s_at[RANK_MAX_PIECES + 1];       // where its window starts, all copied ones one after the other
+  __shared__ uint32_t s_wide;                          // is any window searched in memory?
   const uint32_t tid  = threadIdx.x;
   const uint32_t lane = tid % WAVE, wave = tid / WAVE;
   const uint32_t per_row = pieces * chunks;
@@ -316,18 +326,22 @@ __global__ __launch_bounds__(RANK_CHUNK) void merge_ranks_kernel(const KeyT* __r
   // and some of the window
   uint32_t rank = first + tid;
   if (wave == 0) {
-    uint32_t run = 0;
-    for (uint32_t j0 = 0; j0 < pieces; j0 += WAVE) {
-      const uint32_t j    = j0 + lane;
-      const uint32_t s    = j < pieces ? s_end[1][j] - s_end[0][j] : 0u;
-      const uint32_t incl = wave_inclusive_sum_dpp(s);
-      if (j < pieces) {
-        s_at[j] = run + incl - s;
-      }
-      run += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), WAVE - 1));
+    static_assert(RANK_MAX_PIECES <= WAVE, "a lane per piece");
+    const uint32_t window = lane < pieces ? s_end[1][lane] - s_end[0][lane] : 0u;
+    const uint32_t sum    = wave_inclusive_sum_dpp(window);
+    const uint32_t all    = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(sum), WAVE - 1));
+    const bool in_memory  = all > RANK_MAX_STAGES * RANK_STAGE && window > RANK_WIDE;
+    const uint32_t copied = in_memory ? 0u : window;
+    const uint32_t incl   = wave_inclusive_sum_dpp(copied);
+    if (lane < pieces) {
+      s_at[lane] = incl - copied;
     }
+    if (lane == WAVE - 1) {
+      s_at[pieces] = incl;
+    }
+    const uint64_t wide = __ballot(in_memory);
     if (lane == 0) {
-      s_at[pieces] = run;
+      s_wide = wide != 0 ? 1u : 0u;
     }
   }
   __syncthreads();
@@ -391,6 +405,39 @@ __global__ __launch_bounds__(RANK_CHUNK) void merge_ranks_kernel(const KeyT* __r
       }
     }
     __syncthreads();
+  }
+  if (s_wide != 0) {
+    for (uint32_t j0 = 0; j0 < pieces; j0 += RANK_WIDE_ILP) {
+      uint32_t at[RANK_WIDE_ILP], len[RANK_WIDE_ILP], found[RANK_WIDE_ILP], most = 0;
+#pragma unroll
+      for (int k = 0; k < RANK_WIDE_ILP; ++k) {
+        const uint32_t j = j0 + k < pieces ? j0 + k : pieces - 1;
+        const uint32_t s = s_end[1][j] - s_end[0][j];
+        at[k]            = j * piece + s_end[0][j];  // (n < 2^32)
+        len[k]           = (j0 + k < pieces && s_at[j + 1] == s_at[j]) ? s : 0u;  // (none of it copied)
+        found[k]         = 0;
+        most             = len[k] > most ? len[k] : most;
+      }
+      if (most == 0) {
+        continue;  // uniform
+      }
+      for (uint32_t step = 1u << (31 - __builtin_clz(most)); step != 0; step >>= 1) {
+        KeyT other[RANK_WIDE_ILP];
+#pragma unroll
+        for (int k = 0; k < RANK_WIDE_ILP; ++k) {  // (all loads first; a place inside the row whatever is asked)
+          other[k] = row_keys[found[k] + step <= len[k] ? at[k] + found[k] + step - 1 : 0u];
+        }
+#pragma unroll
+        for (int k = 0; k < RANK_WIDE_ILP; ++k) {
+          const bool earlier = before(image(other[k]), key, j0 + k);
+          found[k]           = (found[k] + step <= len[k] && earlier) ? found[k] + step : found[k];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < RANK_WIDE_ILP; ++k) {
+        rank += found[k];
+      }
+    }
   }
   if (tid < count) {
     if (keys_out != nullptr) {

@@ -54,3 +54,50 @@ def test_level_by_level_still_agrees(lib, torch_cuda):
         _check(lib, torch_cuda, make_input(np.float32, (1, 33_000), seed=6), "level by level")
     finally:
         lib.cpn_set_merge_rows(prev)
+
+
+def _unlike(kind, n, rng):
+    x = rng.random(n)
+    if kind == "one piece wide":
+        x[8192:] = 0.5 + 1e-3 * x[8192:]
+    elif kind == "halves":
+        x[n // 2 :] = 0.5 + 1e-3 * x[n // 2 :]
+    elif kind == "ties":  # whole pieces of one value between two neighbouring keys of another
+        x[8192:] = 0.5
+        x[4000:4200] = 0.5
+    return x
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["one piece wide", "halves", "ties"])
+@pytest.mark.parametrize("n", [24_577, 40_001, 100_003, 212_991])
+def test_unlike_pieces(lib, torch_cuda, dtype, kind, n):
+    """Windows too wide for LDS are searched in memory: some of the pieces, nearly all, the short last one."""
+    x = _unlike(kind, n, np.random.default_rng(n)).astype(dtype)
+    _check(lib, torch_cuda, x.reshape(1, -1), f"{np.dtype(dtype)} {n} {kind}")
+
+
+def test_unlike_pieces_take_no_multiple_of_the_time(torch_cuda):
+    """A workgroup whose windows span the row once copied all of it: 5.4 times what evenly mixed keys take; now the same."""
+    import cupynumeric_amd as num
+
+    torch = torch_cuda
+    n = 262_144
+
+    def best(x):
+        a = num.array(x)
+        times = []
+        for _ in range(20):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(5):
+                num.sort(a)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    rng = np.random.default_rng(0)
+    even = best(rng.random(n).astype(np.float32))
+    for kind in ("one piece wide", "halves"):
+        assert best(_unlike(kind, n, rng).astype(np.float32)) < 2.2 * even, kind
