@@ -293,7 +293,7 @@ uint64_t cpn_local_sort_temp_bytes(int dtype, uint64_t volume, uint64_t sort_dim
   if (sort_dim_size == 0 || volume % sort_dim_size != 0) {
     return 0;
   }
-  return cpn::workspace_bytes(k.bytes, cpn::key_passes(k.bytes, k.codec), volume, sort_dim_size, want_values != 0, want_indices != 0, in_place != 0);
+  return cpn::workspace_bytes(k.bytes, cpn::key_passes(k.bytes, k.codec), k.codec, volume, sort_dim_size, want_values != 0, want_indices != 0, in_place != 0);
 }
 
 int cpn_local_sort(int dtype, const void* values_in, void* values_out, int64_t* indices_out, uint64_t volume,
@@ -364,7 +364,7 @@ int cpn_local_sort_static(int dtype, const void* values_in, void* values_out, in
   if (k.bytes != 0 && k.codec >= 0 && volume != 0 && sort_dim_size != 0 && volume % sort_dim_size == 0) {
     // a well-formed request: does its workspace fit?  (everything else gets cpn_local_sort's own answer)
     const uint64_t need =
-      cpn::workspace_bytes(k.bytes, cpn::key_passes(k.bytes, k.codec), volume, sort_dim_size, values_out != nullptr,
+      cpn::workspace_bytes(k.bytes, cpn::key_passes(k.bytes, k.codec), k.codec, volume, sort_dim_size, values_out != nullptr,
                            indices_out != nullptr, values_out == values_in, /*least=*/true);
     if (need > CPN_STATIC_SCRATCH_BYTES) {
       return CPN_ERR_SCRATCH;

@@ -201,24 +201,37 @@ inline uint64_t merged_row_split_bytes(uint64_t volume, uint64_t seg, int levels
 // Requests of few keys, real keys of 4 and 8 bytes: rows cut into short pieces, all merged by rank in one launch
 // (merge_rows.h).  Returns the pieces' length, 0: another path.  (cpn_set_merge_rows: in the default mode only.)
 // Where the lines lie (us per call through the Python API, this way / the way it took before, sort and argsort):
-//   from where one workgroup per row is left: 14 000 uint32 23, 23 / 24, 24, float32 25, 25 / 34, 33, float64 26,
-//   28 / 46, 51; 8192 float64 26, 28 / 27, 21.  (Only single rows of up to lds_row_capacity keys: the other way
-//   needs no workspace, and several rows keep as many workgroups busy.)
+//   from where one workgroup per row is left (RANK_MIN_ROW_*): normal float64 8193 keys 25, 26 / 24, 28, 10 000 25,
+//   27 / 29, 32, 12 289 26, 27 / 37, 43, uniform 24, 26 / 21, 23, 24, 26 / 23, 26 and 25, 26 / 29, 31, int64 23, 24 /
+//   20, 23, 23, 24 / 23, 26 and 24, 24 / 28, 31; normal float32 12 289 23, 24 / 29, 28, 14 000 23, 24 / 30, 31, 16 384
+//   24, 25 / 28, 34, int32 22, 23 / 21, 22, 23, 23 / 23, 23 and 23, 23 / 21, 25.  What this way loses: rows of equal
+//   keys, which one workgroup sees to without a pass (9000 float64 22 / 13).  (Only single rows of up to
+//   lds_row_capacity keys: the other way needs no workspace, and several rows keep as many workgroups busy.)
 //   to where the work, which grows with the square of the row, eats the launches saved: 262 144 uint32 68, 72 /
 //   86, 98, float32 75, 80 / 89, 99, 400 000 uint32 147, 152 / 86, 106; float64 200 000 104, 96 / 124, 132,
-//   262 144 127, 119 / 123, 131.
+//   262 144 127, 119 / 123, 131.  Levels of merging take 8-byte integers faster: 160 000 74, 73 / 75, 82, 200 000 89,
+//   87 / 83, 91, 230 000 argsort 103 / 92, 262 144 110 / 94.
 //   pieces of 4096 or 8192 keys: fewer pieces to search against a longer sort of each: 32 768 uint32 26, 26
 //   (4096) and 27, 31 (8192), 65 536 34, 35 and 31, 35, 131 072 56, 58 and 39, 44; float64 sort 65 536 40 and 47,
 //   131 072 65 and 59, argsort 32 768 33 and 38, 65 536 41 and 41, 131 072 67 and 51.
 constexpr uint64_t RANK_MAX_VOLUME = 1ull << 18;
+constexpr uint64_t RANK_MIN_ROW_4  = 13312;
+constexpr uint64_t RANK_MIN_ROW_8  = 10240;
 bool merge_rows_default();
-inline uint64_t ranked_row_piece(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_indices)
+inline uint64_t ranked_max_volume_8(int codec, bool want_indices)
+{
+  if (codec == CODEC_FLOAT) {
+    return want_indices ? RANK_MAX_VOLUME : 26 * 8192;
+  }
+  return want_indices ? 26 * 8192 : 20 * 8192;
+}
+inline uint64_t ranked_row_piece(int key_bytes, int passes, int codec, uint64_t volume, uint64_t seg, bool want_indices)
 {
   const uint64_t cap = lds_row_capacity(key_bytes, want_indices);
   if (!merge_rows_default() || (key_bytes != 4 && key_bytes != 8) || passes != key_bytes ||
       lds_row_limit(key_bytes, want_indices) != cap || volume > RANK_MAX_VOLUME ||
-      seg <= (key_bytes == 4 ? 12288u : 8192u) || (seg <= cap && volume != seg) ||
-      (key_bytes == 8 && !want_indices && volume > 26 * 8192)) {
+      seg <= (key_bytes == 4 ? RANK_MIN_ROW_4 : RANK_MIN_ROW_8) || (seg <= cap && volume != seg) ||
+      (key_bytes == 8 && volume > ranked_max_volume_8(codec, want_indices))) {
     return 0;
   }
   const uint64_t few    = key_bytes == 4 ? 40000 : (want_indices ? 40000 : 80000);
@@ -378,11 +391,11 @@ inline uint64_t ranked_workspace_bytes(int key_bytes, uint64_t volume, bool want
   return HEADER_BYTES + align_up(volume * key_bytes, WORKSPACE_ALIGN) + (want_indices ? align_up(volume * 8, WORKSPACE_ALIGN) : 0);
 }
 // What a sort asks for; with `least`, what it can do with.
-inline uint64_t workspace_bytes(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_values,
+inline uint64_t workspace_bytes(int key_bytes, int passes, int codec, uint64_t volume, uint64_t seg, bool want_values,
                                 bool want_indices, bool in_place, bool least = false)
 {
-  if (!least && volume != 0 && ranked_row_piece(key_bytes, passes, volume, seg, want_indices) != 0) {
-    const uint64_t own = workspace_bytes(key_bytes, passes, volume, seg, want_values, want_indices, in_place, true);
+  if (!least && volume != 0 && ranked_row_piece(key_bytes, passes, codec, volume, seg, want_indices) != 0) {
+    const uint64_t own = workspace_bytes(key_bytes, passes, codec, volume, seg, want_values, want_indices, in_place, true);
     const uint64_t all = ranked_workspace_bytes(key_bytes, volume, want_indices);
     return own > all ? own : all;
   }
@@ -1288,7 +1301,7 @@ int sort_typed(const SortRequest& r)
   constexpr int PASSES = KeyTraits<CODEC, KeyT>::PASSES;
   const bool has_idx   = (r.indices_out != nullptr);
   const bool in_place  = (r.values_out == r.values_in);
-  const uint64_t need  = workspace_bytes(KB, PASSES, r.volume, r.seg, r.values_out != nullptr, has_idx, in_place,
+  const uint64_t need  = workspace_bytes(KB, PASSES, CODEC, r.volume, r.seg, r.values_out != nullptr, has_idx, in_place,
                                              /*least=*/true);
   if (need == 0) {
     return CPN_ERR_UNSUPPORTED;
@@ -1297,7 +1310,7 @@ int sort_typed(const SortRequest& r)
     return CPN_ERR_TEMP;
   }
   if constexpr ((KB == 4 || KB == 8) && KeyTraits<CODEC, KeyT>::NWORDS == 1) {
-    const uint64_t piece = ranked_row_piece(KB, PASSES, r.volume, r.seg, has_idx);
+    const uint64_t piece = ranked_row_piece(KB, PASSES, CODEC, r.volume, r.seg, has_idx);
     if (piece != 0 && r.temp_bytes >= ranked_workspace_bytes(KB, r.volume, has_idx)) {
       return has_idx ? sort_rows_ranked<KeyT, CODEC, true>(r, piece) : sort_rows_ranked<KeyT, CODEC, false>(r, piece);
     }

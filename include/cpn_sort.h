@@ -387,8 +387,9 @@ int cpn_set_bitonic_rows(int enabled);
  * into 2, 4, ... pieces that the per-row kernel sorts and that are then merged pairwise, level by
  * level, as long as that is cheaper than the global path's one pass per key byte (mode 1, the default:
  * up to 6 levels for 8-byte keys, 5 with positions, i.e. rows of up to 1 048 576 and 458 752 keys;
- * 2 levels for 4-byte keys, rows of up to 65 536; requests of up to 2^18 keys in all, 212 992 for plain sorts of
- * 8-byte keys, have their pieces merged at once, by rank), or all go down the global path (mode 0).  A mode N >= 2 allows up to N - 1 levels for every key (A/B runs); a
+ * 2 levels for 4-byte keys, rows of up to 65 536; requests of up to 2^18 keys in all -- of 8-byte floats without
+ * positions 212 992, of 8-byte integers 163 840, with positions 212 992 -- have their pieces merged at once, by rank),
+ * or all go down the global path (mode 0).  A mode N >= 2 allows up to N - 1 levels for every key (A/B runs); a
  * negative mode restores the default.  Returns the previous mode.  Also initialised from the
  * environment variable CPN_SORT_MERGE_ROWS.  Changes the sizes returned by
  * cpn_local_sort_temp_bytes: do not change it between the size query and the sort.

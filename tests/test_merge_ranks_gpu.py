@@ -101,3 +101,26 @@ def test_unlike_pieces_take_no_multiple_of_the_time(torch_cuda):
     even = best(rng.random(n).astype(np.float32))
     for kind in ("one piece wide", "halves"):
         assert best(_unlike(kind, n, rng).astype(np.float32)) < 2.2 * even, kind
+
+
+def _merged_by_rank(lib, torch, x, argsort):
+    import ctypes
+
+    lib.cpn_profile_enable(1)
+    try:
+        abi_sort(lib, torch, x, want_values=not argsort, want_indices=argsort)
+    finally:
+        lib.cpn_profile_enable(0)
+    labels, ms = ctypes.create_string_buffer(64 * 64), (ctypes.c_float * 64)()
+    count = lib.cpn_profile_collect(labels, 64, ms, 64)
+    return any(labels.raw[64 * i : 64 * i + 11] == b"merge_ranks" for i in range(count))
+
+
+@pytest.mark.parametrize("dtype,argsort,first,last", [
+    (np.float32, False, 13_313, 262_144), (np.int32, True, 13_313, 262_144),
+    (np.float64, False, 10_241, 212_992), (np.float64, True, 10_241, 262_144),
+    (np.int64, False, 10_241, 163_840), (np.uint64, True, 10_241, 212_992)])
+def test_the_lines_of_the_path(lib, torch_cuda, dtype, argsort, first, last):
+    """Rows outside them are sorted sooner the other way (int64 with positions, 262 144: 94 us against 110)."""
+    for n, by_rank in ((first - 1, False), (first, True), (last, True), (last + 1, False)):
+        assert _merged_by_rank(lib, torch_cuda, make_input(dtype, (1, n), seed=n), argsort) == by_rank, n
