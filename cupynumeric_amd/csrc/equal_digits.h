@@ -358,7 +358,8 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
   if (lane == 0) {
     atomicAdd(&s_repeated, equal);
   }
-  const int mixed = __syncthreads_or(no) | (s_repeated > EQ_SAMPLE / 4 ? 1 : 0);
+  const int any   = __syncthreads_or(no);  // (a statement of its own: the word below is read behind the barrier)
+  const int mixed = any | (s_repeated > EQ_SAMPLE / 4 ? 1 : 0);
   if (tid == 0) {
     eq->origin = origin;
     eq->last   = last;

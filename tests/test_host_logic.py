@@ -406,6 +406,22 @@ def test_no_allocation_calls_in_the_native_sources():
             assert hits == [], f"{path.name} calls {hits}"
 
 
+def test_barriers_that_vote_stand_before_what_is_read_behind_them():
+    """C++ does not order the operands of `|`, `&` and `+`: a shared word read in the same expression as a voting
+    barrier may be read ahead of it."""
+    for path in sorted((ROOT / "cupynumeric_amd" / "csrc").glob("*.h*")):
+        text = re.sub(r"//[^\n]*", "", path.read_text())
+        for statement in re.findall(r"[^;{}]*__syncthreads_(?:or|and|count)\([^;{}]*", text):
+            call = statement.index("__syncthreads_")
+            depth, end = 0, call
+            for end in range(call, len(statement)):
+                depth += {"(": 1, ")": -1}.get(statement[end], 0)
+                if depth == 0 and statement[end] == ")":
+                    break
+            rest = statement[:call].replace("&&", "").replace("||", "") + statement[end + 1 :].replace("&&", "").replace("||", "")
+            assert not re.search(r"[|&+]", rest), (path.name, statement.strip())
+
+
 def test_searchsorted_workspace_holds_the_sorted_values_and_no_more():
     """The bounds of the search windows (8 bytes per 128 values or more, and one) lie in the workspace of the values' sort, behind
     its header of 2048 bytes: a search by windows asks for what one by probes does."""
