@@ -82,6 +82,10 @@ PROTOTYPES: dict[str, tuple] = {
     "cpn_local_sort_static": (
         c_int, [c_int, c_void_p, c_void_p, c_void_p, c_uint64, c_uint64, c_int64, c_int, c_void_p, c_void_p]
     ),
+    "cpn_equal_digit_plan": (
+        c_int,
+        [c_int, c_uint64, c_uint64, c_int, c_int, c_int, c_void_p, c_uint64, c_void_p, c_void_p],
+    ),
     "cpn_local_sort_check": (c_int, [c_void_p, c_void_p]),
     "cpn_real_to_complex": (c_int, [c_int, c_void_p, c_int, c_void_p, c_uint64, c_void_p]),
     "cpn_astype": (c_int, [c_int, c_void_p, c_int, c_void_p, c_uint64, c_void_p]),

@@ -239,6 +239,41 @@ int64_t cpn_set_equal_digit_threshold(int64_t elements)
   return static_cast<int64_t>(cpn::g_equal_threshold.exchange(v));
 }
 
+int cpn_equal_digit_plan(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_values, int want_indices, int in_place,
+                         const void* temp, uint64_t temp_bytes, uint32_t* out, void* stream)
+{
+  const cpn::KeyKind k = cpn::key_kind(dtype);
+  if (k.bytes == 0 || k.codec < 0) {
+    return CPN_ERR_DTYPE;
+  }
+  if (volume == 0 || sort_dim_size == 0 || volume % sort_dim_size != 0) {
+    return CPN_ERR_SHAPE;
+  }
+  if (temp == nullptr || out == nullptr) {
+    return CPN_ERR_NULL;
+  }
+  const int passes          = cpn::key_passes(k.bytes, k.codec);
+  const cpn::GlobalLayout L = cpn::global_layout(k.bytes, passes, volume, sort_dim_size, want_values != 0, want_indices != 0, in_place != 0, true);
+  cpn::EqualPlan plan{};
+  const bool whole          = sort_dim_size > cpn::lds_row_limit(k.bytes, want_indices != 0) &&
+                     cpn::merged_row_levels(k.bytes, passes, volume, sort_dim_size, want_indices != 0) == 0 &&
+                     cpn::ranked_row_piece(k.bytes, passes, k.codec, volume, sort_dim_size, want_indices != 0) == 0;
+  if (whole && L.eq && temp_bytes >= L.eq_total) {
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    if (hipMemcpyAsync(&plan, static_cast<const unsigned char*>(temp) + L.off_eq, offsetof(cpn::EqualPlan, table), hipMemcpyDeviceToHost, st) !=
+          hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess) {
+      return CPN_ERR_HIP;
+    }
+  }
+  out[0] = plan.mode;
+  out[1] = plan.failed;
+  out[2] = plan.n_large;
+  out[3] = plan.n_extra;
+  out[4] = plan.n_list;
+  return CPN_OK;
+}
+
 int64_t cpn_set_lookback_spin_limit(int64_t polls)
 {
   const long long v = (polls < 1 || polls > (1ll << 31)) ? static_cast<long long>(cpn::LOOKBACK_SPIN_LIMIT) : polls;

@@ -453,6 +453,15 @@ int64_t cpn_set_virtual_digit_threshold(int64_t elements);
 int64_t cpn_set_equal_digit_threshold(int64_t elements);
 
 /*
+ * What became of the last sort in the workspace `temp`, which was given with these arguments: out[0] = 1 when the row
+ * was put in order by equalised digits, out[1] = 1 when that failed afterwards and the byte passes went on, and the
+ * lengths of its lists: parts of large buckets, further pieces, pieces of the general sort (out[2..4]).  All 0 where
+ * the sort takes another path.  Five words; waits for `stream`.  For tests and diagnosis.
+ */
+int cpn_equal_digit_plan(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_values, int want_indices,
+                         int in_place, const void* temp, uint64_t temp_bytes, uint32_t* out, void* stream);
+
+/*
  * Per-launch timing.  cpn_profile_enable(1) makes every kernel launch of the library record
  * a pair of HIP events on the stream it is launched on; it returns the previous setting.
  * cpn_profile_collect waits for the recorded events, writes up to `max_records` entries --

@@ -116,3 +116,109 @@ def test_the_smaller_workspace_is_still_taken(lib, torch_cuda):
     assert lib.cpn_local_sort(11, a.data_ptr(), out.data_ptr(), None, n, n, 0, 1, ws.data_ptr(), small, stream) == 0
     assert lib.cpn_local_sort_check(ws.data_ptr(), stream) == 0
     assert_same_bits(out.cpu().numpy(), np.sort(x), "values")
+
+
+def _sort(lib, torch, x, want_values, want_indices, in_place=False, offset=0):
+    """cpn_local_sort on device buffers; returns values, positions and what became of the plan (mode, failed, ...)."""
+    code, n = 11 if x.dtype == np.float64 else (4 if x.dtype == np.int64 else 8), x.size
+    a = torch.from_numpy(x.view(np.int64).copy()).cuda()
+    v = a if in_place else (torch.empty_like(a) if want_values else None)
+    i = torch.empty(n, dtype=torch.int64, device="cuda") if want_indices else None
+    shape = (n, n, int(want_values), int(want_indices), int(in_place))
+    need = lib.cpn_local_sort_temp_bytes(code, *shape)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.cpn_local_sort(code, a.data_ptr(), v.data_ptr() if want_values else None, i.data_ptr() if want_indices else None,
+                              n, n, offset, 1, ws.data_ptr(), need, stream) == 0
+    status = lib.cpn_local_sort_check(ws.data_ptr(), stream)
+    plan = (ctypes.c_uint32 * 5)()
+    assert lib.cpn_equal_digit_plan(code, *shape, ws.data_ptr(), need, plan, stream) == 0
+    return status, (v.cpu().numpy().view(x.dtype) if want_values else None), (i.cpu().numpy() if want_indices else None), tuple(plan)
+
+
+REQUESTS = [(True, False, False), (False, True, False), (True, True, False), (True, False, True), (True, True, True)]
+
+
+def _check(lib, torch, x, mode, failed, what):
+    want_v, want_i = oracle.local_sort(x, argsort=False, threads=8), oracle.local_sort(x, argsort=True, threads=8)
+    for want_values, want_indices, in_place in REQUESTS:
+        status, v, i, plan = _sort(lib, torch, x, want_values, want_indices, in_place)
+        assert status == 0 and plan[:2] == (mode, failed), (what, want_values, want_indices, in_place, plan)
+        if want_values:
+            assert_same_bits(v, want_v, f"{what}: values")
+        if want_indices:
+            assert_same_bits(i, want_i, f"{what}: positions")
+
+
+# (uint64 "bits": few bytes vary; the others that keep the byte passes: a value that occurs often has keys in its cell that
+# do not, +inf in that of the NaNs, any integer in those of the smallest and the largest)
+@pytest.mark.parametrize("dtype,kind,mode,failed", [
+    (np.float64, "spread", 1, 0), (np.float64, "normal", 1, 0), (np.float64, "repeated", 1, 0), (np.float64, "specials", 0, 0),
+    (np.int64, "spread", 1, 0), (np.uint64, "specials", 0, 0), (np.int64, "crowd", 0, 0), (np.uint64, "bits", 0, 0)])
+def test_the_path_that_is_taken(lib, torch_cuda, dtype, kind, mode, failed):
+    x = _keys(kind, dtype, 700_001, np.random.default_rng(7)).astype(dtype, copy=False)
+    _check(lib, torch_cuda, x, mode, failed, kind)
+
+
+def _far_value(x, value, rng):
+    """A quarter of the keys is a value far from the others, with two neighbours that the sample misses."""
+    n = x.size
+    x[rng.random(n) < 0.25] = value
+    x[n // 3], x[n // 2] = value + 1, value - 1
+    return x
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.uint64, np.float64])
+@pytest.mark.parametrize("top", [40, 48, 56])
+def test_late_failure_with_constant_bytes(lib, torch_cuda, dtype, top):
+    """Six, seven and eight bytes vary: an odd number of byte passes takes a copying one more when they go on."""
+    rng = np.random.default_rng(top)
+    x = _far_value(rng.integers(0, 1 << (top - 4), 400_003), 15 << (top - 4), rng).astype(np.int64).view(dtype)
+    _check(lib, torch_cuda, x, 1, 1, f"{np.dtype(dtype)} {top}")
+
+
+@pytest.fixture
+def both_thresholds_lowered(lib):
+    prev = lib.cpn_set_virtual_digit_threshold(1 << 18)
+    yield
+    lib.cpn_set_virtual_digit_threshold(prev)
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.float64])
+def test_few_values_keep_the_pass_on_their_ranks(lib, torch_cuda, both_thresholds_lowered, dtype):
+    rng = np.random.default_rng(1)
+    values = rng.standard_normal(200).view(np.int64).astype(np.int64).view(dtype)
+    _check(lib, torch_cuda, values[rng.integers(0, 200, 300_001)], 0, 0, "few values")
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.float64])
+@pytest.mark.parametrize("bytes_that_vary", [6, 8])
+def test_late_failure_goes_on_with_grouped_digits(lib, torch_cuda, both_thresholds_lowered, dtype, bytes_that_vary):
+    """Few values in every byte: three groups of two bytes (an odd number of passes) and four."""
+    rng = np.random.default_rng(bytes_that_vary)
+    n, x = 500_009, np.zeros(500_009, np.int64)
+    for b in range(bytes_that_vary):
+        x |= (rng.integers(0, 8, n) * 9) << (8 * b)
+    x = _far_value(x, 0x7B << (8 * (bytes_that_vary - 1)), rng)
+    _check(lib, torch_cuda, x.view(dtype), 1, 1, f"{bytes_that_vary} bytes")
+
+
+def test_evenly_spread_keys_with_both_kinds_of_digits_in_force(lib, torch_cuda, both_thresholds_lowered):
+    _check(lib, torch_cuda, np.random.default_rng(3).random(600_011), 1, 0, "evenly spread")
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.float64])
+def test_passes_that_give_up(lib, torch_cuda, dtype):
+    """Every wait for an earlier tile ends at the first unanswered poll: an error is reported, or the result is right."""
+    x = _keys("spread", dtype, 700_001, np.random.default_rng(5)).astype(dtype, copy=False)
+    want = oracle.local_sort(x, argsort=False, threads=8)
+    prev = lib.cpn_set_lookback_spin_limit(1)
+    try:
+        for _ in range(5):
+            status, v, _, plan = _sort(lib, torch_cuda, x, True, False)
+            assert status in (0, -7) and plan[:2] == (1, 0)
+            if status == 0:
+                assert_same_bits(v, want, "values")
+    finally:
+        lib.cpn_set_lookback_spin_limit(prev)
+    assert _sort(lib, torch_cuda, x, True, False)[0] == 0
