@@ -162,19 +162,53 @@ __global__ __launch_bounds__(EQ_GATHER_BLOCK) void eq_gather_kernel(const KeyT* 
 }
 
 // ---- the plan -----------------------------------------------------------------------------
-// One workgroup: the range, the cells, the shares, and whether the row is one for equalised digits.  It is not
+// One workgroup: the range, the cells, the shares, and whether the row is one for equalised digits.  What the LDS
+// sort cannot take costs far more than the two passes save (a row whose pieces all go to the general sort 1.6 times
+// the byte passes, one that fails when it has been sorted as much), so the row keeps the byte passes
 //   - when fewer than EQ_MIN_BYTES bytes of the sampled images vary (that many byte passes are as fast);
 //   - when a bucket that `crowd` and more of the sampled keys fall into holds different ones;
 //   - when such a bucket holds one key, and its cell other keys as well that do not crowd theirs (a value that
 //     occurs often among keys that are close to it: some are bound to share its bucket);
-//   - when a quarter of the sampled keys shares buckets with equal ones only, crowding them by a quarter or more
-//     (values that occur some thousand times each: where a few of them meet, a bucket is too large).
+//   - when `dense` and more sampled keys outside such buckets fall into 2^group_log2 neighbouring buckets: the density
+//     varies too much inside a cell.  (2^26 normal keys of both signs: their images span 2050 octaves, a cell two
+//     of them, and a bucket at 2.0 holds 11 100 keys where the average is 1024; 2^25 of them still fit.  Accepted, they
+//     took 4.1 ms, 2.5 by the byte passes.)
+//   - when `close` and more ordered pairs of sampled keys share a bucket (16384 evenly spread keys: 4700): the keys
+//     stand in clusters narrower than a bucket, e.g. a few thousand groups of neighbouring numbers;
+//   - when `equal` and more sampled keys find an equal one in their bucket: values repeat so often that they crowd
+//     the bins of the LDS sort.
+// (No sample sees a handful of neighbours of a value that occurs often: such a row fails after its two passes.)
 // `veto`: a word that says (non-zero) that the sort runs otherwise.
+struct EqualLimits {
+  uint32_t crowd, group_log2, dense, close, equal;
+};
+// n: length of the row; fits / tile: keys of a bucket that the general sort and the LDS sort can take.
+inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
+{
+  EqualLimits l{};
+  // A bucket that just fits holds fits * EQ_SAMPLE / n sampled keys on average, and one of evenly spread keys 0.29:
+  // the former and six more are a crowd (seven in a bucket of the latter: one row in 700).
+  l.crowd = static_cast<uint32_t>(fits * static_cast<uint64_t>(EQ_SAMPLE) / n) + 6;
+  // Windows of as many buckets (n / 2^22, a power of two) as hold 36 to 72 sampled keys at nine tenths of what fits,
+  // and 2.3 to 9.1 of evenly spread ones.
+  l.group_log2 = 3;
+  while (l.group_log2 < 6 && (1ull << (22 + l.group_log2)) < n) {
+    ++l.group_log2;
+  }
+  l.dense = static_cast<uint32_t>(((9ull * fits * EQ_SAMPLE / 10) << l.group_log2) / n) + 1;
+  // the bucket of an average key: four fifths of the tile, but nine twentieths of a sampled key, which evenly spread ones
+  // stay well below
+  const uint64_t share = 4ull * tile * EQ_SAMPLE * EQ_SAMPLE / (5 * n);
+  l.close              = static_cast<uint32_t>(share > EQ_SAMPLE * 9 / 20 ? share : EQ_SAMPLE * 9 / 20);
+  // every key one of 16 equal ones, or a smaller share of them one of more
+  l.equal = static_cast<uint32_t>((16ull * EQ_SAMPLE * EQ_SAMPLE) / n) + 1;
+  return l;
+}
 constexpr int EQ_MIN_BYTES = 5;
 template <typename KeyT, int CODEC>
 __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __restrict__ ranges,
                                                                   const KeyT* __restrict__ sample,
-                                                                  uint32_t crowd,
+                                                                  const EqualLimits limits,
                                                                   const uint32_t* __restrict__ veto,
                                                                   EqualPlan* __restrict__ eq)
 {
@@ -190,7 +224,8 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
   __shared__ uint64_t s_lo[WAVES], s_hi[WAVES], s_and[WAVES], s_or[WAVES];
   __shared__ uint32_t s_wsum[WAVES];
   __shared__ uint32_t s_cells_crowded[CELLS / 32], s_cells_other[CELLS / 32];  // one bit per cell
-  __shared__ uint32_t s_repeated;
+  __shared__ uint32_t s_group[EQ_BUCKETS / 8 / 2];  // sampled keys per window of buckets, two counters per word
+  __shared__ uint32_t s_dense, s_close, s_equal;
   if (veto != nullptr && *veto != 0) {
     return;  // (the plan is cleared: mode 0)
   }
@@ -214,8 +249,13 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
     s_cells_crowded[tid] = 0;
     s_cells_other[tid]   = 0;
   }
+  for (int j = tid; j < static_cast<int>(EQ_BUCKETS / 16); j += EQ_SAMPLE_BLOCK) {
+    s_group[j] = 0;
+  }
   if (tid == 0) {
-    s_repeated = 0;
+    s_dense = 0;
+    s_close = 0;
+    s_equal = 0;
   }
   KeyT bits_and = static_cast<KeyT>(~static_cast<KeyT>(0)), bits_or = 0;
 #pragma unroll
@@ -306,24 +346,30 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
   __syncthreads();
   // ---- buckets that look too large: do they hold one key each? ----
   uint32_t bucket[EQ_SAMPLE_ITEMS];
+  uint32_t second = 0;  // bit i: key i was the second to arrive in its bucket
 #pragma unroll
   for (int i = 0; i < EQ_SAMPLE_ITEMS; ++i) {
     bucket[i] = eq_bucket<KeyT>(u[i], static_cast<KeyT>(origin), static_cast<KeyT>(last), lshift, s_table, 0);
-    atomicAdd(&s_count[bucket[i] / 2], 1u << (16 * (bucket[i] % 2)));  // (EQ_SAMPLE < 2^16: no carry)
+    const uint32_t half = 16 * (bucket[i] % 2);
+    const uint32_t was  = atomicAdd(&s_count[bucket[i] / 2], 1u << half);  // (EQ_SAMPLE < 2^16: no carry)
+    second |= ((was >> half) & 0xFFFFu) == 1 ? 1u << i : 0u;
   }
   __syncthreads();
-  uint32_t crowded = 0, shared = 0;
+  uint32_t crowded = 0, shared = 0, pairs = 0;
 #pragma unroll
   for (int i = 0; i < EQ_SAMPLE_ITEMS; ++i) {
     const uint32_t c = (s_count[bucket[i] / 2] >> (16 * (bucket[i] % 2))) & 0xFFFFu;
-    if (c >= crowd) {
+    if (c >= limits.crowd) {
       crowded |= 1u << i;
-    } else if (c >= 2 && c >= crowd / 4) {
-      shared |= 1u << i;
+    } else {
+      const uint32_t g = bucket[i] >> limits.group_log2;
+      atomicAdd(&s_group[g / 2], 1u << (16 * (g % 2)));
+      shared |= c >= 2 ? 1u << i : 0u;
+      pairs += c - 1;
     }
     const uint64_t v    = static_cast<uint64_t>(u[i]) - origin;
     const uint32_t cell = static_cast<uint32_t>((v < last ? v : last) >> (TOP - lshift));
-    uint32_t* const map = c >= crowd ? s_cells_crowded : s_cells_other;
+    uint32_t* const map = c >= limits.crowd ? s_cells_crowded : s_cells_other;
     if (((map[cell / 32] >> (cell % 32)) & 1u) == 0) {  // (most find the bit set)
       atomicOr(&map[cell / 32], 1u << (cell % 32));
     }
@@ -340,26 +386,38 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
       s_mark[bucket[i]] = mark_of(u[i]);
     }
   }
+  uint32_t most = 0;
+  for (int j = tid; j < static_cast<int>(EQ_BUCKETS / 16); j += EQ_SAMPLE_BLOCK) {
+    const uint32_t two = s_group[j];
+    most               = (two & 0xFFFFu) > most ? (two & 0xFFFFu) : most;
+    most               = (two >> 16) > most ? (two >> 16) : most;
+  }
   __syncthreads();
-  int no           = 0;
-  uint32_t equal   = 0;
+  // Keys with an equal one in their bucket: those that find their own mark, but for one in every bucket of several
+  // (whose mark it is), i.e. for as many as arrived second.
+  int no         = 0;
+  uint32_t equal = 0;
 #pragma unroll
   for (int i = 0; i < EQ_SAMPLE_ITEMS; ++i) {
     const bool same = s_mark[bucket[i]] == mark_of(u[i]);
     no |= (((crowded >> i) & 1u) != 0 && !same) ? 1 : 0;
     equal += (((shared >> i) & 1u) != 0 && same) ? 1u : 0u;
   }
+  equal -= __popc(shared & second);  // (of the thread: modulo 2^32)
   if (tid < CELLS / 32 && (s_cells_crowded[tid] & s_cells_other[tid]) != 0) {
     no = 1;
   }
-  // (of different keys that share a bucket, the one that left its mark still counts as equal: that alone stays
-  // below a quarter of the sample where a bucket holds a quarter of a sampled key on average)
   equal = static_cast<uint32_t>(__shfl(wave_inclusive_sum_dpp(equal), WAVE - 1, WAVE));
+  pairs = static_cast<uint32_t>(__shfl(wave_inclusive_sum_dpp(pairs), WAVE - 1, WAVE));
   if (lane == 0) {
-    atomicAdd(&s_repeated, equal);
+    atomicAdd(&s_equal, equal);
+    atomicAdd(&s_close, pairs);
   }
-  const int any   = __syncthreads_or(no);  // (a statement of its own: the word below is read behind the barrier)
-  const int mixed = any | (s_repeated > EQ_SAMPLE / 4 ? 1 : 0);
+  if (most >= limits.dense) {
+    s_dense = 1;
+  }
+  const int any   = __syncthreads_or(no);  // (a statement of its own: the words below are read behind the barrier)
+  const int mixed = any | (s_dense != 0 ? 1 : 0) | (s_close >= limits.close ? 1 : 0) | (s_equal >= limits.equal ? 1 : 0);
   if (tid == 0) {
     eq->origin = origin;
     eq->last   = last;

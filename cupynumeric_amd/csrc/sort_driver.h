@@ -901,15 +901,11 @@ inline int sort_equalised(const SortRequest& r, const GlobalLayout& L, EqualPlan
   KeyT* key1               = reinterpret_cast<KeyT*>(ws + L.off_key1);
   uint32_t* idx1           = HAS_IDX ? reinterpret_cast<uint32_t*>(ws + L.off_idx) : nullptr;
   {
-    // A bucket that the LDS sort can just take holds medium * EQ_SAMPLE / n sampled keys on average, and a bucket of
-    // evenly spread keys a quarter of one: the former and 8 more are a crowd.
-    const uint64_t share = static_cast<uint64_t>(medium) * EQ_SAMPLE / r.seg;
-    const uint32_t crowd = static_cast<uint32_t>(share) + 8;
     const KeyT* ranges   = reinterpret_cast<const KeyT*>(ws + L.off_eq_sample);
     ProfileScope prof("equal_plan", r.stream);
     static_assert(VIRT_DISTINCT == 2, "veto word");
     hipLaunchKernelGGL((eq_plan_kernel<KeyT, CODEC>), dim3(1), dim3(EQ_SAMPLE_BLOCK), 0, r.stream, ranges,
-                       ranges + 2 * EQ_GATHER_GRID, crowd,
+                       ranges + 2 * EQ_GATHER_GRID, eq_limits(r.seg, medium, EQ_SORT_TILE),
                        vplan != nullptr ? &vplan->enabled : static_cast<const uint32_t*>(nullptr), eq);
   }
   CPN_HIP_TRY(hipGetLastError());

@@ -222,3 +222,37 @@ def test_passes_that_give_up(lib, torch_cuda, dtype):
     finally:
         lib.cpn_set_lookback_spin_limit(prev)
     assert _sort(lib, torch_cuda, x, True, False)[0] == 0
+
+
+def _long_row(torch, kind, log2):
+    n, gen = 1 << log2, torch.Generator(device="cuda").manual_seed(log2)
+    if kind == "uniform":
+        return torch.rand(n, generator=gen, device="cuda", dtype=torch.float64)
+    x = torch.randn(n, generator=gen, device="cuda", dtype=torch.float64)
+    if kind == "repeated":  # every value forty times
+        return x[: n // 40][torch.randint(0, n // 40, (n,), generator=gen, device="cuda")]
+    if kind.endswith("groups"):  # neighbouring numbers in far groups of n / count keys
+        count = int(kind.split()[0])
+        return (torch.randint(0, count, (n,), generator=gen, device="cuda") << 32) + torch.randint(0, 1 << 16, (n,), generator=gen, device="cuda")
+    return x
+
+
+# The shortest rows that are tried by default, and the length at which 2.0 is too dense among normal keys.
+@pytest.mark.parametrize("kind,log2,mode", [("uniform", 25, 1), ("normal", 25, 1), ("uniform", 26, 1), ("normal", 26, 0), ("repeated", 25, 0),
+                                            ("repeated", 26, 0), ("5000 groups", 26, 0), ("20000 groups", 26, 0)])
+def test_long_rows_that_do_not_fit_keep_the_byte_passes(lib, torch_cuda, kind, log2, mode):
+    """The plan declines them; none is sorted twice (2^26 normal keys: 2.5 ms, and 4.1 when that was seen too late)."""
+    torch = torch_cuda
+    lib.cpn_set_equal_digit_threshold(-1)
+    a = _long_row(torch, kind, log2)
+    n, code = a.numel(), 11 if a.dtype == torch.float64 else 4
+    v = torch.empty_like(a)
+    need = lib.cpn_local_sort_temp_bytes(code, n, n, 1, 0, 0)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.cpn_local_sort(code, a.data_ptr(), v.data_ptr(), None, n, n, 0, 1, ws.data_ptr(), need, stream) == 0
+    assert lib.cpn_local_sort_check(ws.data_ptr(), stream) == 0
+    plan = (ctypes.c_uint32 * 5)()
+    assert lib.cpn_equal_digit_plan(code, n, n, 1, 0, 0, ws.data_ptr(), need, plan, stream) == 0
+    assert tuple(plan[:2]) == (mode, 0), tuple(plan)
+    assert torch.equal(v, torch.sort(a).values)
