@@ -640,8 +640,10 @@ __global__ __launch_bounds__(EQ_SEGMENT_BLOCK) void eq_segments_kernel(const Key
 // The pieces, dealt to the workgroups in turn.  A piece is split into EQ_BINS bins that cover its buckets evenly
 // (the bucket's fraction goes on where its number ends) and every key is put into its bin in the order in which
 // the counting atomic saw it; then the thread that owns a bin puts the few keys of it in order.  Equal keys go
-// by place (plain sorts: they are the same bits) or by position.
-// Pieces that hold a NaN or a -0.0, or crowd a bin, go on the general sort's list.
+// by place (plain sorts: they are the same bits) or by position.  Bins of more than EQ_BIN_LIMIT keys (values that
+// repeat) are put in order one after the other by the whole workgroup, a key per thread, which compares it with all of
+// its bin.
+// Pieces that hold a NaN or a -0.0, or more than a workgroup's worth of keys in a bin, go on the general sort's list.
 // Bound by vector instructions.  Comparing every key with the others of its bin, as lds_row_sort_kernel does,
 // took 156 of them per key: 2^26 float64 keys 0.46 ms, and 0.50 ms in that kernel.
 constexpr int EQ_SORT_BLOCK       = 512;
@@ -662,6 +664,8 @@ struct EqualSort {
     alignas(16) uint32_t bins[EQ_BINS / 2 + 4];
     uint16_t idx[HAS_IDX ? EQ_SORT_TILE : 1];
     uint32_t wsum[WAVES];
+    uint32_t n_crowded;
+    uint16_t crowded[EQ_SORT_TILE / (EQ_BIN_LIMIT + 1) + 1];  // bins
   };
   // The image of a key that is neither a NaN nor a -0.0, and back.
   static __device__ __forceinline__ KeyT image(KeyT k)
@@ -697,6 +701,9 @@ struct EqualSort {
       static_cast<uint32_t>((static_cast<uint64_t>(EQ_BINS) << 32) / (static_cast<uint64_t>(b1 - b0 + 1) << EQ_FRACTION_BITS));
     uint4* const my_bins = reinterpret_cast<uint4*>(sh.bins) + tid;
     *my_bins             = make_uint4(0u, 0u, 0u, 0u);
+    if (tid == 0) {
+      sh.n_crowded = 0;
+    }
     uint32_t at[R];  // bin, and above it how many keys of the bin were counted before
 #pragma unroll
     for (int i = 0; i < R; ++i) {
@@ -723,7 +730,7 @@ struct EqualSort {
     const uint4 c4            = *my_bins;
     const uint32_t counts[4]  = {c4.x, c4.y, c4.z, c4.w};
     uint32_t pairs = 0, most = 0;  // both halves of the words summed at once: a piece has fewer than 2^16 keys
-    uint32_t several = 0;          // bit j: bin j of this thread holds more than one key
+    uint32_t several = 0;          // bit j: bin j of this thread holds more than one key (and not too many)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       pairs += counts[k];
@@ -732,12 +739,21 @@ struct EqualSort {
       most = b > most ? b : most;
       several |= (a > 1 ? 1u << (2 * k) : 0u) | (b > 1 ? 2u << (2 * k) : 0u);
     }
+    if (most > EQ_BIN_LIMIT) {  // (rare)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (((counts[k / 2] >> (16 * (k % 2))) & 0xFFFFu) > EQ_BIN_LIMIT) {
+          several &= ~(1u << k);
+          sh.crowded[atomicAdd(&sh.n_crowded, 1u)] = static_cast<uint16_t>(tid * (2 * WORDS) + k);
+        }
+      }
+    }
     const uint32_t sum  = (pairs & 0xFFFFu) + (pairs >> 16);
     const uint32_t incl = wave_inclusive_sum_dpp(sum);
     if (lane == WAVE - 1) {
       sh.wsum[tid / WAVE] = incl;
     }
-    if (__syncthreads_or(most > EQ_BIN_LIMIT ? 1 : 0) != 0) {
+    if (__syncthreads_or(most > BLOCK ? 1 : 0) != 0) {
       return false;
     }
     uint32_t run = incl - sum;
@@ -810,6 +826,30 @@ struct EqualSort {
         } else {
           last     = k;
           last_idx = k_idx;
+        }
+      }
+    }
+    const uint32_t n_crowded = sh.n_crowded;
+    for (uint32_t c = 0; c < n_crowded; ++c) {  // uniform
+      const uint32_t bin  = sh.crowded[c];
+      const uint32_t from = starts[bin], to = starts[bin + 1];
+      const uint32_t mine = from + tid;
+      KeyT k              = 0;
+      uint32_t k_idx = 0, place = from;
+      if (mine < to) {
+        k     = sh.keys[mine];
+        k_idx = HAS_IDX ? sh.idx[mine] : mine;
+        for (uint32_t p = from; p < to; ++p) {
+          const KeyT x         = sh.keys[p];
+          const uint32_t x_idx = HAS_IDX ? sh.idx[p] : p;
+          place += (x < k || (x == k && x_idx < k_idx)) ? 1u : 0u;
+        }
+      }
+      __syncthreads();
+      if (mine < to) {
+        sh.keys[place] = k;
+        if constexpr (HAS_IDX) {
+          sh.idx[place] = static_cast<uint16_t>(k_idx);
         }
       }
     }

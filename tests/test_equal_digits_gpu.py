@@ -256,3 +256,37 @@ def test_long_rows_that_do_not_fit_keep_the_byte_passes(lib, torch_cuda, kind, l
     assert lib.cpn_equal_digit_plan(code, n, n, 1, 0, 0, ws.data_ptr(), need, plan, stream) == 0
     assert tuple(plan[:2]) == (mode, 0), tuple(plan)
     assert torch.equal(v, torch.sort(a).values)
+
+
+def _repeated(n, repeats, share, rng):
+    """A share of the keys are values that occur `repeats` times each, the others are all different."""
+    x = rng.random(n)
+    count = int(n * share)
+    if count:
+        x[:count] = np.repeat(rng.random(count // repeats + 1), repeats)[:count]
+        rng.shuffle(x)
+    return x
+
+
+# bins of up to 24 keys, of up to a workgroup's worth, and of more
+@pytest.mark.parametrize("repeats,share", [(24, 1.0), (25, 1.0), (40, 0.5), (200, 0.3), (511, 0.3), (512, 0.3), (513, 0.3), (700, 0.2)])
+def test_repeated_values(lib, torch_cuda, repeats, share):
+    x = _repeated(700_001, repeats, share, np.random.default_rng(repeats))
+    _check(lib, torch_cuda, x, 1, 0, f"{repeats} times each")
+    if repeats < 400:  # (a bin may hold two such values)
+        plan = _sort(lib, torch_cuda, x, True, True)[3]
+        assert plan[4] == 0, plan  # no piece went to the general sort
+
+
+def test_crowded_bins_of_different_keys(lib, torch_cuda):
+    """Clusters of neighbouring numbers narrower than a bin: 25 to 500 keys each, in no order."""
+    rng = np.random.default_rng(11)
+    x = rng.integers(0, 1 << 62, 600_007)
+    at = 0
+    for size in (25, 64, 100, 300, 500):
+        for centre in rng.integers(0, 1 << 62, 60):
+            x[at : at + size] = centre + rng.integers(0, 200, size)
+            at += size
+    rng.shuffle(x)
+    _check(lib, torch_cuda, x, 1, 0, "clusters")
+    _check(lib, torch_cuda, (x - (1 << 61)).view(np.uint64), 1, 0, "clusters, unsigned")
