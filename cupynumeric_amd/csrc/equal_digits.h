@@ -175,8 +175,8 @@ __global__ __launch_bounds__(EQ_GATHER_BLOCK) void eq_gather_kernel(const KeyT* 
 //     took 4.1 ms, 2.5 by the byte passes.)
 //   - when `close` and more ordered pairs of sampled keys share a bucket (16384 evenly spread keys: 4700): the keys
 //     stand in clusters narrower than a bucket, e.g. a few thousand groups of neighbouring numbers;
-//   - when `equal` and more sampled keys find an equal one in their bucket: values repeat so often that they crowd
-//     the bins of the LDS sort.
+//   - when `equal` and more sampled keys find one in their bucket that would share a bin of the LDS sort with them:
+//     values repeat, or stand in clusters so narrow, that they crowd the bins.
 // (No sample sees a handful of neighbours of a value that occurs often: such a row fails after its two passes.)
 // `veto`: a word that says (non-zero) that the sort runs otherwise.
 struct EqualLimits {
@@ -205,6 +205,7 @@ inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
   return l;
 }
 constexpr int EQ_MIN_BYTES = 5;
+constexpr int EQ_MARK_BITS = 11;  // a bucket of evenly spread keys is 910 (2^25 keys) to 3640 bins (2^27) of the LDS sort
 template <typename KeyT, int CODEC>
 __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __restrict__ ranges,
                                                                   const KeyT* __restrict__ sample,
@@ -345,24 +346,26 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
   }
   __syncthreads();
   // ---- buckets that look too large: do they hold one key each? ----
-  uint32_t bucket[EQ_SAMPLE_ITEMS];
+  uint32_t bucket[EQ_SAMPLE_ITEMS];  // and, behind it, EQ_MARK_BITS bits of the place in it
   uint32_t second = 0;  // bit i: key i was the second to arrive in its bucket
 #pragma unroll
   for (int i = 0; i < EQ_SAMPLE_ITEMS; ++i) {
-    bucket[i] = eq_bucket<KeyT>(u[i], static_cast<KeyT>(origin), static_cast<KeyT>(last), lshift, s_table, 0);
-    const uint32_t half = 16 * (bucket[i] % 2);
-    const uint32_t was  = atomicAdd(&s_count[bucket[i] / 2], 1u << half);  // (EQ_SAMPLE < 2^16: no carry)
+    bucket[i] = eq_bucket<KeyT>(u[i], static_cast<KeyT>(origin), static_cast<KeyT>(last), lshift, s_table, EQ_MARK_BITS);
+    const uint32_t b    = bucket[i] >> EQ_MARK_BITS;
+    const uint32_t half = 16 * (b % 2);
+    const uint32_t was  = atomicAdd(&s_count[b / 2], 1u << half);  // (EQ_SAMPLE < 2^16: no carry)
     second |= ((was >> half) & 0xFFFFu) == 1 ? 1u << i : 0u;
   }
   __syncthreads();
   uint32_t crowded = 0, shared = 0, pairs = 0;
 #pragma unroll
   for (int i = 0; i < EQ_SAMPLE_ITEMS; ++i) {
-    const uint32_t c = (s_count[bucket[i] / 2] >> (16 * (bucket[i] % 2))) & 0xFFFFu;
+    const uint32_t b = bucket[i] >> EQ_MARK_BITS;
+    const uint32_t c = (s_count[b / 2] >> (16 * (b % 2))) & 0xFFFFu;
     if (c >= limits.crowd) {
       crowded |= 1u << i;
     } else {
-      const uint32_t g = bucket[i] >> limits.group_log2;
+      const uint32_t g = b >> limits.group_log2;
       atomicAdd(&s_group[g / 2], 1u << (16 * (g % 2)));
       shared |= c >= 2 ? 1u << i : 0u;
       pairs += c - 1;
@@ -375,15 +378,17 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
     }
   }
   __syncthreads();
-  // (some key of a bucket leaves 16 bits of itself there; the others compare)
+  // (some key of a bucket leaves a mark there; the others compare: 16 bits of the key itself in a crowded bucket, the
+  // place in the others)
   uint16_t* const s_mark = reinterpret_cast<uint16_t*>(s_count);
-  auto mark_of           = [](KeyT k) -> uint16_t {
-    return static_cast<uint16_t>((static_cast<uint64_t>(k) * 0x9E3779B97F4A7C15ull) >> 48);
+  auto mark_of           = [&](int i) -> uint16_t {
+    return ((crowded >> i) & 1u) != 0 ? static_cast<uint16_t>((static_cast<uint64_t>(u[i]) * 0x9E3779B97F4A7C15ull) >> 48)
+                                      : static_cast<uint16_t>(bucket[i] & ((1u << EQ_MARK_BITS) - 1));
   };
 #pragma unroll
   for (int i = 0; i < EQ_SAMPLE_ITEMS; ++i) {
     if (((crowded | shared) >> i) & 1u) {
-      s_mark[bucket[i]] = mark_of(u[i]);
+      s_mark[bucket[i] >> EQ_MARK_BITS] = mark_of(i);
     }
   }
   uint32_t most = 0;
@@ -393,13 +398,13 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
     most               = (two >> 16) > most ? (two >> 16) : most;
   }
   __syncthreads();
-  // Keys with an equal one in their bucket: those that find their own mark, but for one in every bucket of several
+  // Keys with another one of their place in the bucket: those that find their own mark, but for one in every bucket of several
   // (whose mark it is), i.e. for as many as arrived second.
   int no         = 0;
   uint32_t equal = 0;
 #pragma unroll
   for (int i = 0; i < EQ_SAMPLE_ITEMS; ++i) {
-    const bool same = s_mark[bucket[i]] == mark_of(u[i]);
+    const bool same = s_mark[bucket[i] >> EQ_MARK_BITS] == mark_of(i);
     no |= (((crowded >> i) & 1u) != 0 && !same) ? 1 : 0;
     equal += (((shared >> i) & 1u) != 0 && same) ? 1u : 0u;
   }
@@ -641,8 +646,8 @@ __global__ __launch_bounds__(EQ_SEGMENT_BLOCK) void eq_segments_kernel(const Key
 // (the bucket's fraction goes on where its number ends) and every key is put into its bin in the order in which
 // the counting atomic saw it; then the thread that owns a bin puts the few keys of it in order.  Equal keys go
 // by place (plain sorts: they are the same bits) or by position.  Bins of more than EQ_BIN_LIMIT keys (values that
-// repeat) are put in order one after the other by the whole workgroup, a key per thread, which compares it with all of
-// its bin.
+// repeat) are put in order by a wave each, larger ones by the whole workgroup one after the other: a thread compares
+// its key with all of the bin.
 // Pieces that hold a NaN or a -0.0, or more than a workgroup's worth of keys in a bin, go on the general sort's list.
 // Bound by vector instructions.  Comparing every key with the others of its bin, as lds_row_sort_kernel does,
 // took 156 of them per key: 2^26 float64 keys 0.46 ms, and 0.50 ms in that kernel.
@@ -659,13 +664,14 @@ struct EqualSort {
   static constexpr int WAVES = BLOCK / WAVE;
   static constexpr int WORDS = EQ_BINS / 2 / BLOCK;  // words of counters per thread
   static_assert(WORDS == 4, "one 16-byte access");
+  static constexpr uint32_t CROWDED = EQ_SORT_TILE / (EQ_BIN_LIMIT + 1);  // bins of more than EQ_BIN_LIMIT keys, at most
   struct Shared {
     alignas(16) KeyT keys[EQ_SORT_TILE];
     alignas(16) uint32_t bins[EQ_BINS / 2 + 4];
     uint16_t idx[HAS_IDX ? EQ_SORT_TILE : 1];
     uint32_t wsum[WAVES];
-    uint32_t n_crowded;
-    uint16_t crowded[EQ_SORT_TILE / (EQ_BIN_LIMIT + 1) + 1];  // bins
+    uint32_t n_crowded, n_large;
+    uint16_t crowded[CROWDED];  // bins for a wave, and from the end on those for the workgroup
   };
   // The image of a key that is neither a NaN nor a -0.0, and back.
   static __device__ __forceinline__ KeyT image(KeyT k)
@@ -703,6 +709,7 @@ struct EqualSort {
     *my_bins             = make_uint4(0u, 0u, 0u, 0u);
     if (tid == 0) {
       sh.n_crowded = 0;
+      sh.n_large   = 0;
     }
     uint32_t at[R];  // bin, and above it how many keys of the bin were counted before
 #pragma unroll
@@ -742,9 +749,11 @@ struct EqualSort {
     if (most > EQ_BIN_LIMIT) {  // (rare)
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        if (((counts[k / 2] >> (16 * (k % 2))) & 0xFFFFu) > EQ_BIN_LIMIT) {
+        const uint32_t c = (counts[k / 2] >> (16 * (k % 2))) & 0xFFFFu;
+        if (c > EQ_BIN_LIMIT) {
           several &= ~(1u << k);
-          sh.crowded[atomicAdd(&sh.n_crowded, 1u)] = static_cast<uint16_t>(tid * (2 * WORDS) + k);
+          const uint32_t entry = c <= WAVE ? atomicAdd(&sh.n_crowded, 1u) : CROWDED - 1 - atomicAdd(&sh.n_large, 1u);
+          sh.crowded[entry]    = static_cast<uint16_t>(tid * (2 * WORDS) + k);
         }
       }
     }
@@ -829,24 +838,43 @@ struct EqualSort {
         }
       }
     }
-    const uint32_t n_crowded = sh.n_crowded;
-    for (uint32_t c = 0; c < n_crowded; ++c) {  // uniform
+    // (the lists are complete: there have been barriers since)
+    auto rank_in_bin = [&](uint32_t from, uint32_t to, KeyT k, uint32_t k_idx) -> uint32_t {
+      uint32_t place = from;
+#pragma unroll 4
+      for (uint32_t p = from; p < to; ++p) {
+        const KeyT x         = sh.keys[p];
+        const uint32_t x_idx = HAS_IDX ? sh.idx[p] : p;
+        place += (x < k || (x == k && x_idx < k_idx)) ? 1u : 0u;
+      }
+      return place;
+    };
+    const uint32_t n_crowded = sh.n_crowded, n_large = sh.n_large;
+    for (uint32_t c = tid / WAVE; c < n_crowded; c += WAVES) {  // uniform in a wave
       const uint32_t bin  = sh.crowded[c];
       const uint32_t from = starts[bin], to = starts[bin + 1];
-      const uint32_t mine = from + tid;
-      KeyT k              = 0;
-      uint32_t k_idx = 0, place = from;
-      if (mine < to) {
-        k     = sh.keys[mine];
-        k_idx = HAS_IDX ? sh.idx[mine] : mine;
-        for (uint32_t p = from; p < to; ++p) {
-          const KeyT x         = sh.keys[p];
-          const uint32_t x_idx = HAS_IDX ? sh.idx[p] : p;
-          place += (x < k || (x == k && x_idx < k_idx)) ? 1u : 0u;
+      const uint32_t mine = from + lane < to ? from + lane : from;
+      const KeyT k         = sh.keys[mine];
+      const uint32_t k_idx = HAS_IDX ? sh.idx[mine] : mine;
+      const uint32_t place = rank_in_bin(from, to, k, k_idx);
+      __builtin_amdgcn_wave_barrier();  // (every lane has read the bin)
+      if (from + lane < to) {
+        sh.keys[place] = k;
+        if constexpr (HAS_IDX) {
+          sh.idx[place] = static_cast<uint16_t>(k_idx);
         }
       }
+    }
+    for (uint32_t c = 0; c < n_large; ++c) {  // uniform
+      const uint32_t bin  = sh.crowded[CROWDED - 1 - c];
+      const uint32_t from = starts[bin], to = starts[bin + 1];
+      const bool in        = from + tid < to;
+      const uint32_t mine  = in ? from + tid : from;
+      const KeyT k         = sh.keys[mine];
+      const uint32_t k_idx = HAS_IDX ? sh.idx[mine] : mine;
+      const uint32_t place = rank_in_bin(from, in ? to : from, k, k_idx);
       __syncthreads();
-      if (mine < to) {
+      if (in) {
         sh.keys[place] = k;
         if constexpr (HAS_IDX) {
           sh.idx[place] = static_cast<uint16_t>(k_idx);

@@ -290,3 +290,9 @@ def test_crowded_bins_of_different_keys(lib, torch_cuda):
     rng.shuffle(x)
     _check(lib, torch_cuda, x, 1, 0, "clusters")
     _check(lib, torch_cuda, (x - (1 << 61)).view(np.uint64), 1, 0, "clusters, unsigned")
+
+
+def test_rows_of_narrow_clusters_keep_the_byte_passes(lib, torch_cuda):
+    """300 000 groups of a hundred neighbouring numbers each, all of a group in one bin of the LDS sort: 4 to 8 times the
+    byte passes' time when every piece had its bins put in order one by one."""
+    test_long_rows_that_do_not_fit_keep_the_byte_passes(lib, torch_cuda, "300000 groups", 25, 0)
