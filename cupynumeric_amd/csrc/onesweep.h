@@ -373,7 +373,8 @@ __device__ __forceinline__ void make_plan(const uint32_t* varying, SortPlan* __r
   const bool resume = eq_failed(rq.eq);
   if (resume && (k & 1u) != 0) {
     // The first pass may not write the buffer it reads: an even number of passes, one of them on a
-    // digit on which all keys agree (it copies).
+    // digit on which all keys agree (it copies).  Under grouped virtual digits that is the first number that no group
+    // has: its count is 0, which makes every digit 0, and its histogram, cleared and scanned like the others, starts at 0.
     for (uint32_t p = 0; p < rq.passes; ++p) {
       if (((flags >> p) & 1u) == 0) {
         flags |= 1u << p;

@@ -1155,7 +1155,8 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
           const uint64_t vgrid  = (r.seg + vchunk - 1) / vchunk;
           ProfileScope prof("virtual_histogram", r.stream);
           hipLaunchKernelGGL((vhist_kernel<KeyT, CODEC, OffT>), dim3(static_cast<uint32_t>(vgrid)), dim3(VHIST_BLOCK), 0,
-                             r.stream, static_cast<const KeyT*>(r.values_in), hist, vplan, r.seg, vchunk);
+                             r.stream, static_cast<const KeyT*>(r.values_in), hist, vplan, r.seg, vchunk,
+                             static_cast<const EqualPlan*>(eq), reinterpret_cast<const KeyT*>(ws + L.off_key1));
         }
         CPN_HIP_TRY(hipGetLastError());
         {

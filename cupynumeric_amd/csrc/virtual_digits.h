@@ -31,6 +31,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "equal_digits.h"
 #include "radix_common.h"
 
 namespace cpn {
@@ -543,13 +544,17 @@ __device__ __forceinline__ uint32_t virtual_digit(uint64_t ordered, uint32_t cou
 
 // Histograms of the virtual digits: hist[g][256] += counts over the row (cleared by
 // vplan_kernel).  Exits at once unless the plan runs on grouped virtual digits.
+// `resumed`: what the passes go on from when equalised digits have failed (the caller's array may have been
+// overwritten by then).
 constexpr int VHIST_BLOCK = 256;
 template <typename KeyT, int CODEC, typename OffT>
 __global__ __launch_bounds__(VHIST_BLOCK) void vhist_kernel(const KeyT* __restrict__ keys,
                                                              OffT* __restrict__ hist,
                                                              const VirtPlan* __restrict__ plan,
                                                              uint64_t seg,
-                                                             uint64_t chunk)
+                                                             uint64_t chunk,
+                                                             const EqualPlan* __restrict__ eq,
+                                                             const KeyT* __restrict__ resumed)
 {
   constexpr int COPIES    = 4;
   constexpr int POSITIONS = static_cast<int>(sizeof(KeyT));  // byte positions of the ordered key
@@ -562,6 +567,7 @@ __global__ __launch_bounds__(VHIST_BLOCK) void vhist_kernel(const KeyT* __restri
   if (plan->enabled != VIRT_GROUPS) {
     return;
   }
+  keys                  = eq_failed(eq) ? resumed : keys;
   const int tid         = threadIdx.x;
   const uint32_t groups = plan->n_groups;
   for (int j = tid; j < VIRT_MAX_POSITIONS * RADIX * COPIES; j += VHIST_BLOCK) {
