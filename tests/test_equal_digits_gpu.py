@@ -268,8 +268,8 @@ def _repeated(n, repeats, share, rng):
     return x
 
 
-# bins of up to 24 keys, of up to a workgroup's worth, and of more
-@pytest.mark.parametrize("repeats,share", [(24, 1.0), (25, 1.0), (40, 0.5), (200, 0.3), (511, 0.3), (512, 0.3), (513, 0.3), (700, 0.2)])
+# bins for a thread (up to 8 keys), for a wave (64), for the workgroup (512), and of more
+@pytest.mark.parametrize("repeats,share", [(8, 1.0), (9, 1.0), (24, 1.0), (40, 0.5), (64, 0.5), (65, 0.5), (200, 0.3), (511, 0.3), (512, 0.3), (513, 0.3), (700, 0.2)])
 def test_repeated_values(lib, torch_cuda, repeats, share):
     x = _repeated(700_001, repeats, share, np.random.default_rng(repeats))
     _check(lib, torch_cuda, x, 1, 0, f"{repeats} times each")
