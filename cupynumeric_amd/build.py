@@ -57,7 +57,10 @@ HIPCC_FLAGS = [
 # registers; one that spills runs several times slower without failing any test (a 16-keys-per-
 # thread shape once spilled 516 bytes per lane and took 3.3 ms instead of 0.8), so the build
 # refuses it.  The scatter pass of the global sort is allowed the few words it is known to park.
-SCRATCH_LIMITS = (("row_sort_kernel", 0), ("count16_", 0), ("onesweep_kernel", 32))
+# (So is the sort of equalised pieces, csrc/equal_digits.h, and their plan, a single workgroup.)
+SCRATCH_LIMITS = (("row_sort_kernel", 0), ("count16_", 0), ("onesweep_kernel", 32), ("merge_ranks_kernel", 0),
+                  ("eq_sweep_kernel", 0), ("eq_sort_kernel", 80), ("eq_plan_kernel", 96), ("eq_gather_kernel", 0),
+                  ("eq_histogram_kernel", 0), ("eq_segments_kernel", 0))
 
 
 def hipcc_path() -> str:

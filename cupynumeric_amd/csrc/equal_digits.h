@@ -653,6 +653,11 @@ __global__ __launch_bounds__(EQ_SEGMENT_BLOCK) void eq_segments_kernel(const Key
 // took 156 of them per key: 2^26 float64 keys 0.46 ms, and 0.50 ms in that kernel.
 constexpr int EQ_SORT_BLOCK       = 512;
 constexpr int EQ_SORT_ITEMS       = 6;
+// Waves per SIMD, and with them workgroups per CU (three).  At 80 registers a dozen values are spilled, addresses and
+// bounds of the loop over the pieces for the most part; without that (108 registers, two workgroups) 2^26 float64 keys
+// take 1409 us instead of 1368, with positions 1748 instead of 1672.
+constexpr int EQ_SORT_WAVES       = 6;
+constexpr int EQ_SORT_GROUPS      = EQ_SORT_WAVES * 4 / (EQ_SORT_BLOCK / WAVE);
 constexpr int EQ_SORT_TILE        = EQ_SORT_BLOCK * EQ_SORT_ITEMS;
 constexpr int EQ_BINS             = 4096;  // two 16-bit counters per word
 // (Evenly spread keys: 0.56 in a bin on average.  With 24, 2^26 float64 keys of which half occur 20 times each took 4.2 ms
@@ -917,7 +922,7 @@ struct EqualSort {
 };
 
 template <typename KeyT, int CODEC, bool HAS_IDX>
-__global__ __launch_bounds__(EQ_SORT_BLOCK) __attribute__((amdgpu_waves_per_eu(6)))
+__global__ __launch_bounds__(EQ_SORT_BLOCK) __attribute__((amdgpu_waves_per_eu(EQ_SORT_WAVES)))
 void eq_sort_kernel(const KeyT* __restrict__ keys,
                                                                 KeyT* __restrict__ keys_out,
                                                                 const uint32_t* __restrict__ pos,
