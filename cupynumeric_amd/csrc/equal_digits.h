@@ -648,7 +648,8 @@ __global__ __launch_bounds__(EQ_SEGMENT_BLOCK) void eq_segments_kernel(const Key
 // by place (plain sorts: they are the same bits) or by position.  Bins of more than EQ_BIN_LIMIT keys (values that
 // repeat) are put in order by a wave each, larger ones by the whole workgroup one after the other: a thread compares
 // its key with all of the bin.
-// Pieces that hold a NaN or a -0.0, or more than a workgroup's worth of keys in a bin, go on the general sort's list.
+// Pieces that hold a NaN or a -0.0, more than a workgroup's worth of keys in a bin, or too many bins for the workgroup, go
+// on the general sort's list.
 // Bound by vector instructions.  Comparing every key with the others of its bin, as lds_row_sort_kernel does,
 // took 156 of them per key: 2^26 float64 keys 0.46 ms, and 0.50 ms in that kernel.
 constexpr int EQ_SORT_BLOCK       = 512;
@@ -663,6 +664,10 @@ constexpr int EQ_BINS             = 4096;  // two 16-bit counters per word
 // (Evenly spread keys: 0.56 in a bin on average.  With 24, 2^26 float64 keys of which half occur 20 times each took 4.2 ms
 // with positions, whose order the counting atomic leaves mixed; 2.3 now, the byte passes 3.2.)
 constexpr uint32_t EQ_BIN_LIMIT   = 8;
+// Bins for the whole workgroup, one after the other: with more of them the general sort is the faster one.  (Pieces of
+// many sparse buckets and a full one, whose keys share a few bins: the sort of 2^25 normal float64 keys 802 us without
+// this limit, now 742.)
+constexpr uint32_t EQ_LARGE_BINS  = 6;
 constexpr int EQ_FRACTION_BITS    = 14;    // of a bucket, for the bins
 
 template <typename KeyT, int CODEC, bool HAS_IDX>
@@ -769,7 +774,7 @@ struct EqualSort {
     if (lane == WAVE - 1) {
       sh.wsum[tid / WAVE] = incl;
     }
-    if (__syncthreads_or(most > BLOCK ? 1 : 0) != 0) {
+    if (__syncthreads_or(most > BLOCK ? 1 : 0) != 0 || sh.n_large > EQ_LARGE_BINS) {
       return false;
     }
     uint32_t run = incl - sum;
