@@ -186,16 +186,20 @@ struct EqualLimits {
 inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
 {
   EqualLimits l{};
-  // A bucket that just fits holds fits * EQ_SAMPLE / n sampled keys on average, and one of evenly spread keys 0.29:
-  // the former and six more are a crowd (seven in a bucket of the latter: one row in 700).
-  l.crowd = static_cast<uint32_t>(fits * static_cast<uint64_t>(EQ_SAMPLE) / n) + 6;
-  // Windows of as many buckets (n / 2^22, a power of two) as hold 36 to 72 sampled keys at nine tenths of what fits,
-  // and 2.3 to 9.1 of evenly spread ones.
-  l.group_log2 = 3;
-  while (l.group_log2 < 6 && (1ull << (22 + l.group_log2)) < n) {
+  // A bucket that just fits holds `mean` sampled keys on average (5 of 2^25 keys, 1.25 of 2^27), and one of evenly
+  // spread keys 0.29: three and a half standard deviations above the former are a crowd, and never fewer than seven
+  // (which one row in 700 of the latter has in some bucket).
+  const double mean = static_cast<double>(fits) * EQ_SAMPLE / static_cast<double>(n);
+  l.crowd           = static_cast<uint32_t>(mean + 3.5 * __builtin_sqrt(mean));
+  l.crowd           = l.crowd > 7 ? l.crowd : 7;
+  // Windows of as many buckets (n / 2^21, a power of two) as hold 60 to 120 sampled keys at three quarters of what fits,
+  // and 4.6 to 18 of evenly spread ones.  The densest of 2^25 normal keys holds 43 (and is taken for too dense once in
+  // 250 rows), of 2^26 of them 87 (and is missed once in 100).
+  l.group_log2 = 4;
+  while (l.group_log2 < 7 && (1ull << (21 + l.group_log2)) < n) {
     ++l.group_log2;
   }
-  l.dense = static_cast<uint32_t>(((9ull * fits * EQ_SAMPLE / 10) << l.group_log2) / n) + 1;
+  l.dense = static_cast<uint32_t>(((3ull * fits * EQ_SAMPLE / 4) << l.group_log2) / n) + 1;
   // the bucket of an average key: four fifths of the tile, but nine twentieths of a sampled key, which evenly spread ones
   // stay well below
   const uint64_t share = 4ull * tile * EQ_SAMPLE * EQ_SAMPLE / (5 * n);
@@ -225,7 +229,7 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
   __shared__ uint64_t s_lo[WAVES], s_hi[WAVES], s_and[WAVES], s_or[WAVES];
   __shared__ uint32_t s_wsum[WAVES];
   __shared__ uint32_t s_cells_crowded[CELLS / 32], s_cells_other[CELLS / 32];  // one bit per cell
-  __shared__ uint32_t s_group[EQ_BUCKETS / 8 / 2];  // sampled keys per window of buckets, two counters per word
+  __shared__ uint32_t s_group[EQ_BUCKETS / 16 / 2];  // sampled keys per window of buckets, two counters per word
   __shared__ uint32_t s_dense, s_close, s_equal;
   if (veto != nullptr && *veto != 0) {
     return;  // (the plan is cleared: mode 0)
@@ -250,7 +254,7 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
     s_cells_crowded[tid] = 0;
     s_cells_other[tid]   = 0;
   }
-  for (int j = tid; j < static_cast<int>(EQ_BUCKETS / 16); j += EQ_SAMPLE_BLOCK) {
+  for (int j = tid; j < static_cast<int>(EQ_BUCKETS / 32); j += EQ_SAMPLE_BLOCK) {
     s_group[j] = 0;
   }
   if (tid == 0) {
@@ -392,7 +396,7 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
     }
   }
   uint32_t most = 0;
-  for (int j = tid; j < static_cast<int>(EQ_BUCKETS / 16); j += EQ_SAMPLE_BLOCK) {
+  for (int j = tid; j < static_cast<int>(EQ_BUCKETS / 32); j += EQ_SAMPLE_BLOCK) {
     const uint32_t two = s_group[j];
     most               = (two & 0xFFFFu) > most ? (two & 0xFFFFu) : most;
     most               = (two >> 16) > most ? (two >> 16) : most;

@@ -56,6 +56,15 @@ constexpr uint64_t VIRT_MIN_ROW_ELEMENTS = 1ull << 26;
 uint64_t virtual_digit_threshold();
 // Row lengths that are tried with equalised digits (equal_digits.h), real keys of 8 bytes: from the threshold in
 // force (cpn_set_equal_digit_threshold; tests move it) to EQ_MAX_ROW_ELEMENTS.
+// Why the lines lie there (us per call, this way / byte passes, sort and argsort):
+//   from 2^25: uniform float64 720, 864 / 1300, 1682, int64 711, 877 / 1294, 1655.  Shorter rows that suit it gain as
+//   well (2^24 428, 517 / 698, 918, 2^22 174, 201 / 228, 261), but a row that the plan declines pays for the sample, the
+//   plan and seven launches that find nothing to do: 2^22 values that repeat 40 times 274, 305 / 228, 258 (20 %), 2^24
+//   758, 964 / 710, 918 (7 %), 2^25 1345, 1749 / 1290, 1687 (4 %), 2^26 2542, 3262 / 2479, 3200 (2 %), 2^27 2 %; 2^26
+//   keys of 100 values, which take one pass on their ranks, 833, 662 / 792, 626 (5 %).
+//   to 2^27: a bucket of 2^28 evenly spread keys holds more than the tile of the LDS sort.
+// What the sample cannot see costs most: 2^25 keys, a quarter of them one value with two neighbours that share its
+// bucket, are sorted twice, 2201, 2863 / 1347, 1715.
 constexpr uint64_t EQ_MIN_ROW_ELEMENTS = 1ull << 25;
 constexpr uint64_t EQ_MAX_ROW_ELEMENTS = 1ull << 27;
 uint64_t equal_digit_threshold();
