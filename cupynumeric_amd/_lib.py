@@ -86,6 +86,7 @@ PROTOTYPES: dict[str, tuple] = {
         c_int,
         [c_int, c_uint64, c_uint64, c_int, c_int, c_int, c_void_p, c_uint64, c_void_p, c_void_p],
     ),
+    "cpn_local_sort_may_fail": (c_int, [c_int, c_uint64, c_uint64, c_int, c_uint64]),
     "cpn_local_sort_check": (c_int, [c_void_p, c_void_p]),
     "cpn_real_to_complex": (c_int, [c_int, c_void_p, c_int, c_void_p, c_uint64, c_void_p]),
     "cpn_astype": (c_int, [c_int, c_void_p, c_int, c_void_p, c_uint64, c_void_p]),

@@ -98,9 +98,9 @@ def sort_task(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable
         return temp
 
     temp = issue()
-    # Rows sorted by the per-row kernels cannot fail on the device (the request then needs nothing but
-    # the workspace header).  The global sort can: a bounded wait between its tiles may run out.
-    if runtime.check_mode == "off" or temp_bytes == lib.cpn_local_sort_temp_bytes(code, 0, 0, 1, 0, 0):
+    # Rows sorted by the per-row kernels, whole or in pieces that are merged, cannot fail on the device.
+    # The global sort can: a bounded wait between its tiles may run out.
+    if runtime.check_mode == "off" or not lib.cpn_local_sort_may_fail(code, volume, seg, int(indices_out is not None), temp_bytes):
         return
     if runtime.check_mode == "lazy":
         runtime.defer_status(temp)

@@ -239,6 +239,25 @@ int64_t cpn_set_equal_digit_threshold(int64_t elements)
   return static_cast<int64_t>(cpn::g_equal_threshold.exchange(v));
 }
 
+int cpn_local_sort_may_fail(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_indices, uint64_t temp_bytes)
+{
+  const cpn::KeyKind k = cpn::key_kind(dtype);
+  if (k.bytes == 0 || k.codec < 0 || volume == 0 || sort_dim_size == 0 || volume % sort_dim_size != 0) {
+    return 0;
+  }
+  const bool has_idx = want_indices != 0;
+  const int passes   = cpn::key_passes(k.bytes, k.codec);
+  // (the order of sort_typed)
+  if (cpn::ranked_row_piece(k.bytes, passes, k.codec, volume, sort_dim_size, has_idx) != 0 &&
+      temp_bytes >= cpn::ranked_workspace_bytes(k.bytes, volume, has_idx)) {
+    return 0;
+  }
+  return sort_dim_size > cpn::lds_row_limit(k.bytes, has_idx) &&
+             cpn::merged_row_levels(k.bytes, passes, volume, sort_dim_size, has_idx) == 0
+           ? 1
+           : 0;
+}
+
 int cpn_equal_digit_plan(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_values, int want_indices, int in_place,
                          const void* temp, uint64_t temp_bytes, uint32_t* out, void* stream)
 {
@@ -255,10 +274,7 @@ int cpn_equal_digit_plan(int dtype, uint64_t volume, uint64_t sort_dim_size, int
   const int passes          = cpn::key_passes(k.bytes, k.codec);
   const cpn::GlobalLayout L = cpn::global_layout(k.bytes, passes, volume, sort_dim_size, want_values != 0, want_indices != 0, in_place != 0, true);
   cpn::EqualPlan plan{};
-  const bool whole          = sort_dim_size > cpn::lds_row_limit(k.bytes, want_indices != 0) &&
-                     cpn::merged_row_levels(k.bytes, passes, volume, sort_dim_size, want_indices != 0) == 0 &&
-                     cpn::ranked_row_piece(k.bytes, passes, k.codec, volume, sort_dim_size, want_indices != 0) == 0;
-  if (whole && L.eq && temp_bytes >= L.eq_total) {
+  if (cpn_local_sort_may_fail(dtype, volume, sort_dim_size, want_indices, temp_bytes) != 0 && L.eq && temp_bytes >= L.eq_total) {
     const hipStream_t st = static_cast<hipStream_t>(stream);
     if (hipMemcpyAsync(&plan, static_cast<const unsigned char*>(temp) + L.off_eq, offsetof(cpn::EqualPlan, table), hipMemcpyDeviceToHost, st) !=
           hipSuccess ||

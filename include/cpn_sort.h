@@ -175,6 +175,13 @@ int cpn_local_sort_static(int dtype, const void* values_in, void* values_out, in
 int cpn_local_sort_check(const void* temp, void* stream);
 
 /*
+ * 1 when a sort of these arguments, in a workspace of `temp_bytes`, has a bounded wait that can run out, so that its
+ * status word is worth a check; 0 when none of its kernels can fail on the device (rows sorted by one workgroup each,
+ * or in pieces that are merged).  A host function; follows the switches below.
+ */
+int cpn_local_sort_may_fail(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_indices, uint64_t temp_bytes);
+
+/*
  * out = in with axes `axis_a` and `axis_b` exchanged, both dense row-major; `shape` is the
  * shape of `in`.  Replaces the UNARY_OP(COPY) of a transposed store that sort_swapped
  * issues (cupynumeric/_thunk/_sort.py:50-76, src/cupynumeric/unary/unary_op.cu:85-96,124-170).

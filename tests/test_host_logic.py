@@ -391,6 +391,20 @@ def test_merged_row_levels_and_workspace_over_the_limits(lib):
     assert 65537 * 4 < temp(f32, 65537, False) < 2 * 65536 * 4
 
 
+def test_only_sorts_with_a_bounded_wait_need_a_check(lib):
+    """Requests that one workgroup per row sorts, or whose sorted pieces are merged, have no status to look at: an eager
+    caller waited for the device to read it."""
+    f32, f64, i64, f16 = 10, 11, 4, 9
+    for code, n, idx, fails in [(f32, 1000, 0, 0), (f32, 16384, 0, 0), (f64, 12_000, 1, 0), (f32, 14_000, 1, 0), (f32, 100_000, 0, 0),
+                                (f64, 200_000, 1, 0), (f64, 400_000, 1, 0), (i64, 1 << 20, 0, 0), (f16, 100_000, 0, 1),
+                                (f32, 300_000, 0, 1), (f64, (1 << 20) + 1, 0, 1), (f64, 1 << 26, 1, 1)]:
+        need = lib.cpn_local_sort_temp_bytes(code, n, n, 1, idx, 0)
+        assert lib.cpn_local_sort_may_fail(code, n, n, idx, need) == fails, (code, n, idx)
+    # a workspace too small for the merge by rank: the passes of the global sort run instead
+    assert lib.cpn_local_sort_may_fail(f32, 100_000, 100_000, 1, 2048) == 1
+    assert lib.cpn_local_sort_may_fail(99, 100, 100, 0, 4096) == 0 and lib.cpn_local_sort_may_fail(f32, 0, 0, 0, 4096) == 0
+
+
 def test_no_allocation_calls_in_the_native_sources():
     """cpn_local_sort_static promises that nothing on its path allocates: no translation unit of the
     library calls hipMalloc, hipFree or creates events outside the profiling helper, which is off
