@@ -424,12 +424,13 @@ struct SearchLayout {
   uint64_t sort_bytes, off_values, off_origin, total;
 };
 
-static SearchLayout search_layout(int dtype, int key_bytes, uint64_t num_values)
+// With `least`, the sort's workspace is what it can do with instead of what it asks for (callers that kept a size).
+static SearchLayout search_layout(KeyKind k, uint64_t num_values, bool least)
 {
   SearchLayout L{};
-  L.sort_bytes = cpn_local_sort_temp_bytes(dtype, num_values, num_values, 1, 1, 0);
+  L.sort_bytes = workspace_bytes(k.bytes, key_passes(k.bytes, k.codec), k.codec, num_values, num_values, true, true, false, least);
   L.off_values = align_up(L.sort_bytes, WORKSPACE_ALIGN);
-  L.off_origin = L.off_values + align_up(num_values * static_cast<uint64_t>(key_bytes), WORKSPACE_ALIGN);
+  L.off_origin = L.off_values + align_up(num_values * static_cast<uint64_t>(k.bytes), WORKSPACE_ALIGN);
   L.total      = L.off_origin + align_up(num_values * 8, WORKSPACE_ALIGN);
   return L;
 }
@@ -442,7 +443,7 @@ extern "C" uint64_t cpn_searchsorted_temp_bytes(int dtype, uint64_t n, uint64_t 
   if (k.bytes == 0 || k.codec < 0 || !cpn::presort_pays(k.bytes, n, num_values)) {
     return 0;
   }
-  const cpn::SearchLayout L = cpn::search_layout(dtype, k.bytes, num_values);
+  const cpn::SearchLayout L = cpn::search_layout(k, num_values, false);
   return L.sort_bytes == 0 ? 0 : L.total;
 }
 
@@ -468,7 +469,10 @@ extern "C" int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const
   const int64_t* origin = nullptr;
   uint64_t* bounds      = nullptr;
   if (temp != nullptr && presort_pays(k.bytes, n, num_values)) {
-    const SearchLayout L = search_layout(dtype, k.bytes, num_values);
+    SearchLayout L = search_layout(k, num_values, false);
+    if (temp_bytes < L.total) {
+      L = search_layout(k, num_values, true);
+    }
     if (L.sort_bytes != 0 && temp_bytes >= L.total) {
       if ((reinterpret_cast<uintptr_t>(temp) % WORKSPACE_ALIGN) != 0) {
         return CPN_ERR_TEMP;

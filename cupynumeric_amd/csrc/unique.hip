@@ -219,11 +219,12 @@ struct UniqueLayout {
   uint64_t tiles;
 };
 
-static UniqueLayout unique_layout(int dtype, uint64_t volume)
+// With `least`, the sort's workspace is what it can do with instead of what it asks for (callers that kept a size).
+static UniqueLayout unique_layout(int dtype, uint64_t volume, bool least)
 {
   UniqueLayout L{};
   const KeyKind k = key_kind(dtype);
-  L.sort_bytes    = cpn_local_sort_temp_bytes(dtype, volume, volume, 1, 0, 0);
+  L.sort_bytes    = workspace_bytes(k.bytes, key_passes(k.bytes, k.codec), k.codec, volume, volume, true, false, false, least);
   L.tiles         = (volume + UNIQUE_TILE - 1) / UNIQUE_TILE;
   L.off_sorted    = align_up(L.sort_bytes, WORKSPACE_ALIGN);
   L.off_counts    = L.off_sorted + align_up(volume * static_cast<uint64_t>(k.bytes), WORKSPACE_ALIGN);
@@ -270,7 +271,7 @@ extern "C" uint64_t cpn_unique_temp_bytes(int dtype, uint64_t volume)
   if (volume == 0) {
     return cpn::HEADER_BYTES;
   }
-  const cpn::UniqueLayout L = cpn::unique_layout(dtype, volume);
+  const cpn::UniqueLayout L = cpn::unique_layout(dtype, volume, false);
   return L.sort_bytes == 0 ? 0 : L.total;
 }
 
@@ -298,9 +299,12 @@ extern "C" int cpn_unique(int dtype, const void* values_in, void* values_out, ui
   if (values_in == nullptr || values_out == nullptr) {
     return CPN_ERR_NULL;
   }
-  const UniqueLayout L = unique_layout(dtype, volume);
+  UniqueLayout L = unique_layout(dtype, volume, false);
   if (L.sort_bytes == 0) {
     return CPN_ERR_UNSUPPORTED;
+  }
+  if (temp_bytes < L.total) {
+    L = unique_layout(dtype, volume, true);
   }
   if (temp == nullptr || temp_bytes < L.total || (reinterpret_cast<uintptr_t>(temp) % WORKSPACE_ALIGN) != 0) {
     return CPN_ERR_TEMP;

@@ -357,3 +357,39 @@ def test_random_consumers(seed):
                 keys.append(k)
         got = np.asarray(num.lexsort(tuple(num.array(k) for k in keys), axis=axis))
         assert np.array_equal(got, oracle.lexsort(tuple(keys), axis=axis)), what + f" lexsort {shape} axis={axis}"
+
+
+def test_consumers_take_the_workspace_that_the_sort_takes():
+    """A size asked for while the sort had no use for more (equalised digits out of force) is still enough: unique runs,
+    and searchsorted still sorts its values."""
+    torch, lib = pytest.importorskip("torch"), _lib.load()
+    n, m = 1 << 23, 300_001  # 8-byte keys
+    prev = lib.cpn_set_equal_digit_threshold(1 << 40)
+    merged = lib.cpn_set_merge_rows(0)
+    try:
+        unique_bytes, search_bytes = lib.cpn_unique_temp_bytes(4, m), lib.cpn_searchsorted_temp_bytes(4, n, m)
+        lib.cpn_set_equal_digit_threshold(1 << 18)
+        assert unique_bytes < lib.cpn_unique_temp_bytes(4, m) and search_bytes < lib.cpn_searchsorted_temp_bytes(4, n, m)
+        gen = torch.Generator(device="cuda").manual_seed(1)
+        table = torch.sort(torch.randint(0, 1 << 62, (n,), generator=gen, device="cuda")).values
+        v = torch.randint(0, 1 << 62, (m,), generator=gen, device="cuda")
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        out, count = torch.empty_like(v), torch.zeros(1, dtype=torch.int64, device="cuda")
+        ws = torch.empty(unique_bytes, dtype=torch.uint8, device="cuda")
+        assert lib.cpn_unique(4, v.data_ptr(), out.data_ptr(), m, count.data_ptr(), ws.data_ptr(), unique_bytes, stream) == 0
+        want = torch.unique(v)
+        assert int(count) == want.numel() and torch.equal(out[: want.numel()], want)
+        where = torch.empty(m, dtype=torch.int64, device="cuda")
+        ws = torch.empty(search_bytes, dtype=torch.uint8, device="cuda")
+        lib.cpn_profile_enable(1)
+        _lib.profile_collect()
+        status = lib.cpn_searchsorted(4, table.data_ptr(), n, v.data_ptr(), m, 1, where.data_ptr(), ws.data_ptr(), search_bytes, stream)
+        labels = {k for k, _ in _lib.profile_collect()}
+        lib.cpn_profile_enable(0)
+        assert status == 0 and "onesweep" in labels, labels
+        assert torch.equal(where, torch.searchsorted(table, v))
+        small = unique_bytes - 256 * ((m * 8) // 256)  # less than that is refused
+        assert lib.cpn_unique(4, v.data_ptr(), out.data_ptr(), m, count.data_ptr(), ws.data_ptr(), small, stream) == _lib.CPN_ERR_TEMP
+    finally:
+        lib.cpn_set_equal_digit_threshold(prev)
+        lib.cpn_set_merge_rows(merged)
