@@ -997,7 +997,7 @@ inline int sort_equalised(const SortRequest& r, const GlobalLayout& L, EqualPlan
 
 // A pass in small tiles.
 template <typename KeyT, int CODEC, bool HAS_IDX, bool CAN_ORDER_KEYS>
-inline bool launch_small_sweep(const SweepArgs<false>& a, int items, bool ordered_keys, dim3 grid, hipStream_t stream)
+inline void launch_small_sweep(const SweepArgs<false>& a, int items, bool ordered_keys, dim3 grid, hipStream_t stream)
 {
   auto launch = [&](auto xform, auto count) {
     hipLaunchKernelGGL((onesweep_kernel<KeyT, CODEC, decltype(xform)::value, false, HAS_IDX, SMALL_BLOCK, decltype(count)::value>),
@@ -1013,11 +1013,10 @@ inline bool launch_small_sweep(const SweepArgs<false>& a, int items, bool ordere
   if constexpr (CAN_ORDER_KEYS) {
     if (ordered_keys) {
       shape(std::true_type{});
-      return true;
+      return;
     }
   }
   shape(std::false_type{});
-  return true;
 }
 
 template <typename KeyT, int CODEC, bool BIG, bool HAS_IDX>
@@ -1254,7 +1253,8 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
       bool launched = false;
       if constexpr (SMALL_OK) {
         if (L.small_items != 0) {
-          launched = launch_small_sweep<KeyT, CODEC, HAS_IDX, CAN_ORDER_KEYS>(a, L.small_items, ordered_keys, grid, r.stream);
+          launch_small_sweep<KeyT, CODEC, HAS_IDX, CAN_ORDER_KEYS>(a, L.small_items, ordered_keys, grid, r.stream);
+          launched = true;
         }
       }
       if constexpr (VIRT_OK) {
