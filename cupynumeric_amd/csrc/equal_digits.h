@@ -204,7 +204,8 @@ inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
   // stay well below
   const uint64_t share = 4ull * tile * EQ_SAMPLE * EQ_SAMPLE / (5 * n);
   l.close              = static_cast<uint32_t>(share > EQ_SAMPLE * 9 / 20 ? share : EQ_SAMPLE * 9 / 20);
-  // every key one of 16 equal ones, or a smaller share of them one of more
+  // Every key one of 32 equal ones, or a smaller share of them one of more (a pair counts once; of three keys in a bucket,
+  // two of them equal, it depends on the third, so that rows near the limit may go either way).
   l.equal = static_cast<uint32_t>((16ull * EQ_SAMPLE * EQ_SAMPLE) / n) + 1;
   return l;
 }

@@ -229,16 +229,15 @@ def _long_row(torch, kind, log2):
     if kind == "uniform":
         return torch.rand(n, generator=gen, device="cuda", dtype=torch.float64)
     x = torch.randn(n, generator=gen, device="cuda", dtype=torch.float64)
-    if kind == "repeated":  # every value forty times
-        return x[: n // 40][torch.randint(0, n // 40, (n,), generator=gen, device="cuda")]
+    if kind == "repeated":  # every value two hundred times
+        return x[: n // 200][torch.randint(0, n // 200, (n,), generator=gen, device="cuda")]
     if kind.endswith("groups"):  # neighbouring numbers in far groups of n / count keys
         count = int(kind.split()[0])
         return (torch.randint(0, count, (n,), generator=gen, device="cuda") << 32) + torch.randint(0, 1 << 16, (n,), generator=gen, device="cuda")
     return x
 
 
-# The shortest rows that are tried by default, and the length at which 2.0 is too dense among normal keys.  (The sample is
-# drawn at fixed places: the same rows give the same plan every time.)
+# The shortest rows that are tried by default, and the length at which 2.0 is too dense among normal keys.
 @pytest.mark.parametrize("kind,log2,mode", [("uniform", 25, 1), ("normal", 25, 1), ("uniform", 26, 1), ("normal", 26, 0), ("repeated", 25, 0),
                                             ("repeated", 26, 0), ("5000 groups", 26, 0), ("20000 groups", 26, 0)])
 def test_long_rows_that_do_not_fit_keep_the_byte_passes(lib, torch_cuda, kind, log2, mode):
