@@ -210,12 +210,13 @@ inline uint64_t merged_row_split_bytes(uint64_t volume, uint64_t seg, int levels
 // Requests of few keys, real keys of 4 and 8 bytes: rows cut into short pieces, all merged by rank in one launch
 // (merge_rows.h).  Returns the pieces' length, 0: another path.  (cpn_set_merge_rows: in the default mode only.)
 // Where the lines lie (us per call through the Python API, this way / the way it took before, sort and argsort):
-//   from where one workgroup per row is left (RANK_MIN_ROW_*): normal float64 8193 keys 25, 26 / 24, 28, 10 000 25,
-//   27 / 29, 32, 12 289 26, 27 / 37, 43, uniform 24, 26 / 21, 23, 24, 26 / 23, 26 and 25, 26 / 29, 31, int64 23, 24 /
-//   20, 23, 23, 24 / 23, 26 and 24, 24 / 28, 31; normal float32 12 289 23, 24 / 29, 28, 14 000 23, 24 / 30, 31, 16 384
-//   24, 25 / 28, 34, int32 22, 23 / 21, 22, 23, 23 / 23, 23 and 23, 23 / 21, 25.  What this way loses: rows of equal
-//   keys, which one workgroup sees to without a pass (9000 float64 22 / 13).  (Only single rows of up to
-//   lds_row_capacity keys: the other way needs no workspace, and several rows keep as many workgroups busy.)
+//   from where one workgroup per row is left (ranked_min_row): normal float64 10 000 keys with positions 25 / 33, 11 000
+//   24, 25 / 32, 36, 12 289 24, 25 / 39, 42, uniform 10 000 with positions 24 / 26, 11 000 22, 25 / 24, 28, int64 23 /
+//   26 and 22, 23 / 25, 28; normal float32 12 289 21, 22 / 29, 29, 16 384 22, 23 / 27, 35, int32 19, 20 / 22, 22 and 20,
+//   21 / 23, 26.  Below, 9000 evenly spread float64 keys took 24, 26 / 21, 24 (two of them a status word that this way no
+//   longer copies), normal ones 25, 26 / 25, 30.  What this way loses: rows of equal keys, which one workgroup sees to
+//   without a pass (9000 float64 22 / 13).  (Only single rows of up to lds_row_capacity keys: the other way needs no
+//   workspace, and several rows keep as many workgroups busy.)
 //   to where the work, which grows with the square of the row, eats the launches saved: 262 144 uint32 68, 72 /
 //   86, 98, float32 75, 80 / 89, 99, 400 000 uint32 147, 152 / 86, 106; float64 200 000 104, 96 / 124, 132,
 //   262 144 127, 119 / 123, 131.  Levels of merging take 8-byte integers faster: 160 000 74, 73 / 75, 82, 200 000 89,
@@ -224,9 +225,8 @@ inline uint64_t merged_row_split_bytes(uint64_t volume, uint64_t seg, int levels
 //   (4096) and 27, 31 (8192), 65 536 34, 35 and 31, 35, 131 072 56, 58 and 39, 44; float64 sort 65 536 40 and 47,
 //   131 072 65 and 59, argsort 32 768 33 and 38, 65 536 41 and 41, 131 072 67 and 51.
 constexpr uint64_t RANK_MAX_VOLUME = 1ull << 18;
-constexpr uint64_t RANK_MIN_ROW_4  = 13312;
-constexpr uint64_t RANK_MIN_ROW_8  = 10240;
 bool merge_rows_default();
+inline uint64_t ranked_min_row(int key_bytes, bool want_indices) { return key_bytes == 4 ? 12288 : (want_indices ? 9216 : 10240); }
 inline uint64_t ranked_max_volume_8(int codec, bool want_indices)
 {
   if (codec == CODEC_FLOAT) {
@@ -239,7 +239,7 @@ inline uint64_t ranked_row_piece(int key_bytes, int passes, int codec, uint64_t 
   const uint64_t cap = lds_row_capacity(key_bytes, want_indices);
   if (!merge_rows_default() || (key_bytes != 4 && key_bytes != 8) || passes != key_bytes ||
       lds_row_limit(key_bytes, want_indices) != cap || volume > RANK_MAX_VOLUME ||
-      seg <= (key_bytes == 4 ? RANK_MIN_ROW_4 : RANK_MIN_ROW_8) || (seg <= cap && volume != seg) ||
+      seg <= ranked_min_row(key_bytes, want_indices) || (seg <= cap && volume != seg) ||
       (key_bytes == 8 && volume > ranked_max_volume_8(codec, want_indices))) {
     return 0;
   }

@@ -117,9 +117,9 @@ def _merged_by_rank(lib, torch, x, argsort):
 
 
 @pytest.mark.parametrize("dtype,argsort,first,last", [
-    (np.float32, False, 13_313, 262_144), (np.int32, True, 13_313, 262_144),
-    (np.float64, False, 10_241, 212_992), (np.float64, True, 10_241, 262_144),
-    (np.int64, False, 10_241, 163_840), (np.uint64, True, 10_241, 212_992)])
+    (np.float32, False, 12_289, 262_144), (np.int32, True, 12_289, 262_144),
+    (np.float64, False, 10_241, 212_992), (np.float64, True, 9217, 262_144),
+    (np.int64, False, 10_241, 163_840), (np.uint64, True, 9217, 212_992)])
 def test_the_lines_of_the_path(lib, torch_cuda, dtype, argsort, first, last):
     """Rows outside them are sorted sooner the other way (int64 with positions, 262 144: 94 us against 110)."""
     for n, by_rank in ((first - 1, False), (first, True), (last, True), (last + 1, False)):
