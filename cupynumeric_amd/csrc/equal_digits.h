@@ -14,8 +14,8 @@
 // too large for it are in order already when all their keys are equal (that is what makes most of
 // them large: a value that occurs often).
 //
-// When the sample shows buckets that are too large and hold different keys, the row keeps the byte
-// passes.  When that is seen only after the two passes, the byte passes run on what those left, which
+// When the sample shows buckets that are too large and hold different keys, or keys so close that the sort in LDS would
+// not take them (eq_limits), the row keeps the byte passes.  When that is seen only after the two passes, the byte passes run on what those left, which
 // is a stable arrangement of the input and therefore sorts to the same result.
 //
 // The reference's cub::DeviceRadixSort (src/cupynumeric/sort/cub_sort.cuh:60-182) always runs
@@ -655,8 +655,9 @@ __global__ __launch_bounds__(EQ_SEGMENT_BLOCK) void eq_segments_kernel(const Key
 // its key with all of the bin.
 // Pieces that hold a NaN or a -0.0, more than a workgroup's worth of keys in a bin, or too many bins for the workgroup, go
 // on the general sort's list.
-// Bound by vector instructions.  Comparing every key with the others of its bin, as lds_row_sort_kernel does,
-// took 156 of them per key: 2^26 float64 keys 0.46 ms, and 0.50 ms in that kernel.
+// Bound by vector instructions: 2^26 float64 keys 0.40 ms (1.07 GB).  Comparing every key with the others of its bin, as
+// lds_row_sort_kernel does, takes 156 of them per key (0.50 ms in that kernel when this one took 0.46, with a grid that
+// did not fit at once).
 constexpr int EQ_SORT_BLOCK       = 512;
 constexpr int EQ_SORT_ITEMS       = 6;
 // Waves per SIMD, and with them workgroups per CU (three).  At 80 registers a dozen values are spilled, addresses and
