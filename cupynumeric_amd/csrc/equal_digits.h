@@ -169,10 +169,14 @@ __global__ __launch_bounds__(EQ_GATHER_BLOCK) void eq_gather_kernel(const KeyT* 
 //   - when a bucket that `crowd` and more of the sampled keys fall into holds different ones;
 //   - when such a bucket holds one key, and its cell other keys as well that do not crowd theirs (a value that
 //     occurs often among keys that are close to it: some are bound to share its bucket);
+//   - when the cells of floats are half an octave or wider: rows that span zero, or hold one, whose images reach over
+//     the magnitudes that do not occur (2050 octaves for both signs, cells of two).  A density that falls off inside such
+//     a cell leaves a few buckets too large, and those of the tails hold too few sampled keys to show it: of 2^26 normal
+//     keys a bucket at 2.0 holds 11 100, and 45 10^6 keys of three times that spread failed in 15 of 16 rows, of a
+//     logistic distribution in 2, 2^26 of the latter in 15; accepted and then sorted again they took 1.65 times the byte
+//     passes (which 2^25 normal keys, that would fit, keep as well: 1290 us instead of 740);
 //   - when `dense` and more sampled keys outside such buckets fall into 2^group_log2 neighbouring buckets: the density
-//     varies too much inside a cell.  (2^26 normal keys of both signs: their images span 2050 octaves, a cell two
-//     of them, and a bucket at 2.0 holds 11 100 keys where the average is 1024; 2^25 of them still fit.  Accepted, they
-//     took 4.1 ms, 2.5 by the byte passes.)
+//     varies too much inside a cell;
 //   - when `close` and more ordered pairs of sampled keys share a bucket (16384 evenly spread keys: 4700): the keys
 //     stand in clusters narrower than a bucket, e.g. a few thousand groups of neighbouring numbers;
 //   - when `equal` and more sampled keys find one in their bucket that would share a bin of the LDS sort with them:
@@ -193,8 +197,7 @@ inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
   l.crowd           = static_cast<uint32_t>(mean + 3.5 * __builtin_sqrt(mean));
   l.crowd           = l.crowd > 7 ? l.crowd : 7;
   // Windows of as many buckets (n / 2^21, a power of two) as hold 60 to 120 sampled keys at three quarters of what fits,
-  // and 4.6 to 18 of evenly spread ones.  The densest of 2^25 normal keys holds 43 (and is taken for too dense once in
-  // 250 rows), of 2^26 of them 87 (and is missed once in 100).
+  // and 4.6 to 18 of evenly spread ones.
   l.group_log2 = 4;
   while (l.group_log2 < 7 && (1ull << (21 + l.group_log2)) < n) {
     ++l.group_log2;
@@ -210,6 +213,8 @@ inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
   return l;
 }
 constexpr int EQ_MIN_BYTES = 5;
+// Cells of half an octave (2^52 images of 8-byte floats) and wider: see above.
+constexpr uint32_t EQ_MAX_FLOAT_SHIFT = 51;
 constexpr int EQ_MARK_BITS = 11;  // a bucket of evenly spread keys is 910 (2^25 keys) to 3640 bins (2^27) of the LDS sort
 template <typename KeyT, int CODEC>
 __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __restrict__ ranges,
@@ -306,6 +311,9 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
   uint32_t shift = 0;
   while (((hi - lo) >> shift) > static_cast<uint64_t>(CELLS - 2 * EXTRA - 2)) {
     ++shift;
+  }
+  if (CODEC == CODEC_FLOAT && shift >= EQ_MAX_FLOAT_SHIFT) {
+    return;  // uniform; mode 0
   }
   constexpr uint32_t TOP  = 8 * sizeof(KeyT) - CB;  // (shift <= TOP: the whole range is CELLS cells then)
   const uint64_t below    = static_cast<uint64_t>(EXTRA) << shift;
@@ -671,8 +679,8 @@ constexpr int EQ_BINS             = 4096;  // two 16-bit counters per word
 // with positions, whose order the counting atomic leaves mixed; 2.3 now, the byte passes 3.2.)
 constexpr uint32_t EQ_BIN_LIMIT   = 8;
 // Bins for the whole workgroup, one after the other: with more of them the general sort is the faster one.  (Pieces of
-// many sparse buckets and a full one, whose keys share a few bins: the sort of 2^25 normal float64 keys 802 us without
-// this limit, now 742.)
+// many sparse buckets and a full one, whose keys share a few bins: 2^25 keys with a dozen such pieces took 802 us
+// without this limit, 742 with it.)
 constexpr uint32_t EQ_LARGE_BINS  = 6;
 constexpr int EQ_FRACTION_BITS    = 14;    // of a bucket, for the bins
 

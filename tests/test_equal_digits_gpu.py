@@ -151,9 +151,9 @@ def _check(lib, torch, x, mode, failed, what):
 
 
 # (uint64 "bits": few bytes vary; the others that keep the byte passes: a value that occurs often has keys in its cell that
-# do not, +inf in that of the NaNs, any integer in those of the smallest and the largest)
+# do not, any integer in those of the smallest and the largest; float rows that span zero have cells of two octaves)
 @pytest.mark.parametrize("dtype,kind,mode,failed", [
-    (np.float64, "spread", 1, 0), (np.float64, "normal", 1, 0), (np.float64, "repeated", 1, 0), (np.float64, "specials", 0, 0),
+    (np.float64, "spread", 1, 0), (np.float64, "normal", 0, 0), (np.float64, "repeated", 0, 0), (np.float64, "specials", 0, 0),
     (np.int64, "spread", 1, 0), (np.uint64, "specials", 0, 0), (np.int64, "crowd", 0, 0), (np.uint64, "bits", 0, 0)])
 def test_the_path_that_is_taken(lib, torch_cuda, dtype, kind, mode, failed):
     x = _keys(kind, dtype, 700_001, np.random.default_rng(7)).astype(dtype, copy=False)
@@ -191,8 +191,7 @@ def test_few_values_keep_the_pass_on_their_ranks(lib, torch_cuda, both_threshold
     _check(lib, torch_cuda, values[rng.integers(0, 200, 300_001)], 0, 0, "few values")
 
 
-@pytest.mark.parametrize("dtype", [np.int64, np.float64])
-@pytest.mark.parametrize("bytes_that_vary", [6, 8])
+@pytest.mark.parametrize("dtype,bytes_that_vary", [(np.int64, 6), (np.int64, 8), (np.float64, 6), (np.uint64, 8)])
 def test_late_failure_goes_on_with_grouped_digits(lib, torch_cuda, both_thresholds_lowered, dtype, bytes_that_vary):
     """Few values in every byte: three groups of two bytes (an odd number of passes) and four."""
     rng = np.random.default_rng(bytes_that_vary)
@@ -229,7 +228,13 @@ def _long_row(torch, kind, log2):
     if kind == "uniform":
         return torch.rand(n, generator=gen, device="cuda", dtype=torch.float64)
     x = torch.randn(n, generator=gen, device="cuda", dtype=torch.float64)
+    if kind == "logistic":
+        u = torch.rand(n, generator=gen, device="cuda", dtype=torch.float64)
+        return torch.log(u / (1 - u))
+    if kind == "wide":
+        return 3 * x
     if kind == "repeated":  # every value two hundred times
+        x = x.abs()
         return x[: n // 200][torch.randint(0, n // 200, (n,), generator=gen, device="cuda")]
     if kind.endswith("groups"):  # neighbouring numbers in far groups of n / count keys
         count = int(kind.split()[0])
@@ -237,9 +242,9 @@ def _long_row(torch, kind, log2):
     return x
 
 
-# The shortest rows that are tried by default, and the length at which 2.0 is too dense among normal keys.
-@pytest.mark.parametrize("kind,log2,mode", [("uniform", 25, 1), ("normal", 25, 1), ("uniform", 26, 1), ("normal", 26, 0), ("repeated", 25, 0),
-                                            ("repeated", 26, 0), ("5000 groups", 26, 0), ("20000 groups", 26, 0)])
+# (The shortest rows that are tried by default.)
+@pytest.mark.parametrize("kind,log2,mode", [("uniform", 25, 1), ("normal", 25, 0), ("uniform", 26, 1), ("normal", 26, 0), ("repeated", 25, 0),
+                                            ("repeated", 26, 0), ("5000 groups", 26, 0), ("20000 groups", 26, 0), ("logistic", 26, 0), ("wide", 26, 0)])
 def test_long_rows_that_do_not_fit_keep_the_byte_passes(lib, torch_cuda, kind, log2, mode):
     """The plan declines them; none is sorted twice (2^26 normal keys: 2.5 ms, and 4.1 when that was seen too late)."""
     torch = torch_cuda
@@ -296,3 +301,22 @@ def test_rows_of_narrow_clusters_keep_the_byte_passes(lib, torch_cuda):
     """300 000 groups of a hundred neighbouring numbers each, all of a group in one bin of the LDS sort: 4 to 8 times the
     byte passes' time when every piece had its bins put in order one by one."""
     test_long_rows_that_do_not_fit_keep_the_byte_passes(lib, torch_cuda, "300000 groups", 25, 0)
+
+
+@pytest.mark.parametrize("n", [(1 << 18), (1 << 18) + 1, 16384 * 17 - 1, 16384 * 17, 2304 * 120, 2304 * 120 + 1, 3072 * 100 - 1])
+def test_lengths_of_evenly_spread_rows(lib, torch_cuda, n):
+    """As test_lengths, with keys that take the path."""
+    rng = np.random.default_rng(n)
+    _check(lib, torch_cuda, rng.random(n), 1, 0, f"{n}")
+    _check(lib, torch_cuda, rng.integers(-(1 << 63), (1 << 63) - 1, n), 1, 0, f"{n} int64")
+
+
+def test_special_values_among_huge_keys(lib, torch_cuda):
+    """Keys so large that the cells reach the infinity and the NaNs above them: pieces that hold a NaN go the general way."""
+    rng = np.random.default_rng(2)
+    x = 10.0 ** rng.uniform(280, 308, 500_003)
+    x[rng.random(x.size) < 0.0005] = np.nan
+    x[rng.random(x.size) < 0.0005] = np.inf
+    x.view(np.uint64)[::50_021] = 0x7FF8_0000_0000_1234  # a payload
+    _check(lib, torch_cuda, x, 1, 0, "huge keys")
+    assert _sort(lib, torch_cuda, x, True, True)[3][4] > 0
