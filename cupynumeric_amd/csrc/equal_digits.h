@@ -190,14 +190,14 @@ struct EqualLimits {
 inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
 {
   EqualLimits l{};
-  // A bucket that just fits holds `mean` sampled keys on average (5 of 2^25 keys, 1.25 of 2^27), and one of evenly
+  // A bucket that just fits holds `mean` sampled keys on average (5 of 2^25 keys, 2.5 of 2^26), and one of evenly
   // spread keys 0.29: three and a half standard deviations above the former are a crowd, and never fewer than seven
   // (which one row in 700 of the latter has in some bucket).
   const double mean = static_cast<double>(fits) * EQ_SAMPLE / static_cast<double>(n);
   l.crowd           = static_cast<uint32_t>(mean + 3.5 * __builtin_sqrt(mean));
   l.crowd           = l.crowd > 7 ? l.crowd : 7;
   // Windows of as many buckets (n / 2^21, a power of two) as hold 60 to 120 sampled keys at three quarters of what fits,
-  // and 4.6 to 18 of evenly spread ones.
+  // and 4.6 to 9.1 of evenly spread ones.
   l.group_log2 = 4;
   while (l.group_log2 < 7 && (1ull << (21 + l.group_log2)) < n) {
     ++l.group_log2;
@@ -215,7 +215,7 @@ inline EqualLimits eq_limits(uint64_t n, uint32_t fits, uint32_t tile)
 constexpr int EQ_MIN_BYTES = 5;
 // Cells of half an octave (2^52 images of 8-byte floats) and wider: see above.
 constexpr uint32_t EQ_MAX_FLOAT_SHIFT = 51;
-constexpr int EQ_MARK_BITS = 11;  // a bucket of evenly spread keys is 910 (2^25 keys) to 3640 bins (2^27) of the LDS sort
+constexpr int EQ_MARK_BITS = 11;  // a bucket of evenly spread keys is 910 (2^25 keys) or 1820 bins (2^26) of the LDS sort
 template <typename KeyT, int CODEC>
 __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __restrict__ ranges,
                                                                   const KeyT* __restrict__ sample,

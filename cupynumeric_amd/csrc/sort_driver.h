@@ -60,13 +60,17 @@ uint64_t virtual_digit_threshold();
 //   from 2^25: uniform float64 720, 864 / 1300, 1682, int64 711, 877 / 1294, 1655.  Shorter rows that suit it gain as
 //   well (2^24 428, 517 / 698, 918, 2^22 174, 201 / 228, 261), but a row that the plan declines pays for the sample, the
 //   plan and seven launches that find nothing to do: 2^22 values that repeat 40 times 274, 305 / 228, 258 (20 %), 2^24
-//   758, 964 / 710, 918 (7 %), 2^25 1345, 1749 / 1290, 1687 (4 %), 2^26 2542, 3262 / 2479, 3200 (2 %), 2^27 2 %; 2^26
+//   758, 964 / 710, 918 (7 %), 2^25 1345, 1749 / 1290, 1687 (4 %), 2^26 2542, 3262 / 2479, 3200 (2 %); 2^26
 //   keys of 100 values, which take one pass on their ranks, 833, 662 / 792, 626 (5 %).
-//   to 2^27: a bucket of 2^28 evenly spread keys holds more than the tile of the LDS sort.
+//   to 2^26: a cell that the sample misses gets four buckets, which fit up to 41 000 keys between them, the share of ten
+//   sampled ones in 2^26 keys (missed once in 22 000) and of five in 2^27 (once in 150, and a row has hundreds of such
+//   cells).  Of 2^27 keys, evenly spread ones took 2762, 3367 / 4782, 6182, but 5 of 68 rows of other distributions (the
+//   square of normal keys, Weibull, normal around 1000, int64 spread over magnitudes) failed after their passes, at 1.65 times
+//   the byte passes' time; none of 144 of 2^26 keys did.
 // What the sample cannot see costs most: 2^25 keys, a quarter of them one value with two neighbours that share its
 // bucket, are sorted twice, 2201, 2863 / 1347, 1715.
 constexpr uint64_t EQ_MIN_ROW_ELEMENTS = 1ull << 25;
-constexpr uint64_t EQ_MAX_ROW_ELEMENTS = 1ull << 27;
+constexpr uint64_t EQ_MAX_ROW_ELEMENTS = 1ull << 26;
 uint64_t equal_digit_threshold();
 // The stretch of the row whose bucket starts make one piece of the LDS sort (the rest of its tile is for the last
 // bucket to reach into), and the shape of the general sort that takes what that one does not.

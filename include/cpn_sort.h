@@ -451,7 +451,7 @@ int64_t cpn_set_virtual_digit_threshold(int64_t elements);
 
 /*
  * Process-wide tunable: a 1-D sort of real 8-byte keys with at least `elements` elements (and 2^18, and at most
- * 2^27) lets the device sort it by two passes on digits made from a sample of the keys and one sort in LDS
+ * 2^26) lets the device sort it by two passes on digits made from a sample of the keys and one sort in LDS
  * instead of the byte passes (cupynumeric_amd/csrc/equal_digits.h).  Results do not depend on it.  The default is
  * 2^25; a negative value restores it and the previous setting is returned.  It changes the workspace that
  * cpn_local_sort_temp_bytes asks for; the sort also takes the smaller one, and then runs the byte passes.  Also

@@ -391,6 +391,18 @@ def test_merged_row_levels_and_workspace_over_the_limits(lib):
     assert 65537 * 4 < temp(f32, 65537, False) < 2 * 65536 * 4
 
 
+def test_rows_that_are_tried_with_equalised_digits(lib):
+    """2^25 to 2^26 real 8-byte keys in one row; longer ones have cells that a sample of 16 384 keys misses."""
+    sizes = [(1 << 25) - 1, 1 << 25, 1 << 26, (1 << 26) + 1, 1 << 27]
+    asked = [lib.cpn_local_sort_temp_bytes(11, n, n, 1, 0, 0) for n in sizes]
+    prev = lib.cpn_set_equal_digit_threshold(1 << 40)
+    try:
+        without = [lib.cpn_local_sort_temp_bytes(11, n, n, 1, 0, 0) for n in sizes]
+    finally:
+        lib.cpn_set_equal_digit_threshold(prev)
+    assert [a > w for a, w in zip(asked, without)] == [False, True, True, False, False]
+
+
 def test_only_sorts_with_a_bounded_wait_need_a_check(lib):
     """Requests that one workgroup per row sorts, or whose sorted pieces are merged, have no status to look at: an eager
     caller waited for the device to read it."""
