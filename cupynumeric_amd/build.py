@@ -59,7 +59,7 @@ HIPCC_FLAGS = [
 # refuses it.  The scatter pass of the global sort is allowed the few words it is known to park.
 # (So is the sort of equalised pieces, csrc/equal_digits.h, and their plan, a single workgroup.)
 SCRATCH_LIMITS = (("row_sort_kernel", 0), ("count16_", 0), ("onesweep_kernel", 32), ("merge_ranks_kernel", 0),
-                  ("eq_sweep_kernel", 0), ("eq_sort_kernel", 80), ("eq_plan_kernel", 96), ("eq_gather_kernel", 0),
+                  ("eq_sweep_kernel", 0), ("eq_sort_kernel", 80), ("eq_plan_kernel", 128), ("eq_gather_kernel", 0),
                   ("eq_histogram_kernel", 0), ("eq_segments_kernel", 0))
 
 
