@@ -196,7 +196,7 @@ void lds_row_sort_kernel(const KeyT* keys_in,
   constexpr int CTR_WORDS = (BUCKETS_OK && BINS > WAVES * RADIX) ? BINS : WAVES * RADIX;
   __shared__ __align__(16) uint32_t s_ctr[CTR_WORDS];
   uint32_t* const s_bins = s_ctr;
-  __shared__ uint32_t s_wsum[DT::WAVES];
+  __shared__ uint32_t s_wsum[WAVES > DT::WAVES ? WAVES : DT::WAVES];  // (the split sums every wave, the passes those that scan digits)
   __shared__ SW s_red[2 * WAVES * NW];
 
   do {
