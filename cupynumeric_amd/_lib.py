@@ -49,6 +49,7 @@ CPN_ERR_SCRATCH = -9
 
 # include/cpn_sort.h: options of cpn_local_sort_ex
 CPN_SORT_SINGLE_TICKET = 1
+CPN_SORT_SPLIT = 4
 
 # include/cpn_sort.h: workspace of cpn_local_sort_static
 STATIC_SCRATCH_BYTES = 64 << 20
@@ -70,6 +71,7 @@ PROTOTYPES: dict[str, tuple] = {
     "cpn_dtype_size": (c_uint64, [c_int]),
     "cpn_key_order_bits": (c_uint64, [c_int, c_uint64]),
     "cpn_local_sort_temp_bytes": (c_uint64, [c_int, c_uint64, c_uint64, c_int, c_int, c_int]),
+    "cpn_local_sort_split_temp_bytes": (c_uint64, [c_int, c_uint64, c_uint64, c_int]),
     "cpn_local_sort": (
         c_int,
         [c_int, c_void_p, c_void_p, c_void_p, c_uint64, c_uint64, c_int64, c_int, c_void_p, c_uint64, c_void_p],

@@ -17,6 +17,10 @@ if TYPE_CHECKING:
     from ._thunk import DeviceArray
 
 
+# Shorter rows are never split (`cpn_local_sort_split_temp_bytes`); asking would cost them a call.
+SPLIT_MIN_ROW = 6145
+
+
 def sort_flattened(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable: bool) -> None:
     """`axis=None` on an array of several dimensions (`cupynumeric/_thunk/_sort.py:37-47`): the
     C-order flattening is a view of the same dense storage, its 1-D sort is the result."""
@@ -69,6 +73,16 @@ def sort_task(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable
         values_out = output.base.ptr()
         indices_out = None
 
+    stream = ctypes.c_void_p(runtime.stream_handle())
+    if seg >= SPLIT_MIN_ROW:
+        temp_bytes = lib.cpn_local_sort_split_temp_bytes(code, volume, seg, int(argsort))
+        if temp_bytes != 0:  # two launches that cannot fail on the device: no status to look at
+            temp = runtime.empty_bytes(temp_bytes)
+            status = lib.cpn_local_sort_ex(code, values_in, values_out, indices_out, volume, seg, 0, int(stable),
+                                           _lib.CPN_SORT_SPLIT, temp.data_ptr(), temp_bytes, stream)
+            _lib.check(status, "cpn_local_sort")
+            return
+
     temp_bytes = lib.cpn_local_sort_temp_bytes(code, volume, seg, int(not argsort), int(argsort), int(in_place))
     if temp_bytes == 0:
         _lib.check(
@@ -76,7 +90,6 @@ def sort_task(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable
             "cpn_local_sort",
         )
         raise NotImplementedError(f"cpn_local_sort: no workspace layout for dtype={input.dtype}, shape={input.shape}")
-    stream = ctypes.c_void_p(runtime.stream_handle())
 
     def issue(options: int = 0):
         temp = runtime.empty_bytes(temp_bytes)

@@ -101,6 +101,23 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_dpp_impl(uint32_t v)
 __device__ __forceinline__ uint32_t wave_inclusive_sum_dpp(uint32_t v) { return wave_inclusive_scan_dpp_impl<false>(v); }
 __device__ __forceinline__ uint32_t wave_inclusive_max_dpp(uint32_t v) { return wave_inclusive_scan_dpp_impl<true>(v); }
 
+// The largest value of a wave (any unsigned type of 4 or 8 bytes; of 8: the largest upper half, then the largest lower
+// half beside it); uniform.
+template <typename T>
+__device__ __forceinline__ T wave_max_dpp(T v)
+{
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32- or 64-bit values");
+  auto last = [](uint32_t x) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), WAVE - 1)); };
+  if constexpr (sizeof(T) == 4) {
+    return static_cast<T>(last(wave_inclusive_max_dpp(static_cast<uint32_t>(v))));
+  } else {
+    const uint32_t upper = static_cast<uint32_t>(static_cast<uint64_t>(v) >> 32);
+    const uint32_t hi    = last(wave_inclusive_max_dpp(upper));
+    const uint32_t lo    = last(wave_inclusive_max_dpp(upper == hi ? static_cast<uint32_t>(v) : 0u));
+    return static_cast<T>((static_cast<uint64_t>(hi) << 32) | lo);
+  }
+}
+
 // AND / OR of one 32-bit value per lane over the whole wave, through the same DPP steps (lanes
 // without a source keep the identity); the result is read from the last lane and is uniform.
 template <bool IS_AND>

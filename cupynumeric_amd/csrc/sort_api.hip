@@ -10,6 +10,7 @@
 #include <mutex>
 
 #include "sort_driver.h"
+#include "split_plan.h"
 
 // Device memory for cpn_local_sort_static: the workspace of a sort that may not allocate.  One
 // copy of the array exists on every GPU that loads this library, for the life of the process.
@@ -347,6 +348,17 @@ uint64_t cpn_local_sort_temp_bytes(int dtype, uint64_t volume, uint64_t sort_dim
   return cpn::workspace_bytes(k.bytes, cpn::key_passes(k.bytes, k.codec), k.codec, volume, sort_dim_size, want_values != 0, want_indices != 0, in_place != 0);
 }
 
+uint64_t cpn_local_sort_split_temp_bytes(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_indices)
+{
+  const cpn::KeyKind k = cpn::key_kind(dtype);
+  if (k.bytes == 0 || k.codec < 0 || volume == 0 || sort_dim_size == 0 || volume % sort_dim_size != 0) {
+    return 0;
+  }
+  const bool has_idx        = want_indices != 0;
+  const cpn::SplitPlan plan = cpn::split_plan(k.bytes, cpn::key_passes(k.bytes, k.codec), volume, sort_dim_size, has_idx);
+  return plan.buckets == 0 ? 0 : cpn::split_layout(plan, k.bytes, volume, has_idx).total;
+}
+
 int cpn_local_sort(int dtype, const void* values_in, void* values_out, int64_t* indices_out, uint64_t volume,
                    uint64_t sort_dim_size, int64_t index_offset, int stable, void* temp, uint64_t temp_bytes,
                    void* stream)
@@ -360,7 +372,7 @@ int cpn_local_sort_ex(int dtype, const void* values_in, void* values_out, int64_
                       uint64_t temp_bytes, void* stream)
 {
   (void)stable;  // every path is stable
-  if ((options & ~static_cast<uint32_t>(CPN_SORT_SINGLE_TICKET)) != 0) {
+  if ((options & ~static_cast<uint32_t>(CPN_SORT_SINGLE_TICKET | CPN_SORT_SPLIT)) != 0) {
     return CPN_ERR_UNSUPPORTED;
   }
   const cpn::KeyKind k = cpn::key_kind(dtype);
@@ -395,6 +407,13 @@ int cpn_local_sort_ex(int dtype, const void* values_in, void* values_out, int64_
   r.temp_bytes   = temp_bytes;
   r.stream       = static_cast<hipStream_t>(stream);
   r.single_ticket = (options & CPN_SORT_SINGLE_TICKET) != 0;
+  if ((options & CPN_SORT_SPLIT) != 0 && temp != nullptr && (reinterpret_cast<uintptr_t>(temp) % cpn::WORKSPACE_ALIGN) == 0) {
+    const bool has_idx        = indices_out != nullptr;
+    const cpn::SplitPlan plan = cpn::split_plan(k.bytes, cpn::key_passes(k.bytes, k.codec), volume, sort_dim_size, has_idx);
+    if (plan.buckets != 0 && temp_bytes >= cpn::split_layout(plan, k.bytes, volume, has_idx).total) {
+      return k.bytes == 4 ? cpn::sort_split32(k.codec, r, plan) : cpn::sort_split64(k.codec, r, plan);
+    }
+  }
   switch (k.bytes) {
     case 1: return cpn::sort_keys8(k.codec, r);
     case 2: return cpn::sort_keys16(k.codec, r);

@@ -1,0 +1,84 @@
+// Host side of split_sort.h: one call sorts the row of a request that split_plan (split_plan.h) accepts.
+#pragma once
+
+#include "split_plan.h"
+
+namespace cpn {
+
+template <typename KeyT, int CODEC, bool HAS_IDX>
+inline int sort_row_split(const SortRequest& r, const SplitPlan& p)
+{
+  // (float keys that tie need not be the same bits, but a bucket's keys stay in the order of the row on both ways, so
+  // nothing but a request for positions needs their places)
+  const SplitLayout L = split_layout(p, sizeof(KeyT), r.seg, HAS_IDX);
+  uint8_t* const ws   = static_cast<uint8_t*>(r.temp);
+  KeyT* grouped       = reinterpret_cast<KeyT*>(ws + L.off_keys);
+  uint16_t* places    = HAS_IDX ? reinterpret_cast<uint16_t*>(ws + L.off_places) : nullptr;
+  uint16_t* starts    = reinterpret_cast<uint16_t*>(ws + L.off_starts);
+  const uint32_t n    = static_cast<uint32_t>(r.seg);
+  KeyT* sample        = nullptr;
+  if (p.gathered) {
+    sample                 = reinterpret_cast<KeyT*>(ws + L.off_sample);
+    const uint32_t samples = p.buckets * p.per_bucket;
+    ProfileScope prof("split_gather", r.stream);
+    hipLaunchKernelGGL((split_gather_kernel<KeyT>), dim3(samples / 256), dim3(256), 0, r.stream,
+                       static_cast<const KeyT*>(r.values_in), n, samples, sample);
+    CPN_HIP_TRY(hipGetLastError());
+  }
+  {
+    ProfileScope prof("split_tiles", r.stream);
+    const dim3 grid(p.tiles);
+    auto launch = [&](auto per_thread, auto per_bucket) {
+      hipLaunchKernelGGL((split_tile_kernel<KeyT, CODEC, HAS_IDX, decltype(per_thread)::value, decltype(per_bucket)::value, SPLIT_TILE_ITEMS>),
+                         grid, dim3(SPLIT_BLOCK), 0, r.stream, static_cast<const KeyT*>(r.values_in), n, p.tile_len,
+                         sample, grouped, places, starts, static_cast<uint32_t*>(r.temp));
+    };
+    using C1 = std::integral_constant<int, 1>;
+    using C8 = std::integral_constant<int, 8>;
+    switch (p.buckets) {
+      case 128: launch(C1{}, C8{}); break;
+      case 256:
+        if (p.per_bucket == 4) {
+          launch(C1{}, std::integral_constant<int, 4>{});
+        } else {
+          launch(std::integral_constant<int, 2>{}, C8{});
+        }
+        break;
+      case 512: launch(std::integral_constant<int, 4>{}, C8{}); break;
+      case 1024: launch(C8{}, C8{}); break;
+      default: return CPN_ERR_UNSUPPORTED;
+    }
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    SplitBuckets<KeyT> sb{};
+    sb.grouped  = grouped;
+    sb.places   = places;
+    sb.starts   = starts;
+    sb.ids      = reinterpret_cast<uint32_t*>(ws + L.off_ids);
+    sb.n        = n;
+    sb.tiles    = p.tiles;
+    sb.tile_len = p.tile_len;
+    sb.buckets  = p.buckets;
+    ProfileScope prof("split_buckets", r.stream);
+    hipLaunchKernelGGL((split_bucket_kernel<KeyT, CODEC, HAS_IDX, SPLIT_BUCKET_BLOCK, SPLIT_BUCKET_ITEMS>),
+                       dim3(p.buckets), dim3(SPLIT_BUCKET_BLOCK), 0, r.stream, sb,
+                       static_cast<KeyT*>(r.values_out), r.indices_out, r.index_offset);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  return CPN_OK;
+}
+
+template <typename KeyT>
+inline int sort_split(int codec, const SortRequest& r, const SplitPlan& p)
+{
+  const bool idx = r.indices_out != nullptr;
+  switch (codec) {
+    case CODEC_UNSIGNED: return idx ? sort_row_split<KeyT, CODEC_UNSIGNED, true>(r, p) : sort_row_split<KeyT, CODEC_UNSIGNED, false>(r, p);
+    case CODEC_SIGNED: return idx ? sort_row_split<KeyT, CODEC_SIGNED, true>(r, p) : sort_row_split<KeyT, CODEC_SIGNED, false>(r, p);
+    case CODEC_FLOAT: return idx ? sort_row_split<KeyT, CODEC_FLOAT, true>(r, p) : sort_row_split<KeyT, CODEC_FLOAT, false>(r, p);
+    default: return CPN_ERR_DTYPE;
+  }
+}
+
+}  // namespace cpn

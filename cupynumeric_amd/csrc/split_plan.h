@@ -1,0 +1,68 @@
+// Which requests are split by sampled keys (split_sort.h), into what, and in which workspace.
+#pragma once
+
+#include "sort_driver.h"
+#include "split_sort.h"
+
+namespace cpn {
+
+// Single rows split once by sampled keys (split_sort.h), real keys of 4 and 8 bytes.  buckets == 0: another way.
+// (cpn_set_merge_rows: in the default mode only, and with the row kernels in use.)
+struct SplitPlan {
+  uint32_t buckets;     // a power of two
+  uint32_t per_bucket;  // sampled keys
+  uint32_t tiles, tile_len;
+  bool gathered;        // the sample, by a launch of its own
+};
+// Where the lines lie (us per call, before / this way; normal float keys, sort and argsort):
+//   from where one workgroup has more than 6144 8-byte or 8192 4-byte keys to sort (until 8 or 16 keys per thread, about 12
+//   us, two launches cost as much): float64 6144 16, 19 / 15, 15, 8192 26, 21 / 15, 15, int64 6144 13, 15 / 14, 14, 8192 19, 18
+//   / 14, 14, float32 8192 15, 19 / 13, 14, 9000 22, 21 / 14, 14, int32 8192 12, 16 / 13, 13, 9000 19, 18 / 13, 13.  Rows of a hundred
+//   values cost the network for the sample and passes in the buckets: 8192 float32 15, 17 / 18, 18, float64 27, 27 / 21, 21.
+//   in between: 40 000 float32 29, 30 / 14, 15, float64 33, 34 / 16, 16; 100 000 41, 46 / 16, 17 and 53, 48 / 18, 18;
+//   262 144 68, 75 / 23, 26 and 125, 115 / 26, 27; 524 288 65, 71 / 31, 34 and 152, 146 / 35, 37
+//   to where 8192 sampled keys, which every tile's workgroup sorts, take half of its time: 10^6 float32 76, 86 / 48, 52,
+//   float64 193, 176 / 54, 57, int64 148, 172 / 50, 52
+constexpr uint64_t SPLIT_MAX_ROW = SPLIT_MAX_TILES * SPLIT_BLOCK * SPLIT_TILE_ITEMS;
+constexpr uint64_t split_min_row(int key_bytes) { return key_bytes == 8 ? 6145 : 8193; }
+inline SplitPlan split_plan(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_indices)
+{
+  SplitPlan p{};
+  if (!merge_rows_default() || (key_bytes != 4 && key_bytes != 8) || passes != key_bytes || seg < split_min_row(key_bytes) ||
+      seg > SPLIT_MAX_ROW || volume != seg || lds_row_limit(key_bytes, want_indices) != lds_row_capacity(key_bytes, want_indices)) {
+    return p;
+  }
+  // A bucket of 1024 keys at most, eight of them sampled, or of 512, four of them sampled (and room for 4096).  A tile of as
+  // few keys as leaves no compute unit without one.
+  p.buckets      = seg <= 65536 ? 128 : (seg <= 262144 ? 256 : (seg <= 524288 ? 512 : 1024));
+  p.per_bucket   = p.buckets == 256 && seg <= 131072 ? 4 : 8;
+  p.gathered     = p.buckets * p.per_bucket >= 4096;
+  uint64_t tiles = (seg + SPLIT_BLOCK - 1) / SPLIT_BLOCK;
+  tiles          = tiles > SPLIT_MAX_TILES ? SPLIT_MAX_TILES : tiles;
+  p.tile_len     = static_cast<uint32_t>((seg + tiles - 1) / tiles);
+  p.tiles        = static_cast<uint32_t>((seg + p.tile_len - 1) / p.tile_len);
+  return p;
+}
+// Workspace: header, the sample, the keys in the order of the buckets of each tile, their places, the table, two words
+// per key.
+struct SplitLayout {
+  uint64_t off_sample, off_keys, off_places, off_starts, off_ids, total;
+};
+inline SplitLayout split_layout(const SplitPlan& p, int key_bytes, uint64_t n, bool want_indices)
+{
+  const uint64_t table = static_cast<uint64_t>(p.tiles) * (p.buckets + 1) * sizeof(uint16_t);
+  SplitLayout L{};
+  L.off_sample = HEADER_BYTES;
+  L.off_keys   = L.off_sample + (p.gathered ? align_up(static_cast<uint64_t>(p.buckets) * p.per_bucket * key_bytes, WORKSPACE_ALIGN) : 0);
+  L.off_places = L.off_keys + align_up(n * key_bytes, WORKSPACE_ALIGN);
+  L.off_starts = L.off_places + (want_indices ? align_up(n * sizeof(uint16_t), WORKSPACE_ALIGN) : 0);
+  L.off_ids    = L.off_starts + align_up(table, WORKSPACE_ALIGN);
+  L.total      = L.off_ids + align_up(2 * n * sizeof(uint32_t), WORKSPACE_ALIGN);
+  return L;
+}
+
+// (split_keys32.hip, split_keys64.hip: requests that split_plan accepts, with a workspace of split_layout)
+int sort_split32(int codec, const SortRequest& r, const SplitPlan& plan);
+int sort_split64(int codec, const SortRequest& r, const SplitPlan& plan);
+
+}  // namespace cpn

@@ -96,6 +96,14 @@ uint64_t cpn_local_sort_temp_bytes(int dtype, uint64_t volume, uint64_t sort_dim
                                    int want_values, int want_indices, int in_place);
 
 /*
+ * Workspace size, in bytes, with which cpn_local_sort_ex and its option CPN_SORT_SPLIT sort this request faster than
+ * with cpn_local_sort_temp_bytes: one row of ten thousand to a few million real keys of 4 or 8 bytes.
+ * 0 for every other request.  (The smaller size goes on being enough for
+ * cpn_local_sort.)  Pure host arithmetic, follows the switches below.
+ */
+uint64_t cpn_local_sort_split_temp_bytes(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_indices);
+
+/*
  * Stable sort of `volume / sort_dim_size` independent rows of `sort_dim_size` elements,
  * dense row-major.  Replaces local_sort<CODE> (src/cupynumeric/sort/sort.cu:63-96) together
  * with the index initialisation that precedes it (sort.cu:1851-1863, sort.h:83-92).
@@ -130,8 +138,13 @@ int cpn_local_sort(int dtype, const void* values_in, void* values_out, int64_t* 
  *                           launch: the way to repeat a sort that came back with CPN_ERR_DEVICE
  *                           (cpn_local_sort_check), without touching process-wide state.  Results do
  *                           not depend on it.
+ *   CPN_SORT_SPLIT          `temp` holds cpn_local_sort_split_temp_bytes(...) bytes, which is not 0: rows are split by
+ *                           sampled keys and the parts sorted side by side, two launches that cannot fail on the
+ *                           device.  With a smaller workspace, or where that size is 0, the option changes nothing.
+ *                           Results do not depend on it.
  */
 #define CPN_SORT_SINGLE_TICKET 1u
+#define CPN_SORT_SPLIT 4u
 int cpn_local_sort_ex(int dtype, const void* values_in, void* values_out, int64_t* indices_out,
                       uint64_t volume, uint64_t sort_dim_size, int64_t index_offset, int stable,
                       uint32_t options, void* temp, uint64_t temp_bytes, void* stream);
