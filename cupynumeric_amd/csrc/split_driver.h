@@ -6,6 +6,66 @@
 namespace cpn {
 
 template <typename KeyT, int CODEC, bool HAS_IDX>
+inline int sort_row_split(const SortRequest& r, const SplitPlan& p);
+
+// The launches ahead of a wide row's tiles, and these.
+template <typename KeyT, int CODEC, bool HAS_IDX, int BITS>
+inline int split_wide_tiles(const SortRequest& r, const SplitPlan& p, const SplitLayout& L)
+{
+  uint8_t* const ws      = static_cast<uint8_t*>(r.temp);
+  const uint32_t n       = static_cast<uint32_t>(r.seg);
+  const uint32_t samples = p.buckets * p.per_bucket;
+  KeyT* sample           = reinterpret_cast<KeyT*>(ws + L.off_sample);
+  KeyT* sorted           = reinterpret_cast<KeyT*>(ws + L.off_sorted);
+  int64_t* numbers       = reinterpret_cast<int64_t*>(ws + L.off_numbers);
+  KeyT* images           = reinterpret_cast<KeyT*>(ws + L.off_images);
+  uint32_t* at           = reinterpret_cast<uint32_t*>(ws + L.off_at);
+  float* values          = reinterpret_cast<float*>(ws + L.off_values);
+  uint16_t* before       = reinterpret_cast<uint16_t*>(ws + L.off_before);
+  SplitBins* bins        = reinterpret_cast<SplitBins*>(ws + L.off_bins);
+  {
+    ProfileScope prof("split_gather", r.stream);
+    hipLaunchKernelGGL((split_gather_kernel<KeyT>), dim3(samples / 256), dim3(256), 0, r.stream,
+                       static_cast<const KeyT*>(r.values_in), n, samples, sample);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    SortRequest c  = r;
+    c.values_in    = sample;
+    c.values_out   = sorted;
+    c.indices_out  = numbers;
+    c.volume       = samples;
+    c.seg          = samples;
+    c.index_offset = 0;
+    c.temp         = ws + L.off_inner;
+    const int rc   = sort_row_split<KeyT, CODEC, true>(c, split_plan(sizeof(KeyT), sizeof(KeyT), samples, samples, true));
+    if (rc != CPN_OK) {
+      return rc;
+    }
+  }
+  {
+    ProfileScope prof("split_pick", r.stream);
+    hipLaunchKernelGGL((split_pick_kernel<KeyT, CODEC>), dim3(p.buckets / 256), dim3(256), 0, r.stream, sorted, numbers, n, samples,
+                       p.per_bucket, images, at, values, static_cast<uint32_t*>(r.temp));
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    ProfileScope prof("split_table", r.stream);
+    hipLaunchKernelGGL((split_table_kernel<BITS>), dim3(1), dim3(SPLIT_BLOCK), 0, r.stream, values, before, bins);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    ProfileScope prof("split_tiles", r.stream);
+    hipLaunchKernelGGL((split_wide_tile_kernel<KeyT, CODEC, HAS_IDX, BITS>), dim3(p.tiles), dim3(SPLIT_BLOCK), 0, r.stream,
+                       static_cast<const KeyT*>(r.values_in), n, p.tile_len, images, at, before, bins,
+                       reinterpret_cast<KeyT*>(ws + L.off_keys), HAS_IDX ? reinterpret_cast<uint16_t*>(ws + L.off_places) : nullptr,
+                       reinterpret_cast<uint16_t*>(ws + L.off_starts));
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  return CPN_OK;
+}
+
+template <typename KeyT, int CODEC, bool HAS_IDX>
 inline int sort_row_split(const SortRequest& r, const SplitPlan& p)
 {
   // (float keys that tie need not be the same bits, but a bucket's keys stay in the order of the row on both ways, so
@@ -17,6 +77,19 @@ inline int sort_row_split(const SortRequest& r, const SplitPlan& p)
   uint16_t* starts    = reinterpret_cast<uint16_t*>(ws + L.off_starts);
   const uint32_t n    = static_cast<uint32_t>(r.seg);
   KeyT* sample        = nullptr;
+  if (p.wide) {
+    int rc = CPN_ERR_UNSUPPORTED;
+    if constexpr (sizeof(KeyT) == 8) {  // (split_max_row)
+      switch (p.buckets) {
+        case 1024: rc = split_wide_tiles<KeyT, CODEC, HAS_IDX, 10>(r, p, L); break;
+        case 2048: rc = split_wide_tiles<KeyT, CODEC, HAS_IDX, 11>(r, p, L); break;
+        case 4096: rc = split_wide_tiles<KeyT, CODEC, HAS_IDX, 12>(r, p, L); break;
+      }
+    }
+    if (rc != CPN_OK) {
+      return rc;
+    }
+  }
   if (p.gathered) {
     sample                 = reinterpret_cast<KeyT*>(ws + L.off_sample);
     const uint32_t samples = p.buckets * p.per_bucket;
@@ -25,7 +98,7 @@ inline int sort_row_split(const SortRequest& r, const SplitPlan& p)
                        static_cast<const KeyT*>(r.values_in), n, samples, sample);
     CPN_HIP_TRY(hipGetLastError());
   }
-  {
+  if (!p.wide) {
     ProfileScope prof("split_tiles", r.stream);
     const dim3 grid(p.tiles);
     auto launch = [&](auto per_thread, auto per_bucket) {
@@ -61,9 +134,20 @@ inline int sort_row_split(const SortRequest& r, const SplitPlan& p)
     sb.tile_len = p.tile_len;
     sb.buckets  = p.buckets;
     ProfileScope prof("split_buckets", r.stream);
-    hipLaunchKernelGGL((split_bucket_kernel<KeyT, CODEC, HAS_IDX, SPLIT_BUCKET_BLOCK, SPLIT_BUCKET_ITEMS>),
-                       dim3(p.buckets), dim3(SPLIT_BUCKET_BLOCK), 0, r.stream, sb,
-                       static_cast<KeyT*>(r.values_out), r.indices_out, r.index_offset);
+    auto launch = [&](auto wide) {
+      hipLaunchKernelGGL((split_bucket_kernel<KeyT, CODEC, HAS_IDX, decltype(wide)::value>), dim3(p.buckets), dim3(SPLIT_BUCKET_BLOCK), 0,
+                         r.stream, sb, static_cast<KeyT*>(r.values_out), r.indices_out, r.index_offset);
+    };
+    bool launched = false;
+    if constexpr (sizeof(KeyT) == 8) {
+      if (p.wide) {
+        launch(std::true_type{});
+        launched = true;
+      }
+    }
+    if (!launched) {
+      launch(std::false_type{});
+    }
   }
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;

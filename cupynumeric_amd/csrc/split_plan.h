@@ -13,6 +13,7 @@ struct SplitPlan {
   uint32_t per_bucket;  // sampled keys
   uint32_t tiles, tile_len;
   bool gathered;        // the sample, by a launch of its own
+  bool wide;            // the sample is sorted ahead, as a row of its own
 };
 // Where the lines lie (us per call, before / this way; normal float keys, sort and argsort):
 //   from where one workgroup has more than 6144 8-byte or 8192 4-byte keys to sort (until 8 or 16 keys per thread, about 12
@@ -23,13 +24,26 @@ struct SplitPlan {
 //   262 144 68, 75 / 23, 26 and 125, 115 / 26, 27; 524 288 65, 71 / 31, 34 and 152, 146 / 35, 37
 //   to where 8192 sampled keys, which every tile's workgroup sorts, take half of its time: 10^6 float32 76, 86 / 48, 52,
 //   float64 193, 176 / 54, 57, int64 148, 172 / 50, 52
-constexpr uint64_t SPLIT_MAX_ROW = SPLIT_MAX_TILES * SPLIT_BLOCK * SPLIT_TILE_ITEMS;
+constexpr uint64_t SPLIT_WIDE_ROW = SPLIT_MAX_TILES * SPLIT_BLOCK * SPLIT_TILE_ITEMS + 1;
+constexpr uint64_t split_max_row(int key_bytes) { return key_bytes == 8 ? 4096 * 2560 : SPLIT_WIDE_ROW - 1; }
 constexpr uint64_t split_min_row(int key_bytes) { return key_bytes == 8 ? 6145 : 8193; }
 inline SplitPlan split_plan(int key_bytes, int passes, uint64_t volume, uint64_t seg, bool want_indices)
 {
   SplitPlan p{};
   if (!merge_rows_default() || (key_bytes != 4 && key_bytes != 8) || passes != key_bytes || seg < split_min_row(key_bytes) ||
-      seg > SPLIT_MAX_ROW || volume != seg || lds_row_limit(key_bytes, want_indices) != lds_row_capacity(key_bytes, want_indices)) {
+      seg > split_max_row(key_bytes) || volume != seg || lds_row_limit(key_bytes, want_indices) != lds_row_capacity(key_bytes, want_indices)) {
+    return p;
+  }
+  if (seg >= SPLIT_WIDE_ROW) {
+    // A bucket of 2560 keys at most (and room for 4096): the fuller, the more of them sampled.  Tiles in whole rounds of
+    // the compute units.
+    p.wide         = true;
+    p.buckets      = seg <= (1ull << 21) ? 1024 : (seg <= (1ull << 22) ? 2048 : 4096);
+    p.per_bucket   = seg <= p.buckets * 1365ull ? 16 : (seg <= p.buckets * 2048ull ? 64 : 128);
+    uint64_t tiles = (seg + SPLIT_BLOCK * SPLIT_WIDE_ITEMS - 1) / (SPLIT_BLOCK * SPLIT_WIDE_ITEMS);
+    tiles          = align_up(tiles, 256);
+    p.tile_len     = static_cast<uint32_t>((seg + tiles - 1) / tiles);
+    p.tiles        = static_cast<uint32_t>((seg + p.tile_len - 1) / p.tile_len);
     return p;
   }
   // A bucket of 1024 keys at most, eight of them sampled, or of 512, four of them sampled (and room for 4096).  A tile of as
@@ -44,16 +58,30 @@ inline SplitPlan split_plan(int key_bytes, int passes, uint64_t volume, uint64_t
   return p;
 }
 // Workspace: header, the sample, the keys in the order of the buckets of each tile, their places, the table, two words
-// per key.
+// per key.  Wide: also the sorted sample and the numbers of its keys, the splitters (images, places, values), their table of
+// bins, and the workspace of the sample's own sort.
 struct SplitLayout {
-  uint64_t off_sample, off_keys, off_places, off_starts, off_ids, total;
+  uint64_t off_sample, off_sorted, off_numbers, off_images, off_at, off_values, off_before, off_bins, off_inner;
+  uint64_t off_keys, off_places, off_starts, off_ids, total;
 };
 inline SplitLayout split_layout(const SplitPlan& p, int key_bytes, uint64_t n, bool want_indices)
 {
   const uint64_t table = static_cast<uint64_t>(p.tiles) * (p.buckets + 1) * sizeof(uint16_t);
   SplitLayout L{};
+  const uint64_t samples = static_cast<uint64_t>(p.buckets) * p.per_bucket;
   L.off_sample = HEADER_BYTES;
-  L.off_keys   = L.off_sample + (p.gathered ? align_up(static_cast<uint64_t>(p.buckets) * p.per_bucket * key_bytes, WORKSPACE_ALIGN) : 0);
+  L.off_keys   = L.off_sample + (p.gathered || p.wide ? align_up(samples * key_bytes, WORKSPACE_ALIGN) : 0);
+  if (p.wide) {
+    L.off_sorted  = L.off_keys;
+    L.off_numbers = L.off_sorted + align_up(samples * key_bytes, WORKSPACE_ALIGN);
+    L.off_images  = L.off_numbers + align_up(samples * sizeof(int64_t), WORKSPACE_ALIGN);
+    L.off_at      = L.off_images + align_up(static_cast<uint64_t>(p.buckets) * key_bytes, WORKSPACE_ALIGN);
+    L.off_values  = L.off_at + align_up(p.buckets * sizeof(uint32_t), WORKSPACE_ALIGN);
+    L.off_before  = L.off_values + align_up(p.buckets * sizeof(float), WORKSPACE_ALIGN);
+    L.off_bins    = L.off_before + align_up(p.buckets * SPLIT_WIDE_BINS * sizeof(uint16_t), WORKSPACE_ALIGN);
+    L.off_inner   = L.off_bins + WORKSPACE_ALIGN;
+    L.off_keys    = L.off_inner + split_layout(split_plan(key_bytes, key_bytes, samples, samples, true), key_bytes, samples, true).total;
+  }
   L.off_places = L.off_keys + align_up(n * key_bytes, WORKSPACE_ALIGN);
   L.off_starts = L.off_places + (want_indices ? align_up(n * sizeof(uint16_t), WORKSPACE_ALIGN) : 0);
   L.off_ids    = L.off_starts + align_up(table, WORKSPACE_ALIGN);

@@ -26,7 +26,6 @@
 
 #include <type_traits>
 
-#include "bitonic_row_sort.h"
 #include "radix_common.h"
 
 namespace cpn {
@@ -36,10 +35,15 @@ constexpr int SPLIT_BUCKET_BLOCK = 512;
 constexpr int SPLIT_BUCKET_ITEMS = 8;
 constexpr int SPLIT_WAVES       = SPLIT_BLOCK / WAVE;
 constexpr int SPLIT_TILE_ITEMS  = 4;                       // keys per thread of a tile
-constexpr int SPLIT_SAMPLE_E    = 8;                       // sampled keys per lane of a wave that sorts them
 constexpr int SPLIT_MAX_BUCKETS = 1024;
 constexpr int SPLIT_MAX_TILES   = 256;
-constexpr uint32_t SPLIT_CROWD  = 64;  // most sampled keys of a bin
+// rows whose splitters are found ahead (split_wide_tile_kernel)
+constexpr int SPLIT_WIDE_MAX_TILES = 1280;
+constexpr int SPLIT_WIDE_ITEMS     = 14;
+constexpr int SPLIT_WIDE_BINS      = 2;  // per splitter
+// Most sampled keys of a bin that are compared with each other (64: 10^6 int32 keys of 200 values, 41 of them in every bin, take 80 us, of
+// which the walks are half).
+constexpr uint32_t SPLIT_CROWD  = 24;
 
 // A mixed 32-bit word: which key of its stretch sample i takes.
 __host__ __device__ __forceinline__ uint32_t split_hash(uint32_t x)
@@ -87,65 +91,94 @@ __device__ __forceinline__ uint32_t split_match_rank(uint32_t bucket, bool valid
   return old + lower;
 }
 
-// Exchange of the sample between waves: word r of thread t lies at r * THREADS + t.
-template <typename W>
-struct SplitExchange;
-template <>
-struct SplitExchange<F64Word> {
-  static constexpr int BYTES = 8;
-  static __device__ __forceinline__ void put(unsigned char* s, int, int slot, const F64Word& w) { reinterpret_cast<double*>(s)[slot] = w.v; }
-  static __device__ __forceinline__ F64Word get(const unsigned char* s, int, int slot) { return F64Word{reinterpret_cast<const double*>(s)[slot]}; }
-};
-template <>
-struct SplitExchange<ImagePos> {
-  static constexpr int BYTES = 12;
-  static __device__ __forceinline__ void put(unsigned char* s, int slots, int slot, const ImagePos& w)
-  {
-    reinterpret_cast<uint64_t*>(s)[slot]             = w.image;
-    reinterpret_cast<uint32_t*>(s + 8 * slots)[slot] = static_cast<uint32_t>(w.pos);
-  }
-  static __device__ __forceinline__ ImagePos get(const unsigned char* s, int slots, int slot)
-  {
-    return ImagePos{reinterpret_cast<const uint64_t*>(s)[slot], reinterpret_cast<const uint32_t*>(s + 8 * slots)[slot]};
-  }
-};
-
-// Merges the sorted runs of single waves into one of SW waves (the steps of bitonic_row_sort.h's network that cross
-// waves, through LDS).  Every thread of the workgroup calls; those of the first SW waves hold keys.
-template <int RUN, int SW, typename W>
-__device__ __forceinline__ void split_merge_waves(W (&w)[SPLIT_SAMPLE_E], unsigned char* s, uint32_t tid)
+// Puts the numbers of m keys in LDS in the order of their images' bits [from_bit, top), stably: passes of 8 bits, of which
+// the numbers move and the keys stay where they are.  num: in, any order; ctr: a counter per wave and digit.  Every thread
+// of the workgroup calls, with the same arguments.
+template <int CODEC, int BLOCK, int ITEMS, typename KeyT>
+__device__ __forceinline__ void split_order_passes(const KeyT* keys, uint16_t* num, uint16_t* ctr, uint32_t* s_wave, uint32_t m, int from_bit,
+                                                   int top)
 {
-  if constexpr (RUN <= SW) {
-    constexpr int THREADS = SW * WAVE, SLOTS = THREADS * SPLIT_SAMPLE_E;
-    using X            = SplitExchange<W>;
-    const bool holds   = tid < THREADS;
-    const uint32_t sub = tid % (RUN * WAVE);
+  constexpr int WAVES   = BLOCK / WAVE;
+  const uint32_t tid    = threadIdx.x;
+  const uint32_t lane   = tid & (WAVE - 1);
+  const uint32_t wave   = tid / WAVE;
+  const uint32_t rounds = (m + BLOCK - 1) / BLOCK;  // uniform
+  // (ranks count in the order of waves, rounds and lanes: wave w has numbers [64 rounds w, 64 rounds (w + 1)))
+  uint32_t first = wave * rounds * WAVE + lane;
+  for (int bit = from_bit; bit < top; bit += RADIX_BITS) {
+    asm volatile("" : "+v"(first));  // (or every address below is worked out ahead of the loop, into 160 registers)
+    for (uint32_t j = tid; j < WAVES * RADIX / 2; j += BLOCK) {
+      reinterpret_cast<uint32_t*>(ctr)[j] = 0;
+    }
+    __syncthreads();
+    uint32_t packed[ITEMS], rank[ITEMS];  // number and digit
 #pragma unroll
-    for (int d = RUN; d >= 2; d /= 2) {  // d == RUN: the mirror image in the run; then lanes at distance d * WAVE / 2
-      const bool mirror = d == RUN;
-      __syncthreads();
-      if (holds) {
-#pragma unroll
-        for (int r = 0; r < SPLIT_SAMPLE_E; ++r) {
-          X::put(s, SLOTS, r * THREADS + tid, w[r]);
-        }
-      }
-      __syncthreads();
-      if (holds) {
-        const uint32_t other = mirror ? tid ^ (RUN * WAVE - 1) : tid ^ (d * WAVE / 2);
-        const bool keep_min  = mirror ? sub < RUN * WAVE / 2 : (tid & (d * WAVE / 2)) == 0;
-#pragma unroll
-        for (int r = 0; r < SPLIT_SAMPLE_E; ++r) {
-          const W o = X::get(s, SLOTS, (mirror ? SPLIT_SAMPLE_E - 1 - r : r) * THREADS + other);
-          w[r]      = word_select(word_less(w[r], o) == keep_min, w[r], o);
-        }
+    for (int i = 0; i < ITEMS; ++i) {
+      packed[i] = 0, rank[i] = 0;
+      if (i < static_cast<int>(rounds)) {
+        const uint32_t o = first + i * WAVE;
+        const bool valid = o < m;
+        const uint32_t k = num[valid ? o : m - 1];
+        const uint32_t d = static_cast<uint32_t>(ordered_bits<CODEC, KeyT>(keys[k]) >> bit) & (RADIX - 1);
+        packed[i]        = (k << 8) | d;
+        rank[i]          = split_match_rank<RADIX_BITS>(d, valid, ctr + wave * RADIX);
       }
     }
-    if (holds) {
-      cross_steps<WAVE / 2>(w, tid & (WAVE - 1));
-      lane_sort_bitonic(w);
+    __syncthreads();
+    uint32_t total = 0;
+    if (tid < RADIX) {
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        const uint32_t c     = ctr[w * RADIX + tid];
+        ctr[w * RADIX + tid] = static_cast<uint16_t>(total);
+        total += c;
+      }
     }
-    split_merge_waves<2 * RUN, SW>(w, s, tid);
+    const uint32_t incl = wave_inclusive_sum_dpp(total);
+    if (lane == WAVE - 1) {
+      s_wave[wave] = incl;
+    }
+    __syncthreads();
+    if (tid < RADIX) {
+      uint32_t run = incl - total;
+#pragma unroll
+      for (uint32_t w = 0; w < RADIX / WAVE; ++w) {
+        run += w < wave ? s_wave[w] : 0u;
+      }
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        ctr[w * RADIX + tid] = static_cast<uint16_t>(ctr[w * RADIX + tid] + run);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      if (i < static_cast<int>(rounds) && first + i * WAVE < m) {
+        num[ctr[wave * RADIX + (packed[i] & (RADIX - 1))] + rank[i]] = static_cast<uint16_t>(packed[i] >> 8);
+      }
+    }
+    __syncthreads();
+  }
+}
+// The same for all `top` bits, of which the leading 40 put almost every row in order: passes over them, a look at every pair of
+// neighbours, and passes over all bits if one is not in order.
+template <int CODEC, int BLOCK, int ITEMS, typename KeyT>
+__device__ __forceinline__ void split_order(const KeyT* keys, uint16_t* num, uint16_t* ctr, uint32_t* s_wave, uint32_t m, int top)
+{
+  int from_bit = top > 40 ? top - 40 : 0;
+  for (;;) {
+    split_order_passes<CODEC, BLOCK, ITEMS>(keys, num, ctr, s_wave, m, from_bit, top);
+    if (from_bit == 0) {
+      return;
+    }
+    int bad = 0;
+    for (uint32_t o = threadIdx.x; o + 1 < m; o += BLOCK) {
+      bad |= ordered_bits<CODEC, KeyT>(keys[num[o]]) > ordered_bits<CODEC, KeyT>(keys[num[o + 1]]) ? 1 : 0;
+    }
+    if (__syncthreads_or(bad) == 0) {
+      return;
+    }
+    from_bit = 0;
   }
 }
 
@@ -181,15 +214,15 @@ __device__ __forceinline__ uint32_t split_waves_before(const uint32_t* s_wave, u
 }
 
 // What a workgroup needs in LDS to find the splitters of a row, PER_THREAD sampled keys each: a word per sampled key, and
-// room for the network's exchanges (the keys in the order of their bins, and their numbers, take less).
+// room for their images, their numbers, and the counters of passes over them.
 template <typename KeyT, int PER_THREAD, int PER_BUCKET>
 struct SplitSample {
-  using W                        = std::conditional_t<sizeof(KeyT) == 8, ImagePos, F64Word>;
   static constexpr int SAMPLES   = PER_THREAD * SPLIT_BLOCK;
-  static constexpr int SORTERS   = SAMPLES / SPLIT_SAMPLE_E;  // threads of the network
   static constexpr int SPLITTERS = SAMPLES / PER_BUCKET;
-  static constexpr int BYTES     = SAMPLES * SplitExchange<W>::BYTES;
-  static_assert(SPLIT_SAMPLE_E % PER_BUCKET == 0, "the first of a lane's sampled keys is a splitter");
+  static constexpr int WHICH     = SAMPLES * static_cast<int>(sizeof(KeyT));
+  static constexpr int COUNTERS  = WHICH + SAMPLES * 2;
+  static constexpr int EXTREMES  = COUNTERS + SPLIT_WAVES * RADIX * 2;
+  static constexpr int BYTES     = EXTREMES + 2 * SPLIT_WAVES * static_cast<int>(sizeof(KeyT));
 };
 
 // The bin of a value: subtraction, scaling and truncation do not decrease with it.  (Clamped before the conversion, NaN to
@@ -212,19 +245,18 @@ __device__ __forceinline__ uint32_t split_splitters_before(uint32_t from)
 // Splitter j of a row is the smallest of the j-th PER_BUCKET sampled keys: put(j, image, place) for every j; s_bins is left
 // with the number of sampled keys before each bin.  The whole workgroup calls.  The sample is spread over as many bins of equal width in the value as it has keys; one atomic per key
 // says which of its bin it is, a scan where the bin starts, and a walk over the bin how many of its keys come before.  A
-// sample that crowds its bins (few different values, values of many magnitudes) goes through a sorting network.
-template <int CODEC, int PER_THREAD, int PER_BUCKET, typename KeyT, typename Get, typename Put>
+// sample that crowds its bins (few different values, values of many magnitudes) goes through passes over its bytes.
+template <int CODEC, int PER_THREAD, int PER_BUCKET, typename KeyT, typename Put>
 __device__ __forceinline__ SplitBins split_find_splitters(uint32_t n, unsigned char* s_mem, uint32_t* s_bins, uint32_t* s_wave, uint32_t* s_low,
-                                                          const KeyT (&got)[PER_THREAD], Get get, Put put)
+                                                          const KeyT (&got)[PER_THREAD], Put put)
 {
   using S                = SplitSample<KeyT, PER_THREAD, PER_BUCKET>;
-  using W                = typename S::W;
   constexpr int SAMPLES  = S::SAMPLES;
   const uint32_t tid     = threadIdx.x;
   const uint32_t lane    = tid & (WAVE - 1);
   const uint32_t wave    = tid / WAVE;
   KeyT* const s_image     = reinterpret_cast<KeyT*>(s_mem);
-  uint16_t* const s_which = reinterpret_cast<uint16_t*>(s_mem + SAMPLES * sizeof(KeyT));
+  uint16_t* const s_which = reinterpret_cast<uint16_t*>(s_mem + S::WHICH);
 #pragma unroll
   for (int r = 0; r < PER_THREAD; ++r) {
     s_bins[r * SPLIT_BLOCK + tid] = 0;
@@ -321,32 +353,34 @@ __device__ __forceinline__ SplitBins split_find_splitters(uint32_t n, unsigned c
       }
     }
   } else {
-    W w[SPLIT_SAMPLE_E];
-    if (tid < S::SORTERS) {
+    KeyT* const s_ext = reinterpret_cast<KeyT*>(s_mem + S::EXTREMES);
+    KeyT top_image = 0, low_image = 0;  // the largest, the complement of the smallest
 #pragma unroll
-      for (int r = 0; r < SPLIT_SAMPLE_E; ++r) {
-        const uint32_t i = number * SPLIT_SAMPLE_E + r;
-        const KeyT image = ordered_bits<CODEC, KeyT>(get(i));
-        if constexpr (sizeof(KeyT) == 8) {
-          w[r] = ImagePos{image, i};
-        } else {
-          w[r] = pack_image_pos(image, i);
-        }
-      }
-      blocked_sort<WAVE>(w, lane);
+    for (int r = 0; r < PER_THREAD; ++r) {
+      const KeyT image                 = ordered_bits<CODEC, KeyT>(got[r]);
+      top_image                        = image > top_image ? image : top_image;
+      low_image                        = static_cast<KeyT>(~image) > low_image ? static_cast<KeyT>(~image) : low_image;
+      s_image[r * SPLIT_BLOCK + tid]   = image;
+      s_which[r * SPLIT_BLOCK + tid]   = static_cast<uint16_t>(r * SPLIT_BLOCK + tid);
     }
-    split_merge_waves<2, S::SORTERS / WAVE>(w, s_mem, tid);
-    if (tid < S::SORTERS) {
+    top_image = wave_max_dpp(top_image);
+    low_image = wave_max_dpp(low_image);
+    if (lane == 0) {
+      s_ext[wave]               = top_image;
+      s_ext[SPLIT_WAVES + wave] = low_image;
+    }
+    __syncthreads();
 #pragma unroll
-      for (int r = 0; r < SPLIT_SAMPLE_E; r += PER_BUCKET) {
-        KeyT image;
-        if constexpr (sizeof(KeyT) == 8) {
-          image = w[r].image;
-        } else {
-          image = static_cast<KeyT>(static_cast<uint64_t>(__double_as_longlong(w[r].v)) >> 20);
-        }
-        put((tid * SPLIT_SAMPLE_E + r) / PER_BUCKET, image, split_sample_place(word_pos(w[r]), SAMPLES, n));
-      }
+    for (int v = 0; v < SPLIT_WAVES; ++v) {
+      top_image = s_ext[v] > top_image ? s_ext[v] : top_image;
+      low_image = s_ext[SPLIT_WAVES + v] > low_image ? s_ext[SPLIT_WAVES + v] : low_image;
+    }
+    const uint64_t vary = static_cast<KeyT>(top_image ^ static_cast<KeyT>(~low_image));
+    split_order<CODEC_UNSIGNED, SPLIT_BLOCK, PER_THREAD>(s_image, s_which, reinterpret_cast<uint16_t*>(s_mem + S::COUNTERS), s_wave,
+                                                         static_cast<uint32_t>(SAMPLES), vary != 0 ? 64 - __builtin_clzll(vary) : 0);
+    for (uint32_t j = number; j < S::SPLITTERS; j += SPLIT_BLOCK) {
+      const uint32_t i = s_which[j * PER_BUCKET];
+      put(j, s_image[i], split_sample_place(i, SAMPLES, n));
     }
   }
   return bins;
@@ -420,7 +454,7 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_tile_kernel(const KeyT* __r
     key[i]           = keys_in[first + (o < len ? o : len - 1)];
   }
   uint32_t* const s_bins = reinterpret_cast<uint32_t*>(s_ctr);
-  const SplitBins bins   = split_find_splitters<CODEC, PER_THREAD, PER_BUCKET>(n, s_mem, s_bins, s_wave, s_low, got, sampled,
+  const SplitBins bins   = split_find_splitters<CODEC, PER_THREAD, PER_BUCKET>(n, s_mem, s_bins, s_wave, s_low, got,
                                                                              [&](uint32_t j, KeyT image, uint32_t place) {
                                                                                s_split[j]    = image;
                                                                                s_split_at[j] = place;
@@ -516,6 +550,270 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_tile_kernel(const KeyT* __r
   KeyT* const out = grouped + first;
   for (uint32_t o = tid; o < len; o += SPLIT_BLOCK) {
     out[o] = s_keys[o];
+    if constexpr (HAS_POS) {
+      places[first + o] = s_place[o];
+    }
+  }
+}
+
+// ---- rows whose splitters are found ahead ----
+// Longer rows take more buckets and more sampled keys than a tile's workgroup can sort by the way: the sample is gathered,
+// sorted as a row of its own (by the kernels above), and every (samples / buckets)-th key of it is a splitter.
+
+// The splitters: of the sorted sample and the numbers of its keys, every `step`-th.  A launch of several workgroups: the
+// reads are scattered.
+template <typename KeyT, int CODEC>
+__global__ __launch_bounds__(256) void split_pick_kernel(const KeyT* __restrict__ sorted, const int64_t* __restrict__ numbers,
+                                                         uint32_t n, uint32_t samples, uint32_t step, KeyT* __restrict__ images,
+                                                         uint32_t* __restrict__ places, float* __restrict__ values,
+                                                         uint32_t* __restrict__ status)
+{
+  const uint32_t j = blockIdx.x * 256 + threadIdx.x;  // (the buckets are a multiple of the workgroup)
+  if (j == 0) {
+    *status = 0;  // (the workspace's status word: this sort cannot fail on the device)
+  }
+  const KeyT key   = sorted[j * step];
+  images[j]        = ordered_bits<CODEC, KeyT>(key);
+  places[j]        = split_sample_place(static_cast<uint32_t>(numbers[j * step]), samples, n);
+  values[j]        = split_value<CODEC, KeyT>(key);
+}
+
+// The bins of their values, and how many splitters come before each (one workgroup).
+template <int BITS>
+__global__ __launch_bounds__(SPLIT_BLOCK) void split_table_kernel(const float* __restrict__ values, uint16_t* __restrict__ before,
+                                                                  SplitBins* __restrict__ bins_out)
+{
+  constexpr int BUCKETS = 1 << BITS;
+  constexpr int BINS    = BUCKETS * SPLIT_WIDE_BINS;
+  constexpr int OWN     = BUCKETS / SPLIT_BLOCK;  // splitters of a thread
+  constexpr int SPAN    = BINS / SPLIT_BLOCK;     // bins of a thread
+  __shared__ uint32_t s_bins[BINS];
+  __shared__ uint32_t s_wave[SPLIT_WAVES], s_low[SPLIT_WAVES];
+  const uint32_t tid  = threadIdx.x;
+  const uint32_t lane = tid & (WAVE - 1);
+  const uint32_t wave = tid / WAVE;
+  float value[OWN];
+  uint32_t low = 0, high = 0;  // as in split_find_splitters
+#pragma unroll
+  for (int r = 0; r < OWN; ++r) {
+    value[r]             = values[r * SPLIT_BLOCK + tid];
+    const bool finite    = __builtin_fabsf(value[r]) < __builtin_huge_valf();
+    const uint32_t image = sign_flip<uint32_t>(__float_as_uint(value[r]));
+    high                 = finite && image > high ? image : high;
+    low                  = finite && ~image > low ? ~image : low;
+  }
+  high = wave_inclusive_max_dpp(high);
+  low  = wave_inclusive_max_dpp(low);
+  if (lane == WAVE - 1) {
+    s_wave[wave] = high;
+    s_low[wave]  = low;
+  }
+#pragma unroll
+  for (int r = 0; r < SPAN; ++r) {
+    s_bins[r * SPLIT_BLOCK + tid] = 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < SPLIT_WAVES; ++v) {
+    high = s_wave[v] > high ? s_wave[v] : high;
+    low  = s_low[v] > low ? s_low[v] : low;
+  }
+  SplitBins bins;
+  bins.lowest      = __uint_as_float(sign_unflip<uint32_t>(~low));
+  const float span = __uint_as_float(sign_unflip<uint32_t>(high)) - bins.lowest;
+  bins.scale       = span > 0.0f ? static_cast<float>(BINS) / span : 0.0f;
+#pragma unroll
+  for (int r = 0; r < OWN; ++r) {
+    if (r * SPLIT_BLOCK + tid != 0) {  // (splitter 0 does not count)
+      atomicAdd(&s_bins[split_bin<BINS>(bins, value[r])], 1u);
+    }
+  }
+  __syncthreads();
+  uint32_t count[SPAN], sum = 0;
+#pragma unroll
+  for (int r = 0; r < SPAN; ++r) {
+    count[r] = s_bins[tid * SPAN + r];
+    sum += count[r];
+  }
+  const uint32_t sums = wave_inclusive_sum_dpp(sum);
+  if (lane == WAVE - 1) {
+    s_wave[wave] = sums;
+  }
+  __syncthreads();
+  uint32_t run = sums - sum + split_waves_before(s_wave, wave);
+#pragma unroll
+  for (int r = 0; r < SPAN; ++r) {
+    before[tid * SPAN + r] = static_cast<uint16_t>(run);
+    run += count[r];
+  }
+  if (tid == 0) {
+    *bins_out = bins;
+  }
+}
+
+// split_tile_kernel for these rows: tiles of up to 14 336 keys, 1024 to 4096 buckets.  The splitters, then the counters of
+// the ranks (a 16-bit word per wave and bucket), then the tile itself take turns in the same 140 KiB.
+template <typename KeyT, int CODEC, bool HAS_POS, int BITS>
+__global__ __launch_bounds__(SPLIT_BLOCK) void split_wide_tile_kernel(const KeyT* __restrict__ keys_in, uint32_t n, uint32_t tile_len,
+                                                                      const KeyT* __restrict__ images,
+                                                                      const uint32_t* __restrict__ split_places,
+                                                                      const uint16_t* __restrict__ before,
+                                                                      const SplitBins* __restrict__ bins_in,
+                                                                      KeyT* __restrict__ grouped, uint16_t* __restrict__ places,
+                                                                      uint16_t* __restrict__ starts)
+{
+  constexpr int ITEMS    = SPLIT_WIDE_ITEMS;
+  constexpr int BUCKETS  = 1 << BITS;
+  constexpr int BINS     = BUCKETS * SPLIT_WIDE_BINS;
+  constexpr int TILE     = SPLIT_BLOCK * ITEMS;
+  constexpr int OWN      = BUCKETS / SPLIT_BLOCK;  // buckets a thread scans
+  constexpr int S_BYTES  = BUCKETS * (static_cast<int>(sizeof(KeyT)) + 4) + BINS * 2;
+  constexpr int C_BYTES  = SPLIT_WAVES * BUCKETS * 2 + BUCKETS * 2;
+  constexpr int K_BYTES  = TILE * (static_cast<int>(sizeof(KeyT)) + (HAS_POS ? 2 : 0));
+  constexpr int SC_BYTES = S_BYTES > C_BYTES ? S_BYTES : C_BYTES;
+  static_assert(OWN == 1 || OWN == 2 || OWN == 4, "a thread's buckets are one word of the counters");
+  using Word = std::conditional_t<OWN == 1, uint16_t, std::conditional_t<OWN == 2, uint32_t, uint64_t>>;
+  __shared__ __align__(16) unsigned char s_mem[SC_BYTES > K_BYTES ? SC_BYTES : K_BYTES];
+  __shared__ uint32_t s_wave[SPLIT_WAVES];
+
+  const uint32_t tid    = threadIdx.x;
+  const uint32_t lane   = tid & (WAVE - 1);
+  const uint32_t wave   = tid / WAVE;
+  const uint32_t first  = blockIdx.x * tile_len;
+  const uint32_t len    = n - first < tile_len ? n - first : tile_len;  // (no tile is empty)
+  const uint32_t rounds = (len + SPLIT_BLOCK - 1) / SPLIT_BLOCK;        // uniform
+  const uint32_t woff   = wave * rounds * WAVE + lane;
+  auto runs             = [&](int i) -> bool { return i < static_cast<int>(rounds); };  // uniform
+
+  KeyT key[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const uint32_t o = woff + i * WAVE;
+    key[i]           = KeyT{};
+    if (runs(i)) {
+      key[i] = keys_in[first + (o < len ? o : len - 1)];
+    }
+  }
+  KeyT* const s_split        = reinterpret_cast<KeyT*>(s_mem);
+  uint32_t* const s_split_at = reinterpret_cast<uint32_t*>(s_mem + BUCKETS * sizeof(KeyT));
+  uint16_t* const s_before   = reinterpret_cast<uint16_t*>(s_mem + BUCKETS * (sizeof(KeyT) + 4));
+#pragma unroll
+  for (int r = 0; r < OWN; ++r) {
+    s_split[r * SPLIT_BLOCK + tid]    = images[r * SPLIT_BLOCK + tid];
+    s_split_at[r * SPLIT_BLOCK + tid] = split_places[r * SPLIT_BLOCK + tid];
+  }
+#pragma unroll
+  for (int r = 0; r < BINS / 2 / SPLIT_BLOCK; ++r) {
+    reinterpret_cast<uint32_t*>(s_before)[r * SPLIT_BLOCK + tid] = reinterpret_cast<const uint32_t*>(before)[r * SPLIT_BLOCK + tid];
+  }
+  const SplitBins bins = *bins_in;
+  __syncthreads();
+  // ---- buckets, as in split_tile_kernel, four keys of a thread at a time ----
+  uint32_t where[ITEMS];  // bucket; later, in the upper half, the rank; then where the key goes
+  constexpr int GROUP = 7;
+  static_assert(ITEMS % GROUP == 0, "whole groups");
+#pragma unroll
+  for (int g = 0; g < ITEMS; g += GROUP) {
+    uint32_t left[GROUP];
+#pragma unroll
+    for (int k = 0; k < GROUP; ++k) {
+      const uint32_t bin = split_bin<BINS>(bins, split_value<CODEC, KeyT>(key[g + k]));
+      where[g + k]       = s_before[bin];
+      left[k]            = (bin + 1 < BINS ? s_before[bin + 1] : static_cast<uint32_t>(BUCKETS - 1)) - where[g + k];
+    }
+    for (;;) {
+      uint32_t most = 0;
+#pragma unroll
+      for (int k = 0; k < GROUP; ++k) {
+        most = left[k] > most ? left[k] : most;
+      }
+      if (__ballot(most != 0) == 0) {
+        break;
+      }
+#pragma unroll
+      for (int k = 0; k < GROUP; ++k) {
+        const uint32_t at   = first + woff + (g + k) * WAVE;
+        const uint32_t half = (left[k] + 1) / 2;
+        const uint32_t c    = where[g + k] + half;
+        const KeyT image    = ordered_bits<CODEC, KeyT>(key[g + k]);
+        const KeyT split    = s_split[c];
+        const bool reached  = (split < image) | ((split == image) & (s_split_at[c] <= at));
+        where[g + k]        = reached ? c : where[g + k];
+        left[k]             = left[k] == 0 ? 0 : (reached ? left[k] - half : half - 1);
+      }
+    }
+  }
+  __syncthreads();
+  // ---- ranks ----
+  uint16_t* const s_ctr  = reinterpret_cast<uint16_t*>(s_mem);
+  uint16_t* const s_base = s_ctr + SPLIT_WAVES * BUCKETS;
+  for (uint32_t j = tid; j < SPLIT_WAVES * BUCKETS * 2 / 16; j += SPLIT_BLOCK) {
+    reinterpret_cast<uint4*>(s_mem)[j] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (runs(i)) {
+      where[i] |= split_match_rank<BITS>(where[i], woff + i * WAVE < len, s_ctr + wave * BUCKETS) << 16;
+    }
+  }
+  __syncthreads();
+  uint64_t totals = 0;  // of the thread's buckets, 16 bits each (a tile has fewer than 2^16 keys)
+  {
+    Word* const own = reinterpret_cast<Word*>(s_ctr) + tid;
+#pragma unroll
+    for (int v = 0; v < SPLIT_WAVES; ++v) {
+      const uint64_t c   = own[v * SPLIT_BLOCK];
+      own[v * SPLIT_BLOCK] = static_cast<Word>(totals);
+      totals += c;
+    }
+  }
+  uint32_t sum = 0;
+#pragma unroll
+  for (int r = 0; r < OWN; ++r) {
+    sum += static_cast<uint32_t>(totals >> (16 * r)) & 0xFFFFu;
+  }
+  const uint32_t sums = wave_inclusive_sum_dpp(sum);
+  if (lane == WAVE - 1) {
+    s_wave[wave] = sums;
+  }
+  __syncthreads();
+  {
+    uint32_t run       = sums - sum + split_waves_before(s_wave, wave);
+    uint16_t* const to = starts + static_cast<uint64_t>(blockIdx.x) * (BUCKETS + 1);
+#pragma unroll
+    for (int r = 0; r < OWN; ++r) {
+      s_base[tid * OWN + r] = static_cast<uint16_t>(run);
+      to[tid * OWN + r]     = static_cast<uint16_t>(run);
+      run += static_cast<uint32_t>(totals >> (16 * r)) & 0xFFFFu;
+    }
+    if (tid == 0) {
+      to[BUCKETS] = static_cast<uint16_t>(len);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const uint32_t b = where[i] & 0xFFFFu;
+    where[i]         = s_base[b] + s_ctr[wave * BUCKETS + b] + (where[i] >> 16);
+  }
+  __syncthreads();
+  // ---- the tile in the order of its buckets ----
+  KeyT* const s_keys      = reinterpret_cast<KeyT*>(s_mem);
+  uint16_t* const s_place = reinterpret_cast<uint16_t*>(s_mem + TILE * sizeof(KeyT));
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const uint32_t o = woff + i * WAVE;
+    if (runs(i) && o < len) {
+      s_keys[where[i]] = key[i];
+      if constexpr (HAS_POS) {
+        s_place[where[i]] = static_cast<uint16_t>(o);
+      }
+    }
+  }
+  __syncthreads();
+  for (uint32_t o = tid; o < len; o += SPLIT_BLOCK) {
+    grouped[first + o] = s_keys[o];
     if constexpr (HAS_POS) {
       places[first + o] = s_place[o];
     }
@@ -638,56 +936,75 @@ template <> struct SplitNative<CODEC_SIGNED, 8> { using type = int64_t; };
 template <> struct SplitNative<CODEC_FLOAT, 4> { using type = float; };
 template <> struct SplitNative<CODEC_FLOAT, 8> { using type = double; };
 
-constexpr uint32_t SPLIT_BIN_LIMIT = 24;  // most keys of a bin that are compared with each other
+// Most keys of a bin that are compared with each other.  (192 of them: 10^5 keys of a hundred values 50 us instead of 19,
+// 10^6 with a hundredth of NaNs and zeros 72 instead of 66: the longest walk of a wave is everyone's.)
+constexpr uint32_t SPLIT_BIN_LIMIT = 24;
 
 // One bucket of a row: its parts of all tiles gathered, sorted, stored.
 //   a bucket of equal images is in order: it was gathered in the order of the row
 //   others are spread over four bins per thread, of equal width between their smallest and their largest key; one atomic per key
 //     says which of its bin it is, a scan where the bin starts, a walk over the bin how many of its keys come before
-//   buckets with a NaN or a crowded bin: passes over the bytes of the images, of which numbers of keys move and the keys
-//     stay where they are in LDS.  One pass where there are two values, else the four leading bytes that vary and, where
-//     that does not put them in order, all
+//   buckets with a crowded bin: passes over the bytes of the images, of which numbers of keys move and the keys
+//     stay where they are in LDS.  One pass where there are two values
 // Ties go by the place in the gathered order.
+// Neighbouring buckets, whose parts of a tile share cache lines, go to neighbouring workgroups of one XCD.
 // Bound by its chain where every bucket has a compute unit (7 to 8 us for buckets of 400 keys; as one more mode of
 // lds_row_sort_kernel, with two reductions and two atomics per key, 11), else by the workgroups that fit, two to a unit of
 // 512 threads with 8-byte keys, three with 4-byte keys.
-template <typename KeyT, int CODEC, bool HAS_IDX, int BLOCK, int ITEMS>
-__global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<KeyT> sb, KeyT* __restrict__ keys_out,
+template <typename KeyT, int CODEC, bool HAS_IDX, bool WIDE>
+__global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const SplitBuckets<KeyT> sb, KeyT* __restrict__ keys_out,
                                                              int64_t* __restrict__ idx_out, int64_t index_offset)
 {
+  constexpr int BLOCK = SPLIT_BUCKET_BLOCK;
+  constexpr int ITEMS = SPLIT_BUCKET_ITEMS;
   constexpr int WAVES = BLOCK / WAVE;
   constexpr int TILE  = BLOCK * ITEMS;
-  constexpr int BINS  = 4 * BLOCK;
+  constexpr int BINS  = (WIDE ? 8 : 4) * BLOCK;
+  constexpr int TILES = WIDE ? SPLIT_WIDE_MAX_TILES : SPLIT_MAX_TILES;
+  constexpr int PARTS = (TILES + BLOCK - 1) / BLOCK;  // tiles per thread
   constexpr int OWN   = BINS / BLOCK;  // bins a thread scans
   static_assert(OWN % 4 == 0, "whole vectors");
-  static_assert(BLOCK >= SPLIT_MAX_TILES && BLOCK >= RADIX, "a thread per tile, and per digit");
+  static_assert(PARTS * BLOCK >= TILES && BLOCK >= RADIX, "a thread per digit");
   static_assert(TILE <= 65536 && BINS <= 65536, "numbers of 16 bits");
   constexpr int WORDS0 = BINS > WAVES * RADIX ? BINS : WAVES * RADIX;
   constexpr int WORDS  = WORDS0 > TILE / 2 ? WORDS0 : TILE / 2;
+  constexpr bool BY_PLACE = HAS_IDX || CODEC == CODEC_FLOAT;  // (integers that tie are the same bits)
   using Native         = typename SplitNative<CODEC, sizeof(KeyT)>::type;
   using Scale          = std::conditional_t<sizeof(KeyT) == 4, float, double>;
   __shared__ __align__(16) KeyT s_keys[TILE + SPLIT_BIN_LIMIT];
   __shared__ uint16_t s_num[TILE + SPLIT_BIN_LIMIT];
   __shared__ __align__(16) uint32_t s_ctr[WORDS];  // marks of tiles, bins, counters of digits
-  __shared__ uint32_t s_from[SPLIT_MAX_TILES], s_slot[SPLIT_MAX_TILES];
+  __shared__ uint32_t s_from[TILES];
+  uint32_t* const s_slot = reinterpret_cast<uint32_t*>(s_keys);  // (an oversized bucket's)
+  static_assert(TILES * 4 <= TILE * sizeof(KeyT), "a word per tile");
   __shared__ uint64_t s_red[2 * WAVES];
   __shared__ uint32_t s_wave[WAVES];
-  __shared__ uint32_t s_digit[RADIX];
+  static_assert(ITEMS * WAVES <= WAVE, "a lane per wave and round");
+  __shared__ uint32_t s_last[WAVE];
+  uint32_t* const s_digit = reinterpret_cast<uint32_t*>(s_num);  // (an oversized bucket's)
+  static_assert(RADIX * 4 <= TILE * 2 && RADIX <= TILES, "a word per digit");
 
   const uint32_t tid    = threadIdx.x;
   const uint32_t lane   = tid & (WAVE - 1);
   const uint32_t wave   = tid / WAVE;
-  const uint32_t bucket = blockIdx.x;
+  constexpr uint32_t XCDS = 8;  // workgroups go round them
+  const uint32_t bucket   = blockIdx.x % XCDS * (sb.buckets / XCDS) + blockIdx.x / XCDS;
 
   // ---- the bucket's part of every tile; m keys in all, `base` keys of the row before them ----
-  uint32_t start = 0, len = 0;
-  if (tid < sb.tiles) {
-    const uint16_t* const at = sb.starts + static_cast<uint64_t>(tid) * (sb.buckets + 1) + bucket;
-    start                    = at[0];
-    len                      = at[1] - start;
+  uint32_t start[PARTS], len[PARTS], starts = 0, lens = 0;
+#pragma unroll
+  for (int k = 0; k < PARTS; ++k) {
+    start[k] = 0, len[k] = 0;
+    if (tid * PARTS + k < sb.tiles) {
+      const uint16_t* const at = sb.starts + static_cast<uint64_t>(tid * PARTS + k) * (sb.buckets + 1) + bucket;
+      start[k]                 = at[0];
+      len[k]                   = at[1] - start[k];
+    }
+    starts += start[k];
+    lens += len[k];
   }
-  const uint32_t incl_len   = wave_inclusive_sum_dpp(len);
-  const uint32_t incl_start = wave_inclusive_sum_dpp(start);
+  const uint32_t incl_len   = wave_inclusive_sum_dpp(lens);
+  const uint32_t incl_start = wave_inclusive_sum_dpp(starts);
   if (lane == WAVE - 1) {
     s_red[wave] = (static_cast<uint64_t>(incl_start) << 32) | incl_len;
   }
@@ -695,7 +1012,7 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
     reinterpret_cast<uint4*>(s_ctr)[j] = make_uint4(0u, 0u, 0u, 0u);
   }
   __syncthreads();
-  uint32_t slot = incl_len - len, m = 0, base = 0;
+  uint32_t slot = incl_len - lens, m = 0, base = 0;
 #pragma unroll
   for (uint32_t w = 0; w < WAVES; ++w) {
     const uint64_t sums = s_red[w];
@@ -706,9 +1023,18 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
   if (m == 0) {
     return;  // uniform
   }
-  if (tid < sb.tiles) {
-    s_from[tid] = tid * sb.tile_len + start - slot;
-    s_slot[tid] = slot;
+  uint32_t part_slot[PARTS];
+#pragma unroll
+  for (int k = 0; k < PARTS; ++k) {
+    const uint32_t t = tid * PARTS + k;
+    part_slot[k]     = slot;
+    if (t < sb.tiles) {
+      s_from[t] = t * sb.tile_len + start[k] - slot;
+      if (m > TILE) {
+        s_slot[t] = slot;
+      }
+    }
+    slot += len[k];
   }
   if (m > TILE) {  // uniform
     __syncthreads();
@@ -717,71 +1043,63 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
   }
   // the number of a tile, plus one, at the first slot of its part
   uint16_t* const marks = reinterpret_cast<uint16_t*>(s_ctr);
-  if (len != 0) {
-    marks[slot] = static_cast<uint16_t>(tid + 1);
+#pragma unroll
+  for (int k = 0; k < PARTS; ++k) {
+    if (len[k] != 0) {
+      marks[part_slot[k]] = static_cast<uint16_t>(tid * PARTS + k + 1);
+    }
   }
   __syncthreads();
 
-  // ---- gather: wave w holds slots [64 rounds w, 64 rounds (w + 1)) ----
-  const uint32_t rounds = (m + BLOCK - 1) / BLOCK;  // uniform
-  const uint32_t first  = wave * rounds * WAVE + lane;
-  auto runs             = [&](int i) -> bool { return i < static_cast<int>(rounds); };  // uniform
-  auto holds            = [&](int i) -> bool { return runs(i) && first + i * WAVE < m; };
+  // ---- gather: slot number i * BLOCK + tid is a thread's i-th ----
+  auto slot_of = [&](int i) -> uint32_t { return i * BLOCK + tid; };
+  auto holds   = [&](int i) -> bool { return slot_of(i) < m; };
   KeyT key[ITEMS];
   uint32_t pos[HAS_IDX ? ITEMS : 1];
   {
-    uint32_t tile[ITEMS], last = 0;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {  // the last mark at or before a slot: in the wave's slots, then in the waves before
-      tile[i] = 0;
-      if (runs(i)) {
-        const uint32_t o = first + i * WAVE;
-        tile[i]          = wave_inclusive_max_dpp(o < m ? marks[o] : 0u);
-        tile[i]          = tile[i] > last ? tile[i] : last;
-        last             = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(tile[i]), WAVE - 1));
-      }
-    }
-    if (lane == 0) {
-      s_wave[wave] = last;
-    }
-    __syncthreads();
-    last = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < WAVES; ++w) {
-      last = (w < wave && s_wave[w] > last) ? s_wave[w] : last;
-    }
+    // the tile that a slot belongs to: the last mark at or before it, among the 64 slots of its wave and round, then in
+    // those before
+    uint32_t tile[ITEMS];
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-      key[i] = KeyT{};
-      if (runs(i)) {
-        const uint32_t o = first + i * WAVE;
-        tile[i]          = (tile[i] > last ? tile[i] : last) - 1u;
-        const uint32_t a = s_from[tile[i]] + (o < m ? o : m - 1);
-        key[i]           = sb.grouped[a];
-        if constexpr (HAS_IDX) {
-          pos[i] = sb.places[a];
-        }
+      tile[i] = wave_inclusive_max_dpp(holds(i) ? marks[slot_of(i)] : 0u);
+      if (lane == WAVE - 1) {
+        s_last[i * WAVES + wave] = tile[i];
+      }
+    }
+    __syncthreads();
+    const uint32_t lasts = wave_inclusive_max_dpp(lane < ITEMS * WAVES ? s_last[lane] : 0u);
+    const int uwave      = __builtin_amdgcn_readfirstlane(static_cast<int>(wave));
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int e           = i * WAVES + uwave;
+      const uint32_t before = e != 0 ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(lasts), e - 1)) : 0u;
+      tile[i]               = (tile[i] > before ? tile[i] : before) - 1u;
+      const uint32_t a      = s_from[tile[i]] + (holds(i) ? slot_of(i) : m - 1);
+      key[i]                = sb.grouped[a];
+      if constexpr (HAS_IDX) {
+        pos[i] = sb.places[a];
       }
     }
     if constexpr (HAS_IDX) {
 #pragma unroll
       for (int i = 0; i < ITEMS; ++i) {
-        pos[i] += runs(i) ? tile[i] * sb.tile_len : 0u;
+        pos[i] += tile[i] * sb.tile_len;
       }
     }
   }
   // ---- the extremes, on the images ----
-  KeyT low = 0, high = 0;  // the complement of the smallest, the largest
-  int special = 0;         // a NaN or a -0.0 (with positions, ties go by the place in any case)
+  constexpr KeyT NAN_IMAGE = static_cast<KeyT>(~KeyT{0});  // (float keys)
+  KeyT low = 0, high = 0;  // the complement of the smallest, the largest that is no NaN
+  int nans = 0;
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     if (holds(i)) {
       const KeyT image = ordered_bits<CODEC, KeyT>(key[i]);
-      high             = image > high ? image : high;
+      const bool nan   = CODEC == CODEC_FLOAT && image == NAN_IMAGE;
+      high             = !nan && image > high ? image : high;
       low              = static_cast<KeyT>(~image) > low ? static_cast<KeyT>(~image) : low;
-      if constexpr (CODEC == CODEC_FLOAT && !HAS_IDX) {
-        special |= is_nan_or_negative_zero(key[i]) ? 1 : 0;
-      }
+      nans |= nan ? 1 : 0;
     }
   }
   high = wave_max_dpp(high);
@@ -794,7 +1112,7 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
   for (uint32_t j = tid; j < BINS / 4; j += BLOCK) {
     reinterpret_cast<uint4*>(s_ctr)[j] = make_uint4(0u, 0u, 0u, 0u);
   }
-  special = __syncthreads_or(special);
+  nans = __syncthreads_or(nans);
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) {
     const KeyT h = static_cast<KeyT>(s_red[2 * w]), l = static_cast<KeyT>(s_red[2 * w + 1]);
@@ -802,11 +1120,11 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
     low  = l > low ? l : low;
   }
   low = static_cast<KeyT>(~low);
-  if (low == high) {  // uniform
+  if (low == NAN_IMAGE ? (CODEC == CODEC_FLOAT || high == NAN_IMAGE) : (low == high && nans == 0)) {  // uniform: one image
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       if (holds(i)) {
-        const uint32_t o = base + first + i * WAVE;
+        const uint32_t o = base + slot_of(i);
         if (keys_out != nullptr) {
           keys_out[o] = key[i];
         }
@@ -819,7 +1137,7 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
   }
   uint32_t to[ITEMS];  // where a key belongs; until then its bin and, in the upper half, which of the bin it is
   bool placed = false;
-  if (special == 0 && (CODEC != CODEC_FLOAT || high != static_cast<KeyT>(~KeyT{0}))) {  // uniform
+  {
     auto native = [](KeyT k) -> Native {
       Native v;
       __builtin_memcpy(&v, &k, sizeof(Native));
@@ -840,14 +1158,16 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
       to[i] = 0;
       if (holds(i)) {
         if constexpr (CODEC == CODEC_FLOAT) {
-          // (subtraction, scaling and truncation do not decrease with the key; clamped before the conversion, NaN to 0: an
-          // infinite extreme or span crowds a bin)
-          const Scale t = (native(key[i]) - origin) * scale;
+          // (subtraction, scaling and truncation do not decrease with the key; clamped before the conversion: an infinite
+          // extreme or span crowds a bin.  NaNs: the last bin)
+          const Native v = native(key[i]);
+          const Scale t  = (v - origin) * scale;
           if constexpr (sizeof(Scale) == 4) {
             to[i] = static_cast<uint32_t>(__builtin_fminf(__builtin_fmaxf(t, 0.0f), static_cast<float>(BINS - 1)));
           } else {
             to[i] = static_cast<uint32_t>(__builtin_fmin(__builtin_fmax(t, 0.0), static_cast<double>(BINS - 1)));
           }
+          to[i] = v != v ? BINS - 1 : to[i];
         } else {
           to[i] = static_cast<uint32_t>(static_cast<KeyT>(ordered_bits<CODEC, KeyT>(key[i]) - low) >> shift);
         }
@@ -891,9 +1211,9 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
       for (int i = 0; i < ITEMS; ++i) {
         if (holds(i)) {
           const uint32_t went = s_ctr[to[i] & 0xFFFFu] + (to[i] >> 16);
-          s_keys[went]        = key[i];
-          if constexpr (HAS_IDX) {
-            s_num[went] = static_cast<uint16_t>(first + i * WAVE);
+          s_keys[went]        = ordered_bits<CODEC, KeyT>(key[i]);
+          if constexpr (BY_PLACE) {
+            s_num[went] = static_cast<uint16_t>(slot_of(i));
           }
         }
       }
@@ -904,9 +1224,6 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
       static_assert(ITEMS % GROUP == 0, "whole groups");
 #pragma unroll
       for (int g = 0; g < ITEMS; g += GROUP) {
-        if (!runs(g)) {
-          break;  // uniform
-        }
         uint32_t from[GROUP], length[GROUP], before[GROUP], longest = 0;
 #pragma unroll
         for (int k = 0; k < GROUP; ++k) {
@@ -920,22 +1237,22 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
         }
         for (uint32_t j = 0; j < longest; ++j) {
           KeyT other[GROUP];
-          uint32_t number[HAS_IDX ? GROUP : 1];
+          uint32_t number[BY_PLACE ? GROUP : 1];
 #pragma unroll
           for (int k = 0; k < GROUP; ++k) {
             other[k] = s_keys[from[k] + j];
-            if constexpr (HAS_IDX) {
+            if constexpr (BY_PLACE) {
               number[k] = s_num[from[k] + j];
             }
           }
 #pragma unroll
           for (int k = 0; k < GROUP; ++k) {
-            const Native a = native(other[k]), b = native(key[g + k]);
+            const KeyT image = ordered_bits<CODEC, KeyT>(key[g + k]);
             bool earlier;
-            if constexpr (HAS_IDX) {
-              earlier = (a < b) | ((a == b) & (number[k] < first + (g + k) * WAVE));
+            if constexpr (BY_PLACE) {
+              earlier = (other[k] < image) | ((other[k] == image) & (number[k] < slot_of(g + k)));
             } else {
-              earlier = (a < b) | ((a == b) & (j < (to[g + k] >> 16)));
+              earlier = (other[k] < image) | ((other[k] == image) & (j < (to[g + k] >> 16)));
             }
             before[k] += (earlier & (j < length[k])) ? 1u : 0u;
           }
@@ -948,6 +1265,7 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
     }
   }
   if (!placed) {
+    high = nans != 0 ? NAN_IMAGE : high;
     // ---- the passes: number o of the order so far is s_num[o] ----
     int other_value = 0;
 #pragma unroll
@@ -955,106 +1273,36 @@ __global__ __launch_bounds__(BLOCK) void split_bucket_kernel(const SplitBuckets<
       if (holds(i)) {
         const KeyT image = ordered_bits<CODEC, KeyT>(key[i]);
         other_value |= (image != low && image != high) ? 1 : 0;
-        s_keys[first + i * WAVE] = key[i];
-        s_num[first + i * WAVE]  = static_cast<uint16_t>(first + i * WAVE);
+        s_keys[slot_of(i)] = key[i];
+        s_num[slot_of(i)]  = static_cast<uint16_t>(slot_of(i));
       }
     }
-    const bool two_values = __syncthreads_or(other_value) == 0;
-    const int top         = 64 - __builtin_clzll(static_cast<unsigned long long>(static_cast<KeyT>(low ^ high)));  // bits that vary: below it
-    int from_bit          = (!two_values && top > 32) ? top - 32 : 0;
-    for (;;) {
-      for (int bit = from_bit; bit < top; bit += RADIX_BITS) {
-        for (uint32_t j = tid; j < WAVES * RADIX; j += BLOCK) {
-          s_ctr[j] = 0;
-        }
-        __syncthreads();
-        uint32_t packed[ITEMS];  // number, digit
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-          if (runs(i)) {
-            const uint32_t o = first + i * WAVE;
-            const bool valid = o < m;
-            const uint32_t k = s_num[valid ? o : m - 1];
-            const KeyT image = ordered_bits<CODEC, KeyT>(s_keys[k]);
-            const uint32_t d = two_values ? (image == high ? 1u : 0u) : static_cast<uint32_t>(image >> bit) & (RADIX - 1);
-            packed[i]        = (k << 8) | d;
-            to[i]            = wave_match_rank(d, valid, s_ctr + wave * RADIX);
-          }
-        }
-        __syncthreads();
-        uint32_t total = 0;
-        if (tid < RADIX) {
-#pragma unroll
-          for (int w = 0; w < WAVES; ++w) {
-            const uint32_t c       = s_ctr[w * RADIX + tid];
-            s_ctr[w * RADIX + tid] = total;
-            total += c;
-          }
-        }
-        const uint32_t incl = wave_inclusive_sum_dpp(total);
-        if (lane == WAVE - 1) {
-          s_wave[wave] = incl;
-        }
-        __syncthreads();
-        if (tid < RADIX) {
-          uint32_t run = incl - total;
-#pragma unroll
-          for (uint32_t w = 0; w < RADIX / WAVE; ++w) {
-            run += w < wave ? s_wave[w] : 0u;
-          }
-          s_digit[tid] = run;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-          if (holds(i)) {
-            const uint32_t d = packed[i] & (RADIX - 1);
-            s_num[s_digit[d] + s_ctr[wave * RADIX + d] + to[i]] = static_cast<uint16_t>(packed[i] >> 8);
-          }
-        }
-        __syncthreads();
-        if (two_values) {
-          break;
-        }
-      }
-      if (from_bit == 0) {
-        break;
-      }
-      int bad = 0;
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) {
-        const uint32_t o = first + i * WAVE;
-        if (runs(i) && o + 1 < m) {
-          bad |= ordered_bits<CODEC, KeyT>(s_keys[s_num[o]]) > ordered_bits<CODEC, KeyT>(s_keys[s_num[o + 1]]) ? 1 : 0;
-        }
-      }
-      if (__syncthreads_or(bad) == 0) {
-        break;
-      }
-      from_bit = 0;
+    int top           = 64 - __builtin_clzll(static_cast<unsigned long long>(static_cast<KeyT>(low ^ high)));  // bits that vary: below it
+    uint16_t* const c = reinterpret_cast<uint16_t*>(s_ctr);
+    if (__syncthreads_or(other_value) == 0) {
+      split_order_passes<CODEC, BLOCK, ITEMS>(s_keys, s_num, c, s_wave, m, top - 1, top);  // two values: they differ in this bit
+    } else {
+      split_order<CODEC, BLOCK, ITEMS>(s_keys, s_num, c, s_wave, m, top);
     }
     // as the walk leaves it: where each key of this thread belongs
     uint32_t number[ITEMS];
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-      if (holds(i)) {
-        number[i] = s_num[first + i * WAVE];
-      }
+      number[i] = s_num[holds(i) ? slot_of(i) : 0u];
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       if (holds(i)) {
-        s_num[number[i]] = static_cast<uint16_t>(first + i * WAVE);
+        s_num[number[i]] = static_cast<uint16_t>(slot_of(i));
       }
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-      if (holds(i)) {
-        to[i]  = s_num[first + i * WAVE];
-        key[i] = s_keys[first + i * WAVE];
-      }
+      const uint32_t o = holds(i) ? slot_of(i) : 0u;
+      to[i]            = s_num[o];
+      key[i]           = s_keys[o];
     }
   }
   // ---- out, through LDS, so that neighbouring lanes store neighbouring elements ----

@@ -24,6 +24,11 @@ def test_requests_in_range(lib):
                 # the keys, two words and a place per key, and a table of at most a word per key and bucket's tile
                 assert n * (kb + 8 + 2 * idx) <= need <= n * (kb + 8 + 2 * idx) + (1 << 20), (code, n, idx)
                 assert need % 256 == 0
+            last = 4096 * 2560 if kb == 8 else 1 << 20
+            assert size(code, last, last, idx) != 0 and size(code, last + 1, last + 1, idx) == 0
+            if kb == 8:  # and the sample's own sort
+                for n in ((1 << 20) + 1, last):
+                    assert n * (kb + 8 + 2 * idx) < size(code, n, n, idx) < n * (kb + 8 + 2 * idx) + 40 * (1 << 20), (code, n, idx)
     for code in (F16, C64):
         assert size(code, 100_000, 100_000, 0) == 0
     assert size(F32, 200_000, 100_000, 0) == 0 and size(F32, 0, 0, 0) == 0 and size(99, 100_000, 100_000, 0) == 0

@@ -58,9 +58,11 @@ def test_lengths(lib, torch_cuda, dtype, n):
     _check(lib, torch_cuda, make_input(dtype, (n,), seed=n % 1000), f"{np.dtype(dtype)} {n}")
 
 
+# 8-byte keys only; from 2^20 the sample is sorted ahead (ends of the numbers of buckets, of sampled keys and of tiles)
 @pytest.mark.parametrize("dtype", [np.float64, np.int64, np.uint64])
-@pytest.mark.parametrize("n", [6145, 8192])
-def test_short_rows_of_wide_keys(lib, torch_cuda, dtype, n):
+@pytest.mark.parametrize("n", [6145, 8192, (1 << 20) + 1, 1024 * 1365, 1024 * 1365 + 1, 1 << 21, (1 << 21) + 1, 256 * 14336, 256 * 14336 + 1,
+                               1 << 22, (1 << 22) + 1, 4096 * 2048 + 1, 4096 * 2560])
+def test_lengths_of_wide_keys(lib, torch_cuda, dtype, n):
     _check(lib, torch_cuda, make_input(dtype, (n,), seed=n), f"{np.dtype(dtype)} {n}")
 
 
@@ -103,8 +105,10 @@ def _kind(kind, dtype, n):
 @pytest.mark.parametrize("dtype", [np.float32, np.int32, np.float64, np.uint64])
 @pytest.mark.parametrize("kind", ["equal", "two values", "hundred values", "ascending", "descending", "runs", "magnitudes",
                                   "cluster", "far"])
-@pytest.mark.parametrize("n", [9001, 100_003, 200_001, 700_001])
+@pytest.mark.parametrize("n", [9001, 100_003, 200_001, 700_001, 2_500_001])
 def test_kinds_of_keys(lib, torch_cuda, dtype, kind, n):
+    if n > 1 << 20 and np.dtype(dtype).itemsize == 4:
+        pytest.skip("4-byte keys are split up to 2^20")
     _check(lib, torch_cuda, _kind(kind, dtype, n), f"{np.dtype(dtype)} {n} {kind}")
 
 
@@ -120,11 +124,13 @@ def _sample_places(n, samples):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.int32, np.float64, np.uint64])
-@pytest.mark.parametrize("n,samples", [(20_000, 1024), (150_001, 2048), (300_007, 4096)])
+@pytest.mark.parametrize("n,samples", [(20_000, 1024), (150_001, 2048), (300_007, 4096), (1_100_001, 16384)])
 @pytest.mark.parametrize("share", ["all", "some"])
 def test_buckets_beyond_lds(lib, torch_cuda, dtype, n, samples, share):
     """A row made so that its sample says nothing: the sampled keys are the largest.  All others share a bucket, or, where
     an eighth of the sample is left as it is, buckets of several times the room."""
+    if n > 1 << 20 and np.dtype(dtype).itemsize == 4:
+        pytest.skip("4-byte keys are split up to 2^20")
     rng = np.random.default_rng(n)
     x = rng.integers(0, 1 << 30, n).astype(dtype)
     places = _sample_places(n, samples)
@@ -164,14 +170,19 @@ def test_the_public_calls_take_it(lib, torch_cuda):
         assert np.array_equal(np.asarray(got[1]), np.sort(x))
         assert labels(lambda: a.sort()) == launches
         assert np.array_equal(np.asarray(a), np.sort(x))
-    for x in (rng.standard_normal(4000), rng.standard_normal((2, 30_000)), rng.standard_normal((1 << 20) + 1)):
+    x = rng.integers(0, 1 << 40, (1 << 20) + 1)
+    got = []
+    assert labels(lambda: got.append(num.argsort(num.array(x))))[-3:] == ["split_table", "split_tiles", "split_buckets"]
+    assert runtime._status_used == 0 and np.array_equal(np.asarray(got[0]), np.argsort(x, kind="stable"))
+    for x in (rng.standard_normal(4000), rng.standard_normal((2, 30_000)), rng.standard_normal((1 << 20) + 1).astype(np.float32),
+              rng.standard_normal(4096 * 2560 + 1)):
         assert "split_tiles" not in labels(lambda: num.sort(num.array(x)))
 
 
-def test_captured_and_replayed(lib, torch_cuda):
-    """The two launches in a graph, replayed on other keys with eager work between the replays."""
+@pytest.mark.parametrize("n", [150_000, 1_300_000])
+def test_captured_and_replayed(lib, torch_cuda, n):
+    """The launches in a graph, replayed on other keys with eager work between the replays."""
     torch = torch_cuda
-    n = 150_000
     code = _lib.DTYPE_CODES[np.dtype(np.float64)]
     tb = lib.cpn_local_sort_split_temp_bytes(code, n, n, 1)
     x = torch.empty(n, dtype=torch.float64, device="cuda")
