@@ -96,6 +96,11 @@ PROTOTYPES: dict[str, tuple] = {
     "cpn_searchsorted": (
         c_int, [c_int, c_void_p, c_uint64, c_void_p, c_uint64, c_int, c_void_p, c_void_p, c_uint64, c_void_p]
     ),
+    "cpn_unique_sorted_temp_bytes": (c_uint64, [c_int, c_uint64]),
+    "cpn_unique_sorted": (c_int, [c_int, c_void_p, c_void_p, c_uint64, c_void_p, c_void_p, c_uint64, c_void_p]),
+    "cpn_distinct_temp_bytes": (c_uint64, [c_int, c_uint64, ctypes.POINTER(c_uint64)]),
+    "cpn_distinct_plan": (c_int, [c_int, c_void_p, c_uint64, c_void_p, c_uint64, c_void_p]),
+    "cpn_distinct": (c_int, [c_int, c_void_p, c_uint64, c_int, c_void_p, c_uint64, c_void_p]),
     "cpn_unique_temp_bytes": (c_uint64, [c_int, c_uint64]),
     "cpn_unique": (c_int, [c_int, c_void_p, c_void_p, c_uint64, c_void_p, c_void_p, c_uint64, c_void_p]),
     "cpn_quantile_sorted": (

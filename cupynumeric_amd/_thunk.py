@@ -15,6 +15,14 @@ from .runtime import runtime
 if TYPE_CHECKING:
     import torch
 
+# Where in its workspace `cpn_unique` may put the count: beside the status word, in a line that nothing else uses.
+UNIQUE_COUNT_OFFSET = 64
+# Longest array of integers that `unique` splits by sampled keys (`cpn_local_sort_split_temp_bytes`).  Arrays that it is asked
+# of repeat their values, and 8-byte ones mostly leave upper bytes constant, whose passes the sort of `cpn_unique` skips:
+# int64 below 10^9, us per call that way / split: 2^20 + 1 of as many values 204 / 125, of 1000 219 / 145;
+# 2^21 of 1000 169 / 156; 2^22 of as many 206 / 211, of 20000 203 / 253.
+UNIQUE_SPLIT_INTEGERS = 1 << 21
+
 # dtypes the reference supports (`cupynumeric/_utils/array.py:28-43`)
 SUPPORTED_DTYPES = tuple(_lib.DTYPE_CODES.keys())
 
@@ -319,27 +327,70 @@ class DeviceArray:
     def unique(self) -> "DeviceArray":
         """`DeferredArray.unique` (`cupynumeric/_thunk/deferred.py:5375-5395`): sorted distinct
         values of the flattened array.  The result size is only known on the device (an unbound
-        store in the reference); reading it back is the one synchronisation of this call."""
+        store in the reference) and read back before the call returns."""
         if self.size == 0:
             return DeviceArray((0,), self.dtype)
         lib = _lib.load()
         code = _lib.DTYPE_CODES[self.dtype]
-        temp_bytes = lib.cpn_unique_temp_bytes(code, self.size)
+        stream = ctypes.c_void_p(runtime.stream_handle())
+        list_offset = ctypes.c_uint64()
+        few_bytes = lib.cpn_distinct_temp_bytes(code, self.size, ctypes.byref(list_offset))
+        split = self.dtype.kind == "f" or self.size <= UNIQUE_SPLIT_INTEGERS
+        split = split and lib.cpn_local_sort_split_temp_bytes(code, self.size, self.size, 0) != 0
+        temp_bytes = (lib.cpn_unique_sorted_temp_bytes if split else lib.cpn_unique_temp_bytes)(code, self.size)
         if temp_bytes == 0:
             raise NotImplementedError(f"cpn_unique: no workspace layout for dtype={self.dtype}, size={self.size}")
-        temp = runtime.empty_bytes(temp_bytes)
         out = DeviceArray((self.size,), self.dtype)
-        count = runtime.torch.zeros(1, dtype=runtime.torch.int64, device=runtime.require_device())
-        stream = ctypes.c_void_p(runtime.stream_handle())
-        status = lib.cpn_unique(
-            code, self.base.ptr(), out.base.ptr(), self.size, count.data_ptr(), temp.data_ptr(), temp_bytes, stream
-        )
+        temp = runtime.empty_bytes(max(temp_bytes + 8, few_bytes))
+        if few_bytes != 0:
+            few = self._unique_by_hash(lib, code, temp, list_offset.value, stream)
+            if few is not None:
+                return few
+        if split:  # the sort that cannot fail on the device, then what follows it
+            from ._sort import sort_task
+
+            ordered = DeviceArray((self.size,), self.dtype)
+            sort_task(ordered, DeviceArray((self.size,), self.dtype, self.base), False, True)
+            at = temp_bytes
+            status = lib.cpn_unique_sorted(
+                code, ordered.base.ptr(), out.base.ptr(), self.size, temp.data_ptr() + at, temp.data_ptr(), temp_bytes, stream
+            )
+        else:
+            at = UNIQUE_COUNT_OFFSET
+            status = lib.cpn_unique(
+                code, self.base.ptr(), out.base.ptr(), self.size, temp.data_ptr() + at, temp.data_ptr(), temp_bytes, stream
+            )
         _lib.check(status, "cpn_unique")
-        if runtime.check_mode != "off":  # (reading the count below synchronises anyway)
+        if runtime.check_mode != "off":
             runtime.flush_status()  # errors of earlier work first
-            _lib.check(lib.cpn_local_sort_check(temp.data_ptr(), stream), "cpn_unique")
-        n_unique = int(count.item())
+        # one copy brings the count, and the status word where there is one
+        head = temp[0 if not split else at : at + 8].cpu().numpy()
+        if not split and runtime.check_mode != "off" and head[:4].view(np.uint32)[0] != 0:
+            _lib.check(_lib.CPN_ERR_DEVICE, "cpn_unique")
+        n_unique = int(head[-8:].view(np.int64)[0])
         return DeviceArray((n_unique,), self.dtype, out.base)
+
+    def _unique_by_hash(self, lib: Any, code: int, temp: Any, list_offset: int, stream: Any) -> "DeviceArray | None":
+        """`unique` of an integer array with few values for its length: they are collected unsorted
+        (`cpn_distinct`), then sorted.  None: not such an array."""
+        if runtime.check_mode != "off":
+            runtime.flush_status()  # errors of earlier work first
+        args = (code, self.base.ptr(), self.size)
+        _lib.check(lib.cpn_distinct_plan(*args, temp.data_ptr(), temp.numel(), stream), "cpn_distinct_plan")
+        head = temp[:12].view(runtime.torch.int32)
+        mode = head.tolist()[0]  # (waits, so that an array that is sorted after all waits for no more than this)
+        if mode == 0:
+            return None
+        _lib.check(lib.cpn_distinct(*args, mode, temp.data_ptr(), temp.numel(), stream), "cpn_distinct")
+        _, failed, count = head.tolist()
+        if failed != 0:
+            return None
+        found = DeviceArray.from_device(temp[list_offset : list_offset + count * self.dtype.itemsize], (count,), self.dtype)
+        out = DeviceArray((count,), self.dtype)
+        from ._sort import sort_task
+
+        sort_task(out, found, False, True)
+        return out
 
     def to_complex(self, dtype: Any) -> "DeviceArray":
         """Real -> complex cast (`astype` in `sort_complex`, `cupynumeric/_module/ssc_sorting.py:150-159`)."""

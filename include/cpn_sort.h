@@ -245,8 +245,8 @@ int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const void* valu
  * Sorted distinct values.  values_out has room for `volume` elements and receives the
  * distinct values in ascending order (the first of every run of equal keys in the stable
  * sorted order: all NaNs count as one value, -0.0 and +0.0 as one); *count_out (device
- * memory, 8-byte aligned) receives how many there are.  `temp` is a 256-byte aligned
- * workspace of at least cpn_unique_temp_bytes(dtype, volume) bytes; the device status word of
+ * memory, 8-byte aligned) receives how many there are; temp + 64, which lies beside the status
+ * word, may be that place.  `temp` is a 256-byte aligned workspace of at least cpn_unique_temp_bytes(dtype, volume) bytes; the device status word of
  * the sort is at its start, so cpn_local_sort_check(temp, stream) applies.  values_in is not
  * modified.  Replaces UniqueTask::gpu_variant on one processor
  * (src/cupynumeric/set/unique.cu:137-204, cupynumeric/_thunk/deferred.py:5375-5395).
@@ -255,6 +255,29 @@ int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const void* valu
 uint64_t cpn_unique_temp_bytes(int dtype, uint64_t volume);
 int cpn_unique(int dtype, const void* values_in, void* values_out, uint64_t volume,
                uint64_t* count_out, void* temp, uint64_t temp_bytes, void* stream);
+
+/*
+ * The second half of cpn_unique, for 1 or more values that the caller has sorted itself: `sorted` is not modified, and
+ * `temp` is a 256-byte aligned workspace of cpn_unique_sorted_temp_bytes(dtype, volume) bytes without a status word
+ * (nothing here can fail on the device).  The reference does both in one task (src/cupynumeric/set/unique.cu:137-204).
+ */
+uint64_t cpn_unique_sorted_temp_bytes(int dtype, uint64_t volume);
+int cpn_unique_sorted(int dtype, const void* sorted, void* values_out, uint64_t volume, uint64_t* count_out, void* temp,
+                      uint64_t temp_bytes, void* stream);
+
+/*
+ * The distinct values of an integer array (4 or 8 bytes), in no order, where a sample says that there are few of them for
+ * its length: what a caller that can wait for the count sorts instead of calling cpn_unique.  `temp` is a 256-byte aligned
+ * workspace of cpn_distinct_temp_bytes(dtype, volume, &list_offset) bytes (0: not tried for this type and length).
+ * cpn_distinct_plan looks at the sample; when the stream has finished, the first 32-bit word of `temp` is the mode: 0 for
+ * "not this array" (call cpn_unique), otherwise the `mode` of a call of cpn_distinct on the same array and workspace.  After
+ * that the first three words are the mode; not 0 where the attempt came to nothing (call cpn_unique); and the number of
+ * values, which lie in `temp` from list_offset on.  Every kernel ends by itself and nothing outside `temp` is written.  It
+ * has no counterpart in the reference, whose UniqueTask sorts (src/cupynumeric/set/unique.cu:137-204).
+ */
+uint64_t cpn_distinct_temp_bytes(int dtype, uint64_t volume, uint64_t* list_offset);
+int cpn_distinct_plan(int dtype, const void* values, uint64_t volume, void* temp, uint64_t temp_bytes, void* stream);
+int cpn_distinct(int dtype, const void* values, uint64_t volume, int mode, void* temp, uint64_t temp_bytes, void* stream);
 
 /*
  * Quantiles along the middle axis of `sorted`, a dense [outer][n][inner] array that is already
