@@ -17,6 +17,8 @@ if TYPE_CHECKING:
 
 # Where in its workspace `cpn_unique` may put the count: beside the status word, in a line that nothing else uses.
 UNIQUE_COUNT_OFFSET = 64
+# Fewer values are never grouped by the parts of the array (`cpn_searchsorted_grouped`); asking would cost them a call.
+GROUPED_MIN_VALUES = 1 << 16
 # Longest array of integers that `unique` splits by sampled keys (`cpn_local_sort_split_temp_bytes`).  Arrays that it is asked
 # of repeat their values, and 8-byte ones mostly leave upper bytes constant, whose passes the sort of `cpn_unique` skips:
 # int64 below 10^9, us per call that way / split: 2^20 + 1 of as many values 204 / 125, of 1000 219 / 145;
@@ -303,9 +305,19 @@ class DeviceArray:
             raise TypeError("searchsorted: arrays must share one dtype and the result must be int64")
         lib = _lib.load()
         code = _lib.DTYPE_CODES[rhs.dtype]
+        stream = ctypes.c_void_p(runtime.stream_handle())
+        if v.size >= GROUPED_MIN_VALUES:
+            args = (code, rhs.base.ptr() if rhs.size else None, rhs.size)
+            temp_bytes = lib.cpn_searchsorted_grouped_temp_bytes(*args, v.size)
+            if temp_bytes != 0:  # (cannot fail on the device: no status to look at)
+                temp = runtime.empty_bytes(temp_bytes)
+                status = lib.cpn_searchsorted_grouped(
+                    *args, v.base.ptr(), v.size, int(is_left), self.base.ptr(), temp.data_ptr(), temp_bytes, stream
+                )
+                _lib.check(status, "cpn_searchsorted")
+                return
         temp_bytes = lib.cpn_searchsorted_temp_bytes(code, rhs.size, v.size)
         temp = runtime.empty_bytes(temp_bytes) if temp_bytes else None
-        stream = ctypes.c_void_p(runtime.stream_handle())
         status = lib.cpn_searchsorted(
             code,
             rhs.base.ptr() if rhs.size else None,

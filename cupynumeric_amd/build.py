@@ -28,6 +28,7 @@ SOURCES = [
     "convert.hip",
     "gather.hip",
     "searchsorted.hip",
+    "grouped_search.hip",
     "unique.hip",
     "distinct.hip",
     "quantile.hip",
@@ -61,7 +62,7 @@ HIPCC_FLAGS = [
 # thread shape once spilled 516 bytes per lane and took 3.3 ms instead of 0.8), so the build
 # refuses it.  The scatter pass of the global sort is allowed the few words it is known to park.
 # (So is the sort of equalised pieces, csrc/equal_digits.h, and their plan, a single workgroup.)
-SCRATCH_LIMITS = (("row_sort_kernel", 0), ("count16_", 0), ("onesweep_kernel", 32), ("merge_ranks_kernel", 0), ("split_tile_kernel", 0), ("split_gather_kernel", 0), ("split_bucket_kernel", 0), ("split_wide_tile_kernel", 0), ("collect_", 0),
+SCRATCH_LIMITS = (("row_sort_kernel", 0), ("count16_", 0), ("onesweep_kernel", 32), ("merge_ranks_kernel", 0), ("split_tile_kernel", 0), ("split_gather_kernel", 0), ("split_bucket_kernel", 0), ("split_wide_tile_kernel", 0), ("collect_", 0), ("find_", 0),
                   ("eq_sweep_kernel", 0), ("eq_sort_kernel", 80), ("eq_plan_kernel", 128), ("eq_gather_kernel", 0),
                   ("eq_histogram_kernel", 0), ("eq_segments_kernel", 0))
 

@@ -242,6 +242,16 @@ int cpn_searchsorted(int dtype, const void* sorted, uint64_t n, const void* valu
                      uint64_t temp_bytes, void* stream);
 
 /*
+ * The same result by another way, for many values in a long array of real numbers of 4 or 8 bytes that begins on a 16-byte
+ * boundary: the values are grouped by the part of the array that they belong to and not sorted.  The workspace (256-byte
+ * aligned) has cpn_searchsorted_grouped_temp_bytes(...) bytes, 0 where cpn_searchsorted is to be called instead (the call
+ * itself is then CPN_ERR_UNSUPPORTED); it has no status word, since nothing here can fail on the device.
+ */
+uint64_t cpn_searchsorted_grouped_temp_bytes(int dtype, const void* sorted, uint64_t n, uint64_t num_values);
+int cpn_searchsorted_grouped(int dtype, const void* sorted, uint64_t n, const void* values, uint64_t num_values, int left,
+                             int64_t* positions_out, void* temp, uint64_t temp_bytes, void* stream);
+
+/*
  * Sorted distinct values.  values_out has room for `volume` elements and receives the
  * distinct values in ascending order (the first of every run of equal keys in the stable
  * sorted order: all NaNs count as one value, -0.0 and +0.0 as one); *count_out (device
