@@ -50,6 +50,8 @@ CPN_ERR_SCRATCH = -9
 # include/cpn_sort.h: options of cpn_local_sort_ex
 CPN_SORT_SINGLE_TICKET = 1
 CPN_SORT_SPLIT = 4
+CPN_ROUTE_MAY_FAIL = 1
+CPN_ROUTE_STATUS_ONLY = 2
 
 # include/cpn_sort.h: workspace of cpn_local_sort_static
 STATIC_SCRATCH_BYTES = 64 << 20
@@ -88,6 +90,7 @@ PROTOTYPES: dict[str, tuple] = {
         c_int,
         [c_int, c_uint64, c_uint64, c_int, c_int, c_int, c_void_p, c_uint64, c_void_p, c_void_p],
     ),
+    "cpn_local_sort_route": (c_uint64, [c_int, c_uint64, c_uint64, c_int, c_int, c_int]),
     "cpn_local_sort_may_fail": (c_int, [c_int, c_uint64, c_uint64, c_int, c_uint64]),
     "cpn_local_sort_check": (c_int, [c_void_p, c_void_p]),
     "cpn_real_to_complex": (c_int, [c_int, c_void_p, c_int, c_void_p, c_uint64, c_void_p]),

@@ -11,7 +11,7 @@ from numpy.exceptions import AxisError
 from numpy.lib.array_utils import normalize_axis_index
 
 from . import _lib
-from .runtime import runtime
+from .runtime import STATUS_LINE_BYTES, runtime
 
 if TYPE_CHECKING:
     from ._thunk import DeviceArray
@@ -19,6 +19,8 @@ if TYPE_CHECKING:
 
 # Shorter rows are never split (`cpn_local_sort_split_temp_bytes`); asking would cost them a call.
 SPLIT_MIN_ROW = 6145
+# Answer of `cpn_local_sort_route` for rows that are sorted without a workspace.
+STATUS_ONLY = STATUS_LINE_BYTES | _lib.CPN_ROUTE_STATUS_ONLY
 
 
 def sort_flattened(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable: bool) -> None:
@@ -73,7 +75,7 @@ def sort_task(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable
         values_out = output.base.ptr()
         indices_out = None
 
-    stream = ctypes.c_void_p(runtime.stream_handle())
+    stream = runtime.stream_handle()
     if seg >= SPLIT_MIN_ROW:
         temp_bytes = lib.cpn_local_sort_split_temp_bytes(code, volume, seg, int(argsort))
         if temp_bytes != 0:  # two launches that cannot fail on the device: no status to look at
@@ -83,7 +85,16 @@ def sort_task(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable
             _lib.check(status, "cpn_local_sort")
             return
 
-    temp_bytes = lib.cpn_local_sort_temp_bytes(code, volume, seg, int(not argsort), int(argsort), int(in_place))
+    route = lib.cpn_local_sort_route(code, volume, seg, not argsort, argsort, in_place)
+    if route == STATUS_ONLY:
+        line = runtime.status_line()
+        if line is not None:
+            status = lib.cpn_local_sort_ex(
+                code, values_in, values_out, indices_out, volume, seg, 0, stable, 0, line, STATUS_LINE_BYTES, stream
+            )
+            _lib.check(status, "cpn_local_sort")
+            return
+    temp_bytes = route & ~(_lib.CPN_ROUTE_MAY_FAIL | _lib.CPN_ROUTE_STATUS_ONLY)
     if temp_bytes == 0:
         _lib.check(
             lib.cpn_local_sort(code, values_in, values_out, indices_out, volume, seg, 0, int(stable), None, 0, None),
@@ -113,7 +124,7 @@ def sort_task(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable
     temp = issue()
     # Rows sorted by the per-row kernels, whole or in pieces that are merged, cannot fail on the device.
     # The global sort can: a bounded wait between its tiles may run out.
-    if runtime.check_mode == "off" or not lib.cpn_local_sort_may_fail(code, volume, seg, int(indices_out is not None), temp_bytes):
+    if runtime.check_mode == "off" or not route & _lib.CPN_ROUTE_MAY_FAIL:
         return
     if runtime.check_mode == "lazy":
         runtime.defer_status(temp)

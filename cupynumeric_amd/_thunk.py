@@ -10,6 +10,7 @@ from typing import TYPE_CHECKING, Any
 import numpy as np
 
 from . import _lib
+from ._sort import sort_deferred, sort_task
 from .runtime import runtime
 
 if TYPE_CHECKING:
@@ -74,7 +75,7 @@ class DeviceArray:
     do with `output.base = result.base` (`cupynumeric/_thunk/_sort.py:47,73,76`)."""
 
     def __init__(self, shape: tuple[int, ...], dtype: Any, base: Storage | None = None) -> None:
-        self.shape = tuple(int(s) for s in shape)
+        self.shape = tuple(map(int, shape))
         self.dtype = check_dtype(dtype)
         self.base = base if base is not None else Storage(self.size * self.dtype.itemsize)
 
@@ -239,8 +240,6 @@ class DeviceArray:
     ) -> None:
         """`DeferredArray.sort` (`cupynumeric/_thunk/deferred.py:5453-5474`): `self` receives the
         result of sorting `rhs`."""
-        from ._sort import sort_deferred
-
         # (messages and exception types are the reference's: callers and its tests match on them)
         if order is not None:
             raise NotImplementedError(
@@ -264,8 +263,6 @@ class DeviceArray:
     ) -> None:
         """`DeferredArray.partition` (`cupynumeric/_thunk/deferred.py:5476-5494`): falls back to an
         (unstable-flagged) sort, which satisfies the partition property for every `kth`."""
-        from ._sort import sort_deferred
-
         if order is not None:
             raise NotImplementedError(
                 "cuPyNumeric does not support partitioning with 'order' as "
@@ -359,8 +356,6 @@ class DeviceArray:
             if few is not None:
                 return few
         if split:  # the sort that cannot fail on the device, then what follows it
-            from ._sort import sort_task
-
             ordered = DeviceArray((self.size,), self.dtype)
             sort_task(ordered, DeviceArray((self.size,), self.dtype, self.base), False, True)
             at = temp_bytes
@@ -399,8 +394,6 @@ class DeviceArray:
             return None
         found = DeviceArray.from_device(temp[list_offset : list_offset + count * self.dtype.itemsize], (count,), self.dtype)
         out = DeviceArray((count,), self.dtype)
-        from ._sort import sort_task
-
         sort_task(out, found, False, True)
         return out
 

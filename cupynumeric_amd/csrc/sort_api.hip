@@ -259,6 +259,19 @@ int cpn_local_sort_may_fail(int dtype, uint64_t volume, uint64_t sort_dim_size, 
            : 0;
 }
 
+uint64_t cpn_local_sort_route(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_values, int want_indices, int in_place)
+{
+  static_assert(cpn::WORKSPACE_ALIGN > (CPN_ROUTE_MAY_FAIL | CPN_ROUTE_STATUS_ONLY), "sizes leave the bits free");
+  const uint64_t need = cpn_local_sort_temp_bytes(dtype, volume, sort_dim_size, want_values, want_indices, in_place);
+  if (need == 0) {
+    return 0;
+  }
+  if (cpn_local_sort_may_fail(dtype, volume, sort_dim_size, want_indices, need) != 0) {
+    return need | CPN_ROUTE_MAY_FAIL;
+  }
+  return need == cpn::HEADER_BYTES ? need | CPN_ROUTE_STATUS_ONLY : need;
+}
+
 int cpn_equal_digit_plan(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_values, int want_indices, int in_place,
                          const void* temp, uint64_t temp_bytes, uint32_t* out, void* stream)
 {

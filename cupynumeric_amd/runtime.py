@@ -16,6 +16,9 @@ if TYPE_CHECKING:
     import torch
 
 
+STATUS_LINE_BYTES = 2048  # what the sorts that only write a status word ask for
+
+
 class Runtime:
     """Process-wide state: device, settings."""
 
@@ -34,6 +37,10 @@ class Runtime:
         self._torch = None
         self._device_seen = False
         self._devices = {}
+        self._current_device = None
+        self._raw_stream = None
+        self._status_lines: dict[int, int] = {}  # device -> address
+        self._status_memory: list["torch.Tensor"] = []
         self._status_slots = None
         self._status_kinds: list[str] = []
         self._status_used = 0
@@ -99,8 +106,12 @@ class Runtime:
                     "cupynumeric_amd needs a HIP device: no GPU is visible to this process "
                     "(there is no CPU fallback for the sort path)"
                 )
+            index = torch.cuda.current_device()  # (this one initialises the device)
+            self._current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+            self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
             self._device_seen = True
-        index = torch.cuda.current_device()
+        else:
+            index = self._current_device()
         dev = self._devices.get(index)
         if dev is None:
             dev = self._devices[index] = torch.device("cuda", index)
@@ -108,11 +119,27 @@ class Runtime:
 
     def stream_handle(self) -> int:
         """hipStream_t of torch's current stream, as an integer."""
-        torch = self.torch
-        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        if raw is not None:  # (the same handle as current_stream().cuda_stream without building a Stream object)
-            return int(raw(torch.cuda.current_device()))
-        return int(torch.cuda.current_stream().cuda_stream)
+        if not self._device_seen:
+            self.require_device()
+        if self._raw_stream is not None:  # (the same handle as current_stream().cuda_stream without building a Stream object)
+            return self._raw_stream(self._current_device())
+        return int(self.torch.cuda.current_stream().cuda_stream)
+
+    def status_line(self) -> int | None:
+        """Address of a workspace on the current device for sorts that write nothing but a status word of 0 there
+        (`CPN_ROUTE_STATUS_ONLY`): every stream and thread may use it at once.  None while a graph is captured that would
+        own it."""
+        if not self._device_seen:
+            self.require_device()
+        index = self._current_device()
+        line = self._status_lines.get(index)
+        if line is None:
+            if self.torch.cuda.is_current_stream_capturing():
+                return None
+            memory = self.torch.zeros(STATUS_LINE_BYTES, dtype=self.torch.uint8, device=self.require_device())
+            self._status_memory.append(memory)  # (first, should another thread do the same)
+            line = self._status_lines[index] = memory.data_ptr()
+        return line
 
     def empty_bytes(self, nbytes: int) -> "torch.Tensor":
         """Uninitialised device buffer of `nbytes` bytes (at least one, so that it has an address)."""

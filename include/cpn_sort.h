@@ -195,6 +195,15 @@ int cpn_local_sort_check(const void* temp, void* stream);
 int cpn_local_sort_may_fail(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_indices, uint64_t temp_bytes);
 
 /*
+ * cpn_local_sort_temp_bytes, with cpn_local_sort_may_fail for a workspace of that size in its lowest bit (sizes are multiples of
+ * 256), and in the second whether the status word, set to 0, is all that the sort writes in its workspace: sorts on several
+ * streams may then share one.  A caller of many small sorts asks once instead of twice.
+ */
+#define CPN_ROUTE_MAY_FAIL 1u
+#define CPN_ROUTE_STATUS_ONLY 2u
+uint64_t cpn_local_sort_route(int dtype, uint64_t volume, uint64_t sort_dim_size, int want_values, int want_indices, int in_place);
+
+/*
  * out = in with axes `axis_a` and `axis_b` exchanged, both dense row-major; `shape` is the
  * shape of `in`.  Replaces the UNARY_OP(COPY) of a transposed store that sort_swapped
  * issues (cupynumeric/_thunk/_sort.py:50-76, src/cupynumeric/unary/unary_op.cu:85-96,124-170).
