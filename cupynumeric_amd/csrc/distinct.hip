@@ -11,12 +11,13 @@
 //         says where each class starts), then a workgroup per class reads its part of every tile into a hash table in LDS.
 //         Values that the sample has at least eight times are known by then and leave the array with the first step, so that
 //         a frequent value does not fill a class.  The first step is bound by its two passes over memory (85 us for 2^26
-//         int32), the second by the vector and LDS instructions of the look-ups (151 us, 41 of them the reads of LDS alone).
+//         int32), the second by the vector and LDS instructions of the look-ups (146 us, 41 of them the reads of LDS alone; 151
+//         before the next eight tiles were asked for first).
 //   none  the caller sorts (cpn_unique).
 // A table that fills up, where the estimate was wrong (values of very unlike frequency: Chao's is a lower bound), ends the
 // attempt the same way.
 //
-// us per call of `unique`, sorted / this way: 2^26 int32 of 16 values 868 / 119, of 2^20 923 / 338, of 2^26 1016 / 1036; 2^25 int64
+// us per call of `unique`, sorted / this way: 2^26 int32 of 16 values 868 / 119, of 2^20 923 / 330, of 2^26 1016 / 1036; 2^25 int64
 // of 1000 values 834 / 120, of 2^18 849 / 290, of 2^25 935 / 963.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -584,24 +585,34 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_class_kernel(const KeyT
       len                      = at[1] - from;
     }
     const uint32_t here = tiles - t0 < WAVE ? tiles - t0 : WAVE;
+    KeyT next[AHEAD];
+    const auto request = [&](uint32_t j0) {  // (lanes past the last tile hold a length of 0)
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        const uint32_t f = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(from), j0 + j));
+        const uint32_t l = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(len), j0 + j));
+        next[j]          = KeyT{};
+        if (lane < l) {
+          next[j] = grouped[static_cast<uint64_t>(t0 + j0 + j) * COLLECT_TILE + f + lane];
+        }
+      }
+    };
+    request(0);
     for (uint32_t j0 = 0; j0 < here; j0 += AHEAD) {
       KeyT k[AHEAD];
       uint32_t l[AHEAD], f[AHEAD];
-#pragma unroll
-      for (int j = 0; j < AHEAD; ++j) {  // (lanes past the last tile hold a length of 0)
-        f[j] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(from), j0 + j));
-        l[j] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(len), j0 + j));
-        k[j] = KeyT{};
-        if (lane < l[j]) {
-          k[j] = grouped[static_cast<uint64_t>(t0 + j0 + j) * COLLECT_TILE + f[j] + lane];
-        }
-      }
       bool valid[AHEAD];
       uint32_t longest = 0;
 #pragma unroll
       for (int j = 0; j < AHEAD; ++j) {
+        k[j]     = next[j];
+        f[j]     = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(from), j0 + j));
+        l[j]     = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(len), j0 + j));
         valid[j] = lane < l[j];
         longest  = l[j] > longest ? l[j] : longest;
+      }
+      if (j0 + AHEAD < here) {
+        request(j0 + AHEAD);
       }
       table.add(k, valid);
       for (uint32_t more = WAVE; more < longest; more += WAVE) {  // uniform: what is left of segments longer than a wave
