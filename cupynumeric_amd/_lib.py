@@ -115,6 +115,10 @@ PROTOTYPES: dict[str, tuple] = {
         c_int,
         [c_int, c_void_p, c_uint64, c_uint64, c_uint64, c_uint64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p],
     ),
+    "cpn_quantile_sorted_args": (
+        c_int,
+        [c_int, c_void_p, c_uint64, c_uint64, c_uint64, c_uint64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p],
+    ),
     "cpn_quantile_select_temp_bytes": (c_uint64, [c_int, c_uint64, c_uint64]),
     "cpn_quantile_select": (
         c_int,

@@ -114,12 +114,17 @@ def _collapse_axes(a: ndarray, axes: tuple[int, ...]) -> tuple[int, ndarray]:
     return first, ndarray(thunk.shape, thunk.dtype, thunk=thunk)
 
 
-# Vectors from this length on are selected from (`cpn_quantile_select`) instead of sorted.  us per call of normal
-# values, selected / sorted, one, five and sixteen quantiles:
-#   32 768 elements   float32 38 / 102, 45 / 103, 65 / 104   float64 46 / 119, 61 / 120, 69 / 121   int64 56, 67, 85 / 115
-#   10 000 elements   float32 37 /  85, 44 /  84, 61 /  83   float64 42 /  89, 61 /  89, 65 /  89   int64 54, 65, 76 /  89
-# so the line could lie lower; only at 5000 int64 elements do sixteen quantiles lose (76 / 74).
-SELECT_MIN_SIZE = 32768
+# As many quantiles as `cpn_quantile_sorted_args` takes.
+QUANTILE_ARGS = 16
+# Vectors from this length on are selected from (`cpn_quantile_select`) instead of sorted; of float vectors, four quantiles
+# and more from four times as many.  A selection is a chain of about ten launches, a sort of a vector like these two or three.
+# us per call, selected / sorted, one, five and sixteen quantiles, of normal values and of few different ones:
+#   32 768 elements   float32 37/27, 47/29, 66/33   35/30, 56/30, 71/32   float64 50/27, 66/28, 69/32   39/36, 60/37, 72/37
+#   200 000           float32 38/27, 48/29, 67/33   35/37, 56/37, 71/37   float64 51/27, 65/29, 78/33   39/46, 60/46, 72/47
+#   500 000           float32 39/32, 48/32, 68/35   35/45, 56/46, 71/46   float64 49/35, 70/34, 77/35   39/62, 62/63, 73/63
+#   2 000 000         float32 47/99, 56/99, 79/98   41/106, 62/106, 77/107
+#   int64   200 000   59/27, 66/29, 81/33   56/53, 62/53, 74/53     500 000   63/34, 71/34, 85/35   58/75, 64/75, 76/76
+SELECT_MIN_SIZE = 1 << 17
 
 
 def _select_bytes(a: ndarray, num_q: int) -> int:
@@ -165,7 +170,8 @@ def quantile(
 
     # A long vector of which only a few elements are needed is not sorted (SELECT_MIN_SIZE)
     flat = real_axis is None or a_rr.ndim == 1
-    select = flat and not overwrite_input and a_rr.size >= SELECT_MIN_SIZE and _select_bytes(a_rr, q_arr.size) != 0
+    longest_sorted = SELECT_MIN_SIZE * (4 if q_arr.size >= 4 and a_rr.dtype.kind == "f" else 1)
+    select = flat and not overwrite_input and a_rr.size >= longest_sorted and _select_bytes(a_rr, q_arr.size) != 0
     if overwrite_input:
         a_rr.sort(axis=real_axis)
         arr = a_rr
@@ -238,19 +244,19 @@ def quantile(
         )
         _lib.check(status, "cpn_quantile_select")
     elif result.size:
-        d_left = torch.from_numpy(left).to(dev)
-        d_right = torch.from_numpy(right).to(dev)
-        d_gamma = torch.from_numpy(gamma).to(dev)
-        status = lib.cpn_quantile_sorted(
+        if q_arr.size <= QUANTILE_ARGS:  # (they travel with the launch)
+            evaluate, where = lib.cpn_quantile_sorted_args, (left.ctypes.data, right.ctypes.data, gamma.ctypes.data)
+        else:
+            on_device = [torch.from_numpy(x).to(dev) for x in (left, right, gamma)]
+            evaluate, where = lib.cpn_quantile_sorted, tuple(x.data_ptr() for x in on_device)
+        status = evaluate(
             _lib.DTYPE_CODES[arr.dtype],
             arr._thunk.base.ptr(),
             outer,
             n,
             inner,
             q_arr.size,
-            d_left.data_ptr(),
-            d_right.data_ptr(),
-            d_gamma.data_ptr(),
+            *where,
             int(interpolate),
             result.base.ptr(),
             ctypes.c_void_p(runtime.stream_handle()),

@@ -317,7 +317,15 @@ int cpn_quantile_sorted(int dtype, const void* sorted, uint64_t outer, uint64_t 
                         int interpolate, void* out, void* stream);
 
 /*
- * The same for one long vector that is not sorted (outer == inner == 1): the elements that would stand
+ * The same with left, right and gamma in HOST memory (read before the call returns), for up to 16 quantiles: they travel
+ * with the launch.  More are CPN_ERR_UNSUPPORTED, positions outside [0, n) CPN_ERR_SHAPE.
+ */
+int cpn_quantile_sorted_args(int dtype, const void* sorted, uint64_t outer, uint64_t n, uint64_t inner,
+                             uint64_t num_q, const int64_t* left, const int64_t* right, const double* gamma,
+                             int interpolate, void* out, void* stream);
+
+/*
+ * The same as cpn_quantile_sorted for one long vector that is not sorted (outer == inner == 1): the elements that would stand
  * at left[q] and right[q] of the stable ascending sort are selected without sorting, bit for bit.
  * left, right and gamma are HOST arrays of num_q entries (read before the call returns).  Real types
  * of 4 and 8 bytes, 1 <= n < 2^31, 1 <= num_q <= 16; for anything else the size query returns 0.  The call then
