@@ -130,3 +130,27 @@ def test_requests_and_codes(lib, torch_cuda):
     assert call(f4, p, n, v.data_ptr(), m, 1, out.data_ptr() + 4, t, need, None) == _lib.CPN_ERR_ALIGN
     assert call(f4, p, n, v.data_ptr(), m, 1, out.data_ptr(), t, need - 1, None) == _lib.CPN_ERR_TEMP
     assert call(f4, p, n, v.data_ptr(), m, 1, out.data_ptr(), t + 8, need, None) == _lib.CPN_ERR_TEMP
+
+
+def test_captured(torch_cuda):
+    """Every replay counts its pieces anew: other values, spread otherwise, into the same graph."""
+    import cupynumeric_amd as num
+    from cupynumeric_amd._thunk import DeviceArray
+
+    torch, rng = torch_cuda, np.random.default_rng(6)
+    n, m = LEAST // 4 + 9, 100_000
+    a = np.sort(rng.standard_normal(n).astype(np.float32))
+    d_a = num.array(a)
+    buf = torch.zeros(m, dtype=torch.float32, device="cuda")
+    v = num.ndarray((m,), np.float32, thunk=DeviceArray.from_device(buf, (m,), np.float32))
+    num.searchsorted(d_a, v)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = num.searchsorted(d_a, v)
+    for spread in (1.0, 0.001, 100.0, 1.0):
+        x = (rng.standard_normal(m) * spread).astype(np.float32)
+        buf.copy_(torch.from_numpy(x))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out._thunk.base.device().view(torch.int64).cpu().numpy()
+        assert np.array_equal(got, np.searchsorted(a, x)), spread
