@@ -44,6 +44,9 @@ constexpr int SPLIT_WIDE_BINS      = 2;  // per splitter
 // Most sampled keys of a bin that are compared with each other (64: 10^6 int32 keys of 200 values, 41 of them in every bin, take 80 us, of
 // which the walks are half).
 constexpr uint32_t SPLIT_CROWD  = 24;
+// Threads with a bin that is not empty: at most so many, and the keys are of a few values (of a bucket, of the sample).
+constexpr int SPLIT_FEW         = 12;
+constexpr int SPLIT_FEW_SAMPLED = 256;
 
 // A mixed 32-bit word: which key of its stretch sample i takes.
 __host__ __device__ __forceinline__ uint32_t split_hash(uint32_t x)
@@ -160,15 +163,21 @@ __device__ __forceinline__ void split_order_passes(const KeyT* keys, uint16_t* n
     __syncthreads();
   }
 }
-// The same for all `top` bits, of which the leading 40 put almost every row in order: passes over them, a look at every pair of
-// neighbours, and passes over all bits if one is not in order.
+// The same for all bits that vary (`vary` has those in which any key's image differs from another's).  The leading 40 put almost
+// every row in order, the leading 16 one of a few values that repeat: passes over them, a look at every pair of neighbours,
+// and more passes if one is not in order.  (Every pass is stable, and so is what follows another.)  Nothing is done for low bits that
+// all keys share, as those of whole numbers held as floats do.  us a sort, 40 bits of any key at first / this: 10^7 float64 of 20 000
+// whole numbers 370 / 250, 10^6 int64 of 100 values 70 / 55; with 16 bits first for all, normal float64 with 1 % zeros lost 5 %.
 template <int CODEC, int BLOCK, int ITEMS, typename KeyT>
-__device__ __forceinline__ void split_order(const KeyT* keys, uint16_t* num, uint16_t* ctr, uint32_t* s_wave, uint32_t m, int top)
+__device__ __forceinline__ void split_order(const KeyT* keys, uint16_t* num, uint16_t* ctr, uint32_t* s_wave, uint32_t m, uint64_t vary,
+                                            bool few)
 {
-  int from_bit = top > 40 ? top - 40 : 0;
-  for (;;) {
+  const int top    = vary != 0 ? 64 - __builtin_clzll(vary) : 0;
+  const int bottom = vary != 0 ? __builtin_ctzll(vary) : 0;
+  for (int bits = few ? 16 : 40;; bits = bits == 16 ? 40 : 64) {
+    const int from_bit = top - bits > bottom ? top - bits : bottom;
     split_order_passes<CODEC, BLOCK, ITEMS>(keys, num, ctr, s_wave, m, from_bit, top);
-    if (from_bit == 0) {
+    if (from_bit == bottom) {
       return;
     }
     int bad = 0;
@@ -178,7 +187,6 @@ __device__ __forceinline__ void split_order(const KeyT* keys, uint16_t* num, uin
     if (__syncthreads_or(bad) == 0) {
       return;
     }
-    from_bit = 0;
   }
 }
 
@@ -354,30 +362,30 @@ __device__ __forceinline__ SplitBins split_find_splitters(uint32_t n, unsigned c
     }
   } else {
     KeyT* const s_ext = reinterpret_cast<KeyT*>(s_mem + S::EXTREMES);
-    KeyT top_image = 0, low_image = 0;  // the largest, the complement of the smallest
+    const bool few = __syncthreads_count(sum != 0 ? 1 : 0) <= SPLIT_FEW_SAMPLED;
+    KeyT any = 0, all = static_cast<KeyT>(~KeyT{0});  // OR and AND of the images
 #pragma unroll
     for (int r = 0; r < PER_THREAD; ++r) {
       const KeyT image                 = ordered_bits<CODEC, KeyT>(got[r]);
-      top_image                        = image > top_image ? image : top_image;
-      low_image                        = static_cast<KeyT>(~image) > low_image ? static_cast<KeyT>(~image) : low_image;
+      any |= image;
+      all &= image;
       s_image[r * SPLIT_BLOCK + tid]   = image;
       s_which[r * SPLIT_BLOCK + tid]   = static_cast<uint16_t>(r * SPLIT_BLOCK + tid);
     }
-    top_image = wave_max_dpp(top_image);
-    low_image = wave_max_dpp(low_image);
+    any = wave_reduce_or_dpp(any);
+    all = wave_reduce_and_dpp(all);
     if (lane == 0) {
-      s_ext[wave]               = top_image;
-      s_ext[SPLIT_WAVES + wave] = low_image;
+      s_ext[wave]               = any;
+      s_ext[SPLIT_WAVES + wave] = all;
     }
     __syncthreads();
 #pragma unroll
     for (int v = 0; v < SPLIT_WAVES; ++v) {
-      top_image = s_ext[v] > top_image ? s_ext[v] : top_image;
-      low_image = s_ext[SPLIT_WAVES + v] > low_image ? s_ext[SPLIT_WAVES + v] : low_image;
+      any |= s_ext[v];
+      all &= s_ext[SPLIT_WAVES + v];
     }
-    const uint64_t vary = static_cast<KeyT>(top_image ^ static_cast<KeyT>(~low_image));
     split_order<CODEC_UNSIGNED, SPLIT_BLOCK, PER_THREAD>(s_image, s_which, reinterpret_cast<uint16_t*>(s_mem + S::COUNTERS), s_wave,
-                                                         static_cast<uint32_t>(SAMPLES), vary != 0 ? 64 - __builtin_clzll(vary) : 0);
+                                                         static_cast<uint32_t>(SAMPLES), static_cast<uint64_t>(any ^ all), few);
     for (uint32_t j = number; j < S::SPLITTERS; j += SPLIT_BLOCK) {
       const uint32_t i = s_which[j * PER_BUCKET];
       put(j, s_image[i], split_sample_place(i, SAMPLES, n));
@@ -1136,7 +1144,7 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
     return;
   }
   uint32_t to[ITEMS];  // where a key belongs; until then its bin and, in the upper half, which of the bin it is
-  bool placed = false;
+  bool placed = false, few = false;
   {
     auto native = [](KeyT k) -> Native {
       Native v;
@@ -1191,6 +1199,9 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
       s_wave[wave] = incl;
     }
     placed = __syncthreads_or(largest > SPLIT_BIN_LIMIT ? 1 : 0) == 0;
+    if (!placed) {
+      few = __syncthreads_count(total != 0 ? 1 : 0) <= SPLIT_FEW;
+    }
     if (placed) {
       uint32_t run = incl - total;
 #pragma unroll
@@ -1268,21 +1279,32 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
     high = nans != 0 ? NAN_IMAGE : high;
     // ---- the passes: number o of the order so far is s_num[o] ----
     int other_value = 0;
+    KeyT vary       = 0;
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       if (holds(i)) {
         const KeyT image = ordered_bits<CODEC, KeyT>(key[i]);
         other_value |= (image != low && image != high) ? 1 : 0;
+        vary |= image ^ low;
         s_keys[slot_of(i)] = key[i];
         s_num[slot_of(i)]  = static_cast<uint16_t>(slot_of(i));
       }
     }
-    int top           = 64 - __builtin_clzll(static_cast<unsigned long long>(static_cast<KeyT>(low ^ high)));  // bits that vary: below it
+    vary = wave_reduce_or_dpp(vary);
+    if (lane == 0) {
+      s_red[wave] = static_cast<uint64_t>(vary);  // (the extremes in it have been read)
+    }
     uint16_t* const c = reinterpret_cast<uint16_t*>(s_ctr);
     if (__syncthreads_or(other_value) == 0) {
+      const int top = 64 - __builtin_clzll(static_cast<unsigned long long>(static_cast<KeyT>(low ^ high)));
       split_order_passes<CODEC, BLOCK, ITEMS>(s_keys, s_num, c, s_wave, m, top - 1, top);  // two values: they differ in this bit
     } else {
-      split_order<CODEC, BLOCK, ITEMS>(s_keys, s_num, c, s_wave, m, top);
+      uint64_t all_vary = 0;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        all_vary |= s_red[w];
+      }
+      split_order<CODEC, BLOCK, ITEMS>(s_keys, s_num, c, s_wave, m, all_vary, few);
     }
     // as the walk leaves it: where each key of this thread belongs
     uint32_t number[ITEMS];
