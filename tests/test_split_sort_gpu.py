@@ -230,3 +230,31 @@ def test_a_smaller_workspace_sorts_the_other_way(lib, torch_cuda):
                                  stream) == 0
     assert lib.cpn_local_sort_check(temp.data_ptr(), stream) == 0
     assert np.array_equal(i.cpu().numpy(), np.argsort(x.cpu().numpy(), kind="stable"))
+
+
+@pytest.mark.parametrize("dtype", [np.uint32, np.float32, np.int64, np.float64])
+@pytest.mark.parametrize("n", [9001, 100_000, 1 << 20, 2_100_000])
+@pytest.mark.parametrize("low_bits", ["differ", "shared"])
+def test_few_values_that_only_lower_bits_tell_apart(lib, torch_cuda, dtype, n, low_bits):
+    """A bucket of a few values, each too often for a bin: its leading 16 varying bits are not enough, then 40 are not; or
+    the low bits are the same in all keys and take no pass."""
+    key = np.dtype(dtype).itemsize
+    if lib.cpn_local_sort_split_temp_bytes(_lib.DTYPE_CODES[np.dtype(dtype)], n, n, 1) == 0:
+        pytest.skip("not a row that is split")
+    rng = np.random.default_rng(n)
+    clusters = max(1, n // 200)
+    apart = np.array([0, 1, 1 << 12, 1 << 25] if key == 8 else [0, 1, 2, 5], np.uint64)
+    if low_bits == "shared":
+        apart = apart << np.uint64(20 if key == 8 else 3)
+    top, least = (62, 46) if key == 8 else (30, 6)
+    step = max((1 << top) // clusters >> least << least, 1 << least)
+    keys = (rng.integers(0, clusters, n).astype(np.uint64) * np.uint64(step)) + apart[rng.integers(0, 4, n)]
+    x = keys.astype(np.uint64 if key == 8 else np.uint32).view(dtype)
+    _check(lib, torch_cuda, x, f"{np.dtype(dtype)} {n} {low_bits}")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_whole_numbers_held_as_floats(lib, torch_cuda, dtype):
+    for n, values in ((100_000, 500), (300_000, 3000), (1 << 20, 20_000)):
+        x = np.random.default_rng(values).integers(-values, values, n).astype(dtype)
+        _check(lib, torch_cuda, x, f"{np.dtype(dtype)} {n} {values}")
