@@ -29,6 +29,14 @@ namespace cpn {
 
 constexpr int SEARCH_BLOCK  = 256;
 constexpr int SEARCH_PIVOTS = 2048;
+__device__ constexpr uint32_t search_pivot_at(uint32_t j) { return j + (j >> 6); }
+// Up to so many values every lane has one (searchsorted_few_kernel); past it the table that each workgroup loads first costs more than
+// the lanes give.  us per call of `searchsorted`, sixteen values per lane / one:
+//   float32 in 10^4   2048 values 18 / 11   60 000  30 / 11   250 000  30 / 12   600 000  31 / 13   10^6  31 / 15
+//        in 65 536    2048        22 / 11   60 000  38 / 11   250 000  38 / 18   600 000  39 / 35   10^6  41 / 53
+//        in 10^6      2048        27 / 11   60 000  49 / 11   250 000  61 / 23   600 000  65 / 46   10^6  67 / 71
+//   float64 in 10^6   2048        31 / 11   60 000  74 / 12   250 000  79 / 26   600 000  81 / 54   10^6  83 / 83
+constexpr uint64_t SEARCH_FEW = 1ull << 19;
 
 constexpr uint32_t WINDOW_BYTES    = 40960;
 constexpr uint32_t WINDOW_TILE_MAX = 1024;
@@ -115,6 +123,58 @@ __global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_kernel(const KeyT* 
       }
     }
     // `origin` (values sorted beforehand): the position the value had in the caller's array
+    out[origin != nullptr ? static_cast<uint64_t>(origin[i]) : i] = static_cast<int64_t>(lo);
+  }
+}
+
+// The same for real keys and fewer values than the chip has lanes: a lane has one, where the kernel above gives sixteen to each
+// of a few workgroups.  Bound by the chain of dependent loads.  A gap after every 64 elements in LDS keeps elements a power
+// of two apart out of one bank, and what fills the table up saves the test of the bound.
+template <typename KeyT, int CODEC, bool LEFT>
+__global__ __launch_bounds__(SEARCH_BLOCK) void searchsorted_few_kernel(const KeyT* __restrict__ sorted, uint64_t n,
+                                                                        const KeyT* __restrict__ values, uint64_t num_values,
+                                                                        int64_t* __restrict__ out, const int64_t* __restrict__ origin,
+                                                                        uint64_t step, uint32_t num_pivots)
+{
+  constexpr int EACH = SEARCH_PIVOTS / SEARCH_BLOCK;
+  __shared__ KeyT s_pivot[search_pivot_at(SEARCH_PIVOTS)];
+  const uint32_t tid = threadIdx.x;
+  const uint64_t i   = static_cast<uint64_t>(blockIdx.x) * SEARCH_BLOCK + tid;
+  const KeyT v       = ordered_bits<CODEC, KeyT>(values[i < num_values ? i : num_values - 1]);
+  KeyT pivot[EACH];
+#pragma unroll
+  for (int k = 0; k < EACH; ++k) {
+    const uint32_t j = k * SEARCH_BLOCK + tid;
+    pivot[k]         = sorted[j < num_pivots ? j * step : 0];  // (the last pivot is element (num_pivots - 1) * step < n)
+  }
+#pragma unroll
+  for (int k = 0; k < EACH; ++k) {
+    const uint32_t j            = k * SEARCH_BLOCK + tid;
+    s_pivot[search_pivot_at(j)] = j < num_pivots ? ordered_bits<CODEC, KeyT>(pivot[k]) : static_cast<KeyT>(~KeyT{0});
+  }
+  __syncthreads();
+  // (`at` counts gaps as well until the last step: it is a multiple of 2 * half, so that they add up)
+  uint32_t at = 0;
+#pragma unroll
+  for (uint32_t half = SEARCH_PIVOTS / 2; half != 0; half >>= 1) {
+    const KeyT a = s_pivot[at + search_pivot_at(half - 1)];
+    at += (LEFT ? a < v : a <= v) ? search_pivot_at(half) : 0u;
+  }
+  const KeyT last   = s_pivot[at];
+  const uint32_t on = at - at / 65 + ((LEFT ? last < v : last <= v) ? 1u : 0u);
+  const uint32_t c  = on < num_pivots ? on : num_pivots;  // (the largest key of all is not left of what fills the table up)
+  uint64_t lo       = c == 0 ? 0 : static_cast<uint64_t>(c - 1) * step + 1;
+  uint64_t hi       = c == num_pivots ? n : c * step;
+  while (lo < hi) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    const KeyT a       = ordered_bits<CODEC, KeyT>(sorted[mid]);
+    if (LEFT ? a < v : a <= v) {
+      lo = mid + 1;
+    } else {
+      hi = mid;
+    }
+  }
+  if (i < num_values) {
     out[origin != nullptr ? static_cast<uint64_t>(origin[i]) : i] = static_cast<int64_t>(lo);
   }
 }
@@ -389,6 +449,17 @@ static int launch_searchsorted(const void* sorted, uint64_t n, const void* value
   if (n >= 8192 && num_values >= 2048) {
     step       = (n + SEARCH_PIVOTS - 1) / SEARCH_PIVOTS;
     num_pivots = static_cast<uint32_t>((n + step - 1) / step);
+  }
+  if constexpr (CODEC != CODEC_COMPLEX) {
+    if (num_pivots != 0 && num_values <= SEARCH_FEW) {
+      const auto search = left ? &searchsorted_few_kernel<KeyT, CODEC, true> : &searchsorted_few_kernel<KeyT, CODEC, false>;
+      ProfileScope prof("searchsorted", stream);
+      hipLaunchKernelGGL(search, dim3(static_cast<uint32_t>((num_values + SEARCH_BLOCK - 1) / SEARCH_BLOCK)), dim3(SEARCH_BLOCK), 0,
+                         stream, static_cast<const KeyT*>(sorted), n, static_cast<const KeyT*>(values), num_values, out, origin, step,
+                         num_pivots);
+      CPN_HIP_TRY(hipGetLastError());
+      return CPN_OK;
+    }
   }
   // with a pivot table every workgroup should serve a few thousand values
   const uint64_t per_block = (num_pivots != 0) ? 16 * SEARCH_BLOCK : SEARCH_BLOCK;
