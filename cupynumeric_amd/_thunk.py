@@ -18,8 +18,16 @@ if TYPE_CHECKING:
 
 # Where in its workspace `cpn_unique` may put the count: beside the status word, in a line that nothing else uses.
 UNIQUE_COUNT_OFFSET = 64
-# Fewer values are never grouped by the parts of the array (`cpn_searchsorted_grouped`); asking would cost them a call.
-GROUPED_MIN_VALUES = 1 << 16
+# From so many values on they are grouped by the parts of the array (`cpn_searchsorted_grouped`), where that is done, and up to
+# so many of 4 and 8 bytes are not sorted first where it is not.  us per call, grouped (of 2^28: sorted first) / each value by itself,
+# values spread as the array / half of them in a thousandth of it:
+#   float32   in 4*10^6   130 000  39 / 18  55 / 13   262 144  40 / 33  57 / 23   524 288  43 / 57  59 / 41
+#             in 3*10^7   130 000  80 / 25  85 / 18   262 144  81 / 52  92 / 31   524 288  82 / 94  108 / 55
+#             in 2^28     130 000  73 / 38  78 / 25   262 144 122 / 79 118 / 46   524 288 168 / 149 140 / 87
+#   float64   in 3*10^7   130 000 118 / 28 129 / 20   262 144 119 / 57 130 / 33   524 288 121 / 102 140 / 58
+#             in 2^28     130 000  80 / 42  93 / 28   262 144 172 / 88 175 / 53   524 288 257 / 166 227 / 109
+GROUPED_MIN_VALUES = (1 << 18) + 1
+UNSORTED_MAX_VALUES = 1 << 19
 # Longest array of integers that `unique` splits by sampled keys (`cpn_local_sort_split_temp_bytes`).  Arrays that it is asked
 # of repeat their values, and 8-byte ones mostly leave upper bytes constant, whose passes the sort of `cpn_unique` skips:
 # int64 below 10^9, us per call that way / split: 2^20 + 1 of as many values 204 / 125, of 1000 219 / 145;
@@ -313,7 +321,10 @@ class DeviceArray:
                 )
                 _lib.check(status, "cpn_searchsorted")
                 return
-        temp_bytes = lib.cpn_searchsorted_temp_bytes(code, rhs.size, v.size)
+        if v.size <= UNSORTED_MAX_VALUES and rhs.dtype.itemsize >= 4 and rhs.dtype.kind != "c":
+            temp_bytes = 0
+        else:
+            temp_bytes = lib.cpn_searchsorted_temp_bytes(code, rhs.size, v.size)
         temp = runtime.empty_bytes(temp_bytes) if temp_bytes else None
         status = lib.cpn_searchsorted(
             code,

@@ -51,9 +51,13 @@ def test_edges_of_the_range(n, m):
     _check(a, rng.integers(-3, 2 * n + 3, m))
 
 
-def test_sorted_values_of_a_long_array():
-    """Too few values for the parts of the array: they are sorted, then searched."""
-    n, m = (1 << 28) + 5, 1 << 16
+def test_a_long_array():
+    """Around the line from which values are grouped by the parts of the array, and the one from which they are sorted first."""
+    n = (1 << 28) + 5
     rng = np.random.default_rng(1)
     a = np.arange(n, dtype=np.int32)
-    _check(a, rng.integers(-5, n + 5, m).astype(np.int32))
+    for m in (1 << 16, 1 << 18, (1 << 18) + 1, 1 << 19, (1 << 19) + 1):
+        _check(a, rng.integers(-5, n + 5, m).astype(np.int32))
+    a = a[: 1 << 23]
+    for m in (1 << 18, (1 << 18) + 1):
+        _check(a, rng.integers(-5, a.size + 5, m).astype(np.int32))
