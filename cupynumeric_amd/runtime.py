@@ -55,7 +55,9 @@ class Runtime:
         reaches the host (`flush_status`).  The copy is ordered on the stream; nothing waits."""
         torch = self.torch
         if self._status_slots is None:
-            self._status_slots = torch.zeros(self.STATUS_SLOTS, dtype=torch.int32, device=word.device)
+            slots = torch.zeros(self.STATUS_SLOTS, dtype=torch.int32, device=word.device)
+            self._ready_for_every_stream()
+            self._status_slots = slots
             self._status_kinds = []
         if self._status_used == self.STATUS_SLOTS:
             self.flush_status()
@@ -137,9 +139,17 @@ class Runtime:
             if self.torch.cuda.is_current_stream_capturing():
                 return None
             memory = self.torch.zeros(STATUS_LINE_BYTES, dtype=self.torch.uint8, device=self.require_device())
+            self._ready_for_every_stream()
             self._status_memory.append(memory)  # (first, should another thread do the same)
             line = self._status_lines[index] = memory.data_ptr()
         return line
+
+    def _ready_for_every_stream(self) -> None:
+        """Waits for the current stream, whose memory was just allocated for all of them: the allocator hands out a block
+        again as soon as its owner has let go of it, and only this stream comes after the work that was given the block
+        before.  (Not while a graph is captured, whose memory nothing had before.)"""
+        if not self.torch.cuda.is_current_stream_capturing():
+            self.torch.cuda.current_stream().synchronize()
 
     def empty_bytes(self, nbytes: int) -> "torch.Tensor":
         """Uninitialised device buffer of `nbytes` bytes (at least one, so that it has an address)."""

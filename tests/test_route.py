@@ -31,6 +31,64 @@ def test_answers():
     assert lib.cpn_local_sort_route(99, 10, 10, 1, 0, 0) == 0 and lib.cpn_local_sort_route(4, 10, 3, 1, 0, 0) == 0
 
 
+class _Recorder:
+    """Stands for torch: what is allocated, and when its stream is waited for."""
+
+    uint8 = int32 = device = None
+
+    def __init__(self, capturing=False):
+        self.events, self.capturing, self.cuda = [], capturing, self
+
+    def is_current_stream_capturing(self):
+        return self.capturing
+
+    def current_stream(self):
+        return self
+
+    def synchronize(self):
+        self.events.append("wait")
+
+    def zeros(self, *args, **kwargs):
+        self.events.append("allocate")
+        return self
+
+    def data_ptr(self):
+        self.events.append("publish")
+        return 4096
+
+    def __getitem__(self, where):
+        return self
+
+    def copy_(self, word):
+        self.events.append("write")
+
+
+def _runtime_on(torch):
+    r = type(runtime)()
+    r._torch, r._device_seen, r._current_device, r._devices = torch, True, lambda: 0, {0: "device"}
+    return r
+
+
+def test_line_is_published_after_its_stream_was_waited_for():
+    """The line is memory that the allocator may have had from work still queued on the allocating stream: no other stream may
+    write to it before that has run."""
+    torch = _Recorder()
+    r = _runtime_on(torch)
+    assert r.status_line() == 4096 and torch.events == ["allocate", "wait", "publish"]
+    assert r.status_line() == 4096 and torch.events == ["allocate", "wait", "publish"]  # once
+    torch = _Recorder(capturing=True)
+    assert _runtime_on(torch).status_line() is None and torch.events == []
+
+
+def test_deferred_words_lie_where_no_earlier_work_writes():
+    """The same for the words that sorts on any stream leave there."""
+    torch = _Recorder()
+    r = _runtime_on(torch)
+    r.defer_flag(torch, "sort")
+    r.defer_flag(torch, "sort")
+    assert torch.events == ["allocate", "wait", "write", "write"]
+
+
 @pytest.mark.gpu
 def test_streams_and_threads_share_a_status_word():
     import torch
