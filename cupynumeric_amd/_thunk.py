@@ -406,6 +406,8 @@ class DeviceArray:
         found = DeviceArray.from_device(temp[list_offset : list_offset + count * self.dtype.itemsize], (count,), self.dtype)
         out = DeviceArray((count,), self.dtype)
         sort_task(out, found, False, True)
+        if runtime.check_mode != "off":
+            runtime.flush_status()  # (more values than a row split takes: a sort that can fail)
         return out
 
     def to_complex(self, dtype: Any) -> "DeviceArray":

@@ -164,3 +164,28 @@ def test_codes_of_the_entry_points(lib, torch_cuda):
     assert call(code, d.data_ptr(), d.data_ptr(), 0, count.data_ptr(), temp.data_ptr(), small, None) == _lib.CPN_ERR_UNSUPPORTED
     assert call(code, d.data_ptr(), d.data_ptr(), 5000, count.data_ptr(), temp.data_ptr(), small - 1, None) == _lib.CPN_ERR_TEMP
     assert call(code, d.data_ptr(), d.data_ptr(), 5000, count.data_ptr() + 4, temp.data_ptr(), small, None) == _lib.CPN_ERR_ALIGN
+
+
+@pytest.mark.parametrize("mode", ["lazy", "eager", "off"])
+def test_status_of_the_sort_of_the_values(torch_cuda, monkeypatch, mode):
+    """2^20 and more values of 4 bytes are sorted by passes, which can fail on the device: `unique` has looked when it returns."""
+    from cupynumeric_amd import _thunk
+    from cupynumeric_amd.runtime import runtime
+
+    x = _array(np.int32, 1 << 23, np.arange(1_500_000, dtype=np.int32) * 1000, 3)
+    a = num.array(x)
+    monkeypatch.setattr(runtime, "check_mode", mode)
+    assert np.array_equal(np.asarray(num.unique(a)), np.unique(x))
+    if mode != "lazy":
+        return
+    num.unique(a)
+    assert runtime._status_used == 0
+    sort = _thunk.sort_task
+
+    def failing(*args):
+        sort(*args)
+        runtime.defer_flag(torch_cuda.ones(1, dtype=torch_cuda.int32, device="cuda"), "sort")
+
+    monkeypatch.setattr(_thunk, "sort_task", failing)
+    with pytest.raises(RuntimeError, match="failed on the device"):
+        num.unique(a)
