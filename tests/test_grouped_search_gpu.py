@@ -132,25 +132,53 @@ def test_requests_and_codes(lib, torch_cuda):
     assert call(f4, p, n, v.data_ptr(), m, 1, out.data_ptr(), t + 8, need, None) == _lib.CPN_ERR_TEMP
 
 
-def test_captured(torch_cuda):
+def test_captured(lib, torch_cuda):
     """Every replay counts its pieces anew: other values, spread otherwise, into the same graph."""
-    import cupynumeric_amd as num
-    from cupynumeric_amd._thunk import DeviceArray
-
     torch, rng = torch_cuda, np.random.default_rng(6)
     n, m = LEAST // 4 + 9, 100_000
     a = np.sort(rng.standard_normal(n).astype(np.float32))
-    d_a = num.array(a)
+    code = _lib.DTYPE_CODES[a.dtype]
+    d_a = torch.from_numpy(a).cuda()
     buf = torch.zeros(m, dtype=torch.float32, device="cuda")
-    v = num.ndarray((m,), np.float32, thunk=DeviceArray.from_device(buf, (m,), np.float32))
-    num.searchsorted(d_a, v)
+    out = torch.full((m,), -1, dtype=torch.int64, device="cuda")
+    need = lib.cpn_searchsorted_grouped_temp_bytes(code, d_a.data_ptr(), n, m)
+    temp = torch.full((need,), 0xA5, dtype=torch.uint8, device="cuda")
+
+    def search():
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return lib.cpn_searchsorted_grouped(code, d_a.data_ptr(), n, buf.data_ptr(), m, 1, out.data_ptr(), temp.data_ptr(), need, stream)
+
+    assert need != 0 and search() == 0
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        out = num.searchsorted(d_a, v)
+        assert search() == 0
     for spread in (1.0, 0.001, 100.0, 1.0):
         x = (rng.standard_normal(m) * spread).astype(np.float32)
         buf.copy_(torch.from_numpy(x))
+        out.fill_(-1)
         graph.replay()
         torch.cuda.synchronize()
-        got = out._thunk.base.device().view(torch.int64).cpu().numpy()
-        assert np.array_equal(got, np.searchsorted(a, x)), spread
+        assert np.array_equal(out.cpu().numpy(), np.searchsorted(a, x)), spread
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_the_public_call_comes_here(lib, torch_cuda, dtype):
+    """The launches of the public call from the line on, and one value below it."""
+    import cupynumeric_amd as num
+    from cupynumeric_amd._thunk import GROUPED_MIN_VALUES
+
+    rng = np.random.default_rng(9)
+    a = np.sort(rng.standard_normal(LEAST // np.dtype(dtype).itemsize + 5).astype(dtype))
+    d_a = num.array(a)
+    for m, grouped in ((GROUPED_MIN_VALUES, True), (GROUPED_MIN_VALUES - 1, False)):
+        v = rng.standard_normal(m).astype(dtype)
+        d_v = num.array(v)
+        lib.cpn_profile_enable(1)
+        try:
+            _lib.profile_collect()
+            got = np.asarray(num.searchsorted(d_a, d_v))
+            labels = {label for label, _ in _lib.profile_collect()}
+        finally:
+            lib.cpn_profile_enable(0)
+        assert np.array_equal(got, np.searchsorted(a, v))
+        assert ({"find_group", "find_search"} <= labels) == grouped, labels
