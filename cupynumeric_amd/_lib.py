@@ -70,6 +70,7 @@ PROTOTYPES: dict[str, tuple] = {
     "cpn_set_merge_rows": (c_int, [c_int]),
     "cpn_set_bitonic_rows": (c_int, [c_int]),
     "cpn_set_tile_order": (c_int, [c_int]),
+    "cpn_hold_tile_order": (c_int, [c_int, c_void_p]),
     "cpn_dtype_size": (c_uint64, [c_int]),
     "cpn_key_order_bits": (c_uint64, [c_int, c_uint64]),
     "cpn_local_sort_temp_bytes": (c_uint64, [c_int, c_uint64, c_uint64, c_int, c_int, c_int]),

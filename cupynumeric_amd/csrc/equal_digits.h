@@ -47,10 +47,19 @@ struct EqualPlan {
   uint32_t n_extra;  // further pieces for the LDS sort
   uint32_t n_list;   // pieces for the general LDS sort
   uint32_t lshift;   // left shift that brings the cell number to the top of the word
+  uint32_t per_xcd;  // the passes deal their tiles per XCD
   uint64_t origin;   // image where cell 0 starts
   uint64_t last;     // largest distance from the origin inside the table
   alignas(16) uint32_t table[EQ_MAX_CELLS];  // base (low 16 bits) and width (high 16 bits) of every cell
 };
+// The second word of a sort's workspace says whether the sort deals its tiles per XCD (claim_tile, onesweep.h).  One of a
+// device's sorts at a time may: the first launch takes the device's word `order` (null: the sort is not to), the
+// last one gives it back.  (Should a launch in between be refused, it stays taken, and later sorts do without.)
+constexpr uint64_t HEADER_PER_XCD = 4;
+__device__ __forceinline__ uint32_t take_xcd_order(uint32_t* order)
+{
+  return (order != nullptr && atomicCAS(order, 0u, 1u) == 0u) ? 1u : 0u;
+}
 __device__ __forceinline__ bool eq_sorted(const EqualPlan* eq) { return eq != nullptr && eq->mode != 0 && eq->failed == 0; }
 __device__ __forceinline__ bool eq_failed(const EqualPlan* eq) { return eq != nullptr && eq->mode != 0 && eq->failed != 0; }
 
@@ -114,7 +123,8 @@ __global__ __launch_bounds__(EQ_GATHER_BLOCK) void eq_gather_kernel(const KeyT* 
                                                                     uint4* __restrict__ clear,
                                                                     uint64_t n_clear,
                                                                     uint4* __restrict__ clear2,
-                                                                    uint64_t n_clear2)
+                                                                    uint64_t n_clear2,
+                                                                    uint32_t* order)
 {
   constexpr int WAVES = EQ_GATHER_BLOCK / WAVE;
   __shared__ KeyT s_lo[WAVES], s_hi[WAVES];
@@ -129,7 +139,7 @@ __global__ __launch_bounds__(EQ_GATHER_BLOCK) void eq_gather_kernel(const KeyT* 
   // seg >= EQ_RANGE_SAMPLE: no stretch is empty
   const KeyT u = ordered_bits<CODEC, KeyT>(keys[begin + ((static_cast<uint64_t>(h) * (end - begin)) >> 32)]);
   for (uint64_t i = s; i < n_clear; i += EQ_RANGE_SAMPLE) {
-    clear[i] = make_uint4(0u, 0u, 0u, 0u);
+    clear[i] = make_uint4(0u, i == 0 ? take_xcd_order(order) : 0u, 0u, 0u);  // (the workspace, from its head on)
   }
   for (uint64_t i = s; i < n_clear2; i += EQ_RANGE_SAMPLE) {
     clear2[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -221,6 +231,7 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
                                                                   const KeyT* __restrict__ sample,
                                                                   const EqualLimits limits,
                                                                   const uint32_t* __restrict__ veto,
+                                                                  const uint32_t* __restrict__ per_xcd,
                                                                   EqualPlan* __restrict__ eq)
 {
   constexpr int CB           = eq_cell_bits(sizeof(KeyT));
@@ -437,10 +448,11 @@ __global__ __launch_bounds__(EQ_SAMPLE_BLOCK) void eq_plan_kernel(const KeyT* __
   const int any   = __syncthreads_or(no);  // (a statement of its own: the words below are read behind the barrier)
   const int mixed = any | (s_dense != 0 ? 1 : 0) | (s_close >= limits.close ? 1 : 0) | (s_equal >= limits.equal ? 1 : 0);
   if (tid == 0) {
-    eq->origin = origin;
-    eq->last   = last;
-    eq->lshift = lshift;
-    eq->mode   = mixed != 0 ? 0u : 1u;
+    eq->origin  = origin;
+    eq->last    = last;
+    eq->lshift  = lshift;
+    eq->per_xcd = *per_xcd;
+    eq->mode    = mixed != 0 ? 0u : 1u;
   }
 }
 

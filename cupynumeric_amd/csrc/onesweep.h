@@ -69,11 +69,12 @@ constexpr uint32_t DEVICE_ERR_LOOKBACK = 1u;
 // ---------------------------------------------------------------------------------------
 // zero fill (capture-safe replacement for a memset node)
 // ---------------------------------------------------------------------------------------
-static __global__ __launch_bounds__(256) void zero_fill_kernel(uint4* p, uint64_t n_vec)
+// `order` (may be null): the first vector is the head of a sort's workspace, see take_xcd_order (equal_digits.h).
+static __global__ __launch_bounds__(256) void zero_fill_kernel(uint4* p, uint64_t n_vec, uint32_t* order)
 {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n_vec; i += stride) {
-    p[i] = make_uint4(0u, 0u, 0u, 0u);
+    p[i] = make_uint4(0u, i == 0 ? take_xcd_order(order) : 0u, 0u, 0u);
   }
 }
 
@@ -323,13 +324,14 @@ enum IdxBuf : uint32_t { IDX_FINAL = 1, IDX_T1 = 2, IDX_ALIAS = 3 };  // ALIAS: 
 constexpr uint32_t BUF_NONE = 0xFFu;
 
 struct PassPlan {
-  uint32_t active;   // 0: the pass exits at once
+  uint32_t active;   // 0: the pass exits at once; else bit 0, and PLAN_PER_XCD
   uint32_t key_src;  // KeyBuf
   uint32_t key_dst;  // KeyBuf or BUF_NONE (index-only sort, last pass)
   uint32_t idx_src;  // IdxBuf or BUF_NONE (first running pass: positions are synthesised)
   uint32_t idx_dst;  // IdxBuf
   uint32_t first;    // bit 0: first running pass; bit 1: that pass need not be stable (PLAN_FREE_RANK)
 };
+constexpr uint32_t PLAN_PER_XCD   = 2u;  // tiles are dealt per XCD
 constexpr uint32_t PLAN_FIRST     = 1u;
 constexpr uint32_t PLAN_FREE_RANK = 2u;
 
@@ -353,6 +355,7 @@ struct PlanRequest {
   // keys unless the histogram sweep met a NaN or a -0.0 (*specials != 0).
   uint32_t free_rank;
   const uint32_t* specials;
+  const uint32_t* per_xcd;  // of the workspace header
   // Requests that may use equalised digits (may be null).  When those have failed, the byte passes start
   // from the scratch partner of T1 below and from IDX_ALIAS.
   const EqualPlan* eq;
@@ -396,7 +399,7 @@ __device__ __forceinline__ void make_plan(const uint32_t* varying, SortPlan* __r
     if ((flags >> p) & 1u) {
       ++j;
       const uint32_t from_last = k - j;
-      e.active                 = 1;
+      e.active                 = 1u | (__hip_atomic_load(rq.per_xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ? PLAN_PER_XCD : 0u);
       e.first                  = (j == 1) ? PLAN_FIRST : 0u;
       if (j == 1 && rq.free_rank != 0 &&
           (rq.specials == nullptr || __hip_atomic_load(rq.specials, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)) {
@@ -524,8 +527,12 @@ __global__ __launch_bounds__(256) void finalize_kernel(const SortPlan* __restric
                                                         uint64_t volume,
                                                         uint64_t seg,
                                                         int64_t index_offset,
-                                                        PlanRequest rq)
+                                                        PlanRequest rq,
+                                                        uint32_t* order)
 {
+  if (order != nullptr && blockIdx.x == 0 && threadIdx.x == 0 && *rq.per_xcd != 0) {
+    atomicExch(order, 0u);  // the passes have ended: another sort may deal its tiles per XCD
+  }
   if (eq_sorted(rq.eq)) {
     return;
   }
@@ -578,7 +585,6 @@ struct SweepArgs {
   int pass;                // which 8-bit digit this pass sorts by
   int idx_final;           // idx_out is the caller's int64 array
   uint32_t spin_limit;     // polls of one descriptor before the tile gives up (LOOKBACK_SPIN_LIMIT)
-  uint32_t single_ticket;  // hand tiles out through `ticket` alone instead of the per-XCD counters
   const VirtPlan* vplan;   // virtual digits (virtual_digits.h), nullptr when the request cannot use them
   const DistinctTable* dtable;  // with vplan: the row's different keys when there are at most 256
   int free_rank;                // from the plan: this pass need not be stable
@@ -610,9 +616,15 @@ struct SweepArgs {
 // resident workgroups hold lower tiles only, which finish without it.  What the order does
 // assume is that every XCD keeps receiving workgroups of this launch: if other work kept one XCD
 // fully occupied for seconds, tiles elsewhere would wait for that XCD's share until the bounded
-// look-back gave up and the call reported CPN_ERR_DEVICE.  A single counter for all XCDs has no
-// such dependence, at the price of the split lines: cpn_set_tile_order selects it at run time
-// (SweepArgs::single_ticket), and a caller that met CPN_ERR_DEVICE can repeat the sort that way.
+// look-back gave up and the call reported CPN_ERR_DEVICE.  Another sort of this order is such work:
+// sort A, whose workgroups fill one XCD and wait there for its share on a second one, and sort B, whose workgroups fill the
+// second and wait for B's share on the first, wait for each other until both give up (seen with three streams).  So one
+// sort of a device at a time deals its tiles per XCD (take_xcd_order, equal_digits.h), and the others take theirs
+// from a single counter for all XCDs, which has no such dependence: a workgroup waits for tiles that workgroups
+// already run, so these sorts always end and free their slots.  The price is the split lines, us a sort, argsort, per XCD / one
+// counter: 2^26 uint32 keys 791, 1085 / 797, 1160; 2^24 251, 332 / 251, 341; 4 10^6 119, 134 / 115, 133; 2 10^6 (small
+// tiles, which therefore always take the one counter) 92, 102 / 89, 99.  cpn_set_tile_order selects it for all sorts,
+// and a caller that met CPN_ERR_DEVICE can repeat the sort that way.
 constexpr uint32_t XCD_COUNT = 8;
 #ifndef CPN_TILE_GROUP
 #define CPN_TILE_GROUP 8
@@ -1188,8 +1200,8 @@ void onesweep_kernel(const SweepArgs<BIG> a_in)
   a.free_rank      = static_cast<int>((pp.first & PLAN_FREE_RANK) != 0);
 
   const int tid = threadIdx.x;
-  // Tiles are handed out to the workgroups that are actually running, in ascending order per
-  // XCD (claim_tile), so a tile that a look-back waits for is never stuck behind workgroups
+  // Tiles are handed out to the workgroups that are actually running, in ascending order, or in that
+  // order per XCD (claim_tile), so a tile that a look-back waits for is never stuck behind workgroups
   // that wait themselves.
   if (tid == 0) {
     // Once a tile of an earlier pass has given up, the keys in flight no longer match the
@@ -1198,7 +1210,7 @@ void onesweep_kernel(const SweepArgs<BIG> a_in)
     // at the start of this one.  A failure inside this pass leaves its input consistent, every
     // offset stays inside the row, and waiting tiles notice the status word and drain.)
     uint32_t ticket;
-    if (a.single_ticket != 0) {  // tiles in launch-wide ascending order, whichever XCD asks
+    if (small_tile(BIG, BLOCK, ITEMS) || (pp.active & PLAN_PER_XCD) == 0) {  // in launch-wide ascending order, whichever XCD asks
       ticket = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (ticket >= a.num_tiles) {
         ticket = 0xFFFFFFFFu;
@@ -1272,10 +1284,11 @@ void eq_sweep_kernel(SweepArgs<false> a, const EqualPlan* __restrict__ eq, const
   if (eq->mode == 0) {
     return;
   }
-  const int tid = threadIdx.x;
+  const uint32_t per_xcd = eq->per_xcd;
+  const int tid          = threadIdx.x;
   if (tid == 0) {  // (as in onesweep_kernel)
     uint32_t ticket;
-    if (a.single_ticket != 0) {
+    if (per_xcd == 0) {
       ticket = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (ticket >= a.num_tiles) {
         ticket = 0xFFFFFFFFu;

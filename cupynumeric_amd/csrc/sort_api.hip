@@ -18,6 +18,9 @@
 // receive the per-device address kept in g_static_scratch.
 static __device__ __align__(256) unsigned char scratch[CPN_STATIC_SCRATCH_BYTES];
 
+// The word that one sort at a time has (take_xcd_order, equal_digits.h), on every GPU as above.
+static __device__ uint32_t xcd_order;
+
 namespace cpn {
 
 thread_local int g_last_hip_error = 0;
@@ -185,6 +188,35 @@ static int static_scratch_of_current_device(void** out)
   return CPN_OK;
 }
 
+uint32_t* xcd_order_word()
+{
+  static std::atomic<uint32_t*> known[MAX_DEVICES];
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  uint32_t* word = known[dev].load(std::memory_order_relaxed);
+  if (word == nullptr) {
+    void* ptr = nullptr;
+    if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(xcd_order)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    word = static_cast<uint32_t*>(ptr);
+    known[dev].store(word, std::memory_order_relaxed);
+  }
+  return word;
+}
+
+// one thread: takes or gives back the word, in place of a sort
+static __global__ void hold_order_kernel(uint32_t* word, uint32_t value)
+{
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    atomicExch(word, value);
+  }
+}
+
 // one thread: hands the status word of a finished sort to the caller's device memory
 static __global__ void copy_status_kernel(const uint32_t* __restrict__ status, uint32_t* __restrict__ out)
 {
@@ -308,6 +340,17 @@ int64_t cpn_set_lookback_spin_limit(int64_t polls)
 {
   const long long v = (polls < 1 || polls > (1ll << 31)) ? static_cast<long long>(cpn::LOOKBACK_SPIN_LIMIT) : polls;
   return static_cast<int64_t>(cpn::g_spin_limit.exchange(v));
+}
+
+int cpn_hold_tile_order(int hold, void* stream)
+{
+  uint32_t* const word = cpn::xcd_order_word();
+  if (word == nullptr) {
+    return CPN_ERR_HIP;
+  }
+  hipLaunchKernelGGL(cpn::hold_order_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), word, hold != 0 ? 1u : 0u);
+  CPN_HIP_TRY(hipGetLastError());
+  return CPN_OK;
 }
 
 int cpn_set_tile_order(int single) { return cpn::g_tile_order.exchange(single != 0 ? 1 : 0); }

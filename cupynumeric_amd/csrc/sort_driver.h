@@ -80,6 +80,8 @@ constexpr int EQ_MEDIUM_ITEMS  = 10;  // (12 and more spill)
 // How the scatter passes hand out their tiles: per XCD (default) or through one counter
 // (cpn_set_tile_order, CPN_SORT_TILE_ORDER=single).
 bool tile_order_single();
+// The word of the current device that the sort has which deals its tiles per XCD (take_xcd_order); null where there is none.
+uint32_t* xcd_order_word();
 // Rows of at least this many elements use 64-bit counts, descriptors and row positions:
 // BIG_ROW_ELEMENTS unless lowered by cpn_set_wide_row_threshold / CPN_SORT_WIDE_ROW_THRESHOLD
 // (for tests that exercise the 64-bit kernels without a 2^30-element row).
@@ -426,7 +428,7 @@ inline uint64_t workspace_bytes(int key_bytes, int passes, int codec, uint64_t v
   return L.valid ? (least ? L.total : L.eq_total) : 0;
 }
 
-inline int launch_zero_fill(void* p, uint64_t bytes, hipStream_t stream)
+inline int launch_zero_fill(void* p, uint64_t bytes, hipStream_t stream, uint32_t* order)
 {
   const uint64_t n_vec = bytes / 16;  // bytes is a multiple of 256
   uint64_t blocks      = (n_vec + 255) / 256;
@@ -439,7 +441,7 @@ inline int launch_zero_fill(void* p, uint64_t bytes, hipStream_t stream)
   {
     ProfileScope prof("zero_fill", stream);
     hipLaunchKernelGGL(zero_fill_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, stream,
-                       static_cast<uint4*>(p), n_vec);
+                       static_cast<uint4*>(p), n_vec, order);
   }
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;
@@ -919,7 +921,7 @@ inline int sort_equalised(const SortRequest& r, const GlobalLayout& L, EqualPlan
     static_assert(VIRT_DISTINCT == 2, "veto word");
     hipLaunchKernelGGL((eq_plan_kernel<KeyT, CODEC>), dim3(1), dim3(EQ_SAMPLE_BLOCK), 0, r.stream, ranges,
                        ranges + 2 * EQ_GATHER_GRID, eq_limits(r.seg, medium, EQ_SORT_TILE),
-                       vplan != nullptr ? &vplan->enabled : static_cast<const uint32_t*>(nullptr), eq);
+                       vplan != nullptr ? &vplan->enabled : static_cast<const uint32_t*>(nullptr), rq.per_xcd, eq);
   }
   CPN_HIP_TRY(hipGetLastError());
   {
@@ -956,7 +958,6 @@ inline int sort_equalised(const SortRequest& r, const GlobalLayout& L, EqualPlan
     a.num_tiles       = L.eq_tiles;
     a.pass            = p;
     a.spin_limit      = lookback_spin_limit();
-    a.single_ticket   = (r.single_ticket || tile_order_single()) ? 1u : 0u;
     a.free_rank       = (p == 0 && rq.free_rank != 0) ? 1 : 0;
     ProfileScope prof("equal_sweep", r.stream);
     hipLaunchKernelGGL((eq_sweep_kernel<KeyT, CODEC, HAS_IDX, global_block(KB), global_items(KB, false)>),
@@ -1038,18 +1039,20 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   constexpr bool EQ_OK = eq_keys<KeyT, CODEC, OffT>();
   const bool use_eq    = EQ_OK && L.eq && r.temp_bytes >= L.eq_total;
   EqualPlan* eq        = use_eq ? reinterpret_cast<EqualPlan*>(ws + L.off_eq) : nullptr;
+  // (small tiles take the one counter, see onesweep.h)
+  uint32_t* const order = (L.small_items != 0 || r.single_ticket || tile_order_single()) ? nullptr : xcd_order_word();
   if constexpr (EQ_OK) {
     if (use_eq) {  // one launch clears the workspace and looks at a sample of the keys
       KeyT* ranges = reinterpret_cast<KeyT*>(ws + L.off_eq_sample);
       ProfileScope prof("equal_gather", r.stream);
       hipLaunchKernelGGL((eq_gather_kernel<KeyT, CODEC>), dim3(EQ_GATHER_GRID), dim3(EQ_GATHER_BLOCK), 0, r.stream,
                          static_cast<const KeyT*>(r.values_in), r.seg, ranges, ranges + 2 * EQ_GATHER_GRID,
-                         reinterpret_cast<uint4*>(ws), L.zero_bytes / 16, reinterpret_cast<uint4*>(eq), L.eq_zero_bytes / 16);
+                         reinterpret_cast<uint4*>(ws), L.zero_bytes / 16, reinterpret_cast<uint4*>(eq), L.eq_zero_bytes / 16, order);
     }
   }
   if (use_eq) {
     CPN_HIP_TRY(hipGetLastError());
-  } else if (const int rc = launch_zero_fill(ws, L.zero_bytes, r.stream); rc != CPN_OK) {
+  } else if (const int rc = launch_zero_fill(ws, L.zero_bytes, r.stream, order); rc != CPN_OK) {
     return rc;
   }
   uint32_t* status  = reinterpret_cast<uint32_t*>(ws);
@@ -1069,6 +1072,7 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   rq.in_place     = in_place ? 1u : 0u;
   rq.free_rank    = (!HAS_IDX && (CODEC == CODEC_UNSIGNED || CODEC == CODEC_SIGNED || CODEC == CODEC_FLOAT)) ? 1u : 0u;
   rq.specials     = (CODEC == CODEC_FLOAT) ? reinterpret_cast<const uint32_t*>(ws + HEADER_SPECIALS) : nullptr;
+  rq.per_xcd      = reinterpret_cast<const uint32_t*>(ws + HEADER_PER_XCD);
   rq.eq           = eq;
   // what the intermediate byte passes alternate with key buffer 1 (make_plan)
   void* const key_x = (want_vals && !in_place) ? r.values_out : (L.off_key2 ? ws + L.off_key2 : nullptr);
@@ -1229,7 +1233,6 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
     a.num_tiles          = static_cast<uint32_t>(L.num_tiles);
     a.pass               = p;
     a.spin_limit         = lookback_spin_limit();
-    a.single_ticket      = (r.single_ticket || tile_order_single()) ? 1u : 0u;
     a.vplan              = vplan;
     a.dtable             = dtable;
     a.distinct_pass_done = distinct_special ? 1u : 0u;
@@ -1299,7 +1302,7 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
     ProfileScope prof("finalize", r.stream);
     hipLaunchKernelGGL((finalize_kernel<KeyT>), dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, r.stream, plan,
                        static_cast<const KeyT*>(r.values_in), static_cast<KeyT*>(r.values_out),
-                       static_cast<const KeyT*>(key1), r.indices_out, r.volume, r.seg, r.index_offset, rq);
+                       static_cast<const KeyT*>(key1), r.indices_out, r.volume, r.seg, r.index_offset, rq, order);
   }
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;

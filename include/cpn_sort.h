@@ -491,13 +491,21 @@ int64_t cpn_set_lookback_spin_limit(int64_t polls);
  * Process-wide tunable: how the scatter passes of the global sort hand their tiles to workgroups.
  * 0 (default): per XCD, so that neighbouring tiles share an L2 (faster; assumes that every XCD of
  * the device keeps receiving workgroups of the launch: if foreign work held one XCD for seconds,
- * the bounded look-back would give up with CPN_ERR_DEVICE).  Non-zero: one ticket counter for the
+ * the bounded look-back would give up with CPN_ERR_DEVICE).  Of the sorts that run at the same time on a device, on
+ * several streams, one does so, and the others, like sorts of few tiles, as with non-zero: one ticket counter for the
  * whole launch, which has no such dependence (one call at a time: CPN_SORT_SINGLE_TICKET of
  * cpn_local_sort_ex).  Results do not depend on it.  Returns the previous setting.  Also initialised from the
  * environment variable CPN_SORT_TILE_ORDER ("single" selects the one counter).  The reference has no
  * counterpart (cub's onesweep takes tiles from one counter, behind src/cupynumeric/sort/cub_sort.cuh:120-143).
  */
 int cpn_set_tile_order(int single);
+
+/*
+ * For tests: with `hold`, what the sorts enqueued on `stream` behind this call find is that another sort deals its
+ * tiles per XCD; without, that none does.  Which of the two a sort found is in the second 32-bit word of its workspace
+ * (1: it dealt its tiles per XCD itself).  No counterpart in the reference.
+ */
+int cpn_hold_tile_order(int hold, void* stream);
 
 /*
  * Process-wide tunable: a 1-D sort of real 8-byte keys with at least `elements` elements lets
