@@ -686,7 +686,7 @@ static int collect_plan_typed(const void* values_v, uint64_t n, unsigned char* w
   {
     ProfileScope prof("collect_sample", s);
     hipLaunchKernelGGL((split_gather_kernel<KeyT>), dim3(COLLECT_SAMPLES / 256), dim3(256), 0, s, values, static_cast<uint32_t>(n),
-                       static_cast<uint32_t>(COLLECT_SAMPLES), sample);
+                       static_cast<uint32_t>(COLLECT_SAMPLES), sample, static_cast<const uint32_t*>(nullptr));
   }
   CPN_HIP_TRY(hipGetLastError());
   {

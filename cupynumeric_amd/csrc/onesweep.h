@@ -182,7 +182,8 @@ struct EqualResume {
 // grid = rows * blocks_per_row; block b of a row covers elements [b*chunk, min(seg, (b+1)*chunk)).
 // 128-bit loads over the 16-byte aligned middle of the chunk, scalar head and tail.
 // `vplan` (may be null): nothing to do when the sort already runs on the ranks of the row's
-// different keys (virtual_digits.h), or when equalised digits have sorted it (`eq`, may be null).
+// different keys (virtual_digits.h), or when equalised digits have sorted it (`eq`, may be null), or for a row that
+// few passes will not sort (PlanRequest::narrow, may be null).
 // SPECIALS (float keys, keys-only sorts): also tells through `specials` whether a NaN or a -0.0 occurs.
 template <typename KeyT, int CODEC, typename OffT, bool SPECIALS = false>
 __global__ __launch_bounds__(HIST_BLOCK) void histogram_kernel(const KeyT* __restrict__ keys,
@@ -193,10 +194,14 @@ __global__ __launch_bounds__(HIST_BLOCK) void histogram_kernel(const KeyT* __res
                                                                  const VirtPlan* __restrict__ vplan,
                                                                  uint32_t* __restrict__ specials,
                                                                  const EqualPlan* __restrict__ eq,
-                                                                 const EqualResume<KeyT> resume)
+                                                                 const EqualResume<KeyT> resume,
+                                                                 const uint32_t* __restrict__ narrow)
 {
   constexpr int PASSES      = KeyTraits<CODEC, KeyT>::PASSES;
   constexpr int VEC         = 16 / sizeof(KeyT);
+  if (narrow != nullptr && *narrow == 0) {
+    return;
+  }
   constexpr int HIST_COPIES = hist_copies(PASSES);
   if (vplan != nullptr && vplan->enabled == VIRT_DISTINCT) {
     return;
@@ -356,6 +361,10 @@ struct PlanRequest {
   uint32_t free_rank;
   const uint32_t* specials;
   const uint32_t* per_xcd;  // of the workspace header
+  // Rows that are sorted by the passes in `launched` (a bit each) or not at all (may be null): not 0 while they may be,
+  // 2 when there is nothing to sort.
+  uint32_t* narrow;
+  uint32_t launched;
   // Requests that may use equalised digits (may be null).  When those have failed, the byte passes start
   // from the scratch partner of T1 below and from IDX_ALIAS.
   const EqualPlan* eq;
@@ -371,6 +380,15 @@ __device__ __forceinline__ void make_plan(const uint32_t* varying, SortPlan* __r
     if (__hip_atomic_load(&varying[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
       flags |= 1u << p;
       ++k;
+    }
+  }
+  if (rq.narrow != nullptr) {
+    if ((flags & ~rq.launched) != 0) {
+      *rq.narrow = 0;  // (the plan stays cleared: no pass runs)
+      return;
+    }
+    if (k == 0) {
+      *rq.narrow = 2;  // all keys are equal
     }
   }
   const bool resume = eq_failed(rq.eq);
@@ -447,7 +465,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void histogram_scan_kernel(OffT* __rest
                                                                     SortPlan* __restrict__ plan,
                                                                     PlanRequest rq)
 {
-  if (eq_sorted(rq.eq)) {
+  if (eq_sorted(rq.eq) || (rq.narrow != nullptr && *rq.narrow == 0)) {
     return;  // (the plan stays cleared: no byte pass runs)
   }
   // first use (`second` == 0): nothing when the sort already runs on the ranks of the row's

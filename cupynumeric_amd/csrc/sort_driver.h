@@ -1139,7 +1139,8 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
                          reinterpret_cast<uint32_t*>(ws + HEADER_SPECIALS), static_cast<const EqualPlan*>(eq),
                          EqualResume<KeyT>{reinterpret_cast<const KeyT*>(ws + L.off_key1), static_cast<KeyT*>(key_x),
                                            HAS_IDX ? reinterpret_cast<const uint32_t*>(ws + L.off_idx) : nullptr,
-                                           HAS_IDX ? reinterpret_cast<uint32_t*>(r.indices_out) : nullptr});
+                                           HAS_IDX ? reinterpret_cast<uint32_t*>(r.indices_out) : nullptr},
+                         static_cast<const uint32_t*>(nullptr));
     }
     CPN_HIP_TRY(hipGetLastError());
     {
@@ -1307,6 +1308,102 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
   CPN_HIP_TRY(hipGetLastError());
   return CPN_OK;
 }
+
+// ---- rows of which few bytes vary (split_plan.h) ----
+// Where the passes find what they work on.  `head`: a workspace header whose second and later words are cleared but for
+// `narrow`; hist, desc: cleared where a pass is to run.
+struct NarrowBuffers {
+  unsigned char* head;
+  uint32_t* narrow;
+  uint32_t* hist;
+  unsigned char* desc;
+  void* key1;
+  void* key2;
+  uint32_t* idx1;
+};
+inline uint64_t narrow_tiles(uint64_t n) { return (n + global_tile(8, false) - 1) / global_tile(8, false); }
+inline uint64_t narrow_desc_bytes(uint64_t n) { return align_up(narrow_tiles(n) * RADIX * sizeof(uint32_t), WORKSPACE_ALIGN); }
+
+// Byte passes `first` ... `first + count - 1` of one row, the only ones that may have something to do.  The result of
+// a sort in place is left in key2: the input stays what it was until the passes have succeeded.
+template <typename KeyT, int CODEC, bool HAS_IDX>
+inline int sort_narrow(const SortRequest& r, const NarrowBuffers& b, int first, int count)
+{
+  constexpr int KB     = sizeof(KeyT);
+  constexpr int PASSES = KeyTraits<CODEC, KeyT>::PASSES;
+  const bool want_vals = r.values_out != nullptr;
+  void* const out      = r.values_out == r.values_in ? b.key2 : r.values_out;
+  SortPlan* plan       = reinterpret_cast<SortPlan*>(b.head + HEADER_PLAN);
+  PlanRequest rq{};
+  rq.passes       = PASSES;
+  rq.want_values  = want_vals ? 1u : 0u;
+  rq.want_indices = HAS_IDX ? 1u : 0u;
+  rq.free_rank    = HAS_IDX ? 0u : 1u;
+  rq.specials     = (CODEC == CODEC_FLOAT) ? reinterpret_cast<const uint32_t*>(b.head + HEADER_SPECIALS) : nullptr;
+  rq.per_xcd      = reinterpret_cast<const uint32_t*>(b.head + HEADER_PER_XCD);
+  rq.narrow       = b.narrow;
+  rq.launched     = ((1u << count) - 1u) << first;
+  {
+    const uint64_t chunk = align_up((r.seg + 2047) / 2048 < 16384 ? 16384 : (r.seg + 2047) / 2048, 4096);
+    const uint32_t grid  = static_cast<uint32_t>((r.seg + chunk - 1) / chunk);
+    ProfileScope prof("histogram", r.stream);
+    hipLaunchKernelGGL((histogram_kernel<KeyT, CODEC, uint32_t, (CODEC == CODEC_FLOAT) && !HAS_IDX>), dim3(grid), dim3(HIST_BLOCK), 0,
+                       r.stream, static_cast<const KeyT*>(r.values_in), b.hist, r.seg, grid, chunk, static_cast<const VirtPlan*>(nullptr),
+                       reinterpret_cast<uint32_t*>(b.head + HEADER_SPECIALS), static_cast<const EqualPlan*>(nullptr),
+                       EqualResume<KeyT>{}, static_cast<const uint32_t*>(b.narrow));
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  {
+    ProfileScope prof("histogram_scan", r.stream);
+    hipLaunchKernelGGL((histogram_scan_kernel<uint32_t>), dim3(PASSES * WAVE / SCAN_BLOCK), dim3(SCAN_BLOCK), 0, r.stream, b.hist,
+                       reinterpret_cast<uint32_t*>(b.head + HEADER_VARYING), r.seg, static_cast<uint32_t>(PASSES),
+                       static_cast<uint64_t>(PASSES), static_cast<const VirtPlan*>(nullptr), 0u,
+                       reinterpret_cast<uint32_t*>(b.head + HEADER_SCAN_DONE), plan, rq);
+  }
+  CPN_HIP_TRY(hipGetLastError());
+  constexpr bool CAN_ORDER_KEYS = HAS_IDX && (CODEC == CODEC_SIGNED || CODEC == CODEC_FLOAT);
+  const bool ordered_keys       = CAN_ORDER_KEYS && !want_vals;
+  const uint32_t tiles          = static_cast<uint32_t>(narrow_tiles(r.seg));
+  for (int p = first; p < first + count; ++p) {
+    SweepArgs<false> a{};
+    a.key_buf[KEY_IN]    = r.values_in;
+    a.key_buf[KEY_OUT]   = out;
+    a.key_buf[KEY_T1]    = b.key1;
+    a.key_buf[KEY_T2]    = b.key2;
+    a.idx_buf[IDX_FINAL] = r.indices_out;
+    a.idx_buf[IDX_T1]    = b.idx1;
+    a.idx_buf[IDX_ALIAS] = r.indices_out;
+    a.plan               = plan;
+    a.ticket             = reinterpret_cast<uint32_t*>(b.head + HEADER_TICKETS) + p;
+    a.xcd_tickets        = reinterpret_cast<uint32_t*>(b.head + HEADER_XCD_TICKETS) + p * XCD_COUNT;
+    a.hist_excl          = b.hist + p * RADIX;
+    a.desc               = reinterpret_cast<uint32_t*>(b.desc + (p - first) * narrow_desc_bytes(r.seg));
+    a.status             = reinterpret_cast<uint32_t*>(b.head);
+    a.seg                = r.seg;
+    a.hist_row_stride    = static_cast<uint64_t>(PASSES) * RADIX;
+    a.index_offset       = r.index_offset;
+    a.tiles_per_row      = tiles;
+    a.num_tiles          = tiles;
+    a.pass               = p;
+    a.spin_limit         = lookback_spin_limit();
+    a.volume             = r.seg;
+    ProfileScope prof("onesweep", r.stream);
+    if (ordered_keys) {
+      if constexpr (CAN_ORDER_KEYS) {
+        hipLaunchKernelGGL((onesweep_kernel<KeyT, CODEC, true, false, HAS_IDX, global_block(KB), global_items(KB, false)>), dim3(tiles),
+                           dim3(global_block(KB)), 0, r.stream, a);
+      }
+    } else {
+      hipLaunchKernelGGL((onesweep_kernel<KeyT, CODEC, false, false, HAS_IDX, global_block(KB), global_items(KB, false)>), dim3(tiles),
+                         dim3(global_block(KB)), 0, r.stream, a);
+    }
+    CPN_HIP_TRY(hipGetLastError());
+  }
+  return CPN_OK;
+}
+
+// (sort_keys64.hip, beside the other uses of these kernels)
+int sort_narrow64(int codec, const SortRequest& r, const NarrowBuffers& b, int first, int count);
 
 template <typename KeyT, int CODEC>
 int sort_typed(const SortRequest& r)

@@ -16,4 +16,21 @@ int sort_keys64(int codec, const SortRequest& r)
   }
 }
 
+template <int CODEC>
+static int narrow(const SortRequest& r, const NarrowBuffers& b, int first, int count)
+{
+  return r.indices_out != nullptr ? sort_narrow<uint64_t, CODEC, true>(r, b, first, count)
+                                  : sort_narrow<uint64_t, CODEC, false>(r, b, first, count);
+}
+
+int sort_narrow64(int codec, const SortRequest& r, const NarrowBuffers& b, int first, int count)
+{
+  switch (codec) {
+    case CODEC_UNSIGNED: return narrow<CODEC_UNSIGNED>(r, b, first, count);
+    case CODEC_SIGNED: return narrow<CODEC_SIGNED>(r, b, first, count);
+    case CODEC_FLOAT: return narrow<CODEC_FLOAT>(r, b, first, count);
+    default: return CPN_ERR_DTYPE;
+  }
+}
+
 }  // namespace cpn

@@ -57,11 +57,30 @@ inline SplitPlan split_plan(int key_bytes, int passes, uint64_t volume, uint64_t
   p.tiles        = static_cast<uint32_t>((seg + p.tile_len - 1) / p.tile_len);
   return p;
 }
+// Byte passes that a wide row tries ahead of the split: the lowest of whole numbers, the highest of floats (signs, exponents and the
+// leading bits of fractions; whole numbers that go below zero have busy upper bytes and do not try).  A row of which only those
+// bytes vary is sorted by one read that counts and a pass for each byte that does; the split, which does not skip constant
+// bytes, takes up to four times as long.  us a sort and an argsort, split / passes:
+//   int64 of equal keys    2^22 122, 125 / 53, 49    10^7 223, 231 / 81, 69     below 200  114, 117 / 67, 71    207, 217 / 106, 120
+//   below 20 000                119, 124 / 90, 97         232, 244 / 159, 185   below 300 000  131, 147 / 113, 123   244, 255 / 212, 265
+//   float64 of two values       137, 141 / 98, 97         234, 242 / 175, 184
+// Every other row pays for launches that find nothing to do: full int64 keys 2^21 + 1 83, 88 / 94, 100; 2^22 109, 118 / 121, 130;
+// 10^7 218, 238 / 228, 249.  Up to 2^21 keys that is 12 of 60 to 75 us and wins 20 for keys of one byte, none for others
+// (2^21 int64 below 200 77, 78 / 57, 60; below 20 000 76, 78 / 76, 81); a third pass for floats wins nothing (of three bytes, below
+// 200: 2^23 195, 202 split, 187, 202 in passes that have no split behind them).
+inline int narrow_passes(int codec, uint64_t n)
+{
+  if (n <= (1ull << 21)) {
+    return 0;
+  }
+  return codec == CODEC_FLOAT ? 2 : 3;
+}
 // Workspace: header, the sample, the keys in the order of the buckets of each tile, their places, the table, two words
-// per key.  Wide: also the sorted sample and the numbers of its keys, the splitters (images, places, values), their table of
-// bins, and the workspace of the sample's own sort.
+// per key.  Wide: also the splitters (images, places, values), their table of bins, and the workspace of the sample's own sort.
 struct SplitLayout {
-  uint64_t off_sample, off_sorted, off_numbers, off_images, off_at, off_values, off_before, off_bins, off_inner;
+  uint64_t off_hist, off_desc;                        // wide: the passes' histograms and descriptors,
+  uint64_t off_key1, off_key2, off_idx1;              // and what they work on, where the split's own regions are
+  uint64_t off_sample, off_images, off_at, off_values, off_before, off_bins, off_inner;
   uint64_t off_keys, off_places, off_starts, off_ids, total;
 };
 inline SplitLayout split_layout(const SplitPlan& p, int key_bytes, uint64_t n, bool want_indices)
@@ -70,11 +89,14 @@ inline SplitLayout split_layout(const SplitPlan& p, int key_bytes, uint64_t n, b
   SplitLayout L{};
   const uint64_t samples = static_cast<uint64_t>(p.buckets) * p.per_bucket;
   L.off_sample = HEADER_BYTES;
+  if (p.wide && n > (1ull << 21)) {  // (narrow_passes)
+    L.off_hist   = HEADER_BYTES;
+    L.off_desc   = L.off_hist + 8 * RADIX * sizeof(uint32_t);
+    L.off_sample = L.off_desc + 3 * narrow_desc_bytes(n);
+  }
   L.off_keys   = L.off_sample + (p.gathered || p.wide ? align_up(samples * key_bytes, WORKSPACE_ALIGN) : 0);
   if (p.wide) {
-    L.off_sorted  = L.off_keys;
-    L.off_numbers = L.off_sorted + align_up(samples * key_bytes, WORKSPACE_ALIGN);
-    L.off_images  = L.off_numbers + align_up(samples * sizeof(int64_t), WORKSPACE_ALIGN);
+    L.off_images  = L.off_keys;
     L.off_at      = L.off_images + align_up(static_cast<uint64_t>(p.buckets) * key_bytes, WORKSPACE_ALIGN);
     L.off_values  = L.off_at + align_up(p.buckets * sizeof(uint32_t), WORKSPACE_ALIGN);
     L.off_before  = L.off_values + align_up(p.buckets * sizeof(float), WORKSPACE_ALIGN);
@@ -86,6 +108,13 @@ inline SplitLayout split_layout(const SplitPlan& p, int key_bytes, uint64_t n, b
   L.off_starts = L.off_places + (want_indices ? align_up(n * sizeof(uint16_t), WORKSPACE_ALIGN) : 0);
   L.off_ids    = L.off_starts + align_up(table, WORKSPACE_ALIGN);
   L.total      = L.off_ids + align_up(2 * n * sizeof(uint32_t), WORKSPACE_ALIGN);
+  if (L.off_desc != 0) {  // (the sample outlives the passes)
+    L.off_key1         = L.off_images;
+    L.off_key2         = L.off_key1 + align_up(n * key_bytes, WORKSPACE_ALIGN);
+    L.off_idx1         = L.off_key2 + align_up(n * key_bytes, WORKSPACE_ALIGN);
+    const uint64_t end = L.off_idx1 + (want_indices ? align_up(n * sizeof(uint32_t), WORKSPACE_ALIGN) : 0);
+    L.total            = L.total > end ? L.total : end;
+  }
   return L;
 }
 

@@ -58,12 +58,22 @@ __host__ __device__ __forceinline__ uint32_t split_hash(uint32_t x)
   x ^= x >> 16;
   return x;
 }
-// The place in a row of n keys that sample i of `samples` is taken from: one place of each of `samples` equal stretches.
+// The place in a row of n keys that sample i of `samples`, a power of two, is taken from: one place of each of `samples` equal
+// stretches.  (By a shift: with two divisions of 64 bits the 524 288 keys that 10^7 are sampled with took 10.9 us to gather.)
 __host__ __device__ __forceinline__ uint32_t split_sample_place(uint32_t i, uint32_t samples, uint32_t n)
 {
-  const uint32_t from = static_cast<uint32_t>(static_cast<uint64_t>(i) * n / samples);
-  const uint32_t to   = static_cast<uint32_t>(static_cast<uint64_t>(i + 1) * n / samples);
+  const int log2      = __builtin_ctz(samples);
+  const uint32_t from = static_cast<uint32_t>((static_cast<uint64_t>(i) * n) >> log2);
+  const uint32_t to   = static_cast<uint32_t>((static_cast<uint64_t>(i + 1) * n) >> log2);
   return from + static_cast<uint32_t>((static_cast<uint64_t>(split_hash(i)) * (to - from)) >> 32);
+}
+
+// The head of the workspace of a row that byte passes may have sorted ahead (split_plan.h, narrow): the status word, and
+// HEADER_NARROW bytes on whether they were to.  Null: no passes.
+constexpr uint64_t HEADER_NARROW = 8;
+__device__ __forceinline__ bool split_done(const uint32_t* head)
+{
+  return head != nullptr && head[HEADER_NARROW / 4] != 0 && head[0] == 0;
 }
 
 // Stable rank of a lane's bucket among those of its wave (radix_common.h's wave_match_rank, for as many bits as a
@@ -398,10 +408,75 @@ __device__ __forceinline__ SplitBins split_find_splitters(uint32_t n, unsigned c
 // does each of the workgroups that need all of them.
 template <typename KeyT>
 __global__ __launch_bounds__(256) void split_gather_kernel(const KeyT* __restrict__ keys_in, uint32_t n, uint32_t samples,
-                                                           KeyT* __restrict__ out)
+                                                           KeyT* __restrict__ out, const uint32_t* __restrict__ head)
 {
+  if (split_done(head)) {
+    return;
+  }
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;  // (`samples` is a multiple of the workgroup)
   out[i]           = keys_in[split_sample_place(i, samples, n)];
+}
+// The same as the first launch of a row that may be narrow.  It also gathers what the sample's own sort samples (`again` keys of
+// it; 10^7 keys 2 us less than by a launch), clears what the passes count with, from the head of the workspace on, and the first
+// workgroup looks at SPLIT_PROBE keys: where they differ in no bit of `outside`, the passes are to try.
+constexpr uint32_t SPLIT_PROBE = 4096;
+template <typename KeyT, int CODEC>
+__global__ __launch_bounds__(256) void split_front_kernel(const KeyT* __restrict__ keys_in, uint32_t n, uint32_t samples,
+                                                          KeyT* __restrict__ out, uint32_t again, KeyT* __restrict__ out_again,
+                                                          uint4* __restrict__ clear, uint32_t n_clear, KeyT outside)
+{
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  const KeyT own   = keys_in[split_sample_place(i, samples, n)];
+  if (i < again) {
+    out_again[i] = keys_in[split_sample_place(split_sample_place(i, again, samples), samples, n)];
+  }
+  for (uint32_t v = i; v < n_clear; v += samples) {
+    if (v != 0) {
+      clear[v] = make_uint4(0u, 0u, 0u, 0u);
+    }
+  }
+  if (blockIdx.x == 0) {
+    constexpr int EACH = SPLIT_PROBE / 256;
+    KeyT probe[EACH], vary = 0;
+#pragma unroll
+    for (int r = 0; r < EACH; ++r) {
+      probe[r] = keys_in[split_sample_place(r * 256 + threadIdx.x, SPLIT_PROBE, n)];
+    }
+    const KeyT first = ordered_bits<CODEC, KeyT>(keys_in[0]);
+#pragma unroll
+    for (int r = 0; r < EACH; ++r) {
+      vary |= ordered_bits<CODEC, KeyT>(probe[r]) ^ first;
+    }
+    const int wide = __syncthreads_or((vary & outside) != 0 ? 1 : 0);
+    if (threadIdx.x == 0) {
+      static_assert(HEADER_NARROW == 8, "the third word");
+      clear[0] = make_uint4(0u, 0u, wide != 0 ? 0u : 1u, 0u);
+    }
+  }
+  out[i] = own;
+}
+// What passes leave undone: a row of equal keys, and a row sorted in place, which they leave in a buffer.
+template <typename KeyT>
+struct SplitLeft {
+  const KeyT* sorted;  // null: not in place
+  KeyT* keys_out;      // may be null
+  int64_t* idx_out;    // may be null
+  int64_t index_offset;
+};
+template <typename KeyT>
+__device__ __forceinline__ void split_finish(const SplitLeft<KeyT>& left, const KeyT* keys_in, bool equal, uint32_t first, uint32_t len)
+{
+  const KeyT* const from = equal ? keys_in : left.sorted;
+  if (left.keys_out != nullptr && from != nullptr && from != left.keys_out) {
+    for (uint32_t o = first + threadIdx.x; o < first + len; o += SPLIT_BLOCK) {
+      left.keys_out[o] = from[o];
+    }
+  }
+  if (equal && left.idx_out != nullptr) {
+    for (uint32_t o = first + threadIdx.x; o < first + len; o += SPLIT_BLOCK) {
+      left.idx_out[o] = static_cast<int64_t>(o) + left.index_offset;
+    }
+  }
 }
 
 // One tile of a row into the order of its buckets.
@@ -416,7 +491,8 @@ template <typename KeyT, int CODEC, bool HAS_POS, int PER_THREAD, int PER_BUCKET
 __global__ __launch_bounds__(SPLIT_BLOCK) void split_tile_kernel(const KeyT* __restrict__ keys_in, uint32_t n,
                                                                  uint32_t tile_len, const KeyT* __restrict__ sample,
                                                                  KeyT* __restrict__ grouped, uint16_t* __restrict__ places,
-                                                                 uint16_t* __restrict__ starts, uint32_t* __restrict__ status)
+                                                                 uint16_t* __restrict__ starts, uint32_t* __restrict__ status,
+                                                                 const uint32_t* __restrict__ head)
 {
   using S                 = SplitSample<KeyT, PER_THREAD, PER_BUCKET>;
   constexpr int SAMPLES   = S::SAMPLES;
@@ -440,6 +516,9 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_tile_kernel(const KeyT* __r
   const uint32_t tid  = threadIdx.x;
   const uint32_t lane = tid & (WAVE - 1);
   const uint32_t wave = tid / WAVE;
+  if (split_done(head)) {
+    return;  // uniform
+  }
   if (blockIdx.x == 0 && tid == 0) {
     *status = 0;  // (the workspace's status word: this sort cannot fail on the device)
   }
@@ -566,30 +645,23 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_tile_kernel(const KeyT* __r
 
 // ---- rows whose splitters are found ahead ----
 // Longer rows take more buckets and more sampled keys than a tile's workgroup can sort by the way: the sample is gathered,
-// sorted as a row of its own (by the kernels above), and every (samples / buckets)-th key of it is a splitter.
+// sorted as a row of its own (by the kernels above and below), and every (samples / buckets)-th key of it is a splitter.
 
-// The splitters: of the sorted sample and the numbers of its keys, every `step`-th.  A launch of several workgroups: the
-// reads are scattered.
-template <typename KeyT, int CODEC>
-__global__ __launch_bounds__(256) void split_pick_kernel(const KeyT* __restrict__ sorted, const int64_t* __restrict__ numbers,
-                                                         uint32_t n, uint32_t samples, uint32_t step, KeyT* __restrict__ images,
-                                                         uint32_t* __restrict__ places, float* __restrict__ values,
-                                                         uint32_t* __restrict__ status)
-{
-  const uint32_t j = blockIdx.x * 256 + threadIdx.x;  // (the buckets are a multiple of the workgroup)
-  if (j == 0) {
-    *status = 0;  // (the workspace's status word: this sort cannot fail on the device)
-  }
-  const KeyT key   = sorted[j * step];
-  images[j]        = ordered_bits<CODEC, KeyT>(key);
-  places[j]        = split_sample_place(static_cast<uint32_t>(numbers[j * step]), samples, n);
-  values[j]        = split_value<CODEC, KeyT>(key);
-}
+// Where the sort of a sample leaves the splitters.
+template <typename KeyT>
+struct SplitPicks {
+  KeyT* images;
+  uint32_t* places;
+  float* values;
+  uint32_t log2_step;   // of 2^log2_step sampled keys one is a splitter
+  uint32_t samples, n;  // of a row of n keys
+};
 
-// The bins of their values, and how many splitters come before each (one workgroup).
+// The bins of the splitters' values, and how many splitters come before each (one workgroup).
 template <int BITS>
 __global__ __launch_bounds__(SPLIT_BLOCK) void split_table_kernel(const float* __restrict__ values, uint16_t* __restrict__ before,
-                                                                  SplitBins* __restrict__ bins_out)
+                                                                  SplitBins* __restrict__ bins_out, const uint32_t* __restrict__ passes,
+                                                                  uint32_t* __restrict__ head)
 {
   constexpr int BUCKETS = 1 << BITS;
   constexpr int BINS    = BUCKETS * SPLIT_WIDE_BINS;
@@ -600,6 +672,9 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_table_kernel(const float* _
   const uint32_t tid  = threadIdx.x;
   const uint32_t lane = tid & (WAVE - 1);
   const uint32_t wave = tid / WAVE;
+  if (split_done(passes)) {
+    return;
+  }
   float value[OWN];
   uint32_t low = 0, high = 0;  // as in split_find_splitters
 #pragma unroll
@@ -656,6 +731,9 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_table_kernel(const float* _
   }
   if (tid == 0) {
     *bins_out = bins;
+    // (also where passes have given up, see split_done: this sort cannot fail on the device)
+    head[HEADER_NARROW / 4] = 0;
+    head[0]                 = 0;
   }
 }
 
@@ -668,7 +746,8 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_wide_tile_kernel(const KeyT
                                                                       const uint16_t* __restrict__ before,
                                                                       const SplitBins* __restrict__ bins_in,
                                                                       KeyT* __restrict__ grouped, uint16_t* __restrict__ places,
-                                                                      uint16_t* __restrict__ starts)
+                                                                      uint16_t* __restrict__ starts, const uint32_t* __restrict__ head,
+                                                                      const SplitLeft<KeyT> left)
 {
   constexpr int ITEMS    = SPLIT_WIDE_ITEMS;
   constexpr int BUCKETS  = 1 << BITS;
@@ -692,6 +771,10 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_wide_tile_kernel(const KeyT
   const uint32_t rounds = (len + SPLIT_BLOCK - 1) / SPLIT_BLOCK;        // uniform
   const uint32_t woff   = wave * rounds * WAVE + lane;
   auto runs             = [&](int i) -> bool { return i < static_cast<int>(rounds); };  // uniform
+  if (split_done(head)) {
+    split_finish(left, keys_in, head[HEADER_NARROW / 4] == 2, first, len);
+    return;
+  }
 
   KeyT key[ITEMS];
 #pragma unroll
@@ -836,6 +919,7 @@ struct SplitBuckets {
   const uint16_t* starts;
   uint32_t* ids;  // two words per key: what the slow way of an oversized bucket orders
   uint32_t n, tiles, tile_len, buckets;
+  const uint32_t* head;
 };
 
 // A bucket of more keys than LDS has room for, sorted by its workgroup alone: one stable pass per key byte over the
@@ -843,10 +927,11 @@ struct SplitBuckets {
 //   s_from  [tiles]: where the part of a tile lies in `grouped`, less where it lies in the bucket (modulo 2^32)
 //   s_slot  [tiles]: where it lies in the bucket
 //   s_ctr   a counter per digit and wave, s_digit: one per digit
-template <typename KeyT, int CODEC, bool HAS_IDX, int BLOCK>
+//   put_key, put_pos  take the bucket's o-th key and its place in the row
+template <typename KeyT, int CODEC, bool HAS_IDX, int BLOCK, typename PutKey, typename PutPos>
 __device__ __forceinline__ void oversized_bucket(const SplitBuckets<KeyT>& sb, uint32_t m, uint32_t base,
                                                  const uint32_t* s_from, const uint32_t* s_slot, uint32_t* s_ctr,
-                                                 uint32_t* s_digit, KeyT* keys_out, int64_t* idx_out, int64_t index_offset)
+                                                 uint32_t* s_digit, PutKey put_key, PutPos put_pos)
 {
   using KT             = KeyTraits<CODEC, KeyT>;
   constexpr int WAVES  = BLOCK / WAVE;
@@ -924,11 +1009,9 @@ __device__ __forceinline__ void oversized_bucket(const SplitBuckets<KeyT>& sb, u
   const uint32_t* const ids = sb.ids + base + (KT::PASSES % 2 == 0 ? sb.n : 0u);
   for (uint32_t i = tid; i < m; i += BLOCK) {
     const uint32_t id = ids[i], t = tile_of(id), at = s_from[t] + id;
-    if (keys_out != nullptr) {
-      keys_out[base + i] = sb.grouped[at];
-    }
+    put_key(i, sb.grouped[at]);
     if constexpr (HAS_IDX) {
-      idx_out[base + i] = static_cast<int64_t>(t * sb.tile_len + sb.places[at]) + index_offset;
+      put_pos(i, t * sb.tile_len + sb.places[at]);
     }
   }
 }
@@ -959,9 +1042,11 @@ constexpr uint32_t SPLIT_BIN_LIMIT = 24;
 // Bound by its chain where every bucket has a compute unit (7 to 8 us for buckets of 400 keys; as one more mode of
 // lds_row_sort_kernel, with two reductions and two atomics per key, 11), else by the workgroups that fit, two to a unit of
 // 512 threads with 8-byte keys, three with 4-byte keys.
-template <typename KeyT, int CODEC, bool HAS_IDX, bool WIDE>
+// PICK: of a sample's sort nothing is kept but the splitters.  (A launch of its own that looked them up took 4 us.)
+template <typename KeyT, int CODEC, bool HAS_IDX, bool WIDE, bool PICK>
 __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const SplitBuckets<KeyT> sb, KeyT* __restrict__ keys_out,
-                                                             int64_t* __restrict__ idx_out, int64_t index_offset)
+                                                             int64_t* __restrict__ idx_out, int64_t index_offset,
+                                                             const SplitPicks<KeyT> picks)
 {
   constexpr int BLOCK = SPLIT_BUCKET_BLOCK;
   constexpr int ITEMS = SPLIT_BUCKET_ITEMS;
@@ -997,6 +1082,9 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
   const uint32_t wave   = tid / WAVE;
   constexpr uint32_t XCDS = 8;  // workgroups go round them
   const uint32_t bucket   = blockIdx.x % XCDS * (sb.buckets / XCDS) + blockIdx.x / XCDS;
+  if (split_done(sb.head)) {
+    return;  // uniform
+  }
 
   // ---- the bucket's part of every tile; m keys in all, `base` keys of the row before them ----
   uint32_t start[PARTS], len[PARTS], starts = 0, lens = 0;
@@ -1031,6 +1119,28 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
   if (m == 0) {
     return;  // uniform
   }
+  auto put_key = [&](uint32_t o, KeyT key) {
+    if constexpr (PICK) {
+      const uint32_t at = base + o;
+      if ((at & ((1u << picks.log2_step) - 1)) == 0) {
+        picks.images[at >> picks.log2_step] = ordered_bits<CODEC, KeyT>(key);
+        picks.values[at >> picks.log2_step] = split_value<CODEC, KeyT>(key);
+      }
+    } else if (keys_out != nullptr) {
+      keys_out[base + o] = key;
+    }
+  };
+  auto put_pos = [&](uint32_t o, uint32_t pos) {
+    if constexpr (PICK) {
+      const uint32_t at = base + o;
+      if ((at & ((1u << picks.log2_step) - 1)) == 0) {
+        picks.places[at >> picks.log2_step] = split_sample_place(pos, picks.samples, picks.n);
+      }
+    } else {
+      idx_out[base + o] = static_cast<int64_t>(pos) + index_offset;
+    }
+  };
+  static_assert(HAS_IDX || !PICK, "splitters have places");
   uint32_t part_slot[PARTS];
 #pragma unroll
   for (int k = 0; k < PARTS; ++k) {
@@ -1046,7 +1156,7 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
   }
   if (m > TILE) {  // uniform
     __syncthreads();
-    oversized_bucket<KeyT, CODEC, HAS_IDX, BLOCK>(sb, m, base, s_from, s_slot, s_ctr, s_digit, keys_out, idx_out, index_offset);
+    oversized_bucket<KeyT, CODEC, HAS_IDX, BLOCK>(sb, m, base, s_from, s_slot, s_ctr, s_digit, put_key, put_pos);
     return;
   }
   // the number of a tile, plus one, at the first slot of its part
@@ -1132,12 +1242,9 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       if (holds(i)) {
-        const uint32_t o = base + slot_of(i);
-        if (keys_out != nullptr) {
-          keys_out[o] = key[i];
-        }
+        put_key(slot_of(i), key[i]);
         if constexpr (HAS_IDX) {
-          idx_out[o] = static_cast<int64_t>(pos[i]) + index_offset;
+          put_pos(slot_of(i), pos[i]);
         }
       }
     }
@@ -1328,7 +1435,7 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
     }
   }
   // ---- out, through LDS, so that neighbouring lanes store neighbouring elements ----
-  if (keys_out != nullptr) {
+  if (PICK || keys_out != nullptr) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
@@ -1338,7 +1445,7 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
     }
     __syncthreads();
     for (uint32_t o = tid; o < m; o += BLOCK) {
-      keys_out[base + o] = s_keys[o];
+      put_key(o, s_keys[o]);
     }
   }
   if constexpr (HAS_IDX) {
@@ -1352,7 +1459,7 @@ __global__ __launch_bounds__(SPLIT_BUCKET_BLOCK) void split_bucket_kernel(const 
     }
     __syncthreads();
     for (uint32_t o = tid; o < m; o += BLOCK) {
-      idx_out[base + o] = static_cast<int64_t>(s_pos[o]) + index_offset;
+      put_pos(o, s_pos[o]);
     }
   }
 }
