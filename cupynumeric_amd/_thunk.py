@@ -395,12 +395,12 @@ class DeviceArray:
             runtime.flush_status()  # errors of earlier work first
         args = (code, self.base.ptr(), self.size)
         _lib.check(lib.cpn_distinct_plan(*args, temp.data_ptr(), temp.numel(), stream), "cpn_distinct_plan")
-        head = temp[:12].view(runtime.torch.int32)
-        mode = head.tolist()[0]  # (waits, so that an array that is sorted after all waits for no more than this)
-        if mode == 0:
+        head = temp[:24].view(runtime.torch.int32)
+        mode, _, _, _, _, doubt = head.tolist()  # (waits, so that an array that is sorted after all waits for no more than this)
+        if mode == 0 or doubt != 0:
             return None
         _lib.check(lib.cpn_distinct(*args, mode, temp.data_ptr(), temp.numel(), stream), "cpn_distinct")
-        _, failed, count = head.tolist()
+        _, failed, count, *_ = head.tolist()
         if failed != 0:
             return None
         found = DeviceArray.from_device(temp[list_offset : list_offset + count * self.dtype.itemsize], (count,), self.dtype)

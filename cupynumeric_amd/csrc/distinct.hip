@@ -48,6 +48,7 @@ static_assert(collect_class_full(8) + COLLECT_BLOCK < collect_class_slots(8) && 
 constexpr int COLLECT_FEW_PROBES = 512;  // in the table in memory, a fifth full if the estimate is right (every one is a round trip)
 constexpr double COLLECT_FEW_MAX  = 3000.0;
 constexpr double collect_many_max(int key_bytes) { return 64.0 * collect_class_slots(key_bytes); }  // a quarter of the tables
+constexpr double collect_tail_max(int key_bytes) { return 0.9 * COLLECT_CLASSES * collect_class_full(key_bytes); }
 // An array that turns out to be sorted after all has waited for the sample, 28 us.  us per call of `unique`, sorted / asked first:
 // 2^23 int32 of 1000 values 222 / 91, of 2^18 223 / 144, of 2^23 243 / 270; 2^22 int64 of 1000 values 200 / 87, of 2^18
 // 196 / 150, of 2^22 206 / 235; and 2^22 int32 180 / 94, 180 / 144, 187 / 212: too much for what it gives.
@@ -56,13 +57,14 @@ constexpr uint64_t collect_min_volume(int key_bytes) { return 1ull << (key_bytes
 static_assert(COLLECT_FEW_MAX <= COLLECT_KNOWN_MAX && COLLECT_HEAVY_MAX <= COLLECT_KNOWN_MAX, "room for them");
 
 enum : uint32_t { COLLECT_NONE = 0, COLLECT_FEW = 1, COLLECT_MANY = 2 };
-// The head of the workspace; the caller reads the first three words.
+// The head of the workspace; the caller reads the first three words and the last.
 struct CollectPlan {
   uint32_t mode;
   uint32_t failed;
   uint32_t count;      // of the list
   uint32_t saw_empty;  // the key that stands for an empty slot is in the array
   uint32_t n_known;
+  uint32_t doubt;      // there may be far more values than the mode is for
 };
 
 template <typename KeyT>
@@ -198,6 +200,25 @@ struct CollectTable {
   }
 };
 
+// Values of very unlike frequency make Chao's estimate, a lower bound, far too low: of 2^25 keys spread evenly over the logarithm of
+// 2^24 it sees 47 000 values where there are 5.2 million, and the tables fill up after all the work (`unique` 1088 us sorted, 1360
+// this way and then sorted).  Values of like frequencies are seen once, twice and three times as a Poisson law has it, f1 f3 /
+// f2^2 = 2/3 if they are many; a tail of rarer and rarer ones shows in a quotient above.  Then the sample is read as one of
+// values whose frequencies fall with their rank: c / x^2 dx of them are expected x times in the sample, from some least x on, which f1 =
+// c (ln(1 / x) - 0.577) and f2 = c / 2 give, and so many of them are expected in n keys.  (A few frequent values beside very many
+// rare ones of one frequency show in nothing: those still fail.)  2^23 keys over the logarithm of 2^22, 1.4 million values, are still
+// tried: 310 sorted, 209.
+__device__ __forceinline__ double collect_tail(double f1, double f2, double f3, uint64_t n)
+{
+  if (f3 < 10.0 || f1 * f3 <= 2.0 * f2 * f2) {
+    return 0.0;
+  }
+  const double c    = 2.0 * (f2 > 1.0 ? f2 : 1.0);
+  const double x    = exp(-f1 / c - 0.5772);
+  const double more = static_cast<double>(n) / COLLECT_SAMPLES;
+  return x * more < 0.3 ? c * more * (0.4228 - log(x * more)) : c / x;
+}
+
 // The plan, from the sampled keys, by one workgroup.  Their hashes stand for them: two values of one hash count as one, which
 // only the estimate notices.
 template <typename KeyT>
@@ -209,7 +230,7 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_plan_kernel(const KeyT*
   __shared__ uint32_t s_hash[COLLECT_SLOTS];       // 0: empty
   __shared__ uint32_t s_count[COLLECT_SLOTS / 2];  // 16 bits each
   __shared__ uint16_t s_first[COLLECT_SLOTS];      // a sampled key of the value
-  __shared__ uint32_t s_sum[3];
+  __shared__ uint32_t s_sum[4];
   __shared__ uint32_t s_heavy, s_mode, s_empty;
   const uint32_t tid = threadIdx.x;
   KeyT key[EACH];
@@ -223,7 +244,7 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_plan_kernel(const KeyT*
       s_count[j] = 0;
     }
   }
-  if (tid < 3) {
+  if (tid < 4) {
     s_sum[tid] = 0;
   }
   if (tid == 0) {
@@ -251,20 +272,23 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_plan_kernel(const KeyT*
     atomicAdd(&s_count[slot[r] / 2], slot[r] % 2 != 0 ? 0x10000u : 1u);
   }
   __syncthreads();
-  uint32_t once = 0, twice = 0, values = 0;
+  uint32_t once = 0, twice = 0, thrice = 0, values = 0;
   for (uint32_t j = tid; j < COLLECT_SLOTS; j += COLLECT_BLOCK) {
     const uint32_t c = (s_count[j / 2] >> (j % 2 * 16)) & 0xFFFFu;
     values += c != 0 ? 1u : 0u;
     once += c == 1 ? 1u : 0u;
     twice += c == 2 ? 1u : 0u;
+    thrice += c == 3 ? 1u : 0u;
   }
   values = wave_inclusive_sum_dpp(values);
   once   = wave_inclusive_sum_dpp(once);
   twice  = wave_inclusive_sum_dpp(twice);
+  thrice = wave_inclusive_sum_dpp(thrice);
   if (tid % WAVE == WAVE - 1) {
     atomicAdd(&s_sum[0], values);
     atomicAdd(&s_sum[1], once);
     atomicAdd(&s_sum[2], twice);
+    atomicAdd(&s_sum[3], thrice);
   }
   __syncthreads();
   if (tid == 0) {
@@ -276,7 +300,8 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_plan_kernel(const KeyT*
     } else if (all <= collect_many_max(sizeof(KeyT)) && all * 4.0 <= static_cast<double>(n)) {
       mode = COLLECT_MANY;
     }
-    s_mode = mode;
+    plan->doubt = mode == COLLECT_MANY && collect_tail(s_sum[1], s_sum[2], s_sum[3], n) > collect_tail_max(sizeof(KeyT)) ? 1u : 0u;
+    s_mode      = mode;
   }
   __syncthreads();
   const uint32_t mode = s_mode;

@@ -289,7 +289,8 @@ int cpn_unique_sorted(int dtype, const void* sorted, void* values_out, uint64_t 
  * its length: what a caller that can wait for the count sorts instead of calling cpn_unique.  `temp` is a 256-byte aligned
  * workspace of cpn_distinct_temp_bytes(dtype, volume, &list_offset) bytes (0: not tried for this type and length).
  * cpn_distinct_plan looks at the sample; when the stream has finished, the first 32-bit word of `temp` is the mode: 0 for
- * "not this array" (call cpn_unique), otherwise the `mode` of a call of cpn_distinct on the same array and workspace.  After
+ * "not this array" (call cpn_unique), otherwise the `mode` of a call of cpn_distinct on the same array and workspace, which
+ * will likely come to nothing where the sixth word is not 0 (values of very unlike frequency).  After
  * that the first three words are the mode; not 0 where the attempt came to nothing (call cpn_unique); and the number of
  * values, which lie in `temp` from list_offset on.  Every kernel ends by itself and nothing outside `temp` is written.  It
  * has no counterpart in the reference, whose UniqueTask sorts (src/cupynumeric/set/unique.cu:137-204).

@@ -189,3 +189,28 @@ def test_status_of_the_sort_of_the_values(torch_cuda, monkeypatch, mode):
     monkeypatch.setattr(_thunk, "sort_task", failing)
     with pytest.raises(RuntimeError, match="failed on the device"):
         num.unique(a)
+
+
+@pytest.mark.parametrize("dtype, n, values, tried", [
+    (np.int64, 1 << 25, 1 << 24, False),  # 5.2 million different ones: more than the tables hold
+    (np.int64, 1 << 23, 1 << 22, True),  # 1.4 million
+    (np.int32, 1 << 24, 1 << 23, True),  # 2.7 million
+    (np.uint64, (1 << 24) + 9, 1 << 17, True),
+])
+def test_values_whose_frequencies_fall_with_their_rank(lib, torch_cuda, dtype, n, values, tried):
+    """Chao's estimate of them is far too low (47 000 of the first); what the second one does not believe is not tried."""
+    x = (float(values) ** np.random.default_rng(values).random(n)).astype(dtype) * dtype(97)
+    if tried:
+        mode, failed, found = _mode(lib, torch_cuda, x)
+        assert (mode, failed) == (2, 0) and np.array_equal(np.sort(found), np.unique(x))
+    a = num.array(x)
+    num.unique(a)
+    lib.cpn_profile_enable(1)
+    try:
+        _lib.profile_collect()
+        got = np.asarray(num.unique(a))
+        labels = [label for label, _ in _lib.profile_collect()]
+    finally:
+        lib.cpn_profile_enable(0)
+    assert np.array_equal(got, np.unique(x))
+    assert "collect_plan" in labels and ("collect_class" in labels) == tried, labels
