@@ -116,15 +116,21 @@ def _collapse_axes(a: ndarray, axes: tuple[int, ...]) -> tuple[int, ndarray]:
 
 # As many quantiles as `cpn_quantile_sorted_args` takes.
 QUANTILE_ARGS = 16
-# Vectors from this length on are selected from (`cpn_quantile_select`) instead of sorted; of float vectors, four quantiles
-# and more from four times as many.  A selection is a chain of about ten launches, a sort of a vector like these two or three.
-# us per call, selected / sorted, one, five and sixteen quantiles, of normal values and of few different ones:
-#   32 768 elements   float32 37/27, 47/29, 66/33   35/30, 56/30, 71/32   float64 50/27, 66/28, 69/32   39/36, 60/37, 72/37
-#   200 000           float32 38/27, 48/29, 67/33   35/37, 56/37, 71/37   float64 51/27, 65/29, 78/33   39/46, 60/46, 72/47
-#   500 000           float32 39/32, 48/32, 68/35   35/45, 56/46, 71/46   float64 49/35, 70/34, 77/35   39/62, 62/63, 73/63
-#   2 000 000         float32 47/99, 56/99, 79/98   41/106, 62/106, 77/107
-#   int64   200 000   59/27, 66/29, 81/33   56/53, 62/53, 74/53     500 000   63/34, 71/34, 85/35   58/75, 64/75, 76/76
-SELECT_MIN_SIZE = 1 << 17
+# 4-byte vectors from this length on are selected from (`cpn_quantile_select`) instead of sorted, and from twice as many elements on
+# 8-byte ones, and for more than two quantiles floats, for more than eight whole numbers (past 2^20 elements a sort takes more
+# launches, or splits few values into as many parts as many).  A selection is a chain of about ten launches, a sort of a vector like
+# these two to ten.  us per call, selected / sorted, one, three, five and sixteen quantiles of normal values, then of twenty different:
+#   float32     500 000  37/32  46/32  48/32  66/35    35/35  54/35  53/35  69/36
+#               700 000  38/46  44/46  48/46  69/45    35/46  54/46  53/46  69/46
+#             1 048 576  43/50  47/50  50/50  65/50    36/48  56/48  55/49  69/49    2 097 152  41/101 53/100 56/100 78/100   42/65 62/65 60/65 74/65
+#   int32       500 000  38/33  40/34  42/35  58/40    34/33  35/34  35/36  43/40
+#               700 000  39/45  41/45  43/45  59/45    34/40  35/40  36/39  44/41
+#             1 048 576  42/46  44/46  47/47  63/47    34/43  35/43  35/42  42/42    2 097 152  44/93  51/94  55/93  71/93    33/49 34/50 34/51 43/56
+#   float64     700 000  46/50  65/50  74/49  90/50    44/51  57/51  62/52  76/51
+#             1 048 576  55/57  74/56  82/56 100/56    43/53  60/54  65/54  79/54    1 048 577  54/63  73/66  81/65  97/65    43/79 60/79 66/78 79/78
+#   int64       700 000  64/50  69/49  72/50  87/50    41/47  42/47  45/47  50/47
+#             1 048 576  65/54  78/54  81/54  95/55    42/48  43/48  45/48  51/48    1 048 577  75/61  79/63  83/63  95/63    39/74 40/74 43/73 47/73
+SELECT_MIN_SIZE = 1 << 19
 
 
 def _select_bytes(a: ndarray, num_q: int) -> int:
@@ -170,8 +176,9 @@ def quantile(
 
     # A long vector of which only a few elements are needed is not sorted (SELECT_MIN_SIZE)
     flat = real_axis is None or a_rr.ndim == 1
-    longest_sorted = SELECT_MIN_SIZE * (4 if q_arr.size >= 4 and a_rr.dtype.kind == "f" else 1)
-    select = flat and not overwrite_input and a_rr.size >= longest_sorted and _select_bytes(a_rr, q_arr.size) != 0
+    later = a_rr.dtype.itemsize == 8 or q_arr.size > (2 if a_rr.dtype.kind == "f" else 8)
+    shortest_selected = SELECT_MIN_SIZE * (2 if later else 1)
+    select = flat and not overwrite_input and a_rr.size >= shortest_selected and _select_bytes(a_rr, q_arr.size) != 0
     if overwrite_input:
         a_rr.sort(axis=real_axis)
         arr = a_rr

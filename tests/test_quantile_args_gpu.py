@@ -57,3 +57,24 @@ def test_lengths_around_the_line_of_the_selection(dtype):
                 x[rng.integers(0, m, 20)] = -0.0
             for q in ([50.0], [5.0, 25.0, 50.0, 75.0, 95.0], list(np.linspace(0, 100, 17))):
                 assert_same_bits(np.asarray(num.percentile(num.array(x), q)), oracle.percentile(x, q), f"{m} {q}")
+
+
+@pytest.mark.parametrize("dtype, two, three, nine", [(np.float32, 1, 2, 2), (np.int32, 1, 1, 2), (np.float64, 2, 2, 2), (np.int64, 2, 2, 2)])
+def test_which_vectors_are_selected_from(dtype, two, three, nine):
+    """By the launches, at the lines of two, three and nine quantiles, and one element before."""
+    lib = _lib.load()
+    rng = np.random.default_rng(5)
+    for q, times in (([25.0, 75.0], two), ([25.0, 50.0, 75.0], three), (list(np.linspace(10, 90, 9)), nine)):
+        line = times * _stats.SELECT_MIN_SIZE
+        for n in (line - 1, line):
+            x = (rng.standard_normal(n) * 1e6).astype(dtype)
+            a = num.array(x)
+            lib.cpn_profile_enable(1)
+            try:
+                _lib.profile_collect()
+                got = np.asarray(num.percentile(a, q))
+                labels = {label for label, _ in _lib.profile_collect()}
+            finally:
+                lib.cpn_profile_enable(0)
+            assert_same_bits(got, oracle.percentile(x, q), f"{np.dtype(dtype)} {n} {q}")
+            assert any(label.startswith("select") for label in labels) == (n == line), (n, q, labels)
