@@ -18,16 +18,19 @@ if TYPE_CHECKING:
 
 # Where in its workspace `cpn_unique` may put the count: beside the status word, in a line that nothing else uses.
 UNIQUE_COUNT_OFFSET = 64
-# From so many values on they are grouped by the parts of the array (`cpn_searchsorted_grouped`), where that is done, and up to
-# so many of 4 and 8 bytes are not sorted first where it is not.  us per call, grouped (of 2^28: sorted first) / each value by itself,
-# values spread as the array / half of them in a thousandth of it:
-#   float32   in 4*10^6   130 000  39 / 18  55 / 13   262 144  40 / 33  57 / 23   524 288  43 / 57  59 / 41
-#             in 3*10^7   130 000  80 / 25  85 / 18   262 144  81 / 52  92 / 31   524 288  82 / 94  108 / 55
-#             in 2^28     130 000  73 / 38  78 / 25   262 144 122 / 79 118 / 46   524 288 168 / 149 140 / 87
-#   float64   in 3*10^7   130 000 118 / 28 129 / 20   262 144 119 / 57 130 / 33   524 288 121 / 102 140 / 58
-#             in 2^28     130 000  80 / 42  93 / 28   262 144 172 / 88 175 / 53   524 288 257 / 166 227 / 109
-GROUPED_MIN_VALUES = (1 << 18) + 1
-UNSORTED_MAX_VALUES = 1 << 19
+# From so many values on they are grouped by the parts of the array (`cpn_searchsorted_grouped`), where that is done.  us per call,
+# grouped / each value by itself, values spread as the array / half of them in a thousandth of it:
+#   float32   in 2^21     262 144  44 / 25  51 / 19   393 216  48 / 34  53 / 27   524 288  51 / 44  54 / 35   786 432  60 / 65  57 / 50
+#             in 4*10^6   262 144  38 / 33  50 / 23   393 216  39 / 44  52 / 31   524 288  40 / 55  53 / 40   786 432  43 / 79  59 / 58
+#             in 3*10^7   262 144  78 / 51  94 / 31   393 216  79 / 77  95 / 42   524 288  80 / 95 101 / 54   786 432  82 / 126 105 / 79
+#   float64   in 2^20     262 144  50 / 25  54 / 20   393 216  53 / 34  56 / 28   524 288  58 / 44  58 / 36   786 432  65 / 61  60 / 49
+#             in 4*10^6   262 144  49 / 38  59 / 25   393 216  50 / 51  61 / 33   524 288  51 / 64  63 / 43   786 432  52 / 92  68 / 62
+#             in 3*10^7   262 144 116 / 55 129 / 33   393 216 119 / 80 132 / 44   524 288 119 / 100 136 / 57  786 432 123 / 146 142 / 82
+GROUPED_MIN_VALUES = (1 << 19) + 1
+# Up to so many of 4 and 8 bytes are not sorted first in a long array where they are not grouped; sorted / each by itself:
+#   float32   in 2^28     524 288 165 / 149 130 / 87   786 432 253 / 188 215 / 145   2^20 270 / 229 232 / 157   3*2^19 322 / 348 286 / 225
+#   float64   in 2^27     524 288 243 / 152 210 / 94   786 432 353 / 193 317 / 153   2^20 377 / 232 340 / 164   3*2^19 433 / 346 397 / 225
+UNSORTED_MAX_VALUES = 1 << 20
 # Longest array of integers that `unique` splits by sampled keys (`cpn_local_sort_split_temp_bytes`).  Arrays that it is asked
 # of repeat their values, and 8-byte ones mostly leave upper bytes constant, whose passes the sort of `cpn_unique` skips:
 # int64 below 10^9, us per call that way / split: 2^20 + 1 of as many values 204 / 125, of 1000 219 / 145;

@@ -652,7 +652,7 @@ static FindLayout find_layout(int key_bytes, uint64_t n, uint64_t num_values)
   return L;
 }
 
-// From 8 MiB of array and 2^16 values on (a caller that can choose takes searchsorted_few_kernel, without a workspace, up to 2^18):
+// From 8 MiB of array and 2^16 values on (a caller that can choose takes searchsorted_few_kernel, without a workspace, up to 2^19):
 // below, the five launches and parts too few for all CUs (a part has a window at
 // least) cost more than direct probes of the caches; and not for values so sparse that reading the whole array for them is the
 // larger part.  us per call of `searchsorted`, probes or sorted values / this way, values spread as the array / half of

@@ -30,13 +30,21 @@ namespace cpn {
 constexpr int SEARCH_BLOCK  = 256;
 constexpr int SEARCH_PIVOTS = 2048;
 __device__ constexpr uint32_t search_pivot_at(uint32_t j) { return j + (j >> 6); }
-// Up to so many values every lane has one (searchsorted_few_kernel); past it the table that each workgroup loads first costs more than
-// the lanes give.  us per call of `searchsorted`, sixteen values per lane / one:
-//   float32 in 10^4   2048 values 18 / 11   60 000  30 / 11   250 000  30 / 12   600 000  31 / 13   10^6  31 / 15
-//        in 65 536    2048        22 / 11   60 000  38 / 11   250 000  38 / 18   600 000  39 / 35   10^6  41 / 53
-//        in 10^6      2048        27 / 11   60 000  49 / 11   250 000  61 / 23   600 000  65 / 46   10^6  67 / 71
-//   float64 in 10^6   2048        31 / 11   60 000  74 / 12   250 000  79 / 26   600 000  81 / 54   10^6  83 / 83
-constexpr uint64_t SEARCH_FEW = 1ull << 19;
+// Up to so many values in an array of n every lane has one (searchsorted_few_kernel); past it the table that each workgroup loads
+// first costs more than the lanes give.  us per call of `searchsorted`, sixteen values per lane / one:
+//   float32 in 8192   2048 values 18 / 11  250 000  30 / 11  700 000  27 / 11  1 600 000  30 / 18  3 10^6  35 / 30  2^22  40 / 41
+//        in 16 384    2^19            12   700 000  30 / 16  786 432  30 / 17  1 048 576  31 / 22  1 572 864  34 / 30  2^21  35 / 39
+//        in 65 536    2048        22 / 11  250 000  38 / 18  700 000  37 / 36  786 432    37 / 39  900 000  38 / 45
+//        in 2^18                           700 000  44 / 43  786 432    44 / 47
+//        in 2^20      2048        27 / 11  250 000  61 / 23  700 000  65 / 48  786 432    66 / 54  900 000  66 / 62  2^20  66 / 71
+//        in 4 10^6                         600 000  83 / 65  700 000  85 / 72  786 432    86 / 79  900 000  91 / 90
+//        in 3 10^7                         600 000 112 / 107 700 000 122 / 124 786 432   126 / 137
+//        in 2^28                           2^19    149 / 149 600 000 168 / 175 786 432   188 / 223
+//   float64 in 16 384                      600 000  33 / 19  786 432  34 / 22  1 310 720  37 / 34  1 572 864  37 / 39
+//        in 65 536                         600 000  41 / 33  786 432  42 / 41  900 000    42 / 47
+//        in 2^20      2048        31 / 11  250 000  79 / 26  786 432  80 / 61  2^20       83 / 81  1 310 720  99 / 100
+//        in 3 10^7                         600 000 127 / 119 786 432 146 / 148 900 000   160 / 167
+constexpr uint64_t search_few(uint64_t n) { return n <= 16384 ? 3ull << 19 : (n <= (1ull << 24) ? 11ull << 16 : 1ull << 19); }
 
 constexpr uint32_t WINDOW_BYTES    = 40960;
 constexpr uint32_t WINDOW_TILE_MAX = 1024;
@@ -451,7 +459,7 @@ static int launch_searchsorted(const void* sorted, uint64_t n, const void* value
     num_pivots = static_cast<uint32_t>((n + step - 1) / step);
   }
   if constexpr (CODEC != CODEC_COMPLEX) {
-    if (num_pivots != 0 && num_values <= SEARCH_FEW) {
+    if (num_pivots != 0 && num_values <= search_few(n)) {
       const auto search = left ? &searchsorted_few_kernel<KeyT, CODEC, true> : &searchsorted_few_kernel<KeyT, CODEC, false>;
       ProfileScope prof("searchsorted", stream);
       hipLaunchKernelGGL(search, dim3(static_cast<uint32_t>((num_values + SEARCH_BLOCK - 1) / SEARCH_BLOCK)), dim3(SEARCH_BLOCK), 0,

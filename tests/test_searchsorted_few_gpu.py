@@ -61,3 +61,13 @@ def test_a_long_array():
     a = a[: 1 << 23]
     for m in (1 << 18, (1 << 18) + 1):
         _check(a, rng.integers(-5, a.size + 5, m).astype(np.int32))
+
+
+@pytest.mark.parametrize("n, m", [(16384, 3 << 19), (16385, 11 << 16), (1 << 19, 11 << 16)])
+@pytest.mark.parametrize("dtype", [np.float32, np.int64])
+def test_the_line_moves_with_the_array(n, m, dtype):
+    """As many values as have a lane each, and one more; a result is asked for in the order of the values."""
+    rng = np.random.default_rng(n)
+    a = np.arange(n).astype(dtype) * 3
+    for k in (m, m + 1):
+        _check(a, rng.integers(-3, 3 * n + 3, k).astype(dtype))
