@@ -169,6 +169,22 @@ constexpr bool eq_keys()
   return sizeof(KeyT) == 8 && KeyTraits<CODEC, KeyT>::PASSES == 8 && KeyTraits<CODEC, KeyT>::NWORDS == 1 && sizeof(OffT) == 4;
 }
 
+// Rows that a few passes may sort (PlanRequest::narrow): WIDE_FLAGS words, of which one that is not 0 says that they will not.
+constexpr uint32_t WIDE_FLAGS = 16;
+__device__ __forceinline__ bool any_wide(const uint4* flags)
+{
+  if (flags == nullptr) {
+    return false;
+  }
+  uint32_t any = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < WIDE_FLAGS / 4; ++j) {
+    const uint4 q = flags[j];
+    any |= q.x | q.y | q.z | q.w;
+  }
+  return any != 0;
+}
+
 // What the byte passes go on from when equalised digits have failed (equal_digits.h): keys and positions, and the
 // buffers that their first pass reads (make_plan).
 template <typename KeyT>
@@ -183,7 +199,7 @@ struct EqualResume {
 // 128-bit loads over the 16-byte aligned middle of the chunk, scalar head and tail.
 // `vplan` (may be null): nothing to do when the sort already runs on the ranks of the row's
 // different keys (virtual_digits.h), or when equalised digits have sorted it (`eq`, may be null), or for a row that
-// few passes will not sort (PlanRequest::narrow, may be null).
+// few passes will not sort (`wide`, may be null).
 // SPECIALS (float keys, keys-only sorts): also tells through `specials` whether a NaN or a -0.0 occurs.
 template <typename KeyT, int CODEC, typename OffT, bool SPECIALS = false>
 __global__ __launch_bounds__(HIST_BLOCK) void histogram_kernel(const KeyT* __restrict__ keys,
@@ -195,11 +211,11 @@ __global__ __launch_bounds__(HIST_BLOCK) void histogram_kernel(const KeyT* __res
                                                                  uint32_t* __restrict__ specials,
                                                                  const EqualPlan* __restrict__ eq,
                                                                  const EqualResume<KeyT> resume,
-                                                                 const uint32_t* __restrict__ narrow)
+                                                                 const uint4* __restrict__ wide)
 {
   constexpr int PASSES      = KeyTraits<CODEC, KeyT>::PASSES;
   constexpr int VEC         = 16 / sizeof(KeyT);
-  if (narrow != nullptr && *narrow == 0) {
+  if (any_wide(wide)) {
     return;
   }
   constexpr int HIST_COPIES = hist_copies(PASSES);
@@ -361,9 +377,10 @@ struct PlanRequest {
   uint32_t free_rank;
   const uint32_t* specials;
   const uint32_t* per_xcd;  // of the workspace header
-  // Rows that are sorted by the passes in `launched` (a bit each) or not at all (may be null): not 0 while they may be,
-  // 2 when there is nothing to sort.
+  // Rows that are sorted by the passes in `launched` (a bit each) or not at all (may be null): 0 becomes 1 if they are, 2 if
+  // there is nothing to sort.
   uint32_t* narrow;
+  const uint4* wide;  // see any_wide
   uint32_t launched;
   // Requests that may use equalised digits (may be null).  When those have failed, the byte passes start
   // from the scratch partner of T1 below and from IDX_ALIAS.
@@ -384,12 +401,9 @@ __device__ __forceinline__ void make_plan(const uint32_t* varying, SortPlan* __r
   }
   if (rq.narrow != nullptr) {
     if ((flags & ~rq.launched) != 0) {
-      *rq.narrow = 0;  // (the plan stays cleared: no pass runs)
-      return;
+      return;  // (the plan stays cleared: no pass runs)
     }
-    if (k == 0) {
-      *rq.narrow = 2;  // all keys are equal
-    }
+    *rq.narrow = k != 0 ? 1u : 2u;
   }
   const bool resume = eq_failed(rq.eq);
   if (resume && (k & 1u) != 0) {
@@ -465,7 +479,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void histogram_scan_kernel(OffT* __rest
                                                                     SortPlan* __restrict__ plan,
                                                                     PlanRequest rq)
 {
-  if (eq_sorted(rq.eq) || (rq.narrow != nullptr && *rq.narrow == 0)) {
+  if (eq_sorted(rq.eq) || any_wide(rq.wide)) {
     return;  // (the plan stays cleared: no byte pass runs)
   }
   // first use (`second` == 0): nothing when the sort already runs on the ranks of the row's

@@ -1140,7 +1140,7 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
                          EqualResume<KeyT>{reinterpret_cast<const KeyT*>(ws + L.off_key1), static_cast<KeyT*>(key_x),
                                            HAS_IDX ? reinterpret_cast<const uint32_t*>(ws + L.off_idx) : nullptr,
                                            HAS_IDX ? reinterpret_cast<uint32_t*>(r.indices_out) : nullptr},
-                         static_cast<const uint32_t*>(nullptr));
+                         static_cast<const uint4*>(nullptr));
     }
     CPN_HIP_TRY(hipGetLastError());
     {
@@ -1310,11 +1310,11 @@ inline int sort_global(const SortRequest& r, const GlobalLayout& L)
 }
 
 // ---- rows of which few bytes vary (split_plan.h) ----
-// Where the passes find what they work on.  `head`: a workspace header whose second and later words are cleared but for
-// `narrow`; hist, desc: cleared where a pass is to run.
+// Where the passes find what they work on.  `head`: a cleared workspace header; hist, desc: cleared.
 struct NarrowBuffers {
   unsigned char* head;
-  uint32_t* narrow;
+  uint32_t* narrow;   // see PlanRequest
+  const uint4* wide;
   uint32_t* hist;
   unsigned char* desc;
   void* key1;
@@ -1342,6 +1342,7 @@ inline int sort_narrow(const SortRequest& r, const NarrowBuffers& b, int first, 
   rq.specials     = (CODEC == CODEC_FLOAT) ? reinterpret_cast<const uint32_t*>(b.head + HEADER_SPECIALS) : nullptr;
   rq.per_xcd      = reinterpret_cast<const uint32_t*>(b.head + HEADER_PER_XCD);
   rq.narrow       = b.narrow;
+  rq.wide         = b.wide;
   rq.launched     = ((1u << count) - 1u) << first;
   {
     const uint64_t chunk = align_up((r.seg + 2047) / 2048 < 16384 ? 16384 : (r.seg + 2047) / 2048, 4096);
@@ -1350,7 +1351,7 @@ inline int sort_narrow(const SortRequest& r, const NarrowBuffers& b, int first, 
     hipLaunchKernelGGL((histogram_kernel<KeyT, CODEC, uint32_t, (CODEC == CODEC_FLOAT) && !HAS_IDX>), dim3(grid), dim3(HIST_BLOCK), 0,
                        r.stream, static_cast<const KeyT*>(r.values_in), b.hist, r.seg, grid, chunk, static_cast<const VirtPlan*>(nullptr),
                        reinterpret_cast<uint32_t*>(b.head + HEADER_SPECIALS), static_cast<const EqualPlan*>(nullptr),
-                       EqualResume<KeyT>{}, static_cast<const uint32_t*>(b.narrow));
+                       EqualResume<KeyT>{}, b.wide);
   }
   CPN_HIP_TRY(hipGetLastError());
   {

@@ -48,6 +48,7 @@ inline int split_wide_tiles(const SortRequest& r, const SplitPlan& p, const Spli
     NarrowBuffers b{};
     b.head       = ws;
     b.narrow     = head + HEADER_NARROW / 4;
+    b.wide       = reinterpret_cast<const uint4*>(ws + HEADER_WIDE);
     b.hist       = reinterpret_cast<uint32_t*>(ws + L.off_hist);
     b.desc       = ws + L.off_desc;
     b.key1       = ws + L.off_key1;

@@ -57,6 +57,7 @@ inline SplitPlan split_plan(int key_bytes, int passes, uint64_t volume, uint64_t
   p.tiles        = static_cast<uint32_t>((seg + p.tile_len - 1) / p.tile_len);
   return p;
 }
+static_assert(SPLIT_WIDE_FLAGS == WIDE_FLAGS && HEADER_WIDE + 4 * WIDE_FLAGS <= HEADER_TICKETS, "the flags have a place in the header");
 // Byte passes that a wide row tries ahead of the split: the lowest of whole numbers, the highest of floats (signs, exponents and the
 // leading bits of fractions; whole numbers that go below zero have busy upper bytes and do not try).  A row of which only those
 // bytes vary is sorted by one read that counts and a pass for each byte that does; the split, which does not skip constant

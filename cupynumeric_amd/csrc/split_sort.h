@@ -68,9 +68,12 @@ __host__ __device__ __forceinline__ uint32_t split_sample_place(uint32_t i, uint
   return from + static_cast<uint32_t>((static_cast<uint64_t>(split_hash(i)) * (to - from)) >> 32);
 }
 
-// The head of the workspace of a row that byte passes may have sorted ahead (split_plan.h, narrow): the status word, and
-// HEADER_NARROW bytes on whether they were to.  Null: no passes.
-constexpr uint64_t HEADER_NARROW = 8;
+// The head of the workspace of a row that byte passes may have sorted ahead (split_plan.h, narrow): the status word,
+// HEADER_NARROW bytes on whether they did (PlanRequest::narrow, onesweep.h), and, HEADER_WIDE bytes on, what the look at the row
+// found (any_wide).  Null: no passes.
+constexpr uint64_t HEADER_NARROW     = 8;
+constexpr uint64_t HEADER_WIDE       = 64;
+constexpr uint32_t SPLIT_WIDE_FLAGS  = 16;
 __device__ __forceinline__ bool split_done(const uint32_t* head)
 {
   return head != nullptr && head[HEADER_NARROW / 4] != 0 && head[0] == 0;
@@ -418,8 +421,8 @@ __global__ __launch_bounds__(256) void split_gather_kernel(const KeyT* __restric
 }
 // The same as the first launch of a row that may be narrow.  It also gathers what the sample's own sort samples (`again` keys of
 // it; 10^7 keys 2 us less than by a launch), clears what the passes count with, from the head of the workspace on, and the first
-// workgroup looks at SPLIT_PROBE keys: where they differ in no bit of `outside`, the passes are to try.
-constexpr uint32_t SPLIT_PROBE = 4096;
+// SPLIT_WIDE_FLAGS workgroups look at the keys that they gather, 4096 in all: where these differ in no bit of `outside`, the passes are
+// to try.  (One workgroup that looks at 4096 keys of its own takes 5 us longer than all the others.)
 template <typename KeyT, int CODEC>
 __global__ __launch_bounds__(256) void split_front_kernel(const KeyT* __restrict__ keys_in, uint32_t n, uint32_t samples,
                                                           KeyT* __restrict__ out, uint32_t again, KeyT* __restrict__ out_again,
@@ -431,26 +434,15 @@ __global__ __launch_bounds__(256) void split_front_kernel(const KeyT* __restrict
     out_again[i] = keys_in[split_sample_place(split_sample_place(i, again, samples), samples, n)];
   }
   for (uint32_t v = i; v < n_clear; v += samples) {
-    if (v != 0) {
+    if (v < HEADER_WIDE / 16 || v >= HEADER_WIDE / 16 + SPLIT_WIDE_FLAGS / 4) {
       clear[v] = make_uint4(0u, 0u, 0u, 0u);
     }
   }
-  if (blockIdx.x == 0) {
-    constexpr int EACH = SPLIT_PROBE / 256;
-    KeyT probe[EACH], vary = 0;
-#pragma unroll
-    for (int r = 0; r < EACH; ++r) {
-      probe[r] = keys_in[split_sample_place(r * 256 + threadIdx.x, SPLIT_PROBE, n)];
-    }
-    const KeyT first = ordered_bits<CODEC, KeyT>(keys_in[0]);
-#pragma unroll
-    for (int r = 0; r < EACH; ++r) {
-      vary |= ordered_bits<CODEC, KeyT>(probe[r]) ^ first;
-    }
-    const int wide = __syncthreads_or((vary & outside) != 0 ? 1 : 0);
+  if (blockIdx.x < SPLIT_WIDE_FLAGS) {
+    const KeyT vary = ordered_bits<CODEC, KeyT>(own) ^ ordered_bits<CODEC, KeyT>(keys_in[0]);
+    const int wide  = __syncthreads_or((vary & outside) != 0 ? 1 : 0);
     if (threadIdx.x == 0) {
-      static_assert(HEADER_NARROW == 8, "the third word");
-      clear[0] = make_uint4(0u, 0u, wide != 0 ? 0u : 1u, 0u);
+      (reinterpret_cast<uint32_t*>(clear) + HEADER_WIDE / 4)[blockIdx.x] = wide != 0 ? 1u : 0u;
     }
   }
   out[i] = own;

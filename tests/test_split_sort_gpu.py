@@ -3,6 +3,7 @@ lengths at which the plan changes, keys that crowd the sample's bins or a bucket
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -258,3 +259,35 @@ def test_whole_numbers_held_as_floats(lib, torch_cuda, dtype):
     for n, values in ((100_000, 500), (300_000, 3000), (1 << 20, 20_000)):
         x = np.random.default_rng(values).integers(-values, values, n).astype(dtype)
         _check(lib, torch_cuda, x, f"{np.dtype(dtype)} {n} {values}")
+
+
+def test_streams_and_threads_at_once(torch_cuda):
+    """Rows of every kind of plan, sorted by eight threads on streams of their own, whose workspaces come from one allocator."""
+    torch = torch_cuda
+    rng = np.random.default_rng(12)
+    rows = [rng.standard_normal(9000).astype(np.float32), rng.standard_normal(100_000), rng.integers(0, 1 << 30, 600_000).astype(np.int32),
+            rng.integers(0, 1 << 40, 1_100_000), rng.standard_normal(2_300_000), rng.integers(0, 300, 2_300_000),
+            np.full(2_200_000, 5), rng.integers(0, 1 << 62, 5_000_000)]
+    want = [(np.sort(x), np.argsort(x, kind="stable")) for x in rows]
+    arrays = [num.array(x) for x in rows]
+    for a in arrays:
+        num.sort(a)  # (uploads it)
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for turn in range(6):
+                k = (i + turn) % len(rows)
+                got = [num.sort(arrays[k]), num.argsort(arrays[k])]  # both in flight before either is read
+                for g, w in zip(got, want[k]):
+                    if not np.array_equal(np.asarray(g), w):
+                        wrong.append((i, k))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(rows))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong
