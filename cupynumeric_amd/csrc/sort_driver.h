@@ -1321,7 +1321,12 @@ struct NarrowBuffers {
   void* key2;
   uint32_t* idx1;
 };
-inline uint64_t narrow_tiles(uint64_t n) { return (n + global_tile(8, false) - 1) / global_tile(8, false); }
+inline uint64_t narrow_tiles(uint64_t n)
+{
+  const int items     = small_sweep_items(8, 8, n);
+  const uint64_t tile = items != 0 ? SMALL_BLOCK * items : global_tile(8, false);
+  return (n + tile - 1) / tile;
+}
 inline uint64_t narrow_desc_bytes(uint64_t n) { return align_up(narrow_tiles(n) * RADIX * sizeof(uint32_t), WORKSPACE_ALIGN); }
 
 // Byte passes `first` ... `first + count - 1` of one row, the only ones that may have something to do.  The result of
@@ -1364,6 +1369,7 @@ inline int sort_narrow(const SortRequest& r, const NarrowBuffers& b, int first, 
   CPN_HIP_TRY(hipGetLastError());
   constexpr bool CAN_ORDER_KEYS = HAS_IDX && (CODEC == CODEC_SIGNED || CODEC == CODEC_FLOAT);
   const bool ordered_keys       = CAN_ORDER_KEYS && !want_vals;
+  const int items               = small_sweep_items(8, 8, r.seg);
   const uint32_t tiles          = static_cast<uint32_t>(narrow_tiles(r.seg));
   for (int p = first; p < first + count; ++p) {
     SweepArgs<false> a{};
@@ -1389,7 +1395,9 @@ inline int sort_narrow(const SortRequest& r, const NarrowBuffers& b, int first, 
     a.spin_limit         = lookback_spin_limit();
     a.volume             = r.seg;
     ProfileScope prof("onesweep", r.stream);
-    if (ordered_keys) {
+    if (items != 0) {
+      launch_small_sweep<KeyT, CODEC, HAS_IDX, CAN_ORDER_KEYS>(a, items, ordered_keys, dim3(tiles), r.stream);
+    } else if (ordered_keys) {
       if constexpr (CAN_ORDER_KEYS) {
         hipLaunchKernelGGL((onesweep_kernel<KeyT, CODEC, true, false, HAS_IDX, global_block(KB), global_items(KB, false)>), dim3(tiles),
                            dim3(global_block(KB)), 0, r.stream, a);

@@ -62,19 +62,18 @@ static_assert(SPLIT_WIDE_FLAGS == WIDE_FLAGS && HEADER_WIDE + 4 * WIDE_FLAGS <= 
 // leading bits of fractions; whole numbers that go below zero have busy upper bytes and do not try).  A row of which only those
 // bytes vary is sorted by one read that counts and a pass for each byte that does; the split, which does not skip constant
 // bytes, takes up to four times as long.  us a sort and an argsort, split / passes:
-//   int64 of equal keys    2^22 122, 125 / 53, 49    10^7 223, 231 / 81, 69     below 200  114, 117 / 67, 71    207, 217 / 106, 120
-//   below 20 000                119, 124 / 90, 97         232, 244 / 159, 185   below 300 000  131, 147 / 113, 123   244, 255 / 212, 265
+//   int64 of equal keys    2^22 122, 125 / 47, 45    10^7 223, 231 / 76, 66     below 200  114, 117 / 61, 67    207, 217 / 101, 117
+//   below 20 000                119, 124 / 84, 93         232, 244 / 153, 180   below 300 000  131, 147 / 107, 119   244, 255 / 205, 258
 //   float64 of two values       137, 141 / 98, 97         234, 242 / 175, 184
-// Every other row pays for launches that find nothing to do: full int64 keys 2^21 + 1 83, 88 / 94, 100; 2^22 109, 118 / 121, 130;
-// 10^7 218, 238 / 228, 249.  Up to 2^21 keys that is 12 of 60 to 75 us and wins 20 for keys of one byte, none for others
-// (2^21 int64 below 200 77, 78 / 57, 60; below 20 000 76, 78 / 76, 81); a third pass for floats wins nothing (of three bytes, below
-// 200: 2^23 195, 202 split, 187, 202 in passes that have no split behind them).
+// Every other row pays for launches that find nothing to do: full int64 keys 2^21 + 1 83, 88 / 90, 96; 2^22 109, 118 / 117, 125;
+// 10^7 217, 238 / 224, 243.  Up to 2^21 whole numbers a third pass wins nothing (2^21 below 300 000, three bytes: 78, 86 split, 91, 97
+// in passes), nor do passes over floats (of two values 84, 85 / 81, 80; of three bytes, below 200: 2^23 195, 202 / 187, 202).
 inline int narrow_passes(int codec, uint64_t n)
 {
-  if (n <= (1ull << 21)) {
-    return 0;
+  if (codec == CODEC_FLOAT) {
+    return n > (1ull << 21) ? 2 : 0;
   }
-  return codec == CODEC_FLOAT ? 2 : 3;
+  return n > (1ull << 21) ? 3 : 2;
 }
 // Workspace: header, the sample, the keys in the order of the buckets of each tile, their places, the table, two words
 // per key.  Wide: also the splitters (images, places, values), their table of bins, and the workspace of the sample's own sort.
@@ -90,7 +89,7 @@ inline SplitLayout split_layout(const SplitPlan& p, int key_bytes, uint64_t n, b
   SplitLayout L{};
   const uint64_t samples = static_cast<uint64_t>(p.buckets) * p.per_bucket;
   L.off_sample = HEADER_BYTES;
-  if (p.wide && n > (1ull << 21)) {  // (narrow_passes)
+  if (p.wide) {
     L.off_hist   = HEADER_BYTES;
     L.off_desc   = L.off_hist + 8 * RADIX * sizeof(uint32_t);
     L.off_sample = L.off_desc + 3 * narrow_desc_bytes(n);
@@ -109,7 +108,7 @@ inline SplitLayout split_layout(const SplitPlan& p, int key_bytes, uint64_t n, b
   L.off_starts = L.off_places + (want_indices ? align_up(n * sizeof(uint16_t), WORKSPACE_ALIGN) : 0);
   L.off_ids    = L.off_starts + align_up(table, WORKSPACE_ALIGN);
   L.total      = L.off_ids + align_up(2 * n * sizeof(uint32_t), WORKSPACE_ALIGN);
-  if (L.off_desc != 0) {  // (the sample outlives the passes)
+  if (p.wide) {  // (the sample outlives the passes)
     L.off_key1         = L.off_images;
     L.off_key2         = L.off_key1 + align_up(n * key_bytes, WORKSPACE_ALIGN);
     L.off_idx1         = L.off_key2 + align_up(n * key_bytes, WORKSPACE_ALIGN);

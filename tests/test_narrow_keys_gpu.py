@@ -15,7 +15,7 @@ from oracle import sort_oracle as oracle
 pytestmark = pytest.mark.gpu
 
 LONGEST = 4096 * 2560
-NO_PASSES = 1 << 21  # the longest row that is split at once; longer ones of whole numbers try three passes, of floats two
+SHORT = 1 << 21  # rows up to here try two passes, of floats none; longer ones three, of floats two
 
 
 class _Row:
@@ -74,15 +74,15 @@ def _whole(kind, n):
 
 
 @pytest.mark.parametrize("dtype", [np.int64, np.uint64])
-@pytest.mark.parametrize("n", [NO_PASSES, NO_PASSES + 1, 3_000_017])
+@pytest.mark.parametrize("n", [(1 << 20) + 1, SHORT, SHORT + 1, 3_000_017])
 @pytest.mark.parametrize("kind", list(KINDS))
 def test_whole_numbers(lib, torch_cuda, dtype, n, kind):
     vary = KINDS[kind]
     x = _whole(kind, n).astype(np.int64).view(dtype)
-    assert _both(lib, torch_cuda, x, f"{np.dtype(dtype)} {n} {kind}") == (n > NO_PASSES and vary is not None)
+    assert _both(lib, torch_cuda, x, f"{np.dtype(dtype)} {n} {kind}") == (vary is not None and vary <= (2 if n <= SHORT else 3))
 
 
-@pytest.mark.parametrize("n", [NO_PASSES, NO_PASSES + 1, 3_000_017])
+@pytest.mark.parametrize("n", [SHORT, SHORT + 1, 3_000_017])
 @pytest.mark.parametrize("kind", ["equal", "NaN", "zeros of either sign", "flags", "eighths", "NaN among flags", "thousands"])
 def test_floats(lib, torch_cuda, n, kind):
     rng = np.random.default_rng(n)
@@ -94,7 +94,7 @@ def test_floats(lib, torch_cuda, n, kind):
         "thousands": lambda: rng.integers(0, 5000, n).astype(np.float64),
     }[kind]()
     # (the image of a NaN has all bits set)
-    assert _both(lib, torch_cuda, x, f"{n} {kind}") == (n > NO_PASSES and kind not in ("NaN among flags", "thousands"))
+    assert _both(lib, torch_cuda, x, f"{n} {kind}") == (n > SHORT and kind not in ("NaN among flags", "thousands"))
 
 
 def test_the_longest_row(lib, torch_cuda):
@@ -114,7 +114,7 @@ def test_passes_that_give_up(lib, torch_cuda):
     prev = lib.cpn_set_lookback_spin_limit(1)
     by_passes = []
     try:
-        for n in (2_500_000, LONGEST):
+        for n in (1_500_000, 2_500_000, LONGEST):
             x = _whole("two bytes", n)
             for values, indices, in_place in ((True, False, False), (False, True, False), (True, True, True)):
                 row = _Row(lib, torch_cuda, x, values, indices, in_place)
