@@ -78,7 +78,7 @@ def sort_task(output: "DeviceArray", input: "DeviceArray", argsort: bool, stable
     stream = runtime.stream_handle()
     if seg >= SPLIT_MIN_ROW:
         temp_bytes = lib.cpn_local_sort_split_temp_bytes(code, volume, seg, int(argsort))
-        if temp_bytes != 0:  # two launches that cannot fail on the device: no status to look at
+        if temp_bytes != 0:  # a sort that cannot fail on the device: no status to look at
             temp = runtime.empty_bytes(temp_bytes)
             status = lib.cpn_local_sort_ex(code, values_in, values_out, indices_out, volume, seg, 0, int(stable),
                                            _lib.CPN_SORT_SPLIT, temp.data_ptr(), temp_bytes, stream)

@@ -32,10 +32,12 @@ GROUPED_MIN_VALUES = (1 << 19) + 1
 #   float64   in 2^27     524 288 243 / 152 210 / 94   786 432 353 / 193 317 / 153   2^20 377 / 232 340 / 164   3*2^19 433 / 346 397 / 225
 UNSORTED_MAX_VALUES = 1 << 20
 # Longest array of integers that `unique` splits by sampled keys (`cpn_local_sort_split_temp_bytes`).  Arrays that it is asked
-# of repeat their values, and 8-byte ones mostly leave upper bytes constant, whose passes the sort of `cpn_unique` skips:
-# int64 below 10^9, us per call that way / split: 2^20 + 1 of as many values 204 / 125, of 1000 219 / 145;
-# 2^21 of 1000 169 / 156; 2^22 of as many 206 / 211, of 20000 203 / 253.
-UNIQUE_SPLIT_INTEGERS = 1 << 21
+# of repeat their values, and 8-byte ones mostly leave upper bytes constant, whose passes the sort of `cpn_unique` skips.
+# us per call that way / split, int64 below 10^9 of as many values, of a quarter as many, of 1000, and of full range:
+#   2^20 + 1  130 / 116  129 / 117   97 / 102  194 / 118        2^21       149 / 126  148 / 133  106 / 110  229 / 123
+#   3*10^6    161 / 152  160 / 161  115 / 119  251 / 152        2^22 - 1   175 / 177  172 / 185  121 / 126  271 / 173
+#   2^22      206 / 211  162 / 164   (hashed)  299 / 204        2^23       297 / 306  293 / 318   (hashed)  469 / 296
+UNIQUE_SPLIT_INTEGERS = 3 << 20
 
 # dtypes the reference supports (`cupynumeric/_utils/array.py:28-43`)
 SUPPORTED_DTYPES = tuple(_lib.DTYPE_CODES.keys())

@@ -49,8 +49,9 @@ constexpr int COLLECT_FEW_PROBES = 512;  // in the table in memory, a fifth full
 constexpr double COLLECT_FEW_MAX  = 3000.0;
 constexpr double collect_many_max(int key_bytes) { return 64.0 * collect_class_slots(key_bytes); }  // a quarter of the tables
 constexpr double collect_tail_max(int key_bytes) { return 0.9 * COLLECT_CLASSES * collect_class_full(key_bytes); }
-// An array that turns out to be sorted after all has waited for the sample, 28 us.  us per call of `unique`, sorted / asked first:
-// 2^23 int32 of 1000 values 222 / 91, of 2^18 223 / 144, of 2^23 243 / 270; 2^22 int64 of 1000 values 200 / 87, of 2^18
+// An array that turns out to be sorted after all has waited for the sample, 28 us.  (Less than one copy for count and status in place of
+// two, and shorter scans, save: 2^22 int64 of as many values 226 before both, 206 since; 2^23 int32 250 / 230, 2^26 1037 / 1001.)  us per
+// call of `unique`, sorted / asked first: 2^23 int32 of 1000 values 222 / 91, of 2^18 223 / 144, of 2^23 243 / 270; 2^22 int64 of 1000 values 200 / 87, of 2^18
 // 196 / 150, of 2^22 206 / 235; and 2^22 int32 180 / 94, 180 / 144, 187 / 212: too much for what it gives.
 constexpr uint64_t collect_min_volume(int key_bytes) { return 1ull << (key_bytes == 4 ? 23 : 22); }
 

@@ -281,7 +281,7 @@ __global__ __launch_bounds__(FIND_SEARCHERS, find_waves(sizeof(KeyT))) void find
     uint4 pack[find_pack_at(FIND_WINDOW / 16)];
     uint32_t word[ROOM];
   } s;
-    __shared__ uint32_t s_base[FIND_TILES + 1];  // of the part's values in all tiles, those before a tile's
+  __shared__ uint32_t s_base[FIND_TILES + 1];  // of the part's values in all tiles, those before a tile's
   __shared__ uint16_t s_from[FIND_TILES];      // where they are in the tile
   __shared__ uint32_t s_count[FIND_WINDOWS + WAVE];
   __shared__ uint32_t s_first[FIND_WINDOWS + 1];
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(FIND_SEARCHERS, find_waves(sizeof(KeyT))) void find
   const uint32_t count = total - lo < ROOM ? total - lo : ROOM;  // (a piece is not empty)
   const uint32_t hi    = lo + count;
 
-  // ---- the values, `FIND_LANES` lanes per tile and four tiles of theirs at once ----
+  // ---- the values, `FIND_LANES` lanes per tile and `FIND_GATHER` tiles of theirs at once ----
   const uint32_t sub = tid % FIND_LANES;
   for (uint32_t t0 = tid / FIND_LANES; t0 < tiles; t0 += FIND_GATHER * GROUPS) {
     uint32_t at[FIND_GATHER], end[FIND_GATHER];

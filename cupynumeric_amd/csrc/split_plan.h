@@ -18,8 +18,10 @@ struct SplitPlan {
 // Where the lines lie (us per call, before / this way; normal float keys, sort and argsort):
 //   from where one workgroup has more than 6144 8-byte or 8192 4-byte keys to sort (until 8 or 16 keys per thread, about 12
 //   us, two launches cost as much): float64 6144 16, 19 / 15, 15, 8192 26, 21 / 15, 15, int64 6144 13, 15 / 14, 14, 8192 19, 18
-//   / 14, 14, float32 8192 15, 19 / 13, 14, 9000 22, 21 / 14, 14, int32 8192 12, 16 / 13, 13, 9000 19, 18 / 13, 13.  Rows of a hundred
-//   values cost the network for the sample and passes in the buckets: 8192 float32 15, 17 / 18, 18, float64 27, 27 / 21, 21.
+//   / 14, 14, float32 8192 15, 19 / 13, 14, 9000 22, 21 / 14, 14, int32 8192 12, 16 / 13, 13, 9000 19, 18 / 13, 13.  Rows of few values
+//   cost passes over the sample and in the buckets, where one workgroup skips the bytes that all keys share: of a hundred values 9000 float32 19, 22
+//   / 19, 18, float64 34, 32 / 20, 20, int32 13, 13 / 17, 17, int64 14, 14 / 19, 19; of two 27, 25 / 20, 20, 29, 28 / 23, 23, 13,
+//   13 / 20, 20, 15, 14 / 21, 21; of one 13 / 16 to 18
 //   in between: 40 000 float32 29, 30 / 14, 15, float64 33, 34 / 16, 16; 100 000 41, 46 / 16, 17 and 53, 48 / 18, 18;
 //   262 144 68, 75 / 23, 26 and 125, 115 / 26, 27; 524 288 65, 71 / 31, 34 and 152, 146 / 35, 37
 //   to where 8192 sampled keys, which every tile's workgroup sorts, take half of its time: 10^6 float32 76, 86 / 48, 52,
@@ -35,8 +37,11 @@ inline SplitPlan split_plan(int key_bytes, int passes, uint64_t volume, uint64_t
     return p;
   }
   if (seg >= SPLIT_WIDE_ROW) {
-    // A bucket of 2560 keys at most (and room for 4096): the fuller, the more of them sampled.  Tiles in whole rounds of
-    // the compute units.
+    // A bucket of 2560 keys at most (and room for 4096): the fuller, the more of them sampled, or rows with a bucket that does not
+    // fit, which its workgroup sorts alone in about 0.2 ms, are no longer rare.  128 of 2560: none of 400 rows (simulated), 96 one,
+    // 64 one in 15 (and 7 us of 225 less, 10^7 int64 ids); 64 of 2048: none, 32 one in 60 (7 us of 200 less); 16 of 1365: none.
+    // Longer rows would need more buckets than a tile has room to count: of 12 10^6 keys, with 4096 buckets and 128 sampled
+    // keys each, one row in 12 has such a bucket.  Tiles in whole rounds of the compute units.
     p.wide         = true;
     p.buckets      = seg <= (1ull << 21) ? 1024 : (seg <= (1ull << 22) ? 2048 : 4096);
     p.per_bucket   = seg <= p.buckets * 1365ull ? 16 : (seg <= p.buckets * 2048ull ? 64 : 128);

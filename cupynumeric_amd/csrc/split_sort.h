@@ -13,8 +13,9 @@
 //
 // A splitter is a pair of a key and its place in the row, so that equal keys are divided as well as any others: the sizes
 // of the buckets do not depend on how the values are distributed, only on which places are sampled, and
-// these are drawn from a hash of their number.  A bucket lies between eight sampled keys; the room in LDS is four times
-// the mean.  (Of a bucket with more there is one in ten million; only a row that was made for the purpose has many.)
+// these are drawn from a hash of their number.  A bucket lies between four to 128 sampled keys; the room in LDS is four times
+// the mean or more, in the longest rows 1.6 times and more, with as many more sampled keys (split_plan.h).  (Of a bucket with more there is
+// one in a million or fewer; only a row that was made for the purpose has many.)
 // Such a bucket is sorted by its workgroup in memory, one byte after another (oversized_bucket): slow, and still right.
 //
 // Stands where the reference calls cub's radix sort or thrust's merge sort of one row
@@ -35,7 +36,6 @@ constexpr int SPLIT_BUCKET_BLOCK = 512;
 constexpr int SPLIT_BUCKET_ITEMS = 8;
 constexpr int SPLIT_WAVES       = SPLIT_BLOCK / WAVE;
 constexpr int SPLIT_TILE_ITEMS  = 4;                       // keys per thread of a tile
-constexpr int SPLIT_MAX_BUCKETS = 1024;
 constexpr int SPLIT_MAX_TILES   = 256;
 // rows whose splitters are found ahead (split_wide_tile_kernel)
 constexpr int SPLIT_WIDE_MAX_TILES = 1280;
@@ -48,7 +48,8 @@ constexpr uint32_t SPLIT_CROWD  = 24;
 constexpr int SPLIT_FEW         = 12;
 constexpr int SPLIT_FEW_SAMPLED = 256;
 
-// A mixed 32-bit word: which key of its stretch sample i takes.
+// A mixed 32-bit word: which key of its stretch sample i takes.  (Chris Wellons' "lowbias32", published with his search for
+// integer hashes of 32 bits, constants and shifts.)
 __host__ __device__ __forceinline__ uint32_t split_hash(uint32_t x)
 {
   x ^= x >> 16;
@@ -791,7 +792,7 @@ __global__ __launch_bounds__(SPLIT_BLOCK) void split_wide_tile_kernel(const KeyT
   }
   const SplitBins bins = *bins_in;
   __syncthreads();
-  // ---- buckets, as in split_tile_kernel, four keys of a thread at a time ----
+  // ---- buckets, as in split_tile_kernel, GROUP keys of a thread at a time ----
   uint32_t where[ITEMS];  // bucket; later, in the upper half, the rank; then where the key goes
   constexpr int GROUP = 7;
   static_assert(ITEMS % GROUP == 0, "whole groups");
@@ -1025,7 +1026,7 @@ constexpr uint32_t SPLIT_BIN_LIMIT = 24;
 
 // One bucket of a row: its parts of all tiles gathered, sorted, stored.
 //   a bucket of equal images is in order: it was gathered in the order of the row
-//   others are spread over four bins per thread, of equal width between their smallest and their largest key; one atomic per key
+//   others are spread over four bins per thread (WIDE: eight), of equal width between their smallest and their largest key; one atomic per key
 //     says which of its bin it is, a scan where the bin starts, a walk over the bin how many of its keys come before
 //   buckets with a crowded bin: passes over the bytes of the images, of which numbers of keys move and the keys
 //     stay where they are in LDS.  One pass where there are two values

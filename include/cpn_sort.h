@@ -139,7 +139,7 @@ int cpn_local_sort(int dtype, const void* values_in, void* values_out, int64_t* 
  *                           (cpn_local_sort_check), without touching process-wide state.  Results do
  *                           not depend on it.
  *   CPN_SORT_SPLIT          `temp` holds cpn_local_sort_split_temp_bytes(...) bytes, which is not 0: rows are split by
- *                           sampled keys and the parts sorted side by side, two launches that cannot fail on the
+ *                           sampled keys and the parts sorted side by side; the call cannot fail on the
  *                           device.  With a smaller workspace, or where that size is 0, the option changes nothing.
  *                           Results do not depend on it.
  */
