@@ -214,3 +214,10 @@ def test_values_whose_frequencies_fall_with_their_rank(lib, torch_cuda, dtype, n
         lib.cpn_profile_enable(0)
     assert np.array_equal(got, np.unique(x))
     assert "collect_plan" in labels and ("collect_class" in labels) == tried, labels
+
+
+@pytest.mark.parametrize("n", [3 << 20, (3 << 20) + 1])
+@pytest.mark.parametrize("count", [300, 1 << 40])
+def test_the_longest_integers_that_are_split(n, count):
+    rng = np.random.default_rng(n)
+    _check(rng.integers(-(1 << 40), 1 << 40, min(count, n))[rng.integers(0, min(count, n), n)])
