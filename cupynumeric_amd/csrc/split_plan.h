@@ -69,7 +69,7 @@ static_assert(SPLIT_WIDE_FLAGS == WIDE_FLAGS && HEADER_WIDE + 4 * WIDE_FLAGS <= 
 // bytes, takes up to four times as long.  us a sort and an argsort, split / passes:
 //   int64 of equal keys    2^22 122, 125 / 47, 45    10^7 223, 231 / 76, 66     below 200  114, 117 / 61, 67    207, 217 / 101, 117
 //   below 20 000                119, 124 / 84, 93         232, 244 / 153, 180   below 300 000  131, 147 / 107, 119   244, 255 / 205, 258
-//   float64 of two values       137, 141 / 98, 97         234, 242 / 175, 184
+//   float64 of two values       137, 141 / 92, 92         232, 241 / 168, 178
 // Every other row pays for launches that find nothing to do: full int64 keys 2^21 + 1 83, 88 / 90, 96; 2^22 109, 118 / 117, 125;
 // 10^7 217, 238 / 224, 243.  Up to 2^21 whole numbers a third pass wins nothing (2^21 below 300 000, three bytes: 78, 86 split, 91, 97
 // in passes), nor do passes over floats (of two values 84, 85 / 81, 80; of three bytes, below 200: 2^23 195, 202 / 187, 202).
