@@ -45,9 +45,19 @@ constexpr int COLLECT_TILE        = COLLECT_BLOCK * COLLECT_ITEMS;
 constexpr uint32_t collect_class_full(int key_bytes) { return collect_class_slots(key_bytes) / 4 * 3; }
 constexpr uint32_t COLLECT_FEW_FULL = 6144;
 static_assert(collect_class_full(8) + COLLECT_BLOCK < collect_class_slots(8) && COLLECT_FEW_FULL + COLLECT_BLOCK < COLLECT_FEW_SLOTS, "never full");
-constexpr int COLLECT_FEW_PROBES = 512;  // in the table in memory, a fifth full if the estimate is right (every one is a round trip)
+// In the table in memory, a fifth full if the estimate is right.  (Every one is a round trip: in a full table, of 2^23 int32 keys with 20 000
+// different values whose frequencies fall as the power of 1.7 of their rank, `unique` took 890 us with 512 for each value of each
+// workgroup; 480 with 128 until one of a wave has found no place; 250 sorted.)
+constexpr int COLLECT_FEW_PROBES = 128;
 constexpr double COLLECT_FEW_MAX  = 3000.0;
 constexpr double collect_many_max(int key_bytes) { return 64.0 * collect_class_slots(key_bytes); }  // a quarter of the tables
+// Few values of like frequencies, up to 3000, are seen twice more often than once, and so are 2500 whose frequencies fall as the 7/8th power
+// of their rank by a third as often; of those that fall as its power of 1.7, without end, the sample sees a fifth as many twice.  Of these
+// the sample foretells 9000 to 35 000 for 2^23 keys, of which 20 000 are there, and nine in ten samples of them more than the table has places;
+// of the power of 2 one in twenty for 2^25 keys, where the table still does.  us per call of `unique` tried / not, 2^25 int64 of the power of
+// 1.5 3300 / 860, of 1.7 1160 / 850, of 2 214 / 860.
+constexpr double COLLECT_FEW_ONCE   = 3.6;
+constexpr double COLLECT_FEW_GROWTH = COLLECT_SLOTS;
 constexpr double collect_tail_max(int key_bytes) { return 0.9 * COLLECT_CLASSES * collect_class_full(key_bytes); }
 // An array that turns out to be sorted after all has waited for the sample, 28 us.  (Less than one copy for count and status in place of
 // two, and shorter scans, save: 2^22 int64 of as many values 226 before both, 206 since; 2^23 int32 250 / 230, 2^26 1037 / 1001.)  us per
@@ -204,20 +214,27 @@ struct CollectTable {
 // Values of very unlike frequency make Chao's estimate, a lower bound, far too low: of 2^25 keys spread evenly over the logarithm of
 // 2^24 it sees 47 000 values where there are 5.2 million, and the tables fill up after all the work (`unique` 1088 us sorted, 1360
 // this way and then sorted).  Values of like frequencies are seen once, twice and three times as a Poisson law has it, f1 f3 /
-// f2^2 = 2/3 if they are many; a tail of rarer and rarer ones shows in a quotient above.  Then the sample is read as one of
+// f2^2 = 2/3 if they are many; a tail of rarer and rarer ones shows in a larger f3.  Then the sample is read as one of
 // values whose frequencies fall with their rank: c / x^2 dx of them are expected x times in the sample, from some least x on, which f1 =
 // c (ln(1 / x) - 0.577) and f2 = c / 2 give, and so many of them are expected in n keys.  (A few frequent values beside very many
 // rare ones of one frequency show in nothing: those still fail.)  2^23 keys over the logarithm of 2^22, 1.4 million values, are still
 // tried: 310 sorted, 209.
 __device__ __forceinline__ double collect_tail(double f1, double f2, double f3, uint64_t n)
 {
-  if (f3 < 10.0 || f1 * f3 <= 2.0 * f2 * f2) {
+  const double like = f2 * f2 / 1.5 / (f1 > 1.0 ? f1 : 1.0);  // f3 of like frequencies
+  if (f3 <= 3.0 + 2.0 * like + 3.0 * sqrt(like)) {
     return 0.0;
   }
   const double c    = 2.0 * (f2 > 1.0 ? f2 : 1.0);
   const double x    = exp(-f1 / c - 0.5772);
   const double more = static_cast<double>(n) / COLLECT_SAMPLES;
   return x * more < 0.3 ? c * more * (0.4228 - log(x * more)) : c / x;
+}
+// The same for few values: where frequencies fall as a power of the rank without end, n keys have c n^a of them, with an a that is the share
+// of the sample's that it has once.
+__device__ __forceinline__ double collect_growth(double seen, double f1, uint64_t n)
+{
+  return seen * exp2(f1 / seen * log2(static_cast<double>(n) / COLLECT_SAMPLES));
 }
 
 // The plan, from the sampled keys, by one workgroup.  Their hashes stand for them: two values of one hash count as one, which
@@ -301,8 +318,10 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_plan_kernel(const KeyT*
     } else if (all <= collect_many_max(sizeof(KeyT)) && all * 4.0 <= static_cast<double>(n)) {
       mode = COLLECT_MANY;
     }
-    plan->doubt = mode == COLLECT_MANY && collect_tail(s_sum[1], s_sum[2], s_sum[3], n) > collect_tail_max(sizeof(KeyT)) ? 1u : 0u;
-    s_mode      = mode;
+    const double room = collect_tail_max(sizeof(KeyT)), quarter = static_cast<double>(n) / 4.0;
+    const bool tail   = mode == COLLECT_MANY && collect_tail(f1, f2, s_sum[3], n) > (room < quarter ? room : quarter);
+    plan->doubt       = tail || (mode == COLLECT_FEW && f1 > COLLECT_FEW_ONCE * f2 + 4.0 && collect_growth(seen, f1, n) > COLLECT_FEW_GROWTH) ? 1u : 0u;
+    s_mode            = mode;
   }
   __syncthreads();
   const uint32_t mode = s_mode;
@@ -439,34 +458,39 @@ __global__ __launch_bounds__(COLLECT_BLOCK) void collect_few_kernel(const KeyT* 
   if (tid == 0 && s_empty != 0) {
     collect_list_empty<KeyT>(plan, list, room);
   }
-  // the workgroup's values into the table in memory, and those that are new to it into the list
-  for (uint32_t j = tid; j < COLLECT_FEW_SLOTS; j += COLLECT_BLOCK) {
-    const KeyT k = s_table[j];
-    if (k == EMPTY || ((s_listed[j / WAVE] >> (j % WAVE)) & 1u) != 0) {
-      continue;
-    }
-    uint32_t slot = collect_slot<COLLECT_SLOTS, KeyT>(collect_hash(k));
-    bool placed   = false;
-    for (int probe = 0; probe < COLLECT_FEW_PROBES; ++probe) {
+  // The workgroup's values into the table in memory, and those that are new to it into the list, a wave's worth with one addition
+  // to the one counter.  A wave that finds no place gives up.
+  for (uint32_t j0 = 0; j0 < COLLECT_FEW_SLOTS; j0 += COLLECT_BLOCK) {  // uniform
+    const uint32_t j = j0 + tid;
+    const KeyT k     = s_table[j];
+    bool todo        = k != EMPTY && ((s_listed[j / WAVE] >> (j % WAVE)) & 1u) == 0;
+    bool added       = false;
+    uint32_t slot    = collect_slot<COLLECT_SLOTS, KeyT>(collect_hash(k));
+    for (int probe = 0; probe < COLLECT_FEW_PROBES && todo; ++probe) {
       KeyT there = __hip_atomic_load(&table[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (there == EMPTY) {
         there = collect_cas<KeyT>(&table[slot], EMPTY, k);
-        if (there == EMPTY) {
-          const uint32_t at = atomicAdd(&plan->count, 1u);
-          if (at < room) {
-            list[at] = k;
-          }
-          there = k;
-        }
+        added = there == EMPTY;
       }
-      if (there == k) {
-        placed = true;
-        break;
-      }
+      todo = !added && there != k;
       slot = (slot + 1) & (COLLECT_SLOTS - 1);
     }
-    if (!placed) {
-      plan->failed = 1;
+    const uint64_t bal = __ballot(added);
+    if (bal != 0) {
+      uint32_t at = 0;
+      if (tid % WAVE == 0) {
+        at = atomicAdd(&plan->count, static_cast<uint32_t>(__builtin_popcountll(bal)));
+      }
+      at = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at))) + lanes_below(bal);
+      if (added && at < room) {
+        list[at] = k;
+      }
+    }
+    if (__ballot(todo) != 0) {
+      if (tid % WAVE == 0) {
+        plan->failed = 1;
+      }
+      break;
     }
   }
 }

@@ -216,6 +216,28 @@ def test_values_whose_frequencies_fall_with_their_rank(lib, torch_cuda, dtype, n
     assert "collect_plan" in labels and ("collect_class" in labels) == tried, labels
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.uint64])
+@pytest.mark.parametrize("power, tried", [(1.5, False), (2.0, True)])
+def test_frequencies_that_fall_as_a_power_of_the_rank(lib, torch_cuda, dtype, power, tried):
+    """As word counts do.  Of the power of 1.5 there are 69 000 different ones and the estimate says under 3000: it is not tried, and where it is,
+    the table in memory fills up.  Of the power of 2 there are 5000, which it holds."""
+    x = np.minimum((1 - np.random.default_rng(5).random(1 << 23)) ** (-1 / (power - 1)), 2e9).astype(dtype)
+    mode, failed, found = _mode(lib, torch_cuda, x)
+    assert (mode, failed) == (1, 0 if tried else 1)
+    assert not tried or np.array_equal(np.sort(found), np.unique(x))
+    a = num.array(x)
+    num.unique(a)
+    lib.cpn_profile_enable(1)
+    try:
+        _lib.profile_collect()
+        got = np.asarray(num.unique(a))
+        labels = [label for label, _ in _lib.profile_collect()]
+    finally:
+        lib.cpn_profile_enable(0)
+    assert np.array_equal(got, np.unique(x))
+    assert "collect_plan" in labels and ("collect_few" in labels) == tried, labels
+
+
 @pytest.mark.parametrize("n", [3 << 20, (3 << 20) + 1])
 @pytest.mark.parametrize("count", [300, 1 << 40])
 def test_the_longest_integers_that_are_split(n, count):
